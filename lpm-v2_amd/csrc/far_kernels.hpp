@@ -1,0 +1,461 @@
+// far_kernels.hpp -- the FP32 Biot-Savart and Green sums with the well-separated
+// source tiles on the matrix units.
+//
+// The all-VALU pair (pair_kernels.hpp) is bound by VALU issue: 11-12 instructions,
+// 31-36 cycles per 64 pairs and SIMD on MI355X.  Only the reciprocal (or log) has
+// to run there.  For a block of targets and a tile of sources that are well
+// separated, with X and Y the positions relative to the centre of the target block,
+//   |x - y|^2 + e_x + e_y = (|X|^2 + e_x) + (|Y|^2 + e_y) - 2 X.Y
+// loses nothing to cancellation, so it is a matrix product over 4 values, and the
+// sum of s (x - y) is X (sum of s) - (sum of s Y), a matrix product as well:
+//  * denominator: one v_mfma_f32_16x16x32_bf16 per 16 sources x 16 targets.  Every
+//    FP32 value is split exactly into three bf16 values (8 significant bits each)
+//    and the K = 32 slots hold 8 of the 9 partial products of each coordinate
+//    (all but low x low, 2^-32 relative) and the two squared norms: an FP32
+//    product at 16.7 cycles, where v_mfma_f32_16x16x4_f32 takes 32.5;
+//  * rcp / log2 on the VALU, 8.2 cycles per 64 pairs, the floor of this form;
+//  * accumulation (Biot-Savart): v_mfma_f32_4x4x1_16b_f32 with the source weights
+//    (w Y, w) as its 4 rows, in FP32, 9.1 cycles per 64 pairs.  Its column layout
+//    is the row layout of the first product, so nothing is moved between them.
+//    Green sums have 1-2 outputs and accumulate with FMAs.
+// Inner loop: 21.6 cycles per 64 pairs (4 column tiles; 30.6 when rcp and MFMA are
+// interleaved by the scheduler, hence the scheduling barriers).
+// Tiles that are not well separated, or hold a value that is not finite, take the
+// VALU pair, self pairs included.  Records come in spatial order (lpm_order.hip).
+#pragma once
+
+#include "tiles.hpp"
+
+namespace lpm {
+
+typedef float f32x4 __attribute__((ext_vector_type(4)));
+typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
+typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+
+constexpr int FAR_TILE = 256;     // sources per tile, targets per block
+constexpr int FAR_COLS = 4;       // 16-target column tiles per wave
+constexpr int FAR_FOLD = 1024;    // sources per group, the unit of the source splits
+constexpr int FAR_PART = 512;     // sources per FP32 partial sum (128 terms a lane)
+
+// Well separated: every target-source distance is at least the radius of the target
+// block (|Y| >= 2 rho_t).  The norms and products above are then at most 9 times the
+// denominator for the closest pairs and about equal to it for nearly all; errors
+// against FP64 are the same with 3 rho_t, and fewer tiles go the VALU way.  The
+// margins keep a pair of equal points (a self pair) out for any rounding of centres
+// and radii; the lower bound keeps the split's low parts normal.
+__device__ __forceinline__ bool tiles_far(const float4& t, const float4& s) {
+  const float d2 = ball_d2(t, s);
+  const float th = 1.001f * s.w + 2.002f * t.w;
+  return d2 > th * th && d2 > 1e-28f;
+}
+
+// Exact split v = h + m + l into bf16 values, each in the high half of its word.
+__device__ __forceinline__ void split3(float v, unsigned& h, unsigned& m, unsigned& l) {
+  h = __float_as_uint(v) & 0xffff0000u;
+  const float r = v - __uint_as_float(h);
+  m = __float_as_uint(r) & 0xffff0000u;
+  l = __float_as_uint(r - __uint_as_float(m)) & 0xffff0000u;
+}
+// low half of the result: high half of a; high half: high half of b
+__device__ __forceinline__ unsigned pack_hi(unsigned a, unsigned b) { return (a >> 16) | b; }
+constexpr unsigned kOneHi = 0x3f800000u;  // bf16 1.0 in the high half
+
+// Source side (A operand) of one coordinate and of the norm; target side (B).
+// Slots of a coordinate: hh, hm, mh, mm, hl, lh, ml, lm (source part first).
+__device__ __forceinline__ u32x4 frag_src(float v) {
+  unsigned h, m, l;
+  split3(v, h, m, l);
+  return u32x4{pack_hi(h, h), pack_hi(m, m), pack_hi(h, l), pack_hi(m, l)};
+}
+__device__ __forceinline__ u32x4 frag_src_norm(float n2) {
+  unsigned h, m, l;
+  split3(n2, h, m, l);
+  // The bf16 MFMA truncates its sum to FP32: a mean error of -4.2e-8 of the
+  // denominator, the same for every pair, where the VALU pair rounds to nearest.
+  // 2^-24 of the source norm in one of the two free slots makes up for it: mean 1e-9
+  // to 2e-8 and rms 5.0e-8, against an rms of 5.7e-8 of the VALU pair.
+  const unsigned half_ulp = __float_as_uint(__uint_as_float(h) * 0x1p-24f) & 0xffff0000u;
+  return u32x4{pack_hi(h, m), pack_hi(l, kOneHi), pack_hi(kOneHi, kOneHi), half_ulp >> 16};
+}
+__device__ __forceinline__ u32x4 frag_tgt(float v, bool norm) {
+  unsigned h, m, l;
+  split3(v, h, m, l);
+  const u32x4 c{pack_hi(h, m), pack_hi(h, m), pack_hi(l, h), pack_hi(l, m)};
+  const u32x4 n{pack_hi(kOneHi, kOneHi), pack_hi(kOneHi, h), pack_hi(m, l), kOneHi >> 16};
+  return norm ? n : c;
+}
+
+// ----------------------------------------------------------- far policies
+// DIMS coordinates; E: record word 3 holds e; W0 (and W1): weight words; NW weight
+// sums accumulated by FMAs (0: Biot-Savart, by MFMA); trans: the VALU function.
+template <bool USE_E>
+struct FarSphereBS {
+  using Near = SphereBS<float, USE_E>;
+  static constexpr int DIMS = 3, W0 = 4, W1 = 4, NW = 0;
+  static constexpr bool E = USE_E;
+  __device__ __forceinline__ static float trans(float r2) { return fast_rcp(r2); }
+};
+struct FarPlaneBS {
+  using Near = PlaneBS<float>;
+  static constexpr int DIMS = 2, W0 = 2, W1 = 2, NW = 0;
+  static constexpr bool E = false;
+  __device__ __forceinline__ static float trans(float r2) { return fast_rcp(r2); }
+};
+template <bool USE_E>
+struct FarSphereGreen {
+  using Near = SphereGreen<float, USE_E>;
+  static constexpr int DIMS = 3, W0 = 4, W1 = 5, NW = 2;
+  static constexpr bool E = USE_E;
+  __device__ __forceinline__ static float trans(float r2) { return fast_log2(r2); }
+};
+struct FarPlaneGreen {
+  using Near = PlaneGreen<float>;
+  static constexpr int DIMS = 2, W0 = 2, W1 = 2, NW = 1;
+  static constexpr bool E = false;
+  __device__ __forceinline__ static float trans(float r2) { return fast_log2(r2); }
+};
+
+// LDS of one staged source tile: 16 steps of 16 sources, the MFMA A fragments
+// (64 x 16 bytes a step) and the weights (16 x 16 bytes a step).
+struct FarStage {
+  u32x4 frag[16 * 64];
+  f32x4 wgt[16 * 16];
+};
+
+// The direct VALU sum of one near tile for the wave's 64 targets (lane = target);
+// SELF: the tile may hold the targets' own particles.  The records of the next
+// NEAR_AHEAD sources load (scalar) under the arithmetic of these: with 64 targets
+// per source, one record ahead does not cover the latency of the load.
+constexpr int NEAR_AHEAD = 4;
+// Sources per FP32 partial sum.  Sources in spatial order push a partial sum in one
+// direction, so it rounds more than one over scattered sources: with 256 per partial
+// the 100^2 plane velocity was off by 1.05e-7 against 6.1e-8 in the caller's order.
+constexpr int NEAR_FOLD = 64;
+
+template <class N, bool SELF>
+__device__ __forceinline__ void near_source(const Vec4<float>& t, int tid, const float* sv, float p[N::NOUT]) {
+  W4<float> w;
+  N::arg(t, sv, w);
+  const float f = N::trans(w);
+  const bool mine = SELF && rec_index(sv, N::IDX) == tid;
+  if (SELF && __any(mine)) {
+    float tmp[N::NOUT];
+#pragma unroll
+    for (int k = 0; k < N::NOUT; ++k) tmp[k] = 0.f;
+    N::acc(sv, w, f, tmp);
+#pragma unroll
+    for (int k = 0; k < N::NOUT; ++k) p[k] += mine ? 0.f : tmp[k];
+  } else {
+    N::acc(sv, w, f, p);
+  }
+}
+
+template <class N, bool SELF>
+__device__ __forceinline__ void near_tile(const Vec4<float>& t, int tid, const float* __restrict__ src, int jt,
+                                          int jt_end, double S[N::NOUT]) {
+  constexpr int NO = N::NOUT, G = NEAR_AHEAD;
+  float p[NO];
+#pragma unroll
+  for (int k = 0; k < NO; ++k) p[k] = 0.f;
+  int j = jt;
+  if (jt + G <= jt_end) {
+    float sv[G][SREC];
+#pragma unroll
+    for (int g = 0; g < G; ++g)
+#pragma unroll
+      for (int q = 0; q < SREC; ++q) sv[g][q] = src[(size_t)(jt + g) * SREC + q];
+    for (; j + G <= jt_end; j += G) {
+      const int jn = j + 2 * G <= jt_end ? j + G : j;
+      float sn[G][SREC];
+#pragma unroll
+      for (int g = 0; g < G; ++g)
+#pragma unroll
+        for (int q = 0; q < SREC; ++q) sn[g][q] = src[(size_t)(jn + g) * SREC + q];
+#pragma unroll
+      for (int g = 0; g < G; ++g) near_source<N, SELF>(t, tid, sv[g], p);
+#pragma unroll
+      for (int g = 0; g < G; ++g)
+#pragma unroll
+        for (int q = 0; q < SREC; ++q) sv[g][q] = sn[g][q];
+      if (((j - jt) & (NEAR_FOLD - 1)) == NEAR_FOLD - G) {
+#pragma unroll
+        for (int k = 0; k < NO; ++k) {
+          S[k] += (double)p[k];
+          p[k] = 0.f;
+        }
+      }
+    }
+  }
+  for (; j < jt_end; ++j) {
+    float sv[SREC];
+#pragma unroll
+    for (int q = 0; q < SREC; ++q) sv[q] = src[(size_t)j * SREC + q];
+    near_source<N, SELF>(t, tid, sv, p);
+  }
+#pragma unroll
+  for (int k = 0; k < NO; ++k) S[k] += (double)p[k];
+}
+
+// One step: 16 staged sources against the wave's column tiles.
+template <class P>
+struct FarStep {
+  u32x4 a;
+  f32x4 w, w2;
+  __device__ __forceinline__ void read(const FarStage& st, int s, int lane, int wl, int grp) {
+    a = st.frag[s * 64 + lane];
+    w = st.wgt[s * 16 + wl];
+    if constexpr (P::NW == 2) w2 = st.wgt[s * 16 + grp * 4 + 1];
+  }
+  __device__ __forceinline__ void add(const u32x4 B[FAR_COLS], f32x4 D[FAR_COLS]) const {
+    f32x4 r[FAR_COLS];
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int c = 0; c < FAR_COLS; ++c)
+      r[c] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, a), __builtin_bit_cast(bf16x8, B[c]),
+                                                     f32x4{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
+#pragma unroll
+    for (int c = 0; c < FAR_COLS; ++c)
+#pragma unroll
+      for (int v = 0; v < 4; ++v) r[c][v] = P::trans(r[c][v]);
+    if constexpr (P::NW == 0) {
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int v = 0; v < 4; ++v)
+#pragma unroll
+        for (int c = 0; c < FAR_COLS; ++c) D[c] = __builtin_amdgcn_mfma_f32_4x4x1f32(w[v], r[c][v], D[c], 0, 0, 0);
+    } else {
+#pragma unroll
+      for (int c = 0; c < FAR_COLS; ++c)
+#pragma unroll
+        for (int v = 0; v < 4; ++v) {
+          D[c][0] = fmaf(r[c][v], w[v], D[c][0]);
+          if constexpr (P::NW == 2) D[c][1] = fmaf(r[c][v], w2[v], D[c][1]);
+        }
+    }
+  }
+};
+
+// One block's work: targets [t_block, t_block + 256) of the record array tg[0, nt)
+// (particle index order[local]), 64 to a wave, against the ns sources of src in
+// groups of FAR_FOLD: group first_group and every group_step-th after it, so that
+// the near tiles, which lie together in spatial order, spread over the splits.
+// smeta[k] is the ball of sources [k, k + 1) FAR_TILE.  FP64 results go to
+// out[k * out_stride + i].
+template <class P>
+__device__ __forceinline__ void far_block(const Vec4<float>* __restrict__ tg, int nt, int t_block,
+                                          const int* __restrict__ order, const float4 tm, const float* __restrict__ src,
+                                          const float4* __restrict__ smeta, int ns, int first_group,
+                                          int group_step, double* __restrict__ out, int out_stride, FarStage* stage) {
+  using N = typename P::Near;
+  constexpr int NO = N::NOUT;
+  constexpr int NACC = P::NW == 0 ? 4 : P::NW;
+  const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
+  const int grp = lane >> 4;
+  const int t_begin = t_block + wid * 64;
+  const int i = t_begin + lane;
+  const Vec4<float> t = tg[i < nt ? i : nt - 1];
+  const int tid = order[i < nt ? i : nt - 1];
+  double near_sum[NO];
+#pragma unroll
+  for (int k = 0; k < NO; ++k) near_sum[k] = 0.0;
+
+  // this split's tiles, in order
+  auto next_tile = [&](int jt) {
+    jt += FAR_TILE;
+    return jt % FAR_FOLD ? jt : jt + (group_step - 1) * FAR_FOLD;
+  };
+  const int j_begin = first_group * FAR_FOLD;
+
+  // near tiles first: no staging, no barriers
+  int n_far = 0;
+  for (int jt = j_begin; jt < ns; jt = next_tile(jt)) {
+    const float4 sm = smeta[jt / FAR_TILE];
+    if (tiles_far(tm, sm)) {
+      ++n_far;
+      continue;
+    }
+    if (t_begin >= nt) continue;
+    const int jt_end = min(ns, jt + FAR_TILE);
+    if (balls_touch(ball_d2(tm, sm), tm, sm))
+      near_tile<N, true>(t, tid, src, jt, jt_end, near_sum);
+    else
+      near_tile<N, false>(t, tid, src, jt, jt_end, near_sum);
+  }
+
+  double sum[FAR_COLS][NACC];
+#pragma unroll
+  for (int c = 0; c < FAR_COLS; ++c)
+#pragma unroll
+    for (int k = 0; k < NACC; ++k) sum[c][k] = 0.0;
+  const float X[3] = {t.a - tm.x, t.b - tm.y, P::DIMS == 3 ? t.c - tm.z : 0.f};
+
+  if (n_far > 0) {  // block-uniform
+    const float n2t = fmaf(X[0], X[0], fmaf(X[1], X[1], fmaf(X[2], X[2], P::E ? t.d : 0.f)));
+    u32x4 B[FAR_COLS];
+#pragma unroll
+    for (int c = 0; c < FAR_COLS; ++c) {
+      // lane (group g, column l % 16) holds coordinate g (or the norm) of target 16 c + l % 16
+      const int from = 16 * c + (lane & 15);
+      const float a0 = __shfl(X[0], from), a1 = __shfl(X[1], from), a2 = __shfl(X[2], from), a3 = __shfl(n2t, from);
+      const float v = grp == 0 ? a0 : grp == 1 ? a1 : grp == 2 ? a2 : a3;
+      B[c] = frag_tgt(v, grp == 3);
+    }
+    f32x4 D[FAR_COLS];
+#pragma unroll
+    for (int c = 0; c < FAR_COLS; ++c) D[c] = f32x4{0.f, 0.f, 0.f, 0.f};
+
+    auto next_far = [&](int jt) {
+      while (jt < ns && !tiles_far(tm, smeta[jt / FAR_TILE])) jt = next_tile(jt);
+      return jt;
+    };
+    float rec[SREC];
+    bool have;
+    auto load = [&](int jt) {
+      const int j = jt + (int)threadIdx.x;
+      have = j < ns;
+      const float4* r = reinterpret_cast<const float4*>(src + (size_t)(have ? j : ns - 1) * SREC);
+      const float4 lo = r[0], hi = r[1];
+      rec[0] = lo.x, rec[1] = lo.y, rec[2] = lo.z, rec[3] = lo.w;
+      rec[4] = hi.x, rec[5] = hi.y, rec[6] = hi.z, rec[7] = hi.w;
+    };
+    int jt = next_far(j_begin);
+    load(jt);
+    int buf = 0;
+    while (jt < ns) {
+      FarStage& st = stage[buf];
+      {
+        // this thread's source: row threadIdx % 16 of step threadIdx / 16; past the
+        // end a source of weight 0 at distance 1
+        float d[3] = {rec[0] - tm.x, rec[1] - tm.y, P::DIMS == 3 ? rec[2] - tm.z : 0.f};
+        float n2 = fmaf(d[0], d[0], fmaf(d[1], d[1], fmaf(d[2], d[2], P::E ? rec[3] : 0.f)));
+        float w0 = rec[P::W0], w1 = rec[P::W1];
+        if (!have) d[0] = d[1] = d[2] = w0 = w1 = 0.f, n2 = 1.f;
+        const int s = threadIdx.x >> 4, r = threadIdx.x & 15;
+        st.frag[s * 64 + r] = frag_src(-2.f * d[0]);
+        st.frag[s * 64 + 16 + r] = frag_src(-2.f * d[1]);
+        st.frag[s * 64 + 32 + r] = frag_src(-2.f * d[2]);
+        st.frag[s * 64 + 48 + r] = frag_src_norm(n2);
+        float* w = reinterpret_cast<float*>(st.wgt + s * 16 + (r >> 2) * 4) + (r & 3);
+        if constexpr (P::NW == 0) {
+          w[0] = w0 * d[0];
+          w[4] = w0 * d[1];
+          w[8] = w0 * d[2];
+          w[12] = w0;
+        } else {
+          w[0] = w0;
+          if constexpr (P::NW == 2) w[4] = w1;
+        }
+      }
+      const int jn = next_far(next_tile(jt));
+      if (jn < ns) load(jn);
+      // one barrier a tile: a wave writes a buffer again only after the barrier of
+      // the tile between, which every wave reaches after its reads of this one
+      __syncthreads();
+      // two register sets in turn: the next step's LDS reads run under this step
+      const int wl = grp * 4 + (P::NW == 0 ? lane & 3 : 0);
+      FarStep<P> s0, s1;
+      s0.read(st, 0, lane, wl, grp);
+#pragma unroll 1
+      for (int s = 0; s < 16; s += 2) {
+        s1.read(st, s + 1, lane, wl, grp);
+        s0.add(B, D);
+        s0.read(st, s < 14 ? s + 2 : 15, lane, wl, grp);
+        s1.add(B, D);
+      }
+      // fold at fixed places of the source array, so that the split leaves no trace
+      // beyond FP64 rounding
+      if (jn >= ns || jn / FAR_PART != jt / FAR_PART) {
+#pragma unroll
+        for (int c = 0; c < FAR_COLS; ++c)
+#pragma unroll
+          for (int k = 0; k < NACC; ++k) {
+            sum[c][k] += (double)D[c][k];
+            D[c][k] = 0.f;
+          }
+      }
+      buf ^= 1;
+      jt = jn;
+    }
+  }
+
+  // add the four row groups, then give lane l target t_begin + l its column tile
+  double far_sum[NACC];
+#pragma unroll
+  for (int k = 0; k < NACC; ++k) far_sum[k] = 0.0;
+  if (n_far > 0) {
+#pragma unroll
+    for (int c = 0; c < FAR_COLS; ++c)
+#pragma unroll
+      for (int k = 0; k < NACC; ++k) {
+        double v = sum[c][k];
+        v += __shfl_xor(v, 16);
+        v += __shfl_xor(v, 32);
+        if (grp == c) far_sum[k] = v;
+      }
+  }
+  if (i < nt) {
+    double o[NO];
+    if constexpr (P::NW == 0) {
+      double v[3];
+#pragma unroll
+      for (int k = 0; k < 3; ++k) v[k] = (double)X[k] * far_sum[3] - far_sum[k];
+      if constexpr (P::DIMS == 3) {
+#pragma unroll
+        for (int k = 0; k < 3; ++k) o[k] = v[k];
+      } else {  // PlaneBS accumulates (y, x) separations
+        o[0] = v[1];
+        o[1] = v[0];
+      }
+    } else {
+#pragma unroll
+      for (int k = 0; k < NO; ++k) o[k] = far_sum[k];
+    }
+#pragma unroll
+    for (int k = 0; k < NO; ++k) out[(size_t)k * out_stride + i] = near_sum[k] + o[k];
+  }
+}
+
+template <class P>
+static __global__ __launch_bounds__(256, 4) void far_sum_kernel(const void* __restrict__ tgt, const void* __restrict__ srcv,
+                                                         double* __restrict__ partial,
+                                                         const float4* __restrict__ tmeta,
+                                                         const float4* __restrict__ smeta,
+                                                         const int* __restrict__ order, PairArgs a) {
+  __shared__ FarStage stage[2];
+  const int nblk_t = (a.nt + FAR_TILE - 1) / FAR_TILE;
+  const int split = blockIdx.x / nblk_t;
+  const int tb = blockIdx.x - split * nblk_t;
+  far_block<P>(reinterpret_cast<const Vec4<float>*>(tgt), a.nt, tb * FAR_TILE, order, tmeta[tb],
+               reinterpret_cast<const float*>(srcv), smeta, a.ns, split, a.nsplit,
+               partial + (size_t)split * P::Near::NOUT * a.nt, a.nt, stage);
+}
+
+// Batched problems: a persistent launch whose blocks take (problem, target block,
+// split) items from a counter until the list is exhausted.
+template <class P>
+static __global__ __launch_bounds__(256, 4) void far_batch_kernel(
+    const void* __restrict__ tgt, const void* __restrict__ srcv, double* __restrict__ partial,
+    const float4* __restrict__ tballs, const float4* __restrict__ sballs, const int* __restrict__ order,
+    const BatchProblem* __restrict__ probs, const BatchItem* __restrict__ items, int n_items,
+    unsigned int* __restrict__ counter) {
+  __shared__ FarStage stage[2];
+  // the item number passes through a stage: one more word of LDS would leave room
+  // for 3 blocks per CU instead of 4
+  volatile int* next = reinterpret_cast<volatile int*>(stage);
+  for (;;) {
+    __syncthreads();  // every wave is done with the last item's stages
+    if (threadIdx.x == 0) *next = (int)atomicAdd(counter, 1u);
+    __syncthreads();
+    const int item = __builtin_amdgcn_readfirstlane(*next);
+    __syncthreads();
+    if (item >= n_items) break;
+    const BatchItem it = items[item];
+    const BatchProblem pr = probs[it.prob];
+    far_block<P>(reinterpret_cast<const Vec4<float>*>(tgt) + pr.t_off, pr.nt, it.wtile * FAR_TILE, order + pr.t_off,
+                 tballs[pr.tball_off + it.wtile], reinterpret_cast<const float*>(srcv) + (size_t)pr.s_off * SREC,
+                 sballs + pr.sball_off, pr.ns, it.split, pr.nsplit,
+                 partial + pr.part_off + (size_t)it.split * P::Near::NOUT * pr.nt, pr.nt, stage);
+  }
+}
+
+}  // namespace lpm

@@ -288,6 +288,7 @@ int lpm_destroy(lpm_ctx* ctx) {
   ctx->src.release();
   ctx->partial.release();
   ctx->red.release();
+  ctx->order.release();
   for (auto& ep : ctx->pending) {
     (void)hipEventDestroy(ep.a);
     (void)hipEventDestroy(ep.b);

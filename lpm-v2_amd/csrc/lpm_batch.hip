@@ -7,7 +7,10 @@
 // evaluation is: reset the work counter (a one-thread kernel, so the graph
 // holds no memset node), pack FP32/FP64 records for every particle and every
 // active source, one persistent pair_batch_kernel that drains a work list of
-// (problem, wave target tile, source split) items, and a batched finalize.
+// (problem, wave target tile, source split) items, and a batched finalize.  In FP32
+// the problems above kFarMinPairsSphere pairs go to a second persistent launch with
+// their well-separated tiles on the MFMA (far_kernels.hpp); their particles are put
+// in spatial order once per step.
 #include <math.h>
 
 #include <algorithm>
@@ -15,6 +18,7 @@
 #include <string>
 #include <vector>
 
+#include "far_kernels.hpp"
 #include "lpm_internal.hpp"
 #include "pair_kernels.hpp"
 
@@ -33,7 +37,7 @@ __device__ __forceinline__ void project(double& x, double& y, double& z, double 
 }
 
 __global__ void reset_counter(unsigned int* c) {
-  if (threadIdx.x == 0) c[0] = 0u;
+  if (threadIdx.x < 2) c[threadIdx.x] = 0u;
 }
 
 struct StageArgs {
@@ -105,13 +109,15 @@ struct BatchFinArgs {
   const double* partial;
   const double *x, *y, *z;
   double *u, *v, *w;
+  const int* order;  // particle of every target record (null: the record's own index)
 };
 
 __global__ __launch_bounds__(256) void batch_finalize(BatchFinArgs f) {
-  int p = blockIdx.x * blockDim.x + threadIdx.x;
-  if (p >= f.n) return;
+  const int rec = blockIdx.x * blockDim.x + threadIdx.x;
+  if (rec >= f.n) return;
+  const int p = f.order ? f.order[rec] : rec;
   const lpm::BatchProblem pr = f.probs[f.pinst[p]];
-  const int i = p - pr.t_off;
+  const int i = rec - pr.t_off;
   double A0 = 0.0, A1 = 0.0, A2 = 0.0;
   for (int s = 0; s < pr.nsplit; ++s) {
     const double* ps = f.partial + pr.part_off + (size_t)s * 3 * pr.nt;
@@ -145,18 +151,35 @@ BatchFn pick_batch(int prec, bool on_sphere, int r) {
   return on_sphere ? pick_batch_r<double, false>(r) : pick_batch_r<double, true>(r);
 }
 
+// Source groups per far item: 8 groups (8,192 sources) measured best from 49,154 to
+// 1,966,082 targets, within 3 % from 2 to 16.
+constexpr int kBatchFarGroups = 8;
+
+using FarBatchFn = void (*)(const void*, const void*, double*, const float4*, const float4*, const int*,
+                            const lpm::BatchProblem*, const lpm::BatchItem*, int, unsigned int*);
+
+FarBatchFn pick_far(bool on_sphere) {
+  return on_sphere ? lpm::far_batch_kernel<lpm::FarSphereBS<false>> : lpm::far_batch_kernel<lpm::FarSphereBS<true>>;
+}
+
 }  // namespace
 
 struct lpm_bve_batch {
   lpm_ctx* ctx = nullptr;
   int n_inst = 0, n = 0, ns = 0, precision = 0, flags = 0;
-  int r = 4, kt = 256, chunk = 16384;
+  int r = 2, kt = 256, chunk = 16384;
+  bool auto_chunk = true;  // until a shape is given or tuned
   std::vector<int64_t> off;
   std::vector<int> src_host;  // global active indices
   DevBuf x, y, z, q, u, v, w, area, prad, pomg, pinst, list;
   DevBuf k[4][4];  // [stage][x, y, z, q]
   DevBuf xi, yi, zi, qi;
   DevBuf tgt, src, partial, probs, items, counter;
+  // far path: its items and balls, the problems it holds, and the order of a step
+  bool far_on = true;
+  int n_far_items = 0, n_far = 0, n_tballs = 0, n_sballs = 0, far_grid = 0, far_max_n = 0;
+  DevBuf far_items, ball_desc, balls, far_flags, order;
+  const int *tgt_order = nullptr, *src_order = nullptr;
   int n_items = 0;
   int grid = 0;
   hipGraphExec_t exec[4] = {nullptr, nullptr, nullptr, nullptr};
@@ -176,19 +199,44 @@ void drop_graphs(lpm_bve_batch* b) {
   }
 }
 
+// Sources per item of the all-pairs kernel: the longest chunk that still gives
+// kItemRounds items per resident wave.  Items that take most of a launch leave the
+// chip idle behind the last of them: 15 problems of levels 3-5 took 3.86 ms at 16,384
+// sources and 4 targets per lane.
+constexpr int kItemRounds = 6;
+int default_chunk(const lpm_bve_batch* b, long long waves, const std::vector<long long>& pairs) {
+  int chunk = 16384;
+  for (; chunk > 2 * b->kt; chunk /= 2) {
+    long long items = 0;
+    for (long long p : pairs) items += p / (64LL * b->r * chunk);
+    if (items >= kItemRounds * waves) break;
+  }
+  return chunk;
+}
+
 // (Re)build the problem table and work list for the current tile shape.
 int plan(lpm_bve_batch* b) {
   lpm_ctx* ctx = b->ctx;
   const int per_wave = 64 * b->r;
+  const bool on_sphere = (b->flags & LPM_SOLVER_PROJECT_STAGES) != 0;
+  BatchFn fn = pick_batch(b->precision, on_sphere, b->r);
+  b->grid = lpm::blocks_per_cu((const void*)fn) * ctx->num_cus;
+  b->far_grid = lpm::blocks_per_cu((const void*)pick_far(on_sphere)) * ctx->num_cus;
   const size_t wsz = b->precision == LPM_PREC_FP32_KAHAN ? 4 : 8;
   std::vector<lpm::BatchProblem> probs((size_t)b->n_inst);
   struct It {
     lpm::BatchItem it;
     int cost;
   };
-  std::vector<It> items;
+  std::vector<It> items, far_items;
+  std::vector<int2> tdesc, sdesc;
+  std::vector<int> far_flags((size_t)b->n_inst);
+  // (the sort key has room for 2^21 problems beside the coarsest curve)
+  const bool can_far = b->far_on && b->precision == LPM_PREC_FP32_KAHAN && b->n_inst <= (1 << 21);
+  b->n_far = b->far_max_n = 0;
   long long part = 0;
   int s_off = 0;
+  std::vector<long long> direct_pairs;
   for (int k = 0; k < b->n_inst; ++k) {
     lpm::BatchProblem& p = probs[(size_t)k];
     p.t_off = (int)b->off[(size_t)k];
@@ -198,10 +246,35 @@ int plan(lpm_bve_batch* b) {
     p.s_off = s_off;
     p.ns = nsrc;
     s_off += nsrc;
+    p.far = can_far && (double)p.nt * p.ns >= lpm::kFarMinPairsSphere ? 1 : 0;
+    if (!p.far) direct_pairs.push_back((long long)p.nt * p.ns);
+  }
+  if (b->auto_chunk) b->chunk = default_chunk(b, 4LL * b->grid, direct_pairs);
+  for (int k = 0; k < b->n_inst; ++k) {
+    lpm::BatchProblem& p = probs[(size_t)k];
+    const int nsrc = p.ns;
     int chunk = std::max(b->kt, (b->chunk + b->kt - 1) / b->kt * b->kt);
     p.nsplit = nsrc > 0 ? (nsrc + chunk - 1) / chunk : 0;
     p.chunk = chunk;
     p.part_off = part;
+    p.tball_off = (int)tdesc.size();
+    p.sball_off = (int)sdesc.size();
+    far_flags[(size_t)k] = p.far;
+    if (p.far) {
+      ++b->n_far;
+      b->far_max_n = std::max(b->far_max_n, p.nt);
+      const int groups = (p.ns + lpm::FAR_FOLD - 1) / lpm::FAR_FOLD;
+      p.nsplit = (groups + kBatchFarGroups - 1) / kBatchFarGroups;
+      part += (long long)p.nsplit * 3 * p.nt;
+      for (int t = 0; t < p.nt; t += lpm::FAR_TILE)
+        tdesc.push_back(make_int2(p.t_off + t, std::min(lpm::FAR_TILE, p.nt - t)));
+      for (int j = 0; j < p.ns; j += lpm::FAR_TILE)
+        sdesc.push_back(make_int2(p.s_off + j, std::min(lpm::FAR_TILE, p.ns - j)));
+      for (int s = 0; s < p.nsplit; ++s)
+        for (int t = 0; t * lpm::FAR_TILE < p.nt; ++t)
+          far_items.push_back({{k, t, s, 0}, (groups - s + p.nsplit - 1) / p.nsplit});
+      continue;
+    }
     part += (long long)std::max(p.nsplit, 1) * 3 * p.nt;
     const int nw = (p.nt + per_wave - 1) / per_wave;
     // split-major: the waves that take consecutive items read the same source
@@ -217,6 +290,27 @@ int plan(lpm_bve_batch* b) {
   std::vector<lpm::BatchItem> flat(items.size());
   for (size_t i = 0; i < items.size(); ++i) flat[i] = items[i].it;
   b->n_items = (int)flat.size();
+  std::stable_sort(far_items.begin(), far_items.end(), [](const It& a, const It& c) { return a.cost > c.cost; });
+  std::vector<lpm::BatchItem> far_flat(far_items.size());
+  for (size_t i = 0; i < far_items.size(); ++i) far_flat[i] = far_items[i].it;
+  b->n_far_items = (int)far_flat.size();
+  b->n_tballs = (int)tdesc.size();
+  b->n_sballs = (int)sdesc.size();
+  std::vector<int2> desc(tdesc);
+  desc.insert(desc.end(), sdesc.begin(), sdesc.end());
+  if (b->n_far) {
+    LPM_HIP(ctx, b->far_items.ensure(far_flat.size() * sizeof(lpm::BatchItem)));
+    LPM_HIP(ctx, b->ball_desc.ensure(desc.size() * sizeof(int2)));
+    LPM_HIP(ctx, b->balls.ensure(desc.size() * sizeof(float4)));
+    LPM_HIP(ctx, b->far_flags.ensure(far_flags.size() * sizeof(int)));
+    LPM_HIP(ctx, b->order.ensure(lpm::order_bytes(b->n, b->ns)));
+    LPM_HIP(ctx, hipMemcpyAsync(b->far_items.p, far_flat.data(), far_flat.size() * sizeof(lpm::BatchItem),
+                                hipMemcpyHostToDevice, ctx->stream));
+    LPM_HIP(ctx, hipMemcpyAsync(b->ball_desc.p, desc.data(), desc.size() * sizeof(int2), hipMemcpyHostToDevice,
+                                ctx->stream));
+    LPM_HIP(ctx, hipMemcpyAsync(b->far_flags.p, far_flags.data(), far_flags.size() * sizeof(int),
+                                hipMemcpyHostToDevice, ctx->stream));
+  }
   LPM_HIP(ctx, b->probs.ensure(probs.size() * sizeof(lpm::BatchProblem)));
   LPM_HIP(ctx, b->items.ensure(std::max<size_t>(flat.size(), 1) * sizeof(lpm::BatchItem)));
   LPM_HIP(ctx, b->partial.ensure((size_t)std::max<long long>(part, 1) * sizeof(double)));
@@ -229,10 +323,24 @@ int plan(lpm_bve_batch* b) {
     LPM_HIP(ctx, hipMemcpyAsync(b->items.p, flat.data(), flat.size() * sizeof(lpm::BatchItem),
                                 hipMemcpyHostToDevice, ctx->stream));
   LPM_HIP(ctx, hipStreamSynchronize(ctx->stream));
-  const bool on_sphere = (b->flags & LPM_SOLVER_PROJECT_STAGES) != 0;
-  BatchFn fn = pick_batch(b->precision, on_sphere, b->r);
-  b->grid = lpm::blocks_per_cu((const void*)fn) * ctx->num_cus;
+  b->tgt_order = b->src_order = nullptr;
   drop_graphs(b);
+  return LPM_OK;
+}
+
+// Spatial order of the far problems at (x, y, z): valid for the sums until the next
+// call (any order gives the same sums, so a step's stages share one).
+int order_problems(lpm_bve_batch* b, const double* x, const double* y, const double* z) {
+  if (!b->n_far) return LPM_OK;
+  lpm::OrderInput in{x, y, z, 0, b->n, x, y, z, b->list.as<int>(), b->ns, true};
+  in.prob = b->pinst.as<int>();
+  in.sorted = b->far_flags.as<int>();
+  in.n_prob = b->n_inst;
+  in.max_n = b->far_max_n;
+  int *t = nullptr, *s = nullptr;
+  if (int rc = lpm::spatial_order(b->ctx, in, b->order, &t, &s)) return rc;
+  b->tgt_order = t;
+  b->src_order = s;
   return LPM_OK;
 }
 
@@ -241,8 +349,11 @@ int eval_velocity(lpm_bve_batch* b, const double* x, const double* y, const doub
                   double* u, double* v, double* w) {
   lpm_ctx* ctx = b->ctx;
   hipLaunchKernelGGL(reset_counter, dim3(1), dim3(64), 0, ctx->stream, b->counter.as<unsigned int>());
-  lpm::PackArgs pa{x, y, z, q, nullptr, b->area.as<double>(), b->prad.as<double>(), b->list.as<int>(),
-                   0, 0, 1.0, 1.0};
+  if (b->n_far && !b->tgt_order)  // outside a step
+    if (int rc = order_problems(b, x, y, z)) return rc;
+  lpm::PackArgs pa{x, y, z, q, nullptr, b->area.as<double>(), b->prad.as<double>(),
+                   b->n_far ? b->src_order : b->list.as<int>(), 0, 0, 1.0, 1.0};
+  pa.tgt_order = b->n_far ? b->tgt_order : nullptr;
   lpm::launch_pack(LPM_K_SPHERE_BS, b->precision, pa, b->src.p, b->tgt.p, b->ns, b->n, ctx->stream);
   const bool on_sphere = (b->flags & LPM_SOLVER_PROJECT_STAGES) != 0;
   lpm::BatchArgs ba;
@@ -260,6 +371,28 @@ int eval_velocity(lpm_bve_batch* b, const double* x, const double* y, const doub
     e1 = lpm::take_event(ctx);
     if (e0 && e1) LPM_HIP(ctx, hipEventRecord(e0, ctx->stream));
   }
+  if (b->n_far_items > 0) {
+    lpm::BallSet<float> t, sr;
+    t.rec = b->tgt.as<float>();
+    t.words = lpm::TREC;
+    t.finite_mask = 0xfu;
+    t.out = b->balls.as<float4>();
+    t.desc = b->ball_desc.as<int2>();
+    t.balls = b->n_tballs;
+    sr.rec = b->src.as<float>();
+    sr.words = lpm::SREC;
+    sr.finite_mask = 0x1fu;
+    sr.out = t.out + b->n_tballs;
+    sr.desc = t.desc + b->n_tballs;
+    sr.balls = b->n_sballs;
+    t.dims = sr.dims = 3;
+    hipLaunchKernelGGL(lpm::tile_balls<float>, dim3((b->n_tballs + b->n_sballs + 3) / 4), dim3(256), 0, ctx->stream,
+                       t, sr);
+    hipLaunchKernelGGL(pick_far(on_sphere), dim3((unsigned)std::min(b->far_grid, b->n_far_items)), dim3(256), 0,
+                       ctx->stream, b->tgt.p, b->src.p, b->partial.as<double>(), t.out, sr.out, b->tgt_order,
+                       b->probs.as<lpm::BatchProblem>(), b->far_items.as<lpm::BatchItem>(), b->n_far_items,
+                       b->counter.as<unsigned int>() + 1);
+  }
   if (b->n_items > 0)
     hipLaunchKernelGGL(pick_batch(b->precision, on_sphere, b->r), dim3((unsigned)b->grid), dim3(256), 0,
                        ctx->stream, ba.tgt, ba.src, ba.partial, ba.probs, ba.items, ba.n_items, ba.kt, ba.counter);
@@ -268,7 +401,7 @@ int eval_velocity(lpm_bve_batch* b, const double* x, const double* y, const doub
     ctx->pending.push_back({e0, e1, LPM_K_SPHERE_BS});
   }
   BatchFinArgs f{b->n, b->pinst.as<int>(), b->probs.as<lpm::BatchProblem>(), b->partial.as<double>(), x, y, z,
-                 u, v, w};
+                 u, v, w, b->n_far ? b->tgt_order : nullptr};
   hipLaunchKernelGGL(batch_finalize, dim3((b->n + 255) / 256), dim3(256), 0, ctx->stream, f);
   LPM_HIP(ctx, hipGetLastError());
   return LPM_OK;
@@ -299,6 +432,7 @@ int enqueue_stage(lpm_bve_batch* b, int g, double dt) {
   a.zi = b->zi.as<double>();
   a.qi = b->qi.as<double>();
   if (g == 0) {  // stage 1 algebra from the stored velocity
+    if (int rc = order_problems(b, a.x, a.y, a.z)) return rc;
     a.first = 1;
     a.make_input = 1;
     a.h = 0.5;
@@ -526,6 +660,7 @@ int lpm_bve_batch_set_tuning(lpm_bve_batch* b, int targets_per_lane, int tile_so
     return fail(ctx, LPM_ERR_ARG, "lpm_bve_batch_set_tuning: tile_sources must be a multiple of 8 in [8, 65536]");
   if (chunk_sources < tile_sources) return fail(ctx, LPM_ERR_ARG, "lpm_bve_batch_set_tuning: chunk < tile");
   LPM_HIP(ctx, hipStreamSynchronize(ctx->stream));
+  b->far_on = b->auto_chunk = false;  // the caller's shape is one of the all-pairs kernel
   b->r = targets_per_lane;
   b->kt = tile_sources;
   b->chunk = chunk_sources;
@@ -538,7 +673,7 @@ int lpm_bve_batch_get_tuning(lpm_bve_batch* b, int* targets_per_lane, int* tile_
   *targets_per_lane = b->r;
   *tile_sources = b->kt;
   *chunk_sources = b->chunk;
-  *n_items = b->n_items;
+  *n_items = b->n_items + b->n_far_items;
   return LPM_OK;
 }
 
@@ -559,17 +694,23 @@ int lpm_bve_batch_autotune(lpm_bve_batch* b, int* targets_per_lane, int* tile_so
   static const int rs[3] = {2, 4, 8};
   static const int kts[2] = {128, 256};
   static const int chunks[3] = {4096, 16384, 65536};
+  bool best_far = b->far_on;
   int best_r = b->r, best_kt = b->kt, best_chunk = b->chunk;
   float best = 1e30f;
+  b->auto_chunk = false;
   hipEvent_t e0, e1;
   LPM_HIP(ctx, hipEventCreate(&e0));
   LPM_HIP(ctx, hipEventCreate(&e1));
   const bool was_timing = ctx->timing;
   ctx->timing = false;
   int rc = LPM_OK;
-  for (int r : rs)
+  for (int far = 1; far >= 0 && rc == LPM_OK; --far)
+   for (int r : rs)
     for (int kt : kts)
       for (int ch : chunks) {
+        // with the far path on, the shape is that of the small problems
+        if (far && (b->precision == LPM_PREC_FP64 || r == 8 || kt != 256 || ch == 65536)) continue;
+        b->far_on = far != 0;
         if (b->precision == LPM_PREC_FP64 && r == 8) continue;
         b->r = r;
         b->kt = kt;
@@ -589,12 +730,14 @@ int lpm_bve_batch_autotune(lpm_bve_batch* b, int* targets_per_lane, int* tile_so
             best_r = r;
             best_kt = kt;
             best_chunk = ch;
+            best_far = b->far_on;
           }
         }
       }
   ctx->timing = was_timing;
   (void)hipEventDestroy(e0);
   (void)hipEventDestroy(e1);
+  b->far_on = best_far;
   if (rc) return rc;
   b->r = best_r;
   b->kt = best_kt;
@@ -614,7 +757,8 @@ int lpm_bve_batch_delete(lpm_bve_batch* b) {
   drop_graphs(b);
   DevBuf* all[] = {&b->x, &b->y, &b->z, &b->q, &b->u, &b->v, &b->w, &b->area, &b->prad, &b->pomg,
                    &b->pinst, &b->list, &b->xi, &b->yi, &b->zi, &b->qi, &b->tgt, &b->src, &b->partial,
-                   &b->probs, &b->items, &b->counter};
+                   &b->probs, &b->items, &b->counter, &b->far_items, &b->ball_desc, &b->balls, &b->far_flags,
+                   &b->order};
   for (DevBuf* d : all) d->release();
   for (auto& row : b->k)
     for (auto& d : row) d.release();

@@ -75,6 +75,7 @@ struct lpm_ctx {
   lpm::DevBuf list;
   lpm::DevBuf tgt, src, partial;
   lpm::DevBuf red;  // reductions
+  lpm::DevBuf order;  // spatial order of the tile paths
   // this device's copy of the static scratch array (lpm_api.hip), resolved
   // once at lpm_create; used by the allocation-free entry point only
   void* scratch = nullptr;
@@ -142,6 +143,11 @@ struct PairProblem {
   DevBuf* src_buf = nullptr;
   DevBuf* partial_buf = nullptr;
   DevBuf* red_buf = nullptr;  // FP32 sphere Green: the two FP64 source totals
+  DevBuf* order_buf = nullptr;
+  // Spatial order of targets and sources when the caller has it (a solver keeps
+  // one for the four sums of a step); else run_pair_sum makes one where it is used.
+  const int* tgt_order = nullptr;
+  const int* src_order = nullptr;
   // Source count on the device (set by a device-side compaction): ns is then
   // an upper bound that sizes the launches, and the kernels read the count.
   // Such a sum also records no timing events.
@@ -168,6 +174,7 @@ struct PackArgs {
   int m = 1;        // derivative fields
   double aux = 0.0; // SWE: log2(e)/eps^2 (FP32) or 1/eps^2 (FP64)
   const int* count_dev = nullptr;  // sources: record count on the device (count is then a bound)
+  const int* tgt_order = nullptr;  // targets: particle of every record (null: i0 + record)
 };
 
 // Ordered sum over source splits and the FP64 epilogue of one kind.
@@ -183,6 +190,7 @@ struct FinArgs {
   const double* q2 = nullptr;
   double* out3 = nullptr;
   int op = 0;
+  const int* tgt_order = nullptr;  // particle of every target record (null: i0 + record)
 };
 
 // The PSE derivative, interpolation and SWE kinds (lpm_pse_ops.hip).
@@ -196,6 +204,33 @@ int ops_launch_finalize(int kind, int m, const FinArgs& f, hipStream_t st);
 void launch_pack(int kind, int precision, const PackArgs& a, void* srec, void* trec, int ns, int nt,
                  hipStream_t st);
 Tuning default_tuning(int kind, int prec);
+// Where the far path starts, in pairs (see sum_path).
+constexpr double kFarMinPairsSphere = 2e9, kFarMinPairsPlane = 4e9;
+
+// How a sum is scheduled: over all pairs (pair_kernels.hpp) or with the
+// well-separated tiles on the MFMA (far_kernels.hpp), which wants the records in
+// spatial order.
+enum SumPath { kAllPairs = 0, kFarTiles = 1 };
+SumPath sum_path(const lpm_ctx* ctx, int kind, int prec, int nt, int ns);
+
+// Spatial order (lpm_order.hip) of targets tx.. [i0, i0 + nt) and of the sources
+// x..[list[0, ns)]: device arrays of particle indices inside `buf`.
+struct OrderInput {
+  const double *tx, *ty, *tz;
+  int i0, nt;
+  const double *x, *y, *z;
+  const int* list;
+  int ns;
+  bool sphere;
+  // batched sphere problems, ordered problem by problem: the problem of every
+  // particle, whether a problem is sorted at all, and the largest problem's size
+  const int* prob = nullptr;
+  const int* sorted = nullptr;
+  int n_prob = 0, max_n = 0;
+};
+size_t order_bytes(int nt, int ns);  // spatial_order allocates nothing in a buffer of this size
+int spatial_order(lpm_ctx* ctx, const OrderInput& in, DevBuf& buf, int** tgt_order, int** src_order);
+
 int blocks_per_cu(const void* kernel);
 hipEvent_t take_event(lpm_ctx* ctx);
 

@@ -11,6 +11,7 @@
 #include <algorithm>
 #include <mutex>
 
+#include "far_kernels.hpp"
 #include "lpm_internal.hpp"
 #include "pair_kernels.hpp"
 
@@ -105,7 +106,7 @@ template <typename T, int KIND>
 __global__ __launch_bounds__(256) void pack_targets(PackArgs a, Vec4<T>* __restrict__ rec) {
   int i = blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= a.count) return;
-  const int p = a.i0 + i;
+  const int p = a.tgt_order ? a.tgt_order[i] : a.i0 + i;
   const double x = a.x[p], y = a.y[p];
   Vec4<T> t{(T)0, (T)0, (T)0, (T)0};
   if constexpr (KIND == LPM_K_SPHERE_BS || KIND == LPM_K_SPHERE_GREEN) {
@@ -182,7 +183,7 @@ __global__ __launch_bounds__(256) void finalize_kernel(FinArgs f) {
 #pragma unroll
     for (int k = 0; k < NO; ++k) A[k] += ps[(size_t)k * f.nt + i];
   }
-  const int p = f.i0 + i;
+  const int p = f.tgt_order ? f.tgt_order[i] : f.i0 + i;
   if constexpr (KIND == LPM_K_SPHERE_BS) {
     const double x = f.x[p], y = f.y[p], z = f.z[p];
     f.out0[p] = A[1] * z - A[2] * y;
@@ -246,6 +247,9 @@ Tuning default_tuning(int kind, int prec) {
   }
   return t;
 }
+
+constexpr int kFarRounds = 8;   // rounds of resident blocks wanted of a far-tile sum
+constexpr int kFarGroups = 8;   // at most so many groups of FAR_FOLD sources per split
 
 using KernelFn = void (*)(PairArgs);
 
@@ -413,6 +417,85 @@ static int choose_splits(int n_wtiles, int ns, int kt, int slots, int max_split_
   return std::max(1, std::min(max_split, std::max(fill, std::max(by_chunk, rounds_split))));
 }
 
+// ------------------------------------------ sums with far tiles on the MFMA
+using FarFn = void (*)(const void*, const void*, double*, const float4*, const float4*, const int*, PairArgs);
+
+static FarFn pick_far(int kind, bool on_sphere) {
+  switch (kind) {
+    case LPM_K_SPHERE_BS: return on_sphere ? far_sum_kernel<FarSphereBS<false>> : far_sum_kernel<FarSphereBS<true>>;
+    case LPM_K_PLANE_BS: return far_sum_kernel<FarPlaneBS>;
+    case LPM_K_SPHERE_GREEN:
+      return on_sphere ? far_sum_kernel<FarSphereGreen<false>> : far_sum_kernel<FarSphereGreen<true>>;
+    case LPM_K_PLANE_GREEN: return far_sum_kernel<FarPlaneGreen>;
+    default: return nullptr;
+  }
+}
+
+// Where the far path starts, by whole calls (ordering and balls cost 45 us there):
+// sphere velocity 0.95 of the all-pairs rate at 1.2e9 pairs, 1.01 at 2.5e9, 1.23 at
+// 1e10; plane velocity 0.92 at 1.6e9, 1.07 at 4.3e9.
+SumPath sum_path(const lpm_ctx* ctx, int kind, int prec, int nt, int ns) {
+  const Tuning& ov = ctx->tune[kind][prec == LPM_PREC_FP32_KAHAN ? 1 : 0];
+  if (ov.r || ov.kt) return kAllPairs;  // a forced tile shape is one of the all-pairs kernel
+  if ((long long)nt + ns > (1 << 30)) return kAllPairs;  // item counts of the sort are ints
+  const bool vortex = kind == LPM_K_SPHERE_BS || kind == LPM_K_PLANE_BS || kind == LPM_K_SPHERE_GREEN ||
+                      kind == LPM_K_PLANE_GREEN;
+  if (vortex) {
+    const bool plane = kind == LPM_K_PLANE_BS || kind == LPM_K_PLANE_GREEN;
+    const double least = plane ? kFarMinPairsPlane : kFarMinPairsSphere;
+    return prec == LPM_PREC_FP32_KAHAN && (double)nt * ns >= least ? kFarTiles : kAllPairs;
+  }
+  return kAllPairs;
+}
+
+// Words of a source / target record that must be finite for a tile to be treated
+// by its ball: everything but the index word and the constants behind it.
+static unsigned finite_words(int kind, int m, bool tgt) {
+  int words;
+  switch (kind) {
+    case LPM_K_SPHERE_BS: words = tgt ? 4 : 5; break;
+    case LPM_K_SPHERE_GREEN: words = tgt ? 4 : 6; break;
+    case LPM_K_PLANE_BS:
+    case LPM_K_PLANE_GREEN: words = tgt ? 2 : 3; break;
+    case LPM_K_PSE8:
+    case LPM_K_PSE2: words = tgt ? 3 : 4; break;
+    case LPM_K_PSE_SPHERE8: words = tgt ? 4 : 5; break;
+    case LPM_K_PSE_DERIV_PLANE: words = tgt ? 2 : 3 + m; break;
+    case LPM_K_PSE_DERIV_SPHERE: words = tgt ? 3 : 4 + m; break;
+    case LPM_K_PSE_INTERP_PLANE: words = tgt ? 2 : 3; break;
+    case LPM_K_PSE_INTERP_SPHERE: words = tgt ? 3 : 4; break;
+    default: words = tgt ? 3 : 6; break;  // SWE
+  }
+  return (1u << words) - 1u;
+}
+
+static bool sphere_kind(int kind) {
+  return kind == LPM_K_SPHERE_BS || kind == LPM_K_SPHERE_GREEN || kind == LPM_K_PSE_SPHERE8 ||
+         kind == LPM_K_PSE_DERIV_SPHERE || kind == LPM_K_PSE_INTERP_SPHERE;
+}
+
+template <typename T>
+static void launch_balls(int kind, int m, int nw, const void* trec, const void* srec, float4* tballs, float4* sballs,
+                         int nt, int ns, int t_tile, int s_tile, hipStream_t st) {
+  BallSet<T> t, s;
+  t.rec = static_cast<const T*>(trec);
+  t.out = tballs;
+  t.words = TREC;
+  t.n = nt;
+  t.tile = t_tile;
+  t.dims = s.dims = sphere_kind(kind) ? 3 : 2;
+  t.finite_mask = finite_words(kind, m, true);
+  t.balls = (nt + t_tile - 1) / t_tile;
+  s.rec = static_cast<const T*>(srec);
+  s.out = sballs;
+  s.words = nw;
+  s.n = ns;
+  s.tile = s_tile;
+  s.finite_mask = finite_words(kind, m, false);
+  s.balls = (ns + s_tile - 1) / s_tile;
+  hipLaunchKernelGGL(tile_balls<T>, dim3((unsigned)(t.balls + s.balls + 3) / 4), dim3(256), 0, st, t, s);
+}
+
 hipEvent_t take_event(lpm_ctx* ctx) {
   if (!ctx->event_pool.empty()) {
     hipEvent_t e = ctx->event_pool.back();
@@ -455,7 +538,8 @@ int run_pair_sum(lpm_ctx* ctx, const PairProblem& pp) {
   if (ov.kt) tu.kt = ov.kt;
   tu.splits = ov.splits;
 
-  const size_t wsz = prec == LPM_PREC_FP32_KAHAN ? 4 : 8;
+  const bool fp32 = prec == LPM_PREC_FP32_KAHAN;
+  const size_t wsz = fp32 ? 4 : 8;
   const bool ops = is_ops_kind(kind);
   const int no = ops ? ops_nout(kind, pp.m) : nout_of(kind);
   const int nw = ops ? ops_record_words(kind, pp.m) : SREC;
@@ -475,7 +559,11 @@ int run_pair_sum(lpm_ctx* ctx, const PairProblem& pp) {
   DevBuf& sb = pp.src_buf ? *pp.src_buf : ctx->src;
   DevBuf& pb = pp.partial_buf ? *pp.partial_buf : ctx->partial;
 
-  const int per_wave = 64 * tu.r;
+  // a device-side source count cannot be ordered
+  const SumPath path = pp.ns_dev ? kAllPairs : sum_path(ctx, kind, prec, nt, ns);
+  const bool far = path == kFarTiles;
+  const int t_tile = FAR_TILE, s_tile = FAR_TILE;
+  const int per_wave = path != kAllPairs ? 64 : 64 * tu.r;
   const int n_wtiles = (nt + per_wave - 1) / per_wave;
   // sphere PSE kinds: the series form of the distance when 7 eps <= 0.56 R
   // (FP32, 7 terms) or 7 eps <= 0.35 R (FP64, 10 terms)
@@ -483,13 +571,24 @@ int run_pair_sum(lpm_ctx* ctx, const PairProblem& pp) {
                           kind == LPM_K_PSE_INTERP_SPHERE;
   const double series_reach = prec == LPM_PREC_FP32_KAHAN ? 0.56 : 0.35;
   const bool variant = sphere_pse ? (7.0 * pp.eps <= series_reach * pp.radius) : pp.on_sphere;
-  KernelFn fn = ops ? reinterpret_cast<KernelFn>(const_cast<void*>(ops_pick_kernel(kind, prec, tu.r, pp.m, variant)))
+  FarFn far_fn = far ? pick_far(kind, pp.on_sphere) : nullptr;
+  KernelFn fn = far ? reinterpret_cast<KernelFn>(far_fn) : ops ? reinterpret_cast<KernelFn>(const_cast<void*>(ops_pick_kernel(kind, prec, tu.r, pp.m, variant)))
                     : pick_kernel(kind, prec, tu.r, variant);
   if (!fn) return fail(ctx, LPM_ERR_ARG, "no pair kernel for this kind, precision and field count");
   if (pp.ns_dev && (ops || kind == LPM_K_SPHERE_GREEN))
     return fail(ctx, LPM_ERR_UNSUPPORTED, "a device-side source count is not supported for this kind");
   int nsplit = 1, chunk = std::max(ns, 1);
-  if (ns > 0) {
+  if (far) {
+    // whole groups of FAR_FOLD sources per split, kFarRounds rounds of resident blocks
+    const size_t split_bytes = (size_t)no * nt * sizeof(double);
+    const int groups = (ns + FAR_FOLD - 1) / FAR_FOLD, blocks = (nt + FAR_TILE - 1) / FAR_TILE;
+    const long long slots = (long long)blocks_per_cu((const void*)fn) * ctx->num_cus;
+    const long long cap = std::max<long long>(1, std::min<long long>(groups, (long long)(kPartialCap / split_bytes)));
+    long long want = ov.splits > 0 ? ov.splits : std::min(cap, (kFarRounds * slots + blocks - 1) / blocks);
+    want = std::min<long long>(want, groups);
+    const int per = std::min<int>(kFarGroups, std::max<int>(1, (int)(groups / want)));
+    nsplit = ov.splits > 0 ? (int)want : (int)std::min<long long>((groups + per - 1) / per, cap);
+  } else if (ns > 0) {
     const size_t split_bytes = (size_t)no * nt * sizeof(double);
     size_t cap = std::min<size_t>(4096, kPartialCap / split_bytes);
     if (pb.fixed) cap = std::min(cap, pb.bytes / split_bytes);
@@ -504,16 +603,35 @@ int run_pair_sum(lpm_ctx* ctx, const PairProblem& pp) {
     nsplit = (ns + chunk - 1) / chunk;
   }
 
-  LPM_HIP(ctx, tb.ensure((size_t)nt * TREC * wsz));
-  LPM_HIP(ctx, sb.ensure((size_t)std::max(ns, 1) * nw * wsz));
+  // the tile balls lie behind the records
+  const size_t tgt_bytes = (size_t)nt * TREC * wsz, src_bytes = (size_t)std::max(ns, 1) * nw * wsz;
+  const size_t tball_bytes = path == kAllPairs ? 0 : (size_t)((nt + t_tile - 1) / t_tile) * sizeof(float4);
+  const size_t sball_bytes = path == kAllPairs ? 0 : (size_t)((ns + s_tile - 1) / s_tile) * sizeof(float4);
+  LPM_HIP(ctx, tb.ensure(tgt_bytes + tball_bytes));
+  LPM_HIP(ctx, sb.ensure(src_bytes + sball_bytes));
   LPM_HIP(ctx, pb.ensure((size_t)nsplit * no * nt * sizeof(double)));
 
-  const bool fp32 = prec == LPM_PREC_FP32_KAHAN;
-  PackArgs pa{pp.x, pp.y, pp.z, pp.q0, pp.q1, pp.area, nullptr, pp.src_list, 0, pp.i0, pp.radius, 1.0};
+  const int *tgt_order = nullptr, *src_list = pp.src_list;
+  if (path != kAllPairs) {
+    if (pp.tgt_order && pp.src_order) {
+      tgt_order = pp.tgt_order;
+      src_list = pp.src_order;
+    } else {
+      const bool at = pp.tx != nullptr;
+      int *to = nullptr, *so = nullptr;
+      OrderInput oi{at ? pp.tx : pp.x, at ? pp.ty : pp.y, at ? pp.tz : pp.z, pp.i0, nt, pp.x, pp.y, pp.z,
+                    pp.src_list, ns, sphere_kind(kind)};
+      if (int rc = spatial_order(ctx, oi, pp.order_buf ? *pp.order_buf : ctx->order, &to, &so)) return rc;
+      tgt_order = to;
+      src_list = so;
+    }
+  }
+  PackArgs pa{pp.x, pp.y, pp.z, pp.q0, pp.q1, pp.area, nullptr, src_list, 0, pp.i0, pp.radius, 1.0};
   pa.q2 = pp.q2;
   pa.q3 = pp.q3;
   pa.m = pp.m;
   PackArgs pt = pa;  // targets: the count is nt
+  pt.tgt_order = tgt_order;
   pa.count_dev = pp.ns_dev;
   const bool scaled = kind == LPM_K_PSE8 || kind == LPM_K_PSE2 || kind == LPM_K_PSE_SPHERE8 ||
                       kind == LPM_K_PSE_DERIV_PLANE || kind == LPM_K_PSE_DERIV_SPHERE ||
@@ -550,13 +668,25 @@ int run_pair_sum(lpm_ctx* ctx, const PairProblem& pp) {
     a.ns_dev = pp.ns_dev;
     const int nblk_t = (n_wtiles + 3) / 4;
     dim3 grid((unsigned)(nblk_t * nsplit)), block(256);
+    float4* tballs = reinterpret_cast<float4*>(static_cast<char*>(tb.p) + tgt_bytes);
+    float4* sballs = reinterpret_cast<float4*>(static_cast<char*>(sb.p) + src_bytes);
+    if (path != kAllPairs) {
+      if (fp32)
+        launch_balls<float>(kind, pp.m, nw, tb.p, sb.p, tballs, sballs, nt, ns, t_tile, s_tile, ctx->stream);
+      else
+        launch_balls<double>(kind, pp.m, nw, tb.p, sb.p, tballs, sballs, nt, ns, t_tile, s_tile, ctx->stream);
+    }
     hipEvent_t e0 = nullptr, e1 = nullptr;
     if (ctx->timing && !pp.ns_dev) {
       e0 = take_event(ctx);
       e1 = take_event(ctx);
       if (e0 && e1) LPM_HIP(ctx, hipEventRecord(e0, ctx->stream));
     }
-    hipLaunchKernelGGL(fn, grid, block, 0, ctx->stream, a);
+    if (far) {
+      hipLaunchKernelGGL(far_fn, grid, block, 0, ctx->stream, tb.p, sb.p, pb.as<double>(), tballs, sballs, tgt_order,
+                         a);
+    } else
+      hipLaunchKernelGGL(fn, grid, block, 0, ctx->stream, a);
     LPM_HIP(ctx, hipGetLastError());
     if (ctx->timing && e0 && e1) {
       LPM_HIP(ctx, hipEventRecord(e1, ctx->stream));
@@ -592,6 +722,7 @@ int run_pair_sum(lpm_ctx* ctx, const PairProblem& pp) {
   f.q2 = pp.q2;
   f.out3 = pp.out3;
   f.op = pp.op;
+  f.tgt_order = tgt_order;
   const double e4 = pp.eps * pp.eps * pp.eps * pp.eps;
   if (kind == LPM_K_PSE8 || kind == LPM_K_PSE2 || kind == LPM_K_PSE_SPHERE8)
     f.scale = (kind == LPM_K_PSE2 ? 4.0 : 1.0) / (kPi * e4);

@@ -167,13 +167,15 @@ struct lpm_bve_solver {
   DevBuf psi_rel, psi_abs;
   DevBuf tgt, src, partial;
   DevBuf tot;   // FP32 stream functions: FP64 source totals
+  DevBuf order;  // spatial order of the tile paths: one for the four sums of a step
+  const int *tgt_order = nullptr, *src_order = nullptr;  // inside `order`, null between steps
   DevBuf ptrs;  // device pointer tables for rk4_combine
   hipGraph_t graph = nullptr;
   hipGraphExec_t exec = nullptr;
   double graph_dt = 0.0;
   // addresses of the workspaces a captured step uses, as captured; an on-demand
   // stream-function call may regrow them, and then the step is captured again
-  void* graph_bufs[6] = {};
+  void* graph_bufs[7] = {};
   bool has_abs = false;
   bool loaded = false;  // false after a failed particle reload
 };
@@ -203,6 +205,9 @@ int bve_velocity(lpm_bve_solver* s, const double* x, const double* y, const doub
   pp.tgt_buf = &s->tgt;
   pp.src_buf = &s->src;
   pp.partial_buf = &s->partial;
+  pp.order_buf = &s->order;
+  pp.tgt_order = s->tgt_order;
+  pp.src_order = s->src_order;
   return lpm::run_pair_sum(s->ctx, pp);
 }
 
@@ -233,12 +238,15 @@ int bve_stream(lpm_bve_solver* s) {
   pp.tgt_buf = &s->tgt;
   pp.src_buf = &s->src;
   pp.partial_buf = &s->partial;
+  pp.order_buf = &s->order;
+  pp.tgt_order = s->tgt_order;
+  pp.src_order = s->src_order;
   pp.red_buf = &s->tot;
   return lpm::run_pair_sum(ctx, pp);
 }
 
 // Enqueue one RK4 step (no synchronization).
-int bve_enqueue_step(lpm_bve_solver* s, double dt) {
+int bve_enqueue_sums(lpm_bve_solver* s, double dt) {
   lpm_ctx* ctx = s->ctx;
   const int n = s->n;
   dim3 b(256), g((n + 255) / 256);
@@ -271,18 +279,38 @@ int bve_enqueue_step(lpm_bve_solver* s, double dt) {
   return LPM_OK;
 }
 
+// The four sums of a step share the spatial order of its first state: stage points
+// lie within a step of it, and any order gives the same sums.
+template <class Solver, class SumsFn>
+int with_step_order(Solver* s, int kind, const double* z, SumsFn sums) {
+  if (lpm::sum_path(s->ctx, kind, s->precision, s->n, s->ns) == lpm::kAllPairs) return sums();
+  lpm::OrderInput in{s->x.template as<double>(), s->y.template as<double>(), z, 0, s->n, s->x.template as<double>(),
+                     s->y.template as<double>(), z, s->list.template as<int>(), s->ns, z != nullptr};
+  int *t = nullptr, *q = nullptr;
+  if (int rc = lpm::spatial_order(s->ctx, in, s->order, &t, &q)) return rc;
+  s->tgt_order = t;
+  s->src_order = q;
+  const int rc = sums();
+  s->tgt_order = s->src_order = nullptr;
+  return rc;
+}
+
+int bve_enqueue_step(lpm_bve_solver* s, double dt) {
+  return with_step_order(s, LPM_K_SPHERE_BS, s->z.as<double>(), [&] { return bve_enqueue_sums(s, dt); });
+}
+
 // The workspaces a step grows on demand (the state and stage arrays change
 // only in bve_load, which drops the graph).
-void bve_work_bufs(const lpm_bve_solver* s, void* out[6]) {
-  const DevBuf* b[6] = {&s->tgt, &s->src, &s->partial, &s->psi_rel, &s->psi_abs, &s->tot};
-  for (int k = 0; k < 6; ++k) out[k] = b[k]->p;
+void bve_work_bufs(const lpm_bve_solver* s, void* out[7]) {
+  const DevBuf* b[7] = {&s->tgt, &s->src, &s->partial, &s->psi_rel, &s->psi_abs, &s->tot, &s->order};
+  for (int k = 0; k < 7; ++k) out[k] = b[k]->p;
 }
 
 template <class Solver, class BufsFn>
 bool graph_bufs_unchanged(const Solver* s, BufsFn bufs) {
-  void* now[6];
+  void* now[7];
   bufs(s, now);
-  for (int k = 0; k < 6; ++k)
+  for (int k = 0; k < 7; ++k)
     if (now[k] != s->graph_bufs[k]) return false;
   return true;
 }
@@ -523,7 +551,7 @@ int lpm_bve_solver_delete(lpm_bve_solver* s) {
   if (s->graph) (void)hipGraphDestroy(s->graph);
   DevBuf* all[] = {&s->x, &s->y, &s->z, &s->zeta, &s->absv, &s->u, &s->v, &s->w, &s->area,
                    &s->active, &s->list, &s->xi, &s->yi, &s->zi, &s->qi, &s->psi_rel, &s->psi_abs,
-                   &s->tgt, &s->src, &s->partial, &s->tot, &s->ptrs};
+                   &s->tgt, &s->src, &s->partial, &s->tot, &s->order, &s->ptrs};
   for (DevBuf* b : all) b->release();
   for (auto& row : s->k)
     for (auto& b : row) b.release();
@@ -542,11 +570,13 @@ struct lpm_plane_solver {
   DevBuf xi, yi;
   DevBuf psi;
   DevBuf tgt, src, partial;
+  DevBuf order;  // see lpm_bve_solver
+  const int *tgt_order = nullptr, *src_order = nullptr;
   DevBuf ptrs;
   hipGraph_t graph = nullptr;
   hipGraphExec_t exec = nullptr;
   double graph_dt = 0.0;
-  void* graph_bufs[6] = {};  // workspace addresses as captured (see lpm_bve_solver)
+  void* graph_bufs[7] = {};  // workspace addresses as captured (see lpm_bve_solver)
   bool loaded = false;  // false after a failed particle reload
 };
 
@@ -570,6 +600,9 @@ int plane_velocity(lpm_plane_solver* s, const double* x, const double* y, double
   pp.tgt_buf = &s->tgt;
   pp.src_buf = &s->src;
   pp.partial_buf = &s->partial;
+  pp.order_buf = &s->order;
+  pp.tgt_order = s->tgt_order;
+  pp.src_order = s->src_order;
   return lpm::run_pair_sum(s->ctx, pp);
 }
 
@@ -591,10 +624,13 @@ int plane_stream(lpm_plane_solver* s) {
   pp.tgt_buf = &s->tgt;
   pp.src_buf = &s->src;
   pp.partial_buf = &s->partial;
+  pp.order_buf = &s->order;
+  pp.tgt_order = s->tgt_order;
+  pp.src_order = s->src_order;
   return lpm::run_pair_sum(s->ctx, pp);
 }
 
-int plane_enqueue_step(lpm_plane_solver* s, double dt) {
+int plane_enqueue_sums(lpm_plane_solver* s, double dt) {
   lpm_ctx* ctx = s->ctx;
   const int n = s->n;
   dim3 b(256), g((n + 255) / 256);
@@ -620,10 +656,14 @@ int plane_enqueue_step(lpm_plane_solver* s, double dt) {
   return LPM_OK;
 }
 
-void plane_work_bufs(const lpm_plane_solver* s, void* out[6]) {
-  const DevBuf* b[4] = {&s->tgt, &s->src, &s->partial, &s->psi};
-  for (int k = 0; k < 4; ++k) out[k] = b[k]->p;
-  out[4] = out[5] = nullptr;
+int plane_enqueue_step(lpm_plane_solver* s, double dt) {
+  return with_step_order(s, LPM_K_PLANE_BS, nullptr, [&] { return plane_enqueue_sums(s, dt); });
+}
+
+void plane_work_bufs(const lpm_plane_solver* s, void* out[7]) {
+  const DevBuf* b[5] = {&s->tgt, &s->src, &s->partial, &s->psi, &s->order};
+  for (int k = 0; k < 5; ++k) out[k] = b[k]->p;
+  out[5] = out[6] = nullptr;
 }
 
 int plane_step(lpm_plane_solver* s, double dt) {
@@ -822,7 +862,7 @@ int lpm_plane_solver_delete(lpm_plane_solver* s) {
   if (s->exec) (void)hipGraphExecDestroy(s->exec);
   if (s->graph) (void)hipGraphDestroy(s->graph);
   DevBuf* all[] = {&s->x, &s->y, &s->vort, &s->u, &s->v, &s->area, &s->active, &s->list,
-                   &s->xi, &s->yi, &s->psi, &s->tgt, &s->src, &s->partial, &s->ptrs};
+                   &s->xi, &s->yi, &s->psi, &s->tgt, &s->src, &s->partial, &s->order, &s->ptrs};
   for (DevBuf* b : all) b->release();
   for (auto& row : s->k)
     for (auto& b : row) b.release();

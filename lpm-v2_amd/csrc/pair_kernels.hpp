@@ -621,6 +621,8 @@ struct BatchProblem {
   int t_off, nt, s_off, ns;
   int chunk, nsplit;
   long long part_off;
+  int far;                   // takes the far path (far_kernels.hpp)
+  int tball_off, sball_off;  // its balls
 };
 
 struct BatchItem {

@@ -1,0 +1,172 @@
+"""The tile paths of large sums: spatial order, far tiles on the MFMA.
+
+Each call is compared with the all-pairs kernel (a forced tile shape) and with the
+FP64 sum of the same inputs, over input orders, ragged blocks and masks, sizes at
+the edges of tiles, and values that are not finite.  FP32 velocity and stream sums
+are held to 1e-6 of the largest value, the library's FP32 bar on meshes."""
+import numpy as np
+import pytest
+
+from helpers import rel_err_max
+from lpmgpu import BVEBatch, BVESolver, _lib as L
+from lpmgpu import ic, mesh
+
+pytestmark = pytest.mark.gpu
+
+TOL32 = 1e-6
+
+
+def _rows(out):
+    return [out] if isinstance(out, np.ndarray) else [np.asarray(o) for o in out]
+
+
+def _all_pairs(ctx, kind, prec, call):
+    ctx.set_tuning(kind, prec, 2, 256 if prec == "fp32" else 64, 0)
+    try:
+        return _rows(call())
+    finally:
+        ctx.set_tuning(kind, prec, 0, 0, 0)
+
+
+def _sphere(order, seed=3):
+    """Icosahedral level 6 (122,882 particles), turned, in the mesh's order or shuffled."""
+    m = mesh.icosahedral_mesh(6)
+    rng = np.random.default_rng(seed)
+    rot, _ = np.linalg.qr(rng.normal(size=(3, 3)))
+    xyz = m.xyz() @ rot
+    idx = rng.permutation(m.n) if order == "shuffled" else np.arange(m.n)
+    x, y, z = (np.ascontiguousarray(c[idx]) for c in xyz.T)
+    zeta = ic.random_gaussian_vortices(rng, 3, x, y, z) + ic.rh4_vorticity(x, y, z)
+    active = m.active[idx] * (rng.uniform(size=m.n) < 0.8)
+    return x, y, z, zeta, m.area[idx], active.astype(np.int32)
+
+
+@pytest.mark.parametrize("order", ["mesh", "shuffled"])
+@pytest.mark.parametrize("block", [(0, None), (17, 122882 - 255), (5, 5 + 256 * 128 + 1)])
+def test_far_tiles_sphere(ctx, order, block):
+    x, y, z, zeta, area, act = _sphere(order)
+    i0, i1 = block[0], block[1] or x.size
+    for kind, call in (
+            (L.K_SPHERE_BS, lambda p: ctx.bve_sphere_velocity(x, y, z, zeta, area, act, i0=i0, i1=i1, precision=p)),
+            (L.K_SPHERE_GREEN, lambda p: ctx.bve_sphere_stream(x, y, z, zeta, zeta + z, area, act, i0=i0, i1=i1,
+                                                               precision=p))):
+        got, ref = _rows(call("fp32")), _rows(call("fp64"))
+        for g, r in zip(got, ref):
+            assert rel_err_max(g[i0:i1], r[i0:i1]) < TOL32
+            assert not g[:i0].any() and not g[i1:].any()
+        for g, r in zip(got, _all_pairs(ctx, kind, "fp32", lambda: call("fp32"))):
+            assert rel_err_max(g, r) < 2 * TOL32
+        again = _rows(call("fp32"))
+        assert all(np.array_equal(a, b) for a, b in zip(got, again))
+
+
+@pytest.mark.parametrize("shape", ["grid", "strip", "two_clusters", "duplicates"])
+def test_far_tiles_plane(ctx, shape):
+    """Layouts that make balls large, thin, far apart or of radius zero."""
+    rng = np.random.default_rng(7)
+    n = 70000
+    if shape == "grid":
+        x, y, area, _ = mesh.grid_centres(270, 1.0, jitter=5e-4, seed=2)
+    elif shape == "strip":
+        x, y = rng.uniform(-50, 50, n), rng.uniform(-0.01, 0.01, n)
+    elif shape == "two_clusters":
+        x, y = rng.normal(size=n) * 0.1, rng.normal(size=n) * 0.1
+        x[::2] += 40.0
+    else:  # every point 300 times over: the pairs of equal points are self-like, with weight 0
+        x, y = np.repeat(rng.uniform(-1, 1, n // 300), 300), np.repeat(rng.uniform(-1, 1, n // 300), 300)
+    n = x.size
+    area = np.full(n, 1.0 / n)
+    w = 1.0 + 0.5 * np.sin(5 * x)
+    act = np.ones(n, np.int32)
+    if shape == "duplicates":
+        act[:] = 0
+        act[::300] = 1
+        tgt = np.arange(n) % 300 == 0  # the copies sit on top of a source
+    else:
+        tgt = np.ones(n, bool)
+    for kind, call in ((L.K_PLANE_BS, lambda p: ctx.plane_velocity(x, y, w, area, act, precision=p)),
+                       (L.K_PLANE_GREEN, lambda p: ctx.plane_stream(x, y, w, area, act, precision=p))):
+        got, pairs = _rows(call("fp32")), _all_pairs(ctx, kind, "fp32", lambda: call("fp32"))
+        for g, r, e in zip(got, _rows(call("fp64")), pairs):
+            # random points come closer than mesh points: as far off as the all-pairs sum is
+            own = rel_err_max(e[tgt], r[tgt])
+            assert rel_err_max(g[tgt], r[tgt]) < max(TOL32, 1.5 * own), (shape, own)
+
+
+@pytest.mark.parametrize("bad", ["weight_inf", "weight_nan", "source_nan", "target_nan"])
+def test_far_tiles_spread_non_finite_values_like_all_pairs(ctx, bad):
+    x, y, z, zeta, area, act = (np.array(a, copy=True) for a in _sphere("mesh"))
+    j = int(np.flatnonzero(act)[12345])
+    if bad == "weight_inf":
+        zeta[j] = np.inf
+    elif bad == "weight_nan":
+        zeta[j] = np.nan
+    elif bad == "source_nan":
+        x[j] = np.nan
+    else:
+        x[int(np.flatnonzero(act == 0)[777])] = np.nan
+
+    def call():
+        return ctx.bve_sphere_velocity(x, y, z, zeta, area, act, precision="fp32")
+
+    # (the all-pairs kernel's error-free sums turn an infinite sum into NaN)
+    for g, r in zip(_rows(call()), _all_pairs(ctx, L.K_SPHERE_BS, "fp32", call)):
+        assert np.array_equal(np.isfinite(g), np.isfinite(r))
+        if bad != "weight_inf":
+            assert np.array_equal(np.isnan(g), np.isnan(r))
+
+
+def test_far_tiles_split_leaves_no_trace(ctx):
+    x, y, z, zeta, area, act = _sphere("mesh")
+    ref = _rows(ctx.bve_sphere_velocity(x, y, z, zeta, area, act, precision="fp32"))
+    try:
+        for splits in (1, 3, 64):
+            ctx.set_tuning(L.K_SPHERE_BS, "fp32", 0, 0, splits)
+            for g, r in zip(_rows(ctx.bve_sphere_velocity(x, y, z, zeta, area, act, precision="fp32")), ref):
+                assert rel_err_max(g, r) < 1e-13
+    finally:
+        ctx.set_tuning(L.K_SPHERE_BS, "fp32", 0, 0, 0)
+
+
+def test_far_tiles_solver_and_graph(ctx):
+    """One order per step, captured with it: replays equal eager steps."""
+    x, y, z, zeta, area, act = _sphere("shuffled")
+    kw = dict(rotation_rate=2 * np.pi, precision="fp32", project=True)
+    a = BVESolver(ctx, x, y, z, zeta, area, act, **kw)
+    b = BVESolver(ctx, x, y, z, zeta, area, act, use_graph=True, **kw)
+    d = BVESolver(ctx, x, y, z, zeta, area, act, rotation_rate=2 * np.pi, precision="fp64", project=True)
+    for k in range(3):
+        for s in (a, b, d):
+            s.timestep(0.005)
+        sa, sb, sd = a.state(), b.state(), d.state()
+        assert all(np.array_equal(sa[q], sb[q]) for q in sa), k
+        if k == 0:
+            assert rel_err_max((sa["u"], sa["v"], sa["w"]), (sd["u"], sd["v"], sd["w"])) < TOL32
+    for s in (a, b, d):
+        s.delete()
+
+
+@pytest.mark.parametrize("graph", [False, True])
+def test_far_tiles_batch(ctx, graph):
+    """Problems on both sides of the rule in one batch, with a radius other than 1."""
+    rng = np.random.default_rng(4)
+    probs = []
+    for level, radius in ((3, 1.0), (6, 2.5), (4, 1.0), (6, 1.0)):
+        m = mesh.icosahedral_mesh(level, radius=radius)
+        idx = rng.permutation(m.n)
+        x, y, z = m.x[idx], m.y[idx], m.z[idx]
+        probs.append(dict(x=x, y=y, z=z, relvort=ic.random_gaussian_vortices(rng, 2, x / radius, y / radius, z / radius),
+                          area=m.area[idx], active=m.active[idx], radius=radius, rotation_rate=2 * np.pi))
+    a = BVEBatch(ctx, probs, precision="fp32", project=True, use_graph=graph)
+    b = BVEBatch(ctx, probs, precision="fp64", project=True)
+    c = BVEBatch(ctx, probs, precision="fp32", project=True)
+    c.set_tuning(4, 256, 16384)  # all pairs
+    for s in (a, b, c):
+        s.timestep(0.005)
+    for ga, gb, gc in zip(*(s.split(s.state()) for s in (a, b, c))):
+        ref = (gb["u"], gb["v"], gb["w"])
+        assert rel_err_max((ga["u"], ga["v"], ga["w"]), ref) < TOL32
+        assert rel_err_max((ga["u"], ga["v"], ga["w"]), (gc["u"], gc["v"], gc["w"])) < 2 * TOL32
+        assert rel_err_max((ga["x"], ga["y"], ga["z"]), (gb["x"], gb["y"], gb["z"])) < TOL32
+    for s in (a, b, c):
+        s.delete()
