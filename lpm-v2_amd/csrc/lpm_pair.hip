@@ -211,6 +211,10 @@ __global__ __launch_bounds__(256) void finalize_kernel(FinArgs f) {
 }
 
 // ------------------------------------------------------------ dispatching
+static bool is_vortex_kind(int kind) {
+  return kind == LPM_K_SPHERE_BS || kind == LPM_K_PLANE_BS || kind == LPM_K_SPHERE_GREEN || kind == LPM_K_PLANE_GREEN;
+}
+
 static int nout_of(int kind) {
   switch (kind) {
     case LPM_K_SPHERE_BS: return 3;
@@ -391,6 +395,23 @@ constexpr int kChunkMin = 256;
 constexpr int kMinRounds = 12;
 constexpr size_t kPartialCap = size_t(2) << 30;  // bytes of FP64 split partials
 
+// Small sums: one launch is a few waves per SIMD, each
+// waiting for its scalar loads, so its time is the length of a wave's source chunk,
+// and short chunks over more waves win: one target per lane, at least kSmallChunk
+// sources and about kSmallWaves waves.  Kernel times against 2 targets per lane and
+// 256 sources: level 3 FP64 82 -> 16 us, level 4 FP64 82 -> 42 us and FP32 57 -> 30 us,
+// cubed level 5 FP64 92 -> 65 us, level 5 FP64 (6e8 pairs) 420 -> 360 us.  In FP32, and
+// for the longer PSE pairs, 2 targets per lane are as fast at 7.5e7 pairs and 3-6 %
+// faster at 3e8.
+constexpr double kSmallPairs = 1.2e8, kSmallPairsVortex64 = 1e9;
+constexpr int kSmallChunk = 64;
+constexpr int kSmallWaves = 24576;
+
+static int small_splits(int n_wtiles, int ns, int max_split_mem) {
+  const long long chunk = std::max<long long>(kSmallChunk, (long long)n_wtiles * ns / kSmallWaves);
+  return (int)std::max<long long>(1, std::min<long long>((ns + chunk - 1) / chunk, max_split_mem));
+}
+
 static int choose_splits(int n_wtiles, int ns, int kt, int slots, int max_split_mem) {
   const int nblk_t = (n_wtiles + 3) / 4;
   const int min_chunk = std::max(kt, 256);
@@ -438,9 +459,7 @@ SumPath sum_path(const lpm_ctx* ctx, int kind, int prec, int nt, int ns) {
   const Tuning& ov = ctx->tune[kind][prec == LPM_PREC_FP32_KAHAN ? 1 : 0];
   if (ov.r || ov.kt) return kAllPairs;  // a forced tile shape is one of the all-pairs kernel
   if ((long long)nt + ns > (1 << 30)) return kAllPairs;  // item counts of the sort are ints
-  const bool vortex = kind == LPM_K_SPHERE_BS || kind == LPM_K_PLANE_BS || kind == LPM_K_SPHERE_GREEN ||
-                      kind == LPM_K_PLANE_GREEN;
-  if (vortex) {
+  if (is_vortex_kind(kind)) {
     const bool plane = kind == LPM_K_PLANE_BS || kind == LPM_K_PLANE_GREEN;
     const double least = plane ? kFarMinPairsPlane : kFarMinPairsSphere;
     return prec == LPM_PREC_FP32_KAHAN && (double)nt * ns >= least ? kFarTiles : kAllPairs;
@@ -559,6 +578,12 @@ int run_pair_sum(lpm_ctx* ctx, const PairProblem& pp) {
   DevBuf& sb = pp.src_buf ? *pp.src_buf : ctx->src;
   DevBuf& pb = pp.partial_buf ? *pp.partial_buf : ctx->partial;
 
+  const bool small = !ov.r && !ov.kt && !ov.splits && ns > 0 &&
+                     (double)nt * ns < (is_vortex_kind(kind) && !fp32 ? kSmallPairsVortex64 : kSmallPairs);
+  if (small) {
+    tu.r = 1;
+    tu.kt = fp32 ? 64 : 32;
+  }
   // a device-side source count cannot be ordered
   const SumPath path = pp.ns_dev ? kAllPairs : sum_path(ctx, kind, prec, nt, ns);
   const bool far = path == kFarTiles;
@@ -595,6 +620,7 @@ int run_pair_sum(lpm_ctx* ctx, const PairProblem& pp) {
     if (cap < 1) return fail(ctx, LPM_ERR_NOMEM, "partial buffer too small for one source split");
     const int split_mem = (int)cap;
     int want = tu.splits > 0 ? tu.splits
+               : small       ? small_splits(n_wtiles, ns, split_mem)
                              : choose_splits(n_wtiles, ns, tu.kt, blocks_per_cu((const void*)fn) * ctx->num_cus,
                                              split_mem);
     if (pb.fixed) want = std::min(want, split_mem);

@@ -484,6 +484,20 @@ __device__ __forceinline__ void two_sum_acc(T& S, T& C, T p) {
   S = t;
 }
 
+// Sources loaded together: 4 for the FP64 vortex sums (10-12 SGPRs a source), which
+// took the level-4 sphere sum from 82 to 62 us and none slower at full size; the FP32
+// sums and the longer PSE policies lose 5-35 % with 2 or 4 there and keep one ahead.
+template <class P, typename T>
+inline constexpr int LOAD_GROUP = 1;
+template <bool E>
+inline constexpr int LOAD_GROUP<SphereBS<double, E>, double> = 4;
+template <bool E>
+inline constexpr int LOAD_GROUP<SphereGreen<double, E>, double> = 4;
+template <>
+inline constexpr int LOAD_GROUP<PlaneBS<double>, double> = 4;
+template <>
+inline constexpr int LOAD_GROUP<PlaneGreen<double>, double> = 4;
+
 // One wavefront's work: targets [t_begin, t_begin + 64 R) of the record array
 // tg[0, nt) (particle index tgt_idx0 + local) against sources [j_begin, j_end)
 // of src; FP64 results go to out[k * out_stride + i] for valid targets i.
@@ -527,30 +541,52 @@ __device__ __forceinline__ void pair_tile(const Vec4<T>* __restrict__ tg, int nt
       for (int k = 0; k < NO; ++k) p[r][k] = (T)0;
 
     if (!checked) {
-      // the next source's record is loaded before this one's arithmetic, so
-      // the scalar loads' latency overlaps the pair work (the last iteration
-      // reloads its own record).  Measured on MI355X against loading each
-      // record at its use: PSE-8 at 512^2 15.96 -> 14.45 ms, plane gradient
-      // 20.68 -> 18.92 ms, sphere Biot-Savart at icosahedral L7 38.17 -> 37.95 ms.
-      T sv[P::NW];
+      // LOAD_GROUP sources' records load (scalar) under the arithmetic of the group
+      // before them.  A record that another XCD packed takes 700 cycles, so where few
+      // waves share a SIMD one record ahead leaves the loop waiting for each load.
+      constexpr int G = LOAD_GROUP<P, T>;
+      int j = jt;
+      if (jt + G <= jt_end) {
+        T sv[G][P::NW];
 #pragma unroll
-      for (int q = 0; q < P::NW; ++q) sv[q] = src[(size_t)jt * P::NW + q];
+        for (int g = 0; g < G; ++g)
+#pragma unroll
+          for (int q = 0; q < P::NW; ++q) sv[g][q] = src[(size_t)(jt + g) * P::NW + q];
 #pragma unroll 2
-      for (int j = jt; j < jt_end; ++j) {
-        const int jn = j + 1 < jt_end ? j + 1 : j;
-        T sn[P::NW];
+        for (; j + G <= jt_end; j += G) {
+          const int jn = j + 2 * G <= jt_end ? j + G : j;
+          T sn[G][P::NW];
 #pragma unroll
-        for (int q = 0; q < P::NW; ++q) sn[q] = src[(size_t)jn * P::NW + q];
-        W4<T> w[R];
-        T f[R];
+          for (int g = 0; g < G; ++g)
 #pragma unroll
-        for (int r = 0; r < R; ++r) P::arg(t[r], sv, w[r]);
+            for (int q = 0; q < P::NW; ++q) sn[g][q] = src[(size_t)(jn + g) * P::NW + q];
 #pragma unroll
-        for (int r = 0; r < R; ++r) f[r] = P::trans(w[r]);
+          for (int g = 0; g < G; ++g) {
+            W4<T> w[R];
+            T f[R];
 #pragma unroll
-        for (int r = 0; r < R; ++r) P::acc(sv, w[r], f[r], p[r]);
+            for (int r = 0; r < R; ++r) P::arg(t[r], sv[g], w[r]);
 #pragma unroll
-        for (int q = 0; q < P::NW; ++q) sv[q] = sn[q];
+            for (int r = 0; r < R; ++r) f[r] = P::trans(w[r]);
+#pragma unroll
+            for (int r = 0; r < R; ++r) P::acc(sv[g], w[r], f[r], p[r]);
+          }
+#pragma unroll
+          for (int g = 0; g < G; ++g)
+#pragma unroll
+            for (int q = 0; q < P::NW; ++q) sv[g][q] = sn[g][q];
+        }
+      }
+      for (; j < jt_end; ++j) {
+        T sv[P::NW];
+#pragma unroll
+        for (int q = 0; q < P::NW; ++q) sv[q] = src[(size_t)j * P::NW + q];
+#pragma unroll
+        for (int r = 0; r < R; ++r) {
+          W4<T> w;
+          P::arg(t[r], sv, w);
+          P::acc(sv, w, P::trans(w), p[r]);
+        }
       }
     } else {
       for (int j = jt; j < jt_end; ++j) {

@@ -97,3 +97,27 @@ def test_tile_shapes_and_splits_agree(ctx, prec):
                     assert err <= tol, (name, r, kt, sp, k, err)
         finally:
             ctx.set_tuning(kind, prec, 0, 0, 0)
+
+
+@pytest.mark.parametrize("prec", ["fp64", "fp32"])
+@pytest.mark.parametrize("n", [1, 63, 64, 65, 257, 1027])
+def test_small_sums_match_forced_shapes(ctx, prec, n):
+    """The launch shape of small sums (one target per lane, short source chunks)
+    at the edges of waves and chunks, against a forced shape: FP64 to 1e-12,
+    FP32 to 2e-6."""
+    rng = np.random.default_rng(n)
+    p = rng.normal(size=(3, n))
+    x, y, z = p / np.linalg.norm(p, axis=0)
+    w, area = rng.normal(size=n), np.full(n, 4 * np.pi / n)
+    act = (np.arange(n) % 5 != 1).astype(np.int32)
+    tol = 1e-12 if prec == "fp64" else 2e-6
+    for kind, call in ((L.K_SPHERE_BS, lambda: ctx.bve_sphere_velocity(x, y, z, w, area, act, precision=prec)),
+                       (L.K_PLANE_GREEN, lambda: ctx.plane_stream(x, y, w, area, act, precision=prec))):
+        got = _as_rows(call())
+        ctx.set_tuning(kind, prec, 4, 64, 1)
+        try:
+            ref = _as_rows(call())
+        finally:
+            ctx.set_tuning(kind, prec, 0, 0, 0)
+        for g, r in zip(got, ref):
+            assert np.abs(g - r).max() <= tol * max(np.abs(r).max(), 1e-300)
