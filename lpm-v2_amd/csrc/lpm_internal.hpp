@@ -198,6 +198,7 @@ bool is_ops_kind(int kind);
 int ops_nout(int kind, int m);
 int ops_record_words(int kind, int m);
 const void* ops_pick_kernel(int kind, int prec, int r, int m, bool series);
+const void* ops_pick_cull(int kind, int prec, int m, bool series);
 void ops_launch_pack(int kind, int prec, const PackArgs& s, const PackArgs& t, void* srec, void* trec, int ns,
                      int nt, hipStream_t st);
 int ops_launch_finalize(int kind, int m, const FinArgs& f, hipStream_t st);
@@ -207,11 +208,12 @@ Tuning default_tuning(int kind, int prec);
 // Where the far path starts, in pairs (see sum_path).
 constexpr double kFarMinPairsSphere = 2e9, kFarMinPairsPlane = 4e9;
 
-// How a sum is scheduled: over all pairs (pair_kernels.hpp) or with the
-// well-separated tiles on the MFMA (far_kernels.hpp), which wants the records in
-// spatial order.
-enum SumPath { kAllPairs = 0, kFarTiles = 1 };
-SumPath sum_path(const lpm_ctx* ctx, int kind, int prec, int nt, int ns);
+// How a sum is scheduled: over all pairs (pair_kernels.hpp), with the
+// well-separated tiles on the MFMA (far_kernels.hpp), or without the tiles whose
+// terms are zero (cull_kernels.hpp).  The last two want the records in spatial order.
+enum SumPath { kAllPairs = 0, kFarTiles = 1, kCullTiles = 2 };
+// reach: of a PSE kernel on the sphere, in radii
+SumPath sum_path(const lpm_ctx* ctx, int kind, int prec, int nt, int ns, double reach = 0.0);
 
 // Spatial order (lpm_order.hip) of targets tx.. [i0, i0 + nt) and of the sources
 // x..[list[0, ns)]: device arrays of particle indices inside `buf`.

@@ -1,7 +1,7 @@
 // lpm_order.hip -- spatial order of targets and sources.
 //
-// The tile path (far_kernels.hpp) decides per tile of consecutive
-// records, so it wants consecutive records close together, whatever order the
+// The tile paths (far_kernels.hpp, cull_kernels.hpp) decide per tile of consecutive
+// records, so they want consecutive records close together, whatever order the
 // caller's particles come in (row-major grids, mesh levels one after the other,
 // remeshed sets).  Points are sorted by their index along a Hilbert curve: over the
 // bounding box on the plane, over the six faces of the surrounding cube on the

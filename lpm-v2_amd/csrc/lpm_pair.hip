@@ -11,6 +11,7 @@
 #include <algorithm>
 #include <mutex>
 
+#include "cull_kernels.hpp"
 #include "far_kernels.hpp"
 #include "lpm_internal.hpp"
 #include "pair_kernels.hpp"
@@ -252,8 +253,11 @@ Tuning default_tuning(int kind, int prec) {
   return t;
 }
 
+constexpr double kCullMinPairs = 1.5e8;
+constexpr double kCullMaxReach = 1.6;
 constexpr int kFarRounds = 8;   // rounds of resident blocks wanted of a far-tile sum
 constexpr int kFarGroups = 8;   // at most so many groups of FAR_FOLD sources per split
+constexpr int kCullWaves = 12;  // waves per SIMD wanted of a culled sum
 
 using KernelFn = void (*)(PairArgs);
 
@@ -452,10 +456,34 @@ static FarFn pick_far(int kind, bool on_sphere) {
   }
 }
 
-// Where the far path starts, by whole calls (ordering and balls cost 45 us there):
-// sphere velocity 0.95 of the all-pairs rate at 1.2e9 pairs, 1.01 at 2.5e9, 1.23 at
-// 1e10; plane velocity 0.92 at 1.6e9, 1.07 at 4.3e9.
-SumPath sum_path(const lpm_ctx* ctx, int kind, int prec, int nt, int ns) {
+// PSE Laplacians without their zero tiles; the other PSE kinds: ops_pick_cull.
+static CullFn pick_cull(int kind, int prec, int m, bool series) {
+  if (is_ops_kind(kind)) return reinterpret_cast<CullFn>(const_cast<void*>(ops_pick_cull(kind, prec, m, series)));
+  if (prec == LPM_PREC_FP32_KAHAN) {
+    switch (kind) {
+      case LPM_K_PSE8: return cull_sum_kernel<PsePolicy<float, 8>, void, float, 1>;
+      case LPM_K_PSE2: return cull_sum_kernel<PsePolicy<float, 2>, void, float, 1>;
+      default:
+        return series ? cull_sum_kernel<PseSphere<float, true>, void, float, 1>
+                      : cull_sum_kernel<PseSphere<float, false>, void, float, 1>;
+    }
+  }
+  switch (kind) {
+    case LPM_K_PSE8: return cull_sum_kernel<PsePolicy<double, 8>, void, double, 1>;
+    case LPM_K_PSE2: return cull_sum_kernel<PsePolicy<double, 2>, void, double, 1>;
+    default:
+      return series ? cull_sum_kernel<PseSphere<double, true>, void, double, 1>
+                    : cull_sum_kernel<PseSphere<double, false>, void, double, 1>;
+  }
+}
+
+// Where the tile paths start, by whole calls (ordering and balls cost 45 us there):
+// far tiles, sphere velocity 0.95 of the all-pairs rate at 1.2e9 pairs, 1.01 at 2.5e9,
+// 1.23 at 1e10; plane velocity 0.92 at 1.6e9, 1.07 at 4.3e9.  Culled PSE sums: plane
+// 80^2 (4e7 pairs) 0.88, 110^2 (1.5e8) 1.0, 150^2 (5e8) 1.3; sphere FP32 1.0 at 7.5e7
+// and 1.6 at 6e8.  On the sphere the sum must also reach less than kCullMaxReach radii
+// (chord): in FP64 at level 5 it reaches every particle.
+SumPath sum_path(const lpm_ctx* ctx, int kind, int prec, int nt, int ns, double reach) {
   const Tuning& ov = ctx->tune[kind][prec == LPM_PREC_FP32_KAHAN ? 1 : 0];
   if (ov.r || ov.kt) return kAllPairs;  // a forced tile shape is one of the all-pairs kernel
   if ((long long)nt + ns > (1 << 30)) return kAllPairs;  // item counts of the sort are ints
@@ -464,7 +492,7 @@ SumPath sum_path(const lpm_ctx* ctx, int kind, int prec, int nt, int ns) {
     const double least = plane ? kFarMinPairsPlane : kFarMinPairsSphere;
     return prec == LPM_PREC_FP32_KAHAN && (double)nt * ns >= least ? kFarTiles : kAllPairs;
   }
-  return kAllPairs;
+  return !ov.splits && (double)nt * ns >= kCullMinPairs && reach < kCullMaxReach ? kCullTiles : kAllPairs;
 }
 
 // Words of a source / target record that must be finite for a tile to be treated
@@ -585,9 +613,12 @@ int run_pair_sum(lpm_ctx* ctx, const PairProblem& pp) {
     tu.kt = fp32 ? 64 : 32;
   }
   // a device-side source count cannot be ordered
-  const SumPath path = pp.ns_dev ? kAllPairs : sum_path(ctx, kind, prec, nt, ns);
-  const bool far = path == kFarTiles;
-  const int t_tile = FAR_TILE, s_tile = FAR_TILE;
+  const double reach_eps = fp32 ? std::sqrt(CULL_Q32 / kLog2e) : std::sqrt(CULL_Q64);  // in eps
+  const SumPath path = pp.ns_dev ? kAllPairs
+                                 : sum_path(ctx, kind, prec, nt, ns,
+                                            sphere_kind(kind) ? reach_eps * pp.eps / pp.radius : 0.0);
+  const bool far = path == kFarTiles, cull = path == kCullTiles;
+  const int t_tile = far ? FAR_TILE : 64, s_tile = far ? FAR_TILE : CULL_TILE;
   const int per_wave = path != kAllPairs ? 64 : 64 * tu.r;
   const int n_wtiles = (nt + per_wave - 1) / per_wave;
   // sphere PSE kinds: the series form of the distance when 7 eps <= 0.56 R
@@ -597,6 +628,7 @@ int run_pair_sum(lpm_ctx* ctx, const PairProblem& pp) {
   const double series_reach = prec == LPM_PREC_FP32_KAHAN ? 0.56 : 0.35;
   const bool variant = sphere_pse ? (7.0 * pp.eps <= series_reach * pp.radius) : pp.on_sphere;
   FarFn far_fn = far ? pick_far(kind, pp.on_sphere) : nullptr;
+  CullFn cull_fn = cull ? pick_cull(kind, prec, pp.m, variant) : nullptr;
   KernelFn fn = far ? reinterpret_cast<KernelFn>(far_fn) : ops ? reinterpret_cast<KernelFn>(const_cast<void*>(ops_pick_kernel(kind, prec, tu.r, pp.m, variant)))
                     : pick_kernel(kind, prec, tu.r, variant);
   if (!fn) return fail(ctx, LPM_ERR_ARG, "no pair kernel for this kind, precision and field count");
@@ -613,6 +645,12 @@ int run_pair_sum(lpm_ctx* ctx, const PairProblem& pp) {
     want = std::min<long long>(want, groups);
     const int per = std::min<int>(kFarGroups, std::max<int>(1, (int)(groups / want)));
     nsplit = ov.splits > 0 ? (int)want : (int)std::min<long long>((groups + per - 1) / per, cap);
+  } else if (cull) {
+    // enough waves for kCullWaves a SIMD; a split takes every nsplit-th tile
+    const size_t split_bytes = (size_t)no * nt * sizeof(double);
+    while (nsplit < 64 && (long long)n_wtiles * nsplit < (long long)kCullWaves * 4 * ctx->num_cus &&
+           (size_t)(2 * nsplit) * split_bytes <= kPartialCap && ns >= 2 * nsplit * CULL_TILE)
+      nsplit *= 2;
   } else if (ns > 0) {
     const size_t split_bytes = (size_t)no * nt * sizeof(double);
     size_t cap = std::min<size_t>(4096, kPartialCap / split_bytes);
@@ -711,6 +749,14 @@ int run_pair_sum(lpm_ctx* ctx, const PairProblem& pp) {
     if (far) {
       hipLaunchKernelGGL(far_fn, grid, block, 0, ctx->stream, tb.p, sb.p, pb.as<double>(), tballs, sballs, tgt_order,
                          a);
+    } else if (cull) {
+      // records of the scaled kinds hold separations in units of eps / sqrt(log2 e)
+      // (FP32) or eps (FP64); SWE records are unscaled
+      const double unit = kind == LPM_K_SWE_PLANE ? 1.0 / std::sqrt(pa.aux) : 1.0;
+      CullArgs ca{tb.p, sb.p, pb.as<double>(), tballs, sballs, pp.tx ? nullptr : tgt_order, nt, ns, nsplit,
+                  n_wtiles, (ns + CULL_TILE - 1) / CULL_TILE,
+                  (float)(std::sqrt(fp32 ? (double)CULL_Q32 : CULL_Q64) * unit)};
+      hipLaunchKernelGGL(cull_fn, grid, block, 0, ctx->stream, tb.p, sb.p, pb.as<double>(), ca);
     } else
       hipLaunchKernelGGL(fn, grid, block, 0, ctx->stream, a);
     LPM_HIP(ctx, hipGetLastError());

@@ -10,6 +10,7 @@
 // (PSEDirectSum.f90:180-418, 537-579).
 #include <math.h>
 
+#include "cull_kernels.hpp"
 #include "lpm_internal.hpp"
 #include "pair_kernels.hpp"
 
@@ -87,7 +88,7 @@ template <typename T, int KIND>
 __global__ __launch_bounds__(256) void ops_pack_targets(PackArgs a, Vec4<T>* __restrict__ rec) {
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= a.count) return;
-  const int p = a.i0 + i;
+  const int p = a.tgt_order ? a.tgt_order[i] : a.i0 + i;
   const double x = a.x[p], y = a.y[p];
   Vec4<T> t{(T)0, (T)0, (T)0, (T)0};
   if constexpr (sphere_kind(KIND)) {
@@ -124,14 +125,14 @@ __global__ __launch_bounds__(256) void ops_finalize(FinArgs f) {
 #pragma unroll
     for (int k = 0; k < NO; ++k) A[k] += ps[(size_t)k * f.nt + i];
   }
-  const int p = f.i0 + i;
+  const int p = f.tgt_order ? f.tgt_order[i] : f.i0 + i;
   if constexpr (KIND == LPM_K_PSE_INTERP_PLANE || KIND == LPM_K_PSE_INTERP_SPHERE) {
     f.out0[p] = A[0] * f.scale;
   } else if constexpr (KIND == LPM_K_SWE_PLANE) {
     f.out0[p] = A[0];
     f.out1[p] = A[1];
-    f.out2[p] = A[2] * A[2] + 2.0 * A[3] * A[4] + A[5] * A[5];
-    f.out3[p] = A[6] * f.scale;
+    f.out2[p] = 2.0 * (A[2] * A[2] + A[3] * A[3]);  // ux^2 + 2 uy vx + vy^2 with uy = vx, vy = -ux
+    f.out3[p] = A[4] * f.scale;
   } else {
     constexpr int Dm = KIND == LPM_K_PSE_DERIV_SPHERE ? 3 : 2;
     constexpr int M = NO / Dm - 1;
@@ -229,6 +230,29 @@ KernelFn pick_t(int kind, int r, int m, bool series) {
   }
 }
 
+// One wave per 64 targets: with 128 the ball around them reaches more source tiles
+// than the sources' scalar loads, shared by twice the targets, give back.
+template <typename T>
+CullFn pick_cull(int kind, int m, bool series) {
+  switch (kind) {
+    case LPM_K_PSE_DERIV_PLANE:
+      if (m == 1) return cull_sum_kernel<PseDeriv<T, false, 1, false>, void, T, 1>;
+      return cull_sum_kernel<PseDeriv<T, false, 2, false>, void, T, 1>;
+    case LPM_K_PSE_DERIV_SPHERE:
+      if (series)
+        return m == 1 ? cull_sum_kernel<PseDeriv<T, true, 1, true>, void, T, 1>
+                      : cull_sum_kernel<PseDeriv<T, true, 3, true>, void, T, 1>;
+      return m == 1 ? cull_sum_kernel<PseDeriv<T, true, 1, false>, void, T, 1>
+                    : cull_sum_kernel<PseDeriv<T, true, 3, false>, void, T, 1>;
+    case LPM_K_PSE_INTERP_PLANE: return cull_sum_kernel<PseInterp<T, false, false>, void, T, 1>;
+    case LPM_K_PSE_INTERP_SPHERE:
+      return series ? cull_sum_kernel<PseInterp<T, true, true>, void, T, 1>
+                    : cull_sum_kernel<PseInterp<T, true, false>, void, T, 1>;
+    case LPM_K_SWE_PLANE: return cull_sum_kernel<SwePlane<T, true>, SwePlane<T, false>, T, 1>;
+    default: return nullptr;
+  }
+}
+
 template <typename T>
 void pack_t(int kind, int nw, const PackArgs& as, const PackArgs& at, void* srec, void* trec, int ns, int nt,
             hipStream_t st) {
@@ -259,7 +283,7 @@ int ops_nout(int kind, int m) {
   switch (kind) {
     case LPM_K_PSE_DERIV_PLANE: return 2 * (m + 1);
     case LPM_K_PSE_DERIV_SPHERE: return 3 * (m + 1);
-    case LPM_K_SWE_PLANE: return 7;
+    case LPM_K_SWE_PLANE: return 5;
     default: return 1;
   }
 }
@@ -272,6 +296,11 @@ int ops_record_words(int kind, int m) {
 const void* ops_pick_kernel(int kind, int prec, int r, int m, bool series) {
   KernelFn fn = prec == LPM_PREC_FP32_KAHAN ? pick_t<float>(kind, r, m, series) : pick_t<double>(kind, r, m, series);
   return reinterpret_cast<const void*>(fn);
+}
+
+const void* ops_pick_cull(int kind, int prec, int m, bool series) {
+  return reinterpret_cast<const void*>(prec == LPM_PREC_FP32_KAHAN ? pick_cull<float>(kind, m, series)
+                                                                   : pick_cull<double>(kind, m, series));
 }
 
 void ops_launch_pack(int kind, int prec, const PackArgs& s, const PackArgs& t, void* srec, void* trec, int ns,
@@ -303,7 +332,7 @@ int ops_launch_finalize(int kind, int m, const FinArgs& f, hipStream_t st) {
   else if (kind == LPM_K_PSE_INTERP_SPHERE)
     hipLaunchKernelGGL((ops_finalize<LPM_K_PSE_INTERP_SPHERE, 1, 0>), g, b, 0, st, f);
   else if (kind == LPM_K_SWE_PLANE)
-    hipLaunchKernelGGL((ops_finalize<LPM_K_SWE_PLANE, 7, 0>), g, b, 0, st, f);
+    hipLaunchKernelGGL((ops_finalize<LPM_K_SWE_PLANE, 5, 0>), g, b, 0, st, f);
   else
     return LPM_ERR_ARG;  // no epilogue for this kind / field count / operator
   return LPM_OK;

@@ -405,26 +405,28 @@ struct PseInterp {
 };
 
 // Planar shallow-water right-hand side (SWEPlaneSolver.f90:457-538), one pass
-// over the pairs for seven sums: velocity (u, v), velocity gradient
-// (ux, uy, vx, vy) of the point vortices and sources, and the K8 Laplacian of
-// the surface height s = h + bottom.
+// over the pairs for five sums: velocity (u, v) and its x derivative (ux, vx) of
+// the point vortices and sources, and the K8 Laplacian of the surface height
+// s = h + bottom (LAP; left out where its kernel is zero).
 // Source record {x, y, a, b, s A, A, idx, c}: a = zeta A / (2 pi),
 // b = delta A / (2 pi), c = log2(e) / eps^2 (FP32) or 1 / eps^2 (FP64).
-// Target record {x, y, s, .}.  With f = 1 / r^2:
-//   u  += -Y a f + X b f             v  += X a f + Y b f
-//   ux += b f - 2 X (X b - Y a) f^2  uy += -a f - 2 Y (X b - Y a) f^2
-//   vx += a f - 2 X (Y b + X a) f^2  vy += b f - 2 Y (Y b + X a) f^2
+// Target record {x, y, s, .}.  With f = 1 / r^2, p = (X b - Y a) f, q = (Y b + X a) f:
+//   u  += p                      v  += q
+//   ux += f (b - 2 X p)          vx += f (a - 2 X q)
 //   lap += K8'(r^2 c) (s_j - s_i) A_j
-template <typename T>
+// The flow of a pair is analytic away from its source, so uy = vx and vy = -ux
+// for every pair and two of the four gradient sums are enough: 18 instructions
+// per pair without the Laplacian against 35 for seven sums with it.
+template <typename T, bool LAP = true>
 struct SwePlane {
-  static constexpr int NOUT = 7;
+  static constexpr int NOUT = 5;
   static constexpr int IDX = 6;
   static constexpr int NW = SREC;
   __device__ __forceinline__ static void arg(const Vec4<T>& t, const T* s, W4<T>& w) {
     w.a = t.a - s[0];
     w.b = t.b - s[1];
     w.z = fma(w.a, w.a, w.b * w.b);
-    w.c = fma(-t.c, s[5], s[4]);  // (s_j - s_i) A_j
+    if constexpr (LAP) w.c = fma(-t.c, s[5], s[4]);  // (s_j - s_i) A_j
   }
   __device__ __forceinline__ static T trans(const W4<T>& w) {
     if constexpr (sizeof(T) == 4)
@@ -434,18 +436,17 @@ struct SwePlane {
   }
   __device__ __forceinline__ static void acc(const T* s, const W4<T>& w, T f, T a[NOUT]) {
     const T X = w.a, Y = w.b;
-    const T rot = s[2] * f, pot = s[3] * f;
-    a[0] = fma(X, pot, fma(-Y, rot, a[0]));
-    a[1] = fma(Y, pot, fma(X, rot, a[1]));
-    const T hh = (f + f) * f;
-    const T p1 = fma(X, s[3], -Y * s[2]) * hh;
-    const T p2 = fma(Y, s[3], X * s[2]) * hh;
-    a[2] = fma(-X, p1, a[2] + pot);
-    a[3] = fma(-Y, p1, a[3] - rot);
-    a[4] = fma(-X, p2, a[4] + rot);
-    a[5] = fma(-Y, p2, a[5] + pot);
-    const T q = w.z * s[7];
-    a[6] = fma(cubic_in_q(q, 40.0, -40.0, 10.0, -2.0 / 3.0) * exp_neg_q(q), w.c, a[6]);
+    const T p = fma(X, s[3], -Y * s[2]) * f;
+    const T q = fma(Y, s[3], X * s[2]) * f;
+    const T X2 = X + X;
+    a[0] += p;
+    a[1] += q;
+    a[2] = fma(f, fma(-X2, p, s[3]), a[2]);
+    a[3] = fma(f, fma(-X2, q, s[2]), a[3]);
+    if constexpr (LAP) {
+      const T qq = w.z * s[7];
+      a[4] = fma(cubic_in_q(qq, 40.0, -40.0, 10.0, -2.0 / 3.0) * exp_neg_q(qq), w.c, a[4]);
+    }
   }
 };
 

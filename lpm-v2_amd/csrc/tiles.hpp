@@ -1,6 +1,6 @@
 // tiles.hpp -- bounding balls of tiles of consecutive records.
 //
-// The tile paths (far_kernels.hpp) choose a tile's treatment from
+// The tile paths (far_kernels.hpp, cull_kernels.hpp) choose a tile's treatment from
 // two balls, one around its sources and one around a wave's or block's targets.
 // With the records in spatial order (lpm_order.hip) the balls are small.
 #pragma once

@@ -170,3 +170,82 @@ def test_far_tiles_batch(ctx, graph):
         assert rel_err_max((ga["x"], ga["y"], ga["z"]), (gb["x"], gb["y"], gb["z"])) < TOL32
     for s in (a, b, c):
         s.delete()
+
+
+# ------------------------------------------------------- culled PSE and SWE sums
+def _ops(ctx, x, y, z, f, area, act, eps, prec, **kw):
+    """PSE calls on the plane (z None) or the sphere: name -> (kind, call)."""
+    if z is None:
+        u, v = np.sin(2 * y) + x, np.cos(x) * y
+        return {
+            "pse8": (L.K_PSE8, lambda: ctx.pse_plane_laplacian(x, y, f, area, act, eps, order=8, precision=prec, **kw)),
+            "pse2": (L.K_PSE2, lambda: ctx.pse_plane_laplacian(x, y, f, area, act, eps, order=2, precision=prec, **kw)),
+            "gradient": (L.K_PSE_DERIV_PLANE, lambda: ctx.pse_plane_gradient(x, y, f, area, act, eps, precision=prec,
+                                                                             **kw)),
+            "second": (L.K_PSE_DERIV_PLANE, lambda: ctx.pse_plane_second_partials(x, y, u, v, area, act, eps,
+                                                                                  precision=prec, **kw)),
+            "interpolate": (L.K_PSE_INTERP_PLANE, lambda: ctx.pse_plane_interpolate(
+                x, y, f, area, act, eps, 0.9 * x[::2] + 1e-3, 0.9 * y[::2], precision=prec)),
+            "swe": (L.K_SWE_PLANE, lambda: ctx.swe_plane_rhs(x, y, f, 0.2 * f, 1.0 + 0.1 * x, 0.05 * y, area, act, eps,
+                                                             precision=prec, **kw)),
+        }
+    return {
+        "laplacian": (L.K_PSE_SPHERE8, lambda: ctx.pse_sphere_laplacian(x, y, z, f, area, act, eps, precision=prec,
+                                                                        **kw)),
+        "gradient": (L.K_PSE_DERIV_SPHERE, lambda: ctx.pse_sphere_gradient(x, y, z, f, area, act, eps, precision=prec,
+                                                                           **kw)),
+        "divergence": (L.K_PSE_DERIV_SPHERE, lambda: ctx.pse_sphere_divergence(x, y, z, y * z, x * x, z, area, act, eps,
+                                                                               precision=prec, **kw)),
+        "interpolate": (L.K_PSE_INTERP_SPHERE, lambda: ctx.pse_sphere_interpolate(x, y, z, f, area, act, eps, y[::3],
+                                                                                  z[::3], x[::3], precision=prec)),
+    }
+
+
+# The terms are the all-pairs kernel's; only their order of summation differs: FP64
+# to 1e-11 of the largest value, FP32 to 5e-5 (the bar of the forced shapes).
+CULL_TOL = {"fp64": 1e-11, "fp32": 5e-5}
+
+
+@pytest.mark.parametrize("prec", ["fp64", "fp32"])
+@pytest.mark.parametrize("eps_h", [0.7, 2.0, 9.0])
+def test_culled_plane_sums(ctx, prec, eps_h):
+    """Kernel widths from under the spacing to the whole domain, a shuffled grid with
+    passive particles and a block of targets."""
+    x, y, area, h = mesh.grid_centres(131, 1.0, jitter=1e-3, seed=3)
+    rng = np.random.default_rng(9)
+    idx = rng.permutation(x.size)
+    x, y, area = x[idx], y[idx], area[idx]
+    f = np.exp(-4.0 * (x * x + y * y)) + 0.3 * x
+    act = (rng.uniform(size=x.size) < 0.93).astype(np.int32)
+    for kw in ({}, {"i0": 333, "i1": x.size - 70}):
+        for name, (kind, call) in _ops(ctx, x, y, None, f, area, act, eps_h * h, prec, **kw).items():
+            for g, r in zip(_rows(call()), _all_pairs(ctx, kind, prec, call)):
+                assert rel_err_max(g, r) <= CULL_TOL[prec], (name, kw)
+
+
+@pytest.mark.parametrize("prec", ["fp64", "fp32"])
+@pytest.mark.parametrize("eps", [0.01, 0.04])
+def test_culled_sphere_sums(ctx, prec, eps):
+    m = mesh.icosahedral_mesh(5)
+    f = np.sin(3 * m.x) * m.y + m.z
+    for name, (kind, call) in _ops(ctx, m.x, m.y, m.z, f, m.area, m.active, eps, prec).items():
+        for g, r in zip(_rows(call()), _all_pairs(ctx, kind, prec, call)):
+            assert rel_err_max(g, r) <= 4 * CULL_TOL[prec], name
+
+
+@pytest.mark.parametrize("prec", ["fp64", "fp32"])
+@pytest.mark.parametrize("bad", [np.inf, np.nan])
+@pytest.mark.parametrize("where", ["source", "target"])
+def test_culled_sums_spread_non_finite_values_like_all_pairs(ctx, prec, bad, where):
+    x, y, area, h = mesh.grid_centres(120, 1.0, jitter=1e-3, seed=3)
+    f = np.exp(-4.0 * (x * x + y * y))
+    act = np.ones(x.size, np.int32)
+    j = 7000
+    if where == "target":
+        act[j] = 0
+    f[j] = bad
+    for name, (kind, call) in _ops(ctx, x, y, None, f, area, act, 2 * h, prec).items():
+        if name == "second":
+            continue  # does not read f
+        for g, r in zip(_rows(call()), _all_pairs(ctx, kind, prec, call)):
+            assert np.array_equal(np.isfinite(g), np.isfinite(r)), name
