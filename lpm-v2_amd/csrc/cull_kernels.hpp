@@ -94,6 +94,7 @@ template <class P, class FAR, typename T, int R>
 static __global__ __launch_bounds__(256) void cull_sum_kernel(const void* __restrict__ tgt,
                                                               const void* __restrict__ srcv,
                                                               double* __restrict__ partial, CullArgs a) {
+  fill_tables<P::TABLE>();
   constexpr int NO = P::NOUT;
   const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
   const int nblk_t = (a.n_wtiles + 3) >> 2;

@@ -197,8 +197,9 @@ struct FinArgs {
 bool is_ops_kind(int kind);
 int ops_nout(int kind, int m);
 int ops_record_words(int kind, int m);
-const void* ops_pick_kernel(int kind, int prec, int r, int m, bool series);
-const void* ops_pick_cull(int kind, int prec, int m, bool series);
+// series: terms of the sphere distance series, 0 by asin
+const void* ops_pick_kernel(int kind, int prec, int r, int m, int series);
+const void* ops_pick_cull(int kind, int prec, int m, int series);
 void ops_launch_pack(int kind, int prec, const PackArgs& s, const PackArgs& t, void* srec, void* trec, int ns,
                      int nt, hipStream_t st);
 int ops_launch_finalize(int kind, int m, const FinArgs& f, hipStream_t st);

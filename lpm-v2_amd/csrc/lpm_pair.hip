@@ -273,9 +273,18 @@ static KernelFn pick_r(int r) {
 }
 
 // variant: sphere kinds, targets on the sphere (no e terms); sphere PSE, the
-// series form of the distance (FP32 only)
-static KernelFn pick_kernel(int kind, int prec, int r, bool variant) {
-  const bool on_sphere = variant;
+// terms of the series form of the distance (0: by asin)
+template <typename T>
+static KernelFn pick_pse_sphere(int r, int series) {
+  constexpr bool F = sizeof(T) == 4;
+  if (series == 0) return pick_r<PseSphere<T, 0>, T>(r);
+  if (series <= (F ? 7 : 10)) return pick_r<PseSphere<T, F ? 7 : 10>, T>(r);
+  if (series <= (F ? 14 : 16)) return pick_r<PseSphere<T, F ? 14 : 16>, T>(r);
+  return pick_r<PseSphere<T, F ? 14 : 28>, T>(r);
+}
+
+static KernelFn pick_kernel(int kind, int prec, int r, int variant) {
+  const bool on_sphere = variant != 0;
   if (prec == LPM_PREC_FP32_KAHAN) {
     switch (kind) {
       case LPM_K_SPHERE_BS:
@@ -284,7 +293,7 @@ static KernelFn pick_kernel(int kind, int prec, int r, bool variant) {
       case LPM_K_PSE8: return pick_r<PsePolicy<float, 8>, float>(r);
       case LPM_K_PSE2: return pick_r<PsePolicy<float, 2>, float>(r);
       case LPM_K_PSE_SPHERE8:
-        return variant ? pick_r<PseSphere<float, true>, float>(r) : pick_r<PseSphere<float, false>, float>(r);
+        return pick_pse_sphere<float>(r, variant);
       case LPM_K_SPHERE_GREEN:
         return on_sphere ? pick_r<SphereGreen<float, false>, float>(r) : pick_r<SphereGreen<float, true>, float>(r);
       default: return pick_r<PlaneGreen<float>, float>(r);
@@ -297,7 +306,7 @@ static KernelFn pick_kernel(int kind, int prec, int r, bool variant) {
     case LPM_K_PSE8: return pick_r<PsePolicy<double, 8>, double>(r);
     case LPM_K_PSE2: return pick_r<PsePolicy<double, 2>, double>(r);
     case LPM_K_PSE_SPHERE8:
-      return variant ? pick_r<PseSphere<double, true>, double>(r) : pick_r<PseSphere<double, false>, double>(r);
+      return pick_pse_sphere<double>(r, variant);
     case LPM_K_SPHERE_GREEN:
       return on_sphere ? pick_r<SphereGreen<double, false>, double>(r) : pick_r<SphereGreen<double, true>, double>(r);
     default: return pick_r<PlaneGreen<double>, double>(r);
@@ -457,23 +466,30 @@ static FarFn pick_far(int kind, bool on_sphere) {
 }
 
 // PSE Laplacians without their zero tiles; the other PSE kinds: ops_pick_cull.
-static CullFn pick_cull(int kind, int prec, int m, bool series) {
+template <typename T>
+static CullFn pick_cull_sphere(int series) {
+  constexpr bool F = sizeof(T) == 4;
+  if (series == 0) return cull_sum_kernel<PseSphere<T, 0>, void, T, 1>;
+  if (series <= (F ? 7 : 10)) return cull_sum_kernel<PseSphere<T, F ? 7 : 10>, void, T, 1>;
+  if (series <= (F ? 14 : 16)) return cull_sum_kernel<PseSphere<T, F ? 14 : 16>, void, T, 1>;
+  return cull_sum_kernel<PseSphere<T, F ? 14 : 28>, void, T, 1>;
+}
+
+static CullFn pick_cull(int kind, int prec, int m, int series) {
   if (is_ops_kind(kind)) return reinterpret_cast<CullFn>(const_cast<void*>(ops_pick_cull(kind, prec, m, series)));
   if (prec == LPM_PREC_FP32_KAHAN) {
     switch (kind) {
       case LPM_K_PSE8: return cull_sum_kernel<PsePolicy<float, 8>, void, float, 1>;
       case LPM_K_PSE2: return cull_sum_kernel<PsePolicy<float, 2>, void, float, 1>;
       default:
-        return series ? cull_sum_kernel<PseSphere<float, true>, void, float, 1>
-                      : cull_sum_kernel<PseSphere<float, false>, void, float, 1>;
+        return pick_cull_sphere<float>(series);
     }
   }
   switch (kind) {
     case LPM_K_PSE8: return cull_sum_kernel<PsePolicy<double, 8>, void, double, 1>;
     case LPM_K_PSE2: return cull_sum_kernel<PsePolicy<double, 2>, void, double, 1>;
     default:
-      return series ? cull_sum_kernel<PseSphere<double, true>, void, double, 1>
-                    : cull_sum_kernel<PseSphere<double, false>, void, double, 1>;
+      return pick_cull_sphere<double>(series);
   }
 }
 
@@ -570,6 +586,12 @@ int collect_timing(lpm_ctx* ctx) {
   return LPM_OK;
 }
 
+// Terms of the sphere PSE distance series that reach `angle` (see PseSphere).
+static int series_terms(bool fp32, double angle) {
+  if (fp32) return angle <= 0.56 ? 7 : angle <= 1.2 ? 14 : 0;
+  return angle <= 0.35 ? 10 : angle <= 0.70 ? 16 : angle <= 1.16 ? 28 : 0;
+}
+
 int run_pair_sum(lpm_ctx* ctx, const PairProblem& pp) {
   const int kind = pp.kind;
   const int prec = pp.precision;
@@ -621,12 +643,9 @@ int run_pair_sum(lpm_ctx* ctx, const PairProblem& pp) {
   const int t_tile = far ? FAR_TILE : 64, s_tile = far ? FAR_TILE : CULL_TILE;
   const int per_wave = path != kAllPairs ? 64 : 64 * tu.r;
   const int n_wtiles = (nt + per_wave - 1) / per_wave;
-  // sphere PSE kinds: the series form of the distance when 7 eps <= 0.56 R
-  // (FP32, 7 terms) or 7 eps <= 0.35 R (FP64, 10 terms)
   const bool sphere_pse = kind == LPM_K_PSE_SPHERE8 || kind == LPM_K_PSE_DERIV_SPHERE ||
                           kind == LPM_K_PSE_INTERP_SPHERE;
-  const double series_reach = prec == LPM_PREC_FP32_KAHAN ? 0.56 : 0.35;
-  const bool variant = sphere_pse ? (7.0 * pp.eps <= series_reach * pp.radius) : pp.on_sphere;
+  const int variant = sphere_pse ? series_terms(fp32, 7.0 * pp.eps / pp.radius) : pp.on_sphere ? 1 : 0;
   FarFn far_fn = far ? pick_far(kind, pp.on_sphere) : nullptr;
   CullFn cull_fn = cull ? pick_cull(kind, prec, pp.m, variant) : nullptr;
   KernelFn fn = far ? reinterpret_cast<KernelFn>(far_fn) : ops ? reinterpret_cast<KernelFn>(const_cast<void*>(ops_pick_kernel(kind, prec, tu.r, pp.m, variant)))

@@ -205,26 +205,29 @@ KernelFn pick_r(int r) {
   }
 }
 
+template <typename T, int SERIES>
+KernelFn pick_sphere(int kind, int r, int m) {
+  if (kind == LPM_K_PSE_INTERP_SPHERE) return pick_r<PseInterp<T, true, SERIES>, T>(r);
+  if (m == 1) return pick_r<PseDeriv<T, true, 1, SERIES>, T>(r);
+  if (m == 3) return pick_r<PseDeriv<T, true, 3, SERIES>, T>(r);
+  return nullptr;
+}
+
 template <typename T>
-KernelFn pick_t(int kind, int r, int m, bool series) {
+KernelFn pick_t(int kind, int r, int m, int series) {
+  constexpr bool F = sizeof(T) == 4;
   switch (kind) {
     case LPM_K_PSE_DERIV_PLANE:
-      if (m == 1) return pick_r<PseDeriv<T, false, 1, false>, T>(r);
-      if (m == 2) return pick_r<PseDeriv<T, false, 2, false>, T>(r);
+      if (m == 1) return pick_r<PseDeriv<T, false, 1, 0>, T>(r);
+      if (m == 2) return pick_r<PseDeriv<T, false, 2, 0>, T>(r);
       return nullptr;
     case LPM_K_PSE_DERIV_SPHERE:
-      if (series) {
-        if (m == 1) return pick_r<PseDeriv<T, true, 1, true>, T>(r);
-        if (m == 3) return pick_r<PseDeriv<T, true, 3, true>, T>(r);
-        return nullptr;
-      }
-      if (m == 1) return pick_r<PseDeriv<T, true, 1, false>, T>(r);
-      if (m == 3) return pick_r<PseDeriv<T, true, 3, false>, T>(r);
-      return nullptr;
-    case LPM_K_PSE_INTERP_PLANE: return pick_r<PseInterp<T, false, false>, T>(r);
     case LPM_K_PSE_INTERP_SPHERE:
-      if (series) return pick_r<PseInterp<T, true, true>, T>(r);
-      return pick_r<PseInterp<T, true, false>, T>(r);
+      if (series == 0) return pick_sphere<T, 0>(kind, r, m);
+      if (series <= (F ? 7 : 10)) return pick_sphere<T, F ? 7 : 10>(kind, r, m);
+      if (series <= (F ? 14 : 16)) return pick_sphere<T, F ? 14 : 16>(kind, r, m);
+      return pick_sphere<T, F ? 14 : 28>(kind, r, m);
+    case LPM_K_PSE_INTERP_PLANE: return pick_r<PseInterp<T, false, 0>, T>(r);
     case LPM_K_SWE_PLANE: return pick_r<SwePlane<T>, T>(r);
     default: return nullptr;
   }
@@ -232,22 +235,27 @@ KernelFn pick_t(int kind, int r, int m, bool series) {
 
 // One wave per 64 targets: with 128 the ball around them reaches more source tiles
 // than the sources' scalar loads, shared by twice the targets, give back.
+template <typename T, int SERIES>
+CullFn cull_sphere(int kind, int m) {
+  if (kind == LPM_K_PSE_INTERP_SPHERE) return cull_sum_kernel<PseInterp<T, true, SERIES>, void, T, 1>;
+  return m == 1 ? cull_sum_kernel<PseDeriv<T, true, 1, SERIES>, void, T, 1>
+                : cull_sum_kernel<PseDeriv<T, true, 3, SERIES>, void, T, 1>;
+}
+
 template <typename T>
-CullFn pick_cull(int kind, int m, bool series) {
+CullFn pick_cull(int kind, int m, int series) {
+  constexpr bool F = sizeof(T) == 4;
   switch (kind) {
     case LPM_K_PSE_DERIV_PLANE:
-      if (m == 1) return cull_sum_kernel<PseDeriv<T, false, 1, false>, void, T, 1>;
-      return cull_sum_kernel<PseDeriv<T, false, 2, false>, void, T, 1>;
+      if (m == 1) return cull_sum_kernel<PseDeriv<T, false, 1, 0>, void, T, 1>;
+      return cull_sum_kernel<PseDeriv<T, false, 2, 0>, void, T, 1>;
     case LPM_K_PSE_DERIV_SPHERE:
-      if (series)
-        return m == 1 ? cull_sum_kernel<PseDeriv<T, true, 1, true>, void, T, 1>
-                      : cull_sum_kernel<PseDeriv<T, true, 3, true>, void, T, 1>;
-      return m == 1 ? cull_sum_kernel<PseDeriv<T, true, 1, false>, void, T, 1>
-                    : cull_sum_kernel<PseDeriv<T, true, 3, false>, void, T, 1>;
-    case LPM_K_PSE_INTERP_PLANE: return cull_sum_kernel<PseInterp<T, false, false>, void, T, 1>;
     case LPM_K_PSE_INTERP_SPHERE:
-      return series ? cull_sum_kernel<PseInterp<T, true, true>, void, T, 1>
-                    : cull_sum_kernel<PseInterp<T, true, false>, void, T, 1>;
+      if (series == 0) return cull_sphere<T, 0>(kind, m);
+      if (series <= (F ? 7 : 10)) return cull_sphere<T, F ? 7 : 10>(kind, m);
+      if (series <= (F ? 14 : 16)) return cull_sphere<T, F ? 14 : 16>(kind, m);
+      return cull_sphere<T, F ? 14 : 28>(kind, m);
+    case LPM_K_PSE_INTERP_PLANE: return cull_sum_kernel<PseInterp<T, false, 0>, void, T, 1>;
     case LPM_K_SWE_PLANE: return cull_sum_kernel<SwePlane<T, true>, SwePlane<T, false>, T, 1>;
     default: return nullptr;
   }
@@ -293,12 +301,12 @@ int ops_record_words(int kind, int m) {
   return SREC;
 }
 
-const void* ops_pick_kernel(int kind, int prec, int r, int m, bool series) {
+const void* ops_pick_kernel(int kind, int prec, int r, int m, int series) {
   KernelFn fn = prec == LPM_PREC_FP32_KAHAN ? pick_t<float>(kind, r, m, series) : pick_t<double>(kind, r, m, series);
   return reinterpret_cast<const void*>(fn);
 }
 
-const void* ops_pick_cull(int kind, int prec, int m, bool series) {
+const void* ops_pick_cull(int kind, int prec, int m, int series) {
   return reinterpret_cast<const void*>(prec == LPM_PREC_FP32_KAHAN ? pick_cull<float>(kind, m, series)
                                                                    : pick_cull<double>(kind, m, series));
 }

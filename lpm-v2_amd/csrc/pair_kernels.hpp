@@ -47,54 +47,111 @@ struct Vec4 {
 };
 
 __device__ __forceinline__ float fast_rcp(float x) { return __builtin_amdgcn_rcpf(x); }
-// FP64 reciprocal: the hardware estimate (v_rcp_f64) refined by two
-// Newton-Raphson steps r <- r + r (1 - x r), each of which squares the
-// relative error, so the result is within an ulp or two of the correctly
-// rounded 1 / x for normal x.  Five instructions against about ten for the
-// IEEE division sequence; x = 0 gives NaN instead of inf, which the pair
-// sums multiply by a zero separation either way.
+// FP64 reciprocal: the hardware estimate r (v_rcp_f64, 2^-24.4) with the error
+// e = 1 - x r taken out to third order, r (1 + e + e^2): what is left is e^3, 2^-73, so
+// the result is within an ulp of the correctly rounded 1 / x for normal x.  Four
+// instructions, against five for two Newton steps and about ten for the IEEE division
+// sequence; x = 0 gives NaN instead of inf, which the pair sums multiply by a zero
+// separation either way.
 __device__ __forceinline__ double rcp_refined(double x) {
-  double r = __builtin_amdgcn_rcp(x);
-  double e = fma(-x, r, 1.0);
-  r = fma(r, e, r);
-  e = fma(-x, r, 1.0);
-  return fma(r, e, r);
+  const double r = __builtin_amdgcn_rcp(x);
+  const double e = fma(-x, r, 1.0);
+  return fma(r, fma(e, e, e), r);
 }
-// FP64 natural logarithm for the Green's-function sums.  x = m 2^e with m in
-// [sqrt(1/2), sqrt(2)); log m = 2 atanh(s) = 2 (s + s^3/3 + ... + s^21/21),
-// s = (m - 1) / (m + 1), |s| <= 0.1716, so the first dropped term is below
-// 1e-18 relative; e ln 2 uses ln 2 split into a 32-bit head (exact products
-// for |e| < 2^21) and its tail.  Within 2 ulp of the correctly rounded log
-// for positive normal x (the same steps against the C library's log on
-// 1.2e6 arguments from 1e-13 to 7.4); about 30 instructions against ~80 for
-// the library's double-double evaluation.  Zero gives a finite value, not
-// -inf: the pair sums only meet it in the self pair, which they discard.
-__device__ __forceinline__ double log_fp64(double x) {
-  constexpr double kLn2Hi = 0.6931471803691238;      // ln 2 to 32 significant bits
-  constexpr double kLn2Lo = 1.9082149292705877e-10;  // ln 2 - kLn2Hi
-  double m = __builtin_amdgcn_frexp_mant(x);         // [0.5, 1)
-  int e = __builtin_amdgcn_frexp_exp(x);
-  if (m < 0.70710678118654752440) {
-    m *= 2.0;
-    --e;
+// FP64 exponential and logarithm by table.  The FP64 vector rate is 4.6 cycles per
+// instruction and SIMD, so the sums below are bound by the length of these: a table
+// entry from LDS (512 or 2,048 bytes, filled once per block) takes the place of half
+// of the polynomial.  All pairs at icosahedral L6: Green sum 11.8 -> 8.1 ms; PSE-8 at
+// 256^2: 3.6 -> 3.0 ms.  Kernels whose policy names a TABLE call fill_tables first.
+enum Table { kNoTable = 0, kExpTable = 1, kLogTable = 2 };
+constexpr int kExpBits = 6;  // 2^(i / 64)
+constexpr int kLogBits = 7;  // {c_i, -log c_i}, c_i near 1 / m in the i-th 128th of [0.70, 1.41)
+
+__device__ __forceinline__ double* exp_table() {
+  __shared__ double t[1 << kExpBits];
+  return t;
+}
+struct LogEntry {
+  double c, l;
+};
+__device__ __forceinline__ LogEntry* log_table() {
+  __shared__ LogEntry t[1 << kLogBits];
+  return t;
+}
+
+// High word of the lower end of the mantissa interval, about sqrt(1/2).
+constexpr unsigned kLogLow = 0x3fe66000u;
+
+template <int TABLE>
+__device__ __forceinline__ void fill_tables() {
+  if constexpr (TABLE == kExpTable) {
+    if (threadIdx.x < (1 << kExpBits)) exp_table()[threadIdx.x] = exp2(threadIdx.x / (double)(1 << kExpBits));
+    __syncthreads();
+  } else if constexpr (TABLE == kLogTable) {
+    if (threadIdx.x < (1 << kLogBits)) {
+      // the interval's middle; c has 9 bits so that c is exact in the product below,
+      // and is 1 next to m = 1, where log m = log1p(m - 1) must not lose its own digits
+      const unsigned step = 1u << (20 - kLogBits);
+      const unsigned lo = kLogLow + threadIdx.x * step;
+      const double m = __hiloint2double((int)(lo + step / 2), 0);
+      const double m0 = __hiloint2double((int)lo, 0), m1 = __hiloint2double((int)(lo + step), 0);
+      double c = rint(512.0 / m) / 512.0;
+      if (m0 <= 1.0 && 1.0 <= m1) c = 1.0;
+      log_table()[threadIdx.x] = LogEntry{c, c == 1.0 ? 0.0 : -log(c)};
+    }
+    __syncthreads();
   }
-  const double f = m - 1.0;  // exact (Sterbenz)
-  const double s = f * rcp_refined(m + 1.0);
-  const double z = s * s;
-  double p = 1.0 / 21.0;
-  p = fma(p, z, 1.0 / 19.0);
-  p = fma(p, z, 1.0 / 17.0);
-  p = fma(p, z, 1.0 / 15.0);
-  p = fma(p, z, 1.0 / 13.0);
-  p = fma(p, z, 1.0 / 11.0);
-  p = fma(p, z, 1.0 / 9.0);
-  p = fma(p, z, 1.0 / 7.0);
-  p = fma(p, z, 1.0 / 5.0);
-  p = fma(p, z, 1.0 / 3.0);
-  const double s2 = 2.0 * s;
-  const double lm = fma(s2 * z, p, s2);
-  const double de = (double)e;
-  return fma(de, kLn2Hi, fma(de, kLn2Lo, lm));
+}
+
+// exp(-q) for q >= 0: -q = (64 e + i) ln 2 / 64 + r, |r| <= ln 2 / 128, and
+// exp r = 1 + r + ... + r^6 / 720 (first dropped term 2e-19); within an ulp of the
+// correctly rounded value, 0 from q = 745.2 as the library's.  12 FP64 and 4 integer
+// instructions against about 26.  NaN gives exp(-800) = 0 unless NAN_SAFE: the
+// polynomial factor of the 8th-order kernels carries it.
+template <bool NAN_SAFE = false>
+__device__ __forceinline__ double exp_neg_fp64(double q) {
+  constexpr double kInv = 92.332482616893656877;        // 64 / ln 2
+  constexpr double kHi = 0.010830424696223417;          // ln 2 / 64, low 14 bits of the mantissa cleared
+  constexpr double kLo = 2.572804622327669e-14;         // ln 2 / 64 - kHi
+  constexpr double kMagic = 6755399441055744.0;         // 1.5 * 2^52: adds to an integer in the low word
+  const double qc = NAN_SAFE ? (q > 800.0 ? 800.0 : q) : fmin(q, 800.0);
+  const double t = fma(qc, -kInv, kMagic);
+  const int n = __double2loint(t);
+  const double k = t - kMagic;
+  double r = fma(k, -kHi, -qc);
+  r = fma(k, -kLo, r);
+  double p = fma(r, 1.0 / 720.0, 1.0 / 120.0);
+  p = fma(r, p, 1.0 / 24.0);
+  p = fma(r, p, 1.0 / 6.0);
+  p = fma(r, p, 0.5);
+  p = fma(r, p, 1.0);
+  const double e = exp_table()[n & ((1 << kExpBits) - 1)];
+  return ldexp(fma(e * r, p, e), n >> kExpBits);
+}
+
+// log x for positive normal x: x = 2^e m with m in [0.70, 1.41), m c_i = 1 + r with
+// |r| < 2^-7 next to 1 and 2^-8 elsewhere, log x = e ln 2 - log c_i + log1p r, the
+// last through r^8 (first dropped term 1e-18 relative).  Within 2 ulp; 14 FP64 and 6
+// integer instructions against about 30 for the atanh series that it replaces.
+// NaN and infinities give NaN; zero a finite value: the pair sums only meet it in the
+// self pair, which they discard.
+__device__ __forceinline__ double log_fp64(double x) {
+  constexpr double kLn2 = 0.69314718055994530942;
+  const unsigned hi = (unsigned)__double2hiint(x);
+  const int d = (int)(hi - kLogLow);
+  const int e = d >> 20;
+  const LogEntry t = log_table()[(d >> (20 - kLogBits)) & ((1 << kLogBits) - 1)];
+  const double m = __hiloint2double((int)(hi - (unsigned)(d & ~0xfffff)), __double2loint(x));
+  const double r = fma(m, t.c, -1.0);
+  const double r2 = r * r;
+  double p = fma(r, -1.0 / 8.0, 1.0 / 7.0);
+  p = fma(r, p, -1.0 / 6.0);
+  p = fma(r, p, 1.0 / 5.0);
+  p = fma(r, p, -1.0 / 4.0);
+  p = fma(r, p, 1.0 / 3.0);
+  p = fma(r, p, -0.5);
+  const double base = fma((double)e, kLn2, t.l);
+  return fma(x, 0.0, base + fma(r2, p, r));
 }
 __device__ __forceinline__ float fast_exp2(float x) { return __builtin_amdgcn_exp2f(x); }
 __device__ __forceinline__ float fast_log2(float x) { return __builtin_amdgcn_logf(x); }
@@ -118,6 +175,7 @@ struct SphereBS {
   static constexpr int NOUT = 3;
   static constexpr int IDX = 5;
   static constexpr int NW = SREC;
+  static constexpr int TABLE = kNoTable;
   // acc += s * (x_i - y_j),  s = w2 / (|x_i - y_j|^2 + e_i + e_j); with
   // USE_E == false the points are on the sphere and e_i = e_j = 0.
   __device__ __forceinline__ static void arg(const Vec4<T>& t, const T* s, W4<T>& w) {
@@ -151,6 +209,7 @@ struct PlaneBS {
   static constexpr int NOUT = 2;
   static constexpr int IDX = 3;
   static constexpr int NW = SREC;
+  static constexpr int TABLE = kNoTable;
   __device__ __forceinline__ static void arg(const Vec4<T>& t, const T* s, W4<T>& w) {
     w.a = t.a - s[0];
     w.b = t.b - s[1];
@@ -177,6 +236,7 @@ struct PsePolicy {
   static constexpr int NOUT = 1;
   static constexpr int IDX = 4;
   static constexpr int NW = SREC;
+  static constexpr int TABLE = sizeof(T) == 8 ? kExpTable : kNoTable;
   __device__ __forceinline__ static void arg(const Vec4<T>& t, const T* s, W4<T>& w) {
     T dx = t.a - s[0], dy = t.b - s[1];
     w.z = fma(dx, dx, dy * dy);
@@ -186,7 +246,7 @@ struct PsePolicy {
     if constexpr (sizeof(T) == 4)
       return fast_exp2(-w.z);
     else
-      return exp(-w.z);
+      return exp_neg_fp64<ORDER == 2>(w.z);
   }
   __device__ __forceinline__ static void acc(const T* s, const W4<T>& w, T e, T a[NOUT]) {
     if constexpr (ORDER == 8) {
@@ -210,37 +270,31 @@ struct PsePolicy {
 // u = |x'_i - x'_j|^2 / (k R)^2 = (c / R)^2 (c the chord) the scaled squared
 // distance is q = (k R)^2 theta^2, theta = 2 asin(sqrt(u) / 2).
 // SERIES: theta^2 = u g(u), g = sum_n a_n u^(n-1), a_n = 2 / (n^2 binom(2n, n))
-// (the Taylor series of 4 asin^2(s / 2)), through n = 7 in FP32 (the caller
-// uses it when 7 eps <= 0.56 R, where the first dropped term is below 4e-9
-// relative) and n = 10 in FP64 (7 eps <= 0.35 R).  Pairs farther than 7 eps
-// get a slightly low theta^2, but their kernel factor exp(-q) is below e^-49.
+// (the Taylor series of 4 asin^2(s / 2)), through n = SERIES; 0: by asin and sqrt.
+// The caller takes the fewest terms that reach 7 eps (series_terms): in FP32 7 terms
+// to 0.56 R and 14 to 1.2 R (first dropped term below 4e-9 relative), in FP64 10 to
+// 0.35 R, 16 to 0.70 R and 28 to 1.16 R (2e-17).  Pairs farther than 7 eps get a
+// slightly low theta^2, but their kernel factor exp(-q) is below e^-49.  The FP64
+// gradient at level 6 (7 eps = 0.40 R) took 39.3 ms over all pairs by asin, 15.1 ms by
+// 16 terms and the table exponential.
 // Source record: {x', y', z', f A, A, idx, 1/(kR)^2, (kR)^2}; target {x', y', z', f}.
 // Scaled squared great-circle distance q = (k R theta)^2 from the squared
 // chord c2 = |x'_i - x'_j|^2 of directions scaled by k R; inv = 1/(k R)^2,
 // kr2 = (k R)^2.
-template <typename T, bool SERIES>
+// Coefficient a_n of theta^2 = u g(u), g = sum a_n u^(n-1).
+constexpr double theta2_coef(int n) {
+  double a = 1.0;
+  for (int k = 1; k < n; ++k) a *= (double)k * k / ((2.0 * k + 2.0) * (2.0 * k + 1.0));
+  return a;
+}
+
+template <typename T, int SERIES>
 __device__ __forceinline__ T sphere_q(T c2, T inv, T kr2) {
   const T u = c2 * inv;
-  if constexpr (SERIES && sizeof(T) == 8) {
-    // FP64: through n = 10; the caller uses it when 7 eps <= 0.35 R, where the
-    // first dropped term is below 2e-17 relative
-    double g = fma(u, 1.0 / 9237800.0, 1.0 / 1969110.0);
-    g = fma(u, g, 1.0 / 411840.0);
-    g = fma(u, g, 1.0 / 84084.0);
-    g = fma(u, g, 1.0 / 16632.0);
-    g = fma(u, g, 1.0 / 3150.0);
-    g = fma(u, g, 1.0 / 560.0);
-    g = fma(u, g, 1.0 / 90.0);
-    g = fma(u, g, 1.0 / 12.0);
-    g = fma(u, g, 1.0);
-    return c2 * g;
-  } else if constexpr (SERIES) {
-    T g = fma(u, (T)(1.0 / 84084.0), (T)(1.0 / 16632.0));
-    g = fma(u, g, (T)(1.0 / 3150.0));
-    g = fma(u, g, (T)(1.0 / 560.0));
-    g = fma(u, g, (T)(1.0 / 90.0));
-    g = fma(u, g, (T)(1.0 / 12.0));
-    g = fma(u, g, (T)1.0);
+  if constexpr (SERIES > 0) {
+    T g = (T)theta2_coef(SERIES);
+#pragma unroll
+    for (int n = SERIES - 1; n >= 1; --n) g = fma(u, g, (T)theta2_coef(n));
     return c2 * g;
   } else {
     const T th = (T)2.0 * asin(fmin((T)0.5 * sqrt(u), (T)1.0));
@@ -248,11 +302,12 @@ __device__ __forceinline__ T sphere_q(T c2, T inv, T kr2) {
   }
 }
 
-template <typename T, bool SERIES>
+template <typename T, int SERIES>
 struct PseSphere {
   static constexpr int NOUT = 1;
   static constexpr int IDX = 5;
   static constexpr int NW = SREC;
+  static constexpr int TABLE = sizeof(T) == 8 ? kExpTable : kNoTable;
   __device__ __forceinline__ static void arg(const Vec4<T>& t, const T* s, W4<T>& w) {
     const T dx = t.a - s[0], dy = t.b - s[1], dz = t.c - s[2];
     const T c2 = fma(dx, dx, fma(dy, dy, dz * dz));
@@ -270,6 +325,7 @@ struct SphereGreen {
   static constexpr int NOUT = 2;
   static constexpr int IDX = 6;
   static constexpr int NW = SREC;
+  static constexpr int TABLE = sizeof(T) == 8 ? kLogTable : kNoTable;
   __device__ __forceinline__ static void arg(const Vec4<T>& t, const T* s, W4<T>& w) {
     T dx = t.a - s[0], dy = t.b - s[1], dz = t.c - s[2];
     T r2;
@@ -297,6 +353,7 @@ struct PlaneGreen {
   static constexpr int NOUT = 1;
   static constexpr int IDX = 3;
   static constexpr int NW = SREC;
+  static constexpr int TABLE = sizeof(T) == 8 ? kLogTable : kNoTable;
   __device__ __forceinline__ static void arg(const Vec4<T>& t, const T* s, W4<T>& w) {
     T dx = t.a - s[0], dy = t.b - s[1];
     w.z = fma(dx, dx, dy * dy);
@@ -328,7 +385,7 @@ __device__ __forceinline__ T exp_neg_q(T q) {
   if constexpr (sizeof(T) == 4)
     return fast_exp2(-q);
   else
-    return exp(-q);
+    return exp_neg_fp64(q);
 }
 
 // PSE first-derivative sums (PSEDirectSum.f90:180-418, 537-579).  For M source
@@ -341,7 +398,7 @@ __device__ __forceinline__ T exp_neg_q(T q) {
 // Source record: plane {x', y', A, c_0 .. c_{M-1}, idx};
 // sphere {x', y', z', A, c_0 .., idx, 1/(kR)^2, (kR)^2} with x' the unit
 // direction times k R (the separation is taken as R (d_i - d_j)).
-template <typename T, bool SPH, int M, bool SERIES>
+template <typename T, bool SPH, int M, int SERIES>
 struct PseDeriv {
   static constexpr int D = SPH ? 3 : 2;
   static constexpr int NOUT = D * (M + 1);
@@ -351,6 +408,7 @@ struct PseDeriv {
   static constexpr int IINV = IDX + 1;
   static constexpr int IKR2 = IDX + 2;
   static constexpr int NW = (SPH ? IKR2 + 1 : IDX + 1) <= SREC ? SREC : SREC_MAX;
+  static constexpr int TABLE = sizeof(T) == 8 ? kExpTable : kNoTable;
   static_assert((SPH ? IKR2 + 1 : IDX + 1) <= SREC_MAX, "record too long");
   __device__ __forceinline__ static void arg(const Vec4<T>& t, const T* s, W4<T>& w) {
     w.a = t.a - s[0];
@@ -382,13 +440,14 @@ struct PseDeriv {
 // PSE interpolation (PSEDirectSum.f90:121-168): sum_j f_j A_j Kd'(q).
 // Source record: plane {x', y', f A, idx}; sphere {x', y', z', f A, idx,
 // 1/(kR)^2, (kR)^2}.
-template <typename T, bool SPH, bool SERIES>
+template <typename T, bool SPH, int SERIES>
 struct PseInterp {
   static constexpr int D = SPH ? 3 : 2;
   static constexpr int NOUT = 1;
   static constexpr int IFA = D;
   static constexpr int IDX = D + 1;
   static constexpr int NW = SREC;
+  static constexpr int TABLE = sizeof(T) == 8 ? kExpTable : kNoTable;
   __device__ __forceinline__ static void arg(const Vec4<T>& t, const T* s, W4<T>& w) {
     const T dx = t.a - s[0], dy = t.b - s[1];
     if constexpr (SPH) {
@@ -422,6 +481,7 @@ struct SwePlane {
   static constexpr int NOUT = 5;
   static constexpr int IDX = 6;
   static constexpr int NW = SREC;
+  static constexpr int TABLE = sizeof(T) == 8 ? kExpTable : kNoTable;
   __device__ __forceinline__ static void arg(const Vec4<T>& t, const T* s, W4<T>& w) {
     w.a = t.a - s[0];
     w.b = t.b - s[1];
@@ -634,6 +694,7 @@ __device__ __forceinline__ void pair_tile(const Vec4<T>* __restrict__ tg, int nt
 
 template <class P, typename T, int R, bool COMPENSATED>
 __global__ __launch_bounds__(256) void pair_sum_kernel(PairArgs a) {
+  fill_tables<P::TABLE>();
   const int wid = threadIdx.x >> 6;
   const int nblk_t = (a.n_wtiles + 3) >> 2;
   const int split = blockIdx.x / nblk_t;

@@ -102,3 +102,29 @@ def test_fp64_reciprocal_in_biot_savart_sum(ctx):
     got = np.array([st["u"][1:], st["v"][1:], st["w"][1:]])
     err = np.linalg.norm(got - want, axis=0) / (np.abs(s) * np.linalg.norm(d, axis=0))
     assert err.max() < 1e-14, err.max()
+
+
+def test_fp64_exponential_in_pse_sums(ctx):
+    """exp(-rho^2) of the 2nd-order kernel, one source term per target, from 0 to the
+    smallest results.  rho^2 carries a relative rounding of a few ulp (coordinates
+    scaled by 1 / eps, two differences and products), which the exponential turns into
+    an error of rho^2 times that; below e^-700 the terms lose digits to denormals."""
+    rng = np.random.default_rng(10)
+    n = 20000
+    eps = 0.25
+    x = np.concatenate([[0.0], rng.uniform(-6.9, 6.9, n)])
+    y = np.concatenate([[0.0], rng.uniform(-0.5, 0.5, n)])
+    act = np.zeros(n + 1, np.int32)
+    act[0] = 1
+    area = np.zeros(n + 1)
+    area[0] = 0.5
+    f = np.zeros(n + 1)
+    f[0] = 2.0
+    lap = ctx.pse_plane_laplacian(x, y, f, area, act, eps, order=2, precision="fp64")[1:]
+    q = (x[1:] / eps) ** 2 + (y[1:] / eps) ** 2
+    want = 4 / np.pi / eps**4 * f[0] * area[0] * np.exp(-q)
+    ok = q < 690
+    rel = np.abs(lap - want)[ok] / want[ok]
+    assert (rel < 2.3e-16 * (8 + 6 * q[ok])).all()
+    far = q > 760
+    assert far.any() and not lap[far].any()

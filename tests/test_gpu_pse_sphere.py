@@ -84,3 +84,20 @@ def test_bad_arguments(ctx):
         ctx.pse_sphere_laplacian(m.x, m.y, m.z, f, m.area, m.active, 0.1, radius=0.0)
     # the context survives
     ctx.pse_sphere_laplacian(m.x, m.y, m.z, f, m.area, m.active, 0.3)
+
+
+@pytest.mark.parametrize("precision", ["fp64", "fp32"])
+@pytest.mark.parametrize("reach", [0.345, 0.355, 0.555, 0.565, 0.695, 0.705, 1.155, 1.165, 1.195, 1.205])
+def test_distance_series_at_the_ends_of_their_ranges(ctx, oracle, precision, reach):
+    """Each series of the great-circle distance on both sides of the largest 7 eps / R
+    it is used for (FP64 0.35, 0.70, 1.16; FP32 0.56, 1.2), on a radius other than 1,
+    against the oracle's asin form: the bars of the sums above."""
+    radius = 3.0
+    m = icos(4)
+    x, y, z, area = m.x * radius, m.y * radius, m.z * radius, m.area * radius**2
+    f = _harmonic(m)
+    eps = reach / 7.0 * radius
+    ref = oracle.pse_sphere_laplacian(x, y, z, f, area, m.active, eps, radius=radius)
+    got = ctx.pse_sphere_laplacian(x, y, z, f, area, m.active, eps, radius=radius, precision=precision)
+    e = np.abs(got - ref).max() / np.abs(ref).max()
+    assert e < (1e-11 if precision == "fp64" else 1e-4), e
