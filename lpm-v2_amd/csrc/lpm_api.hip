@@ -2,6 +2,9 @@
 // timing and tuning.  Device-resident solvers live in lpm_solver.hip.
 #include <string.h>
 
+#include <algorithm>
+#include <memory>
+#include <new>
 #include <string>
 
 #include "lpm_internal.hpp"
@@ -109,40 +112,153 @@ int check_prec(lpm_ctx* ctx, int precision) {
   return LPM_OK;
 }
 
-// Upload k host arrays of n doubles into ctx->in[0..k).
-int upload(lpm_ctx* ctx, int n, std::initializer_list<const double*> arrays) {
-  int k = 0;
-  for (const double* a : arrays) {
-    DevBuf& b = ctx->in[k++];
-    if (!a) continue;
-    LPM_HIP(ctx, b.ensure((size_t)std::max(n, 1) * sizeof(double)));
-    if (n > 0)
-      LPM_HIP(ctx, hipMemcpyAsync(b.p, a, (size_t)n * sizeof(double), hipMemcpyHostToDevice, ctx->stream));
-  }
-  return LPM_OK;
-}
+// Host arrays of one call in, host arrays out.
+//
+// A call of up to kStageBytes goes through the context's pinned block: inputs and
+// the active list are gathered there and copied up at once, the outputs come down in
+// one copy.  Each copy of pageable memory costs 8-20 us however short it is, and a
+// velocity call made nine of them: at icosahedral level 4 (0.6 MB) 160 of 220 us.
+// Longer calls copy from the caller's arrays: the runtime moves pageable memory at
+// 38 GB/s, a gather of ours would first move it at a quarter of that.
+constexpr size_t kStageBytes = size_t(2) << 20;
 
-int prepare_outputs(lpm_ctx* ctx, int n, int nout) {
-  for (int k = 0; k < nout; ++k) LPM_HIP(ctx, ctx->out[k].ensure((size_t)std::max(n, 1) * sizeof(double)));
-  return LPM_OK;
-}
+class CallIO {
+ public:
+  explicit CallIO(lpm_ctx* ctx) : ctx_(ctx) {}
 
-int download(lpm_ctx* ctx, int i0, int i1, std::initializer_list<double*> outs) {
-  int k = 0;
-  for (double* o : outs) {
-    DevBuf& b = ctx->out[k++];
-    if (!o || i1 <= i0) continue;
-    LPM_HIP(ctx, hipMemcpyAsync(o + i0, b.as<double>() + i0, (size_t)(i1 - i0) * sizeof(double),
-                                hipMemcpyDeviceToHost, ctx->stream));
+  // Inputs: the active mask and `arrays` of n values, then `points` of npts values;
+  // room for nout outputs of `rows` values.
+  int open(int n, const int32_t* active, bool flags, std::initializer_list<const double*> arrays, int rows, int nout,
+           int npts = 0, std::initializer_list<const double*> points = {}) {
+    rows_ = rows;
+    nout_ = nout;
+    const size_t nb = up((size_t)std::max(n, 1) * 8), pb = up((size_t)std::max(npts, 1) * 8);
+    const size_t lb = up((size_t)std::max(n, 1) * 4);
+    const size_t in_bytes = arrays.size() * nb + points.size() * pb + lb + (flags ? lb : 0);
+    const size_t out_bytes = nout * up((size_t)std::max(rows, 1) * 8);
+    staged_ = in_bytes + out_bytes <= kStageBytes;
+    if (staged_) {
+      if (int rc = pinned()) return rc;
+      LPM_HIP(ctx_, ctx_->stage.ensure(kStageBytes));
+      char *h = static_cast<char*>(ctx_->pin), *d = ctx_->stage.as<char>();
+      size_t at = 0;
+      auto gather = [&](const double* a, int count, size_t bytes) {
+        arg_[narg_++] = a ? reinterpret_cast<double*>(d + at) : nullptr;
+        if (a && count > 0) memcpy(h + at, a, (size_t)count * 8);
+        at += bytes;
+      };
+      for (const double* a : arrays) gather(a, n, nb);
+      for (const double* a : points) gather(a, npts, pb);
+      list_ = reinterpret_cast<int*>(d + at);
+      ns_ = compact(active, n, reinterpret_cast<int*>(h + at));
+      at += lb;
+      if (flags) {
+        flags_ = reinterpret_cast<int*>(d + at);
+        if (n > 0) memcpy(h + at, active, (size_t)n * 4);
+        at += lb;
+      }
+      LPM_HIP(ctx_, hipMemcpyAsync(d, h, at, hipMemcpyHostToDevice, ctx_->stream));
+      for (int k = 0; k < nout; ++k) res_[k] = reinterpret_cast<double*>(d + at + k * up((size_t)std::max(rows, 1) * 8));
+      out_at_ = at;
+      return LPM_OK;
+    }
+    int k = 0;
+    auto copy = [&](const double* a, int count) -> int {
+      DevBuf& b = ctx_->in[k++];
+      arg_[narg_++] = nullptr;
+      if (!a) return LPM_OK;
+      LPM_HIP(ctx_, b.ensure((size_t)std::max(count, 1) * 8));
+      if (count > 0) LPM_HIP(ctx_, hipMemcpyAsync(b.p, a, (size_t)count * 8, hipMemcpyHostToDevice, ctx_->stream));
+      arg_[narg_ - 1] = b.as<double>();
+      return LPM_OK;
+    };
+    for (const double* a : arrays)
+      if (int rc = copy(a, n)) return rc;
+    for (const double* a : points)
+      if (int rc = copy(a, npts)) return rc;
+    // built under the copies above, in memory that lasts until the call ends
+    host_list_.reset(new (std::nothrow) int[(size_t)std::max(n, 1)]);
+    if (!host_list_) return fail(ctx_, LPM_ERR_NOMEM, "no host memory for the active list");
+    ns_ = compact(active, n, host_list_.get());
+    LPM_HIP(ctx_, ctx_->list.ensure((size_t)std::max(ns_, 1) * 4));
+    list_ = ctx_->list.as<int>();
+    if (ns_ > 0)
+      LPM_HIP(ctx_, hipMemcpyAsync(list_, host_list_.get(), (size_t)ns_ * 4, hipMemcpyHostToDevice, ctx_->stream));
+    if (flags) {
+      LPM_HIP(ctx_, ctx_->flags.ensure((size_t)std::max(n, 1) * 4));
+      flags_ = ctx_->flags.as<int>();
+      if (n > 0)
+        LPM_HIP(ctx_, hipMemcpyAsync(flags_, active, (size_t)n * 4, hipMemcpyHostToDevice, ctx_->stream));
+    }
+    for (int q = 0; q < nout; ++q) {
+      LPM_HIP(ctx_, ctx_->out[q].ensure((size_t)std::max(rows, 1) * 8));
+      res_[q] = ctx_->out[q].as<double>();
+    }
+    return LPM_OK;
   }
-  LPM_HIP(ctx, hipStreamSynchronize(ctx->stream));
-  return lpm::collect_timing(ctx);
-}
+
+  // Entries [i0, i1) of every output into the caller's arrays.
+  int close(int i0, int i1, std::initializer_list<double*> outs) {
+    const size_t ob = up((size_t)std::max(rows_, 1) * 8), slice = (size_t)(i1 - i0) * 8;
+    char* h = static_cast<char*>(ctx_->pin) + out_at_;
+    if (staged_)
+      LPM_HIP(ctx_, hipMemcpyAsync(h, ctx_->stage.as<char>() + out_at_, nout_ * ob, hipMemcpyDeviceToHost, ctx_->stream));
+    int k = 0;
+    if (!staged_)
+      for (double* o : outs)
+        LPM_HIP(ctx_, hipMemcpyAsync(o + i0, res_[k++] + i0, slice, hipMemcpyDeviceToHost, ctx_->stream));
+    LPM_HIP(ctx_, hipStreamSynchronize(ctx_->stream));
+    open_ = false;
+    if (staged_)
+      for (double* o : outs) memcpy(o + i0, h + (k++) * ob + (size_t)i0 * 8, slice);
+    return lpm::collect_timing(ctx_);
+  }
+
+  // A call that fails half-way may have copies under way from memory of ours.
+  ~CallIO() {
+    if (open_) (void)hipStreamSynchronize(ctx_->stream);
+  }
+  CallIO(const CallIO&) = delete;
+  CallIO& operator=(const CallIO&) = delete;
+
+  const double* arg(int k) const { return arg_[k]; }
+  double* res(int k) const { return k < nout_ ? res_[k] : nullptr; }
+  const int* list() const { return list_; }
+  const int* flags() const { return flags_; }
+  int ns() const { return ns_; }
+
+ private:
+  static size_t up(size_t b) { return (b + 255) / 256 * 256; }
+
+  // Indices of the nonzero flags, ascending (no branch: masks may be random).
+  static int compact(const int32_t* active, int n, int* out) {
+    int k = 0;
+    for (int i = 0; i < n; ++i) {
+      out[k] = i;
+      k += active[i] != 0;
+    }
+    return k;
+  }
+
+  int pinned() {
+    if (!ctx_->pin) LPM_HIP(ctx_, hipHostMalloc(&ctx_->pin, kStageBytes, hipHostMallocDefault));
+    return LPM_OK;
+  }
+
+  lpm_ctx* ctx_;
+  bool staged_ = false, open_ = true;
+  int rows_ = 0, nout_ = 0, narg_ = 0, ns_ = 0;
+  double* arg_[12] = {};
+  double* res_[4] = {};
+  int *list_ = nullptr, *flags_ = nullptr;
+  size_t out_at_ = 0;
+  std::unique_ptr<int[]> host_list_;
+};
 
 // Common body of the PSE operator and SWE entry points.  `inputs` (n doubles
-// each) go to ctx->in[0..) in order, `outputs` to ctx->out[0..); the caller's
-// `bind` maps them onto the pair problem (kind, fields, op).  Points, when
-// given (npts >= 0), are uploaded after the inputs and become the targets.
+// each) are arguments 0, 1, ... in order; the caller's `bind` maps them onto the
+// pair problem (kind, fields, op).  Points, when given (npts >= 0), come after the
+// inputs and become the targets.
 struct OpsCall {
   const char* name;
   int n, i0, i1, precision;
@@ -175,37 +291,25 @@ int run_ops_call(lpm_ctx* ctx, const OpsCall& c, Bind bind) {
   LPM_HIP(ctx, hipSetDevice(ctx->device));
   const int t0 = at_points ? 0 : c.i0, t1 = at_points ? c.npts : c.i1;
   if (t1 == t0) return LPM_OK;
-  int ns = 0;
-  if (int rc = lpm::upload_active_list(ctx, c.active, c.n, ctx->list, nullptr, &ns)) return rc;
-  int k = 0;
-  for (const double* a : c.inputs) {
-    DevBuf& b = ctx->in[k++];
-    LPM_HIP(ctx, b.ensure((size_t)std::max(c.n, 1) * sizeof(double)));
-    if (c.n > 0)
-      LPM_HIP(ctx, hipMemcpyAsync(b.p, a, (size_t)c.n * sizeof(double), hipMemcpyHostToDevice, ctx->stream));
-  }
-  const int k_pts = k;
-  for (const double* a : c.points) {
-    DevBuf& b = ctx->in[k++];
-    LPM_HIP(ctx, b.ensure((size_t)std::max(c.npts, 1) * sizeof(double)));
-    LPM_HIP(ctx, hipMemcpyAsync(b.p, a, (size_t)c.npts * sizeof(double), hipMemcpyHostToDevice, ctx->stream));
-  }
-  const int nout_rows = at_points ? c.npts : c.n;
-  if (int rc = prepare_outputs(ctx, nout_rows, (int)c.outputs.size())) return rc;
+  CallIO io(ctx);
+  if (int rc = io.open(c.n, c.active, false, c.inputs, at_points ? c.npts : c.n, (int)c.outputs.size(),
+                       at_points ? c.npts : 0, c.points))
+    return rc;
+  const int k_pts = (int)c.inputs.size();
   lpm::PairProblem pp;
   pp.precision = c.precision;
   pp.n = c.n;
   pp.i0 = t0;
   pp.i1 = t1;
-  pp.src_list = ctx->list.as<int>();
-  pp.ns = ns;
+  pp.src_list = io.list();
+  pp.ns = io.ns();
   pp.eps = c.eps;
   pp.radius = c.radius;
-  pp.out0 = ctx->out[0].as<double>();
-  pp.out1 = ctx->out[1].as<double>();
-  pp.out2 = ctx->out[2].as<double>();
-  pp.out3 = ctx->out[3].as<double>();
-  auto in = [&](int i) { return ctx->in[i].as<double>(); };
+  pp.out0 = io.res(0);
+  pp.out1 = io.res(1);
+  pp.out2 = io.res(2);
+  pp.out3 = io.res(3);
+  auto in = [&](int i) { return io.arg(i); };
   if (at_points) {
     pp.tx = in(k_pts);
     pp.ty = in(k_pts + 1);
@@ -214,14 +318,7 @@ int run_ops_call(lpm_ctx* ctx, const OpsCall& c, Bind bind) {
   }
   bind(pp, in);
   if (int rc = lpm::run_pair_sum(ctx, pp)) return rc;
-  // outputs are copied back in the order given
-  int o = 0;
-  for (double* out : c.outputs) {
-    LPM_HIP(ctx, hipMemcpyAsync(out + t0, ctx->out[o++].as<double>() + t0, (size_t)(t1 - t0) * sizeof(double),
-                                hipMemcpyDeviceToHost, ctx->stream));
-  }
-  LPM_HIP(ctx, hipStreamSynchronize(ctx->stream));
-  return lpm::collect_timing(ctx);
+  return io.close(t0, t1, c.outputs);
 }
 
 }  // namespace
@@ -289,6 +386,9 @@ int lpm_destroy(lpm_ctx* ctx) {
   ctx->partial.release();
   ctx->red.release();
   ctx->order.release();
+  ctx->flags.release();
+  ctx->stage.release();
+  if (ctx->pin) (void)hipHostFree(ctx->pin);
   for (auto& ep : ctx->pending) {
     (void)hipEventDestroy(ep.a);
     (void)hipEventDestroy(ep.b);
@@ -324,29 +424,27 @@ int lpm_bve_sphere_velocity(lpm_ctx* ctx, double* u, double* v, double* w, const
   if (!(radius > 0.0)) return fail(ctx, LPM_ERR_ARG, "lpm_bve_sphere_velocity: radius must be > 0");
   LPM_HIP(ctx, hipSetDevice(ctx->device));
   if (i1 == i0) return LPM_OK;
-  int ns = 0;
-  if (int rc = lpm::upload_active_list(ctx, active, n, ctx->list, nullptr, &ns)) return rc;
-  if (int rc = upload(ctx, n, {x, y, z, relvort, area})) return rc;
-  if (int rc = prepare_outputs(ctx, n, 3)) return rc;
+  CallIO io(ctx);
+  if (int rc = io.open(n, active, false, {x, y, z, relvort, area}, n, 3)) return rc;
   lpm::PairProblem pp;
   pp.kind = LPM_K_SPHERE_BS;
   pp.precision = precision;
   pp.n = n;
   pp.i0 = i0;
   pp.i1 = i1;
-  pp.x = ctx->in[0].as<double>();
-  pp.y = ctx->in[1].as<double>();
-  pp.z = ctx->in[2].as<double>();
-  pp.q0 = ctx->in[3].as<double>();
-  pp.area = ctx->in[4].as<double>();
-  pp.src_list = ctx->list.as<int>();
-  pp.ns = ns;
+  pp.x = io.arg(0);
+  pp.y = io.arg(1);
+  pp.z = io.arg(2);
+  pp.q0 = io.arg(3);
+  pp.area = io.arg(4);
+  pp.src_list = io.list();
+  pp.ns = io.ns();
   pp.radius = radius;
-  pp.out0 = ctx->out[0].as<double>();
-  pp.out1 = ctx->out[1].as<double>();
-  pp.out2 = ctx->out[2].as<double>();
+  pp.out0 = io.res(0);
+  pp.out1 = io.res(1);
+  pp.out2 = io.res(2);
   if (int rc = lpm::run_pair_sum(ctx, pp)) return rc;
-  return download(ctx, i0, i1, {u, v, w});
+  return io.close(i0, i1, {u, v, w});
 }
 
 int lpm_bve_sphere_velocity_noalloc(lpm_ctx* ctx, double* u, double* v, double* w, const double* x,
@@ -438,26 +536,24 @@ int lpm_plane_velocity(lpm_ctx* ctx, double* u, double* v, const double* x, cons
     return fail(ctx, LPM_ERR_ARG, "lpm_plane_velocity: null array argument");
   LPM_HIP(ctx, hipSetDevice(ctx->device));
   if (i1 == i0) return LPM_OK;
-  int ns = 0;
-  if (int rc = lpm::upload_active_list(ctx, active, n, ctx->list, nullptr, &ns)) return rc;
-  if (int rc = upload(ctx, n, {x, y, vort, area})) return rc;
-  if (int rc = prepare_outputs(ctx, n, 2)) return rc;
+  CallIO io(ctx);
+  if (int rc = io.open(n, active, false, {x, y, vort, area}, n, 2)) return rc;
   lpm::PairProblem pp;
   pp.kind = LPM_K_PLANE_BS;
   pp.precision = precision;
   pp.n = n;
   pp.i0 = i0;
   pp.i1 = i1;
-  pp.x = ctx->in[0].as<double>();
-  pp.y = ctx->in[1].as<double>();
-  pp.q0 = ctx->in[2].as<double>();
-  pp.area = ctx->in[3].as<double>();
-  pp.src_list = ctx->list.as<int>();
-  pp.ns = ns;
-  pp.out0 = ctx->out[0].as<double>();
-  pp.out1 = ctx->out[1].as<double>();
+  pp.x = io.arg(0);
+  pp.y = io.arg(1);
+  pp.q0 = io.arg(2);
+  pp.area = io.arg(3);
+  pp.src_list = io.list();
+  pp.ns = io.ns();
+  pp.out0 = io.res(0);
+  pp.out1 = io.res(1);
   if (int rc = lpm::run_pair_sum(ctx, pp)) return rc;
-  return download(ctx, i0, i1, {u, v});
+  return io.close(i0, i1, {u, v});
 }
 
 int lpm_pse_plane_laplacian(lpm_ctx* ctx, double* lap, const double* x, const double* y,
@@ -474,26 +570,24 @@ int lpm_pse_plane_laplacian(lpm_ctx* ctx, double* lap, const double* x, const do
     return fail(ctx, LPM_ERR_ARG, "lpm_pse_plane_laplacian: order must be 2 or 8");
   LPM_HIP(ctx, hipSetDevice(ctx->device));
   if (i1 == i0) return LPM_OK;
-  int ns = 0;
-  if (int rc = lpm::upload_active_list(ctx, active, n, ctx->list, nullptr, &ns)) return rc;
-  if (int rc = upload(ctx, n, {x, y, f, area})) return rc;
-  if (int rc = prepare_outputs(ctx, n, 1)) return rc;
+  CallIO io(ctx);
+  if (int rc = io.open(n, active, false, {x, y, f, area}, n, 1)) return rc;
   lpm::PairProblem pp;
   pp.kind = order == 8 ? LPM_K_PSE8 : LPM_K_PSE2;
   pp.precision = precision;
   pp.n = n;
   pp.i0 = i0;
   pp.i1 = i1;
-  pp.x = ctx->in[0].as<double>();
-  pp.y = ctx->in[1].as<double>();
-  pp.q0 = ctx->in[2].as<double>();
-  pp.area = ctx->in[3].as<double>();
-  pp.src_list = ctx->list.as<int>();
-  pp.ns = ns;
+  pp.x = io.arg(0);
+  pp.y = io.arg(1);
+  pp.q0 = io.arg(2);
+  pp.area = io.arg(3);
+  pp.src_list = io.list();
+  pp.ns = io.ns();
   pp.eps = eps;
-  pp.out0 = ctx->out[0].as<double>();
+  pp.out0 = io.res(0);
   if (int rc = lpm::run_pair_sum(ctx, pp)) return rc;
-  return download(ctx, i0, i1, {lap});
+  return io.close(i0, i1, {lap});
 }
 
 int lpm_pse_sphere_laplacian(lpm_ctx* ctx, double* lap, const double* x, const double* y, const double* z,
@@ -509,28 +603,26 @@ int lpm_pse_sphere_laplacian(lpm_ctx* ctx, double* lap, const double* x, const d
     return fail(ctx, LPM_ERR_ARG, "lpm_pse_sphere_laplacian: eps and radius must be > 0");
   LPM_HIP(ctx, hipSetDevice(ctx->device));
   if (i1 == i0) return LPM_OK;
-  int ns = 0;
-  if (int rc = lpm::upload_active_list(ctx, active, n, ctx->list, nullptr, &ns)) return rc;
-  if (int rc = upload(ctx, n, {x, y, z, f, area})) return rc;
-  if (int rc = prepare_outputs(ctx, n, 1)) return rc;
+  CallIO io(ctx);
+  if (int rc = io.open(n, active, false, {x, y, z, f, area}, n, 1)) return rc;
   lpm::PairProblem pp;
   pp.kind = LPM_K_PSE_SPHERE8;
   pp.precision = precision;
   pp.n = n;
   pp.i0 = i0;
   pp.i1 = i1;
-  pp.x = ctx->in[0].as<double>();
-  pp.y = ctx->in[1].as<double>();
-  pp.z = ctx->in[2].as<double>();
-  pp.q0 = ctx->in[3].as<double>();
-  pp.area = ctx->in[4].as<double>();
-  pp.src_list = ctx->list.as<int>();
-  pp.ns = ns;
+  pp.x = io.arg(0);
+  pp.y = io.arg(1);
+  pp.z = io.arg(2);
+  pp.q0 = io.arg(3);
+  pp.area = io.arg(4);
+  pp.src_list = io.list();
+  pp.ns = io.ns();
   pp.eps = eps;
   pp.radius = radius;
-  pp.out0 = ctx->out[0].as<double>();
+  pp.out0 = io.res(0);
   if (int rc = lpm::run_pair_sum(ctx, pp)) return rc;
-  return download(ctx, i0, i1, {lap});
+  return io.close(i0, i1, {lap});
 }
 
 int lpm_pse_sphere_laplacian_at_points(lpm_ctx* ctx, double* lap, const double* px, const double* py,
@@ -689,30 +781,28 @@ int lpm_bve_sphere_stream(lpm_ctx* ctx, double* psi_rel, double* psi_abs, const 
   if (!(radius > 0.0)) return fail(ctx, LPM_ERR_ARG, "lpm_bve_sphere_stream: radius must be > 0");
   LPM_HIP(ctx, hipSetDevice(ctx->device));
   if (i1 == i0) return LPM_OK;
-  int ns = 0;
-  if (int rc = lpm::upload_active_list(ctx, active, n, ctx->list, &ctx->in[7], &ns)) return rc;
-  if (int rc = upload(ctx, n, {x, y, z, relvort, absvort, area})) return rc;
-  if (int rc = prepare_outputs(ctx, n, 2)) return rc;
+  CallIO io(ctx);
+  if (int rc = io.open(n, active, true, {x, y, z, relvort, absvort, area}, n, 2)) return rc;
   lpm::PairProblem pp;
   pp.kind = LPM_K_SPHERE_GREEN;
   pp.precision = precision;
   pp.n = n;
   pp.i0 = i0;
   pp.i1 = i1;
-  pp.x = ctx->in[0].as<double>();
-  pp.y = ctx->in[1].as<double>();
-  pp.z = ctx->in[2].as<double>();
-  pp.q0 = ctx->in[3].as<double>();
-  pp.q1 = ctx->in[4].as<double>();
-  pp.area = ctx->in[5].as<double>();
-  pp.active = ctx->in[7].as<int>();
-  pp.src_list = ctx->list.as<int>();
-  pp.ns = ns;
+  pp.x = io.arg(0);
+  pp.y = io.arg(1);
+  pp.z = io.arg(2);
+  pp.q0 = io.arg(3);
+  pp.q1 = io.arg(4);
+  pp.area = io.arg(5);
+  pp.active = io.flags();
+  pp.src_list = io.list();
+  pp.ns = io.ns();
   pp.radius = radius;
-  pp.out0 = ctx->out[0].as<double>();
-  pp.out1 = ctx->out[1].as<double>();
+  pp.out0 = io.res(0);
+  pp.out1 = io.res(1);
   if (int rc = lpm::run_pair_sum(ctx, pp)) return rc;
-  return download(ctx, i0, i1, {psi_rel, psi_abs});
+  return io.close(i0, i1, {psi_rel, psi_abs});
 }
 
 int lpm_plane_stream(lpm_ctx* ctx, double* psi, const double* x, const double* y,
@@ -726,25 +816,23 @@ int lpm_plane_stream(lpm_ctx* ctx, double* psi, const double* x, const double* y
     return fail(ctx, LPM_ERR_ARG, "lpm_plane_stream: null array argument");
   LPM_HIP(ctx, hipSetDevice(ctx->device));
   if (i1 == i0) return LPM_OK;
-  int ns = 0;
-  if (int rc = lpm::upload_active_list(ctx, active, n, ctx->list, nullptr, &ns)) return rc;
-  if (int rc = upload(ctx, n, {x, y, vort, area})) return rc;
-  if (int rc = prepare_outputs(ctx, n, 1)) return rc;
+  CallIO io(ctx);
+  if (int rc = io.open(n, active, false, {x, y, vort, area}, n, 1)) return rc;
   lpm::PairProblem pp;
   pp.kind = LPM_K_PLANE_GREEN;
   pp.precision = precision;
   pp.n = n;
   pp.i0 = i0;
   pp.i1 = i1;
-  pp.x = ctx->in[0].as<double>();
-  pp.y = ctx->in[1].as<double>();
-  pp.q0 = ctx->in[2].as<double>();
-  pp.area = ctx->in[3].as<double>();
-  pp.src_list = ctx->list.as<int>();
-  pp.ns = ns;
-  pp.out0 = ctx->out[0].as<double>();
+  pp.x = io.arg(0);
+  pp.y = io.arg(1);
+  pp.q0 = io.arg(2);
+  pp.area = io.arg(3);
+  pp.src_list = io.list();
+  pp.ns = io.ns();
+  pp.out0 = io.res(0);
   if (int rc = lpm::run_pair_sum(ctx, pp)) return rc;
-  return download(ctx, i0, i1, {psi});
+  return io.close(i0, i1, {psi});
 }
 
 int lpm_pse_eps(double max_edge_length, double power, double* eps) {
@@ -776,15 +864,10 @@ int lpm_diagnostics(lpm_ctx* ctx, const double* u, const double* v, const double
   if (!u || !v || !vort || !area || !active || !ke || !enstrophy || !circulation)
     return fail(ctx, LPM_ERR_ARG, "lpm_diagnostics: null argument");
   LPM_HIP(ctx, hipSetDevice(ctx->device));
-  if (int rc = upload(ctx, n, {u, v, w, vort, area})) return rc;
-  LPM_HIP(ctx, ctx->in[7].ensure((size_t)std::max(n, 1) * sizeof(int)));
-  if (n > 0)
-    LPM_HIP(ctx, hipMemcpyAsync(ctx->in[7].p, active, (size_t)n * sizeof(int), hipMemcpyHostToDevice,
-                                ctx->stream));
+  CallIO io(ctx);
+  if (int rc = io.open(n, active, true, {u, v, w, vort, area}, 0, 0)) return rc;
   double out[3];
-  if (int rc = lpm::run_diagnostics(ctx, n, ctx->in[0].as<double>(), ctx->in[1].as<double>(),
-                                    w ? ctx->in[2].as<double>() : nullptr, ctx->in[3].as<double>(),
-                                    ctx->in[4].as<double>(), ctx->in[7].as<int>(), out))
+  if (int rc = lpm::run_diagnostics(ctx, n, io.arg(0), io.arg(1), io.arg(2), io.arg(3), io.arg(4), io.flags(), out))
     return rc;
   *ke = out[0];
   *enstrophy = out[1];

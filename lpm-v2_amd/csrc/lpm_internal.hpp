@@ -72,7 +72,9 @@ struct lpm_ctx {
   // stateless-call staging
   lpm::DevBuf in[12];
   lpm::DevBuf out[4];
-  lpm::DevBuf list;
+  lpm::DevBuf list, flags;
+  lpm::DevBuf stage;  // the staged calls' inputs and outputs (lpm_api.hip)
+  void* pin = nullptr;  // pinned host block of the same size
   lpm::DevBuf tgt, src, partial;
   lpm::DevBuf red;  // reductions
   lpm::DevBuf order;  // spatial order of the tile paths
@@ -244,7 +246,8 @@ int collect_timing(lpm_ctx* ctx);
 int run_diagnostics(lpm_ctx* ctx, int n, const double* u, const double* v, const double* w,
                     const double* q, const double* area, const int* active, double out[3]);
 
-// Active-particle list on the device from host flags (ascending indices).
+// Active-particle list on the device from host flags (ascending indices), and the
+// flags themselves (any nonzero value is true).
 int upload_active_list(lpm_ctx* ctx, const int32_t* active_host, int n, DevBuf& list,
                        DevBuf* flags, int* ns_out);
 

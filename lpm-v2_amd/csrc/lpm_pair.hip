@@ -9,7 +9,9 @@
 #include <math.h>
 
 #include <algorithm>
+#include <memory>
 #include <mutex>
+#include <new>
 
 #include "cull_kernels.hpp"
 #include "far_kernels.hpp"
@@ -909,25 +911,24 @@ int run_diagnostics(lpm_ctx* ctx, int n, const double* u, const double* v, const
 
 int upload_active_list(lpm_ctx* ctx, const int32_t* active_host, int n, DevBuf& list,
                        DevBuf* flags, int* ns_out) {
-  std::vector<int> idx;
-  idx.reserve((size_t)n);
-  std::vector<int> fl((size_t)n);
-  for (int i = 0; i < n; ++i) {
-    fl[(size_t)i] = active_host[i] != 0;
-    if (fl[(size_t)i]) idx.push_back(i);
+  std::unique_ptr<int[]> idx(new (std::nothrow) int[(size_t)std::max(n, 1)]);
+  if (!idx) return fail(ctx, LPM_ERR_NOMEM, "no host memory for the active list");
+  int ns = 0;
+  for (int i = 0; i < n; ++i) {  // no branch: masks may be random
+    idx[(size_t)ns] = i;
+    ns += active_host[i] != 0;
   }
-  *ns_out = (int)idx.size();
-  LPM_HIP(ctx, list.ensure(std::max<size_t>(idx.size(), 1) * sizeof(int)));
-  if (!idx.empty())
-    LPM_HIP(ctx, hipMemcpyAsync(list.p, idx.data(), idx.size() * sizeof(int), hipMemcpyHostToDevice,
-                                ctx->stream));
+  *ns_out = ns;
+  LPM_HIP(ctx, list.ensure((size_t)std::max(ns, 1) * sizeof(int)));
+  if (ns > 0)
+    LPM_HIP(ctx, hipMemcpyAsync(list.p, idx.get(), (size_t)ns * sizeof(int), hipMemcpyHostToDevice, ctx->stream));
   if (flags) {
     LPM_HIP(ctx, flags->ensure((size_t)std::max(n, 1) * sizeof(int)));
     if (n > 0)
-      LPM_HIP(ctx, hipMemcpyAsync(flags->p, fl.data(), (size_t)n * sizeof(int), hipMemcpyHostToDevice,
+      LPM_HIP(ctx, hipMemcpyAsync(flags->p, active_host, (size_t)n * sizeof(int), hipMemcpyHostToDevice,
                                   ctx->stream));
   }
-  // the host vectors die at return: make the copies complete first
+  // the host list dies at return: make the copies complete first
   LPM_HIP(ctx, hipStreamSynchronize(ctx->stream));
   return LPM_OK;
 }
