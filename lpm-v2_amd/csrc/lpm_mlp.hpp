@@ -20,7 +20,7 @@ struct Mlp {
   int cur_n = 0;
   DevBuf p, grad, m, v;    // FP32 parameters, gradient, Adam moments
   DevBuf frag, bias;       // FP16 MFMA fragments + FP32 biases (inference)
-  DevBuf act, pre, scratch, loss_part, splitk;
+  DevBuf act, scratch, loss_part, splitk;
   DevBuf xb, tb, idx;      // training minibatch staging
   ~Mlp();
   void release();

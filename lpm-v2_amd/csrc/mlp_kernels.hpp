@@ -4,8 +4,8 @@
 // ISRU x / sqrt(1 + x^2), parameters per layer W[out][in] (row-major) then
 // b[out], FP32 master copy.
 //
-// Training path (FP32, VALU): tiled GEMMs C = A op(B) with a fused
-// bias + activation epilogue, the backward GEMMs, column sums and Adam.
+// Training path (FP32 matrix instructions): tiled GEMMs C = A op(B) with the
+// bias + activation, the activation's derivative or the bias gradient fused in, and Adam.
 // Inference path (FP16 MFMA, FP32 accumulate), specialised for the
 // 13 -> 128 -> 128 -> 128 -> 3 surrogate: activations are kept transposed
 // (features = MFMA rows, samples = MFMA columns), so the D registers of one
@@ -90,104 +90,220 @@ __host__ __device__ inline float mlp_hidden_scale(int act) {
 }
 
 // ------------------------------------------------------------ FP32 GEMM
-// C[M][N] = act(alpha * sum_k A(m, k) B(k, n) + bias[n]) (+ beta C), with
-// A(m, k) = TA ? A[k][m] : A[m][k] and B(k, n) = TB ? B[n][k] : B[k][n].
-// 64 x 64 tile per 256-thread block, 4 x 4 outputs per thread, K tiles of 16
-// staged in LDS.  Z (optional) receives the pre-activation.  Split K: with
-// part != nullptr, block z of the grid covers k in [z kchunk, (z+1) kchunk)
-// and writes alpha * its partial product to part[z][M][N] (no bias, beta or
-// activation); gemm_splitk_reduce then sums the partials in a fixed order.
+// C[M][N] = act(sum_k A(m, k) B(k, n) + bias[n]), with A(m, k) = TA ? A[k][m] :
+// A[m][k] and B(k, n) = TB ? B[n][k] : B[k][n]; with H, the product is instead
+// multiplied by the activation's derivative at the output H[m][n] (leading
+// dimension ldc).  sums (TA only) receives sum_k A(m, k), the bias gradient.
+//
+// 64 x 64 tile per 256-thread block on the FP32 matrix instruction
+// v_mfma_f32_16x16x4_f32: each of the 4 waves holds 32 x 32 outputs as four
+// accumulators.  Operands are staged as [row][k] in two LDS buffers of 32 k
+// each, the next tile's global loads in flight during the current tile's
+// products.  Lane group g = lane / 16 reads k = 4 g .. 4 g + 3 of a 16-k block in one
+// ds_read_b128 and step s multiplies its element s, for A and B alike, so a
+// block needs 4 LDS reads per 16 matrix instructions; a row pitch of 36
+// floats spreads the reads over the banks.  B's rows are the instruction's
+// rows: a lane's four results are four consecutive n, one 16-byte store.
+// Split K: with part != nullptr, block z covers k in [z kchunk, (z+1) kchunk)
+// and writes its partial product (and, after it, its partial sums) to
+// part[z][M N (+ M)]; gemm_splitk_reduce adds them in a fixed order.
+// At 32,768 samples and width 128 (1.07 GFLOP, 6.8 us of matrix time; the
+// operands' 34 MB take 7 us) a layer's forward takes 22 us, its input gradient
+// 19.5 and its weight and bias gradient 24 with the reduction; the same on the
+// vector units, with the derivative and the sums in kernels of their own, took
+// 51, 52 and 188.  What is left is the serial load, product, store of a block
+// with 4 K tiles.
+constexpr int kGemmTile = 64;
+constexpr int kGemmK = 32;
+constexpr int kGemmPitch = kGemmK + 4;
+
 struct GemmArgs {
   const float* A;
   const float* B;
   float* C;
-  float* Z;
   const float* bias;
+  const float* H;
+  float* sums;
   int M, N, K;
   int lda, ldb, ldc;
-  float alpha, beta;
   int act;  // 0 none, kActTanh, kActIsru
   float* part;
   int kchunk;
 };
 
-template <bool TA, bool TB>
-__global__ __launch_bounds__(256) void gemm_f32(GemmArgs g) {
-  __shared__ float As[16][64 + 1];
-  __shared__ float Bs[16][64 + 1];
-  const int tx = threadIdx.x & 15, ty = threadIdx.x >> 4;
-  const int m0 = blockIdx.y * 64, n0 = blockIdx.x * 64;
-  const int kb = g.part ? (int)blockIdx.z * g.kchunk : 0;
-  const int ke = g.part ? min(g.K, kb + g.kchunk) : g.K;
-  float acc[4][4] = {};
-  for (int k0 = kb; k0 < ke; k0 += 16) {
-    for (int t = threadIdx.x; t < 16 * 64; t += 256) {
-      const int kk = t / 64, mm = t % 64;
-      const int m = m0 + mm, k = k0 + kk;
-      float a = 0.f;
-      if (m < g.M && k < ke) a = TA ? g.A[(size_t)k * g.lda + m] : g.A[(size_t)m * g.lda + k];
-      As[kk][mm] = a;
-      const int n = n0 + mm;
-      float b = 0.f;
-      if (n < g.N && k < ke) b = TB ? g.B[(size_t)n * g.ldb + k] : g.B[(size_t)k * g.ldb + n];
-      Bs[kk][mm] = b;
-    }
-    __syncthreads();
+// dZ = dH act'(Z) from the output H alone: tanh' = 1 - H^2;
+// ISRU' = (1 + Z^2)^(-3/2) = (1 - H^2)^(3/2)
+__device__ __forceinline__ float act_slope(int act, float h) {
+  const float t = 1.0f - h * h;
+  return act == kActIsru ? t * sqrtf(fmaxf(t, 0.0f)) : t;
+}
+
+// Eight floats of one operand's 64 x 32 tile (rows r0 .., k0 ..) for this thread.
+// ROWS (k contiguous in memory): rows t/8 and t/8 + 32, k = 4 (t%8) .. + 3.
+// Else (rows contiguous): row t%64, k = 4 (t/64) .. + 3 and the same + 16.
+// Rows past the end repeat the last one (their outputs are not stored), k past
+// the end is zero; every load is unconditional, so all are in flight together.
+// vec: the k-contiguous rows start on 16 bytes.
+template <bool ROWS>
+__device__ __forceinline__ void gemm_fetch(const float* __restrict__ X, int ld, int rows, int ke, int r0, int k0,
+                                           bool vec, floatx4_t v[2]) {
+  const int t = threadIdx.x;
+  const bool full = k0 + kGemmK <= ke;
 #pragma unroll
-    for (int kk = 0; kk < 16; ++kk) {
-      float a[4], b[4];
+  for (int j = 0; j < 2; ++j) {
+    const int r = min(ROWS ? r0 + (t >> 3) + 32 * j : r0 + (t & 63), rows - 1);
+    const int k = ROWS ? k0 + 4 * (t & 7) : k0 + 4 * (t >> 6) + 16 * j;
+    const float* x = ROWS ? X + (size_t)r * ld : X + r;
+    const size_t step = ROWS ? 1 : (size_t)ld;
+    if (full) {
+      if (ROWS && vec) {
+        v[j] = *reinterpret_cast<const floatx4_t*>(x + k);
+      } else {
 #pragma unroll
-      for (int i = 0; i < 4; ++i) a[i] = As[kk][ty * 4 + i];
-#pragma unroll
-      for (int j = 0; j < 4; ++j) b[j] = Bs[kk][tx * 4 + j];
-#pragma unroll
-      for (int i = 0; i < 4; ++i)
-#pragma unroll
-        for (int j = 0; j < 4; ++j) acc[i][j] = fmaf(a[i], b[j], acc[i][j]);
-    }
-    __syncthreads();
-  }
-  if (g.part) {
-    float* P = g.part + (size_t)blockIdx.z * g.M * g.N;
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const int m = m0 + ty * 4 + i;
-      if (m >= g.M) continue;
-#pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        const int n = n0 + tx * 4 + j;
-        if (n < g.N) P[(size_t)m * g.N + n] = g.alpha * acc[i][j];
+        for (int e = 0; e < 4; ++e) v[j][e] = x[(size_t)(k + e) * step];
       }
-    }
-    return;
-  }
+    } else {
 #pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    const int m = m0 + ty * 4 + i;
-    if (m >= g.M) continue;
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      const int n = n0 + tx * 4 + j;
-      if (n >= g.N) continue;
-      float v = g.alpha * acc[i][j];
-      if (g.bias) v += g.bias[n];
-      if (g.beta != 0.f) v += g.beta * g.C[(size_t)m * g.ldc + n];
-      if (g.Z) g.Z[(size_t)m * g.ldc + n] = v;
-      if (g.act == kActTanh) v = tanhf(v);
-      else if (g.act == kActIsru) v = v / sqrtf(fmaf(v, v, 1.0f));
-      g.C[(size_t)m * g.ldc + n] = v;
+      for (int e = 0; e < 4; ++e) {
+        const float y = x[(size_t)min(k + e, ke - 1) * step];
+        v[j][e] = k + e < ke ? y : 0.f;
+      }
     }
   }
 }
 
-// C[m][n] = sum over splits z = 0, 1, ... of part[z][m][n] (fixed order)
-static __global__ __launch_bounds__(256) void gemm_splitk_reduce(int splits, int M, int N, const float* __restrict__ part,
-                                                                float* __restrict__ C, int ldc) {
-  const int t = blockIdx.x * blockDim.x + threadIdx.x;
-  if (t >= M * N) return;
+template <bool ROWS>
+__device__ __forceinline__ void gemm_stage(float* __restrict__ S, const floatx4_t v[2]) {
+  const int t = threadIdx.x;
+#pragma unroll
+  for (int j = 0; j < 2; ++j) {
+    const int r = ROWS ? (t >> 3) + 32 * j : (t & 63);
+    const int k = ROWS ? 4 * (t & 7) : 4 * (t >> 6) + 16 * j;
+    *reinterpret_cast<floatx4_t*>(S + r * kGemmPitch + k) = v[j];
+  }
+}
+
+template <bool TA, bool TB>
+__global__ __launch_bounds__(256) void gemm_f32(GemmArgs g) {
+  __shared__ __attribute__((aligned(16))) float As[2][kGemmTile * kGemmPitch];
+  __shared__ __attribute__((aligned(16))) float Bs[2][kGemmTile * kGemmPitch];
+  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+  const int i16 = lane & 15, g4 = lane >> 4;
+  const int m0 = blockIdx.x * kGemmTile, n0 = blockIdx.y * kGemmTile;
+  const int wm = 32 * (w & 1), wn = 32 * (w >> 1);
+  const int kb = g.part ? (int)blockIdx.z * g.kchunk : 0;
+  const int ke = g.part ? min(g.K, kb + g.kchunk) : g.K;
+  const bool va = !TA && (g.lda & 3) == 0 && (reinterpret_cast<uintptr_t>(g.A) & 15) == 0;
+  const bool vb = TB && (g.ldb & 3) == 0 && (reinterpret_cast<uintptr_t>(g.B) & 15) == 0;
+  const bool sums = TA && g.sums && n0 == 0;
+  floatx4_t acc[2][2] = {};  // [n tile][m tile]
+  floatx4_t fa[2], fb[2];
+  float sum = 0.f;
+  gemm_fetch<!TA>(g.A, g.lda, g.M, ke, m0, kb, va, fa);
+  gemm_fetch<TB>(g.B, g.ldb, g.N, ke, n0, kb, vb, fb);
+  int cur = 0;
+  for (int k0 = kb; k0 < ke; k0 += kGemmK, cur ^= 1) {
+    gemm_stage<!TA>(As[cur], fa);
+    gemm_stage<TB>(Bs[cur], fb);
+    if (sums) {
+      const floatx4_t s = fa[0] + fa[1];
+      sum += (s[0] + s[1]) + (s[2] + s[3]);
+    }
+    __syncthreads();  // also: every wave has left the buffer staged next
+    if (k0 + kGemmK < ke) {
+      gemm_fetch<!TA>(g.A, g.lda, g.M, ke, m0, k0 + kGemmK, va, fa);
+      gemm_fetch<TB>(g.B, g.ldb, g.N, ke, n0, k0 + kGemmK, vb, fb);
+    }
+    const float* a = As[cur] + (wm + i16) * kGemmPitch + 4 * g4;
+    const float* b = Bs[cur] + (wn + i16) * kGemmPitch + 4 * g4;
+#pragma unroll
+    for (int kk = 0; kk < kGemmK; kk += 16) {
+      floatx4_t av[2], bv[2];
+#pragma unroll
+      for (int q = 0; q < 2; ++q) {
+        av[q] = *reinterpret_cast<const floatx4_t*>(a + 16 * q * kGemmPitch + kk);
+        bv[q] = *reinterpret_cast<const floatx4_t*>(b + 16 * q * kGemmPitch + kk);
+      }
+#pragma unroll
+      for (int s = 0; s < 4; ++s)
+#pragma unroll
+        for (int p = 0; p < 2; ++p)
+#pragma unroll
+          for (int q = 0; q < 2; ++q)
+            acc[p][q] = __builtin_amdgcn_mfma_f32_16x16x4f32(bv[p][s], av[q][s], acc[p][q], 0, 0, 0);
+    }
+  }
+  const size_t mn = (size_t)g.M * g.N;
+  float* P = g.part ? g.part + (size_t)blockIdx.z * (mn + (g.sums ? g.M : 0)) : nullptr;
+  if (sums) {  // 4 waves' sums of each row, in order; the staging buffers are free after the barrier
+    __syncthreads();
+    As[0][threadIdx.x] = sum;
+    __syncthreads();
+    const int m = m0 + threadIdx.x;
+    if (threadIdx.x < kGemmTile && m < g.M) {
+      const float s = (As[0][threadIdx.x] + As[0][threadIdx.x + 64]) +
+                      (As[0][threadIdx.x + 128] + As[0][threadIdx.x + 192]);
+      (P ? P + mn : g.sums)[m] = s;
+    }
+  }
+  float* C = P ? P : g.C;
+  const int ldc = P ? g.N : g.ldc;
+  const bool vc = (ldc & 3) == 0 && ((reinterpret_cast<uintptr_t>(C) | reinterpret_cast<uintptr_t>(g.H)) & 15) == 0;
+#pragma unroll
+  for (int p = 0; p < 2; ++p) {
+#pragma unroll
+    for (int q = 0; q < 2; ++q) {
+      const int m = m0 + wm + 16 * q + i16, n = n0 + wn + 16 * p + 4 * g4;
+      if (m >= g.M || n >= g.N) continue;
+      const size_t at = (size_t)m * ldc + n;
+      const int cols = min(4, g.N - n);
+      floatx4_t v = acc[p][q];
+      if (!P) {
+        if (g.bias)
+          for (int e = 0; e < cols; ++e) v[e] += g.bias[n + e];
+        if (g.H) {
+          floatx4_t h = {};
+          if (vc && cols == 4) h = *reinterpret_cast<const floatx4_t*>(g.H + at);
+          else
+            for (int e = 0; e < cols; ++e) h[e] = g.H[at + e];
+#pragma unroll
+          for (int e = 0; e < 4; ++e) v[e] *= act_slope(g.act, h[e]);
+        } else if (g.act == kActTanh) {
+#pragma unroll
+          for (int e = 0; e < 4; ++e) v[e] = tanhf(v[e]);
+        } else if (g.act == kActIsru) {
+#pragma unroll
+          for (int e = 0; e < 4; ++e) v[e] = v[e] / sqrtf(fmaf(v[e], v[e], 1.0f));
+        }
+      }
+      if (vc && cols == 4) *reinterpret_cast<floatx4_t*>(C + at) = v;
+      else
+        for (int e = 0; e < cols; ++e) C[at + e] = v[e];
+    }
+  }
+}
+
+// out[t] = sum over splits z of part[z][t]: 64 outputs per block, wave w adds
+// splits w, w + 4, ... with 8 loads in flight, then the four waves' sums (fixed order).
+static __global__ __launch_bounds__(256) void gemm_splitk_reduce(int splits, int n, const float* __restrict__ part,
+                                                                float* __restrict__ out) {
+  __shared__ float sh[256];
+  const int w = threadIdx.x >> 6, t = blockIdx.x * 64 + (threadIdx.x & 63);
   float s = 0.f;
-  for (int z = 0; z < splits; ++z) s += part[(size_t)z * M * N + t];
-  C[(size_t)(t / N) * ldc + t % N] = s;
+  if (t < n) {
+    int z = w;
+    for (; z + 28 < splits; z += 32) {
+      float v[8];
+#pragma unroll
+      for (int e = 0; e < 8; ++e) v[e] = part[(size_t)(z + 4 * e) * n + t];
+#pragma unroll
+      for (int e = 0; e < 8; ++e) s += v[e];
+    }
+    for (; z < splits; z += 4) s += part[(size_t)z * n + t];
+  }
+  sh[threadIdx.x] = s;
+  __syncthreads();
+  if (w == 0 && t < n) out[t] = (sh[threadIdx.x] + sh[threadIdx.x + 64]) + (sh[threadIdx.x + 128] + sh[threadIdx.x + 192]);
 }
 
 // ------------------------------------------------------- FP16 MFMA forward

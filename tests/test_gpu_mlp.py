@@ -73,3 +73,31 @@ def test_training_reduces_loss(ctx):
     y32 = net.forward(x[:2048])
     y16 = net.forward(x[:2048], mfma=True)
     assert np.sqrt(((y16 - y32) ** 2).sum() / (y32**2).sum()) < 3e-2
+
+
+@pytest.mark.parametrize("nin,width,nh,nout,n", [
+    (1, 1, 1, 1, 1),          # one tile, nothing but padding
+    (13, 128, 3, 3, 64),      # whole tiles, no split
+    (4, 64, 2, 4, 511),       # aligned rows, ragged samples, just below the split
+    (5, 65, 2, 7, 513),       # rows that start on no 16 bytes, one column past a tile, two splits
+    (33, 130, 1, 66, 2049),   # input and output wider than a tile, ragged K
+    (31, 63, 3, 2, 40000),    # all splits, the smallest tails
+])
+def test_gradient_at_tile_edges(ctx, oracle, nin, width, nh, nout, n):
+    """The matrix-instruction products (tile 64 x 64 x 32, split at 512 samples) at
+    their edges.  Tolerance: roundings of a random walk, sqrt(layers' K + samples
+    per split) 2^-24 < 3e-6 in norm, times 3."""
+    net = Mlp(ctx, nin, width, nh, nout, seed=7, act=ACT_ISRU)
+    p = net.params()
+    rng = np.random.default_rng(n)
+    x = rng.normal(size=(n, nin)).astype(np.float32)
+    t = rng.normal(size=(n, nout)).astype(np.float32)
+    ref = oracle.mlp_forward(p.astype(np.float64), x.astype(np.float64), nin, width, nh, nout, ACT_ISRU)
+    assert np.linalg.norm(net.forward(x) - ref) < 1e-5 * np.linalg.norm(ref)
+    loss, g = net.loss_grad(x, t)
+    rl, rg = oracle.mlp_loss_grad(p.astype(np.float64), x.astype(np.float64), t.astype(np.float64), nin, width, nh,
+                                  nout, ACT_ISRU)
+    assert abs(loss - rl) < 1e-5 * abs(rl)
+    assert np.linalg.norm(g - rg) < 1e-5 * np.linalg.norm(rg)
+    again = net.loss_grad(x, t)
+    assert again[0] == loss and np.array_equal(again[1], g)
