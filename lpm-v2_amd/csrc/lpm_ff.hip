@@ -37,8 +37,6 @@
 // remainder (~ W l^(P+1) / |x - c|^(P+3)) is O(1) at every distance in the band.
 #include <math.h>
 
-#include <hipcub/hipcub.hpp>
-
 #include <algorithm>
 #include <numeric>
 #include <random>
@@ -67,7 +65,6 @@ constexpr int kCellRec = 40; // floats per far-field cell record
 constexpr int kMlpRec = 32;  // floats per MLP cell record
 constexpr int kMlpNct = 2;   // 16-target column tiles per network pass
 constexpr int kMlpTile = 16 * kMlpNct;  // targets per network work item
-constexpr int kLocR = 2;  // particles per lane in the binning kernel
 // The near and far kernels split their work (near lists, far record lists) in
 // up to kSplitMax parts, enough for about kSplitRounds rounds of resident waves.
 constexpr double kSplitRounds = 6.0;
@@ -263,75 +260,146 @@ __device__ __forceinline__ void project(double& x, double& y, double& z, double 
 // Cell of each particle: the generator with the largest dot product (lowest
 // index on ties); sort keys for targets (all particles) and sources (inactive
 // particles get key ncell and sort last).
-__global__ __launch_bounds__(256) void ff_locate(int n, int ncell, const lpm::Vec4<float>* __restrict__ gen,
-                                                 const double* __restrict__ x, const double* __restrict__ y,
-                                                 const double* __restrict__ z, const int* __restrict__ active,
-                                                 int* __restrict__ cellof, int* __restrict__ key_t,
-                                                 int* __restrict__ key_s, int* __restrict__ iota) {
-  // kLocR particles per lane; generators in groups of 8, so that one wait
-  // covers 8 scalar loads
-  const int i0 = blockIdx.x * blockDim.x * kLocR + threadIdx.x;
-  if (i0 >= n) return;
-  float px[kLocR], py[kLocR], pz[kLocR], best[kLocR];
-  int bs[kLocR];
-#pragma unroll
-  for (int r = 0; r < kLocR; ++r) {
-    const int i = min(i0 + r * (int)blockDim.x, n - 1);
-    px[r] = (float)x[i];
-    py[r] = (float)y[i];
-    pz[r] = (float)z[i];
-    best[r] = -3.f;
-    bs[r] = 0;
+//
+// The generators are fixed, so their search is laid out once: directions fall in
+// 6 g x g bins (faces of the surrounding cube), and a bin lists, in ascending
+// order, every generator that can be the nearest of a direction in it: those
+// whose largest dot product over the bin is not below the largest of all the
+// generators' smallest ones.  Bins of a quarter of a cell's width list 3-4 of
+// them on average.  A bin with more than kBinMax, and a particle whose
+// coordinates are no ordinary numbers, look through all generators.
+// At 491,522 particles and 1,280 cells: 190 us over all generators, 13 in bins.
+constexpr int kBinMax = 15;
+struct LocBin {
+  int count;  // -1: all generators
+  int cell[kBinMax];
+};
+
+__host__ __device__ inline int loc_grid(int ncell) {
+  int g = 4;
+  while (g < 128 && 6 * g * g < 16 * ncell) g *= 2;
+  return g;
+}
+
+// Bin of direction (px, py, pz), not all zero.
+__device__ __forceinline__ int loc_bin(float px, float py, float pz, int g) {
+  const float ax = fabsf(px), ay = fabsf(py), az = fabsf(pz);
+  int face;
+  float m, u, v;
+  if (ax >= ay && ax >= az) {
+    face = px >= 0.f ? 0 : 1, m = ax, u = py, v = pz;
+  } else if (ay >= az) {
+    face = py >= 0.f ? 2 : 3, m = ay, u = px, v = pz;
+  } else {
+    face = pz >= 0.f ? 4 : 5, m = az, u = px, v = py;
   }
-  auto visit = [&](const lpm::Vec4<float>& g, int s) {
-#pragma unroll
-    for (int r = 0; r < kLocR; ++r) {
-      const float d = fmaf(g.a, px[r], fmaf(g.b, py[r], g.c * pz[r]));
-      if (d > best[r]) {  // strict: the lowest index wins a tie
-        best[r] = d;
-        bs[r] = s;
-      }
+  const float h = 0.5f * (float)g, q = h / m;
+  const int iu = min(g - 1, max(0, (int)fmaf(u, q, h))), iv = min(g - 1, max(0, (int)fmaf(v, q, h)));
+  return (face * g + iu) * g + iv;
+}
+
+__global__ __launch_bounds__(256) void ff_locate_bins(int ncell, int g, const lpm::Vec4<float>* __restrict__ gen,
+                                                      LocBin* __restrict__ bins) {
+  const int b = blockIdx.x * 256 + threadIdx.x;
+  if (b >= 6 * g * g) return;
+  const int face = b / (g * g), iu = b / g % g, iv = b % g;
+  auto dir = [&](double u, double v, double d[3]) {
+    const int ax = face >> 1;
+    const double s = face & 1 ? -1.0 : 1.0, r = 1.0 / sqrt(1.0 + u * u + v * v);
+    d[ax] = s * r;
+    d[ax == 0 ? 1 : 0] = u * r;
+    d[ax == 2 ? 1 : 2] = v * r;
+  };
+  const double w = 2.0 / g;
+  double c[3], e[3];
+  dir((iu + 0.5) * w - 1.0, (iv + 0.5) * w - 1.0, c);
+  double half = 0.0;  // angular radius: the farthest corner, with room for the bin's own rounding
+  for (int k = 0; k < 4; ++k) {
+    dir((iu + (k & 1)) * w - 1.0, (iv + (k >> 1)) * w - 1.0, e);
+    half = fmax(half, acos(fmin(1.0, c[0] * e[0] + c[1] * e[1] + c[2] * e[2])));
+  }
+  half += 1e-5;
+  const double ch = cos(half), sh = sin(half);
+  // of a generator at angle a (dot c, sine s): dot products over the bin lie in
+  // [cos(a + half), cos(max(0, a - half))]; a zero generator has 0 everywhere
+  auto bounds = [&](const lpm::Vec4<float>& q, double& lo, double& hi) {
+    const double d = q.a * c[0] + q.b * c[1] + q.c * c[2];
+    const double n2 = (double)q.a * q.a + (double)q.b * q.b + (double)q.c * q.c;
+    const double s = sqrt(fmax(0.0, n2 - d * d)), n = sqrt(n2);
+    lo = d <= -n * ch ? -n : d * ch - s * sh;
+    hi = d >= n * ch ? n : d * ch + s * sh;
+  };
+  double floor_ = -1e300, lo, hi;
+  for (int s = 0; s < ncell; ++s) {
+    bounds(gen[s], lo, hi);
+    floor_ = fmax(floor_, lo);
+  }
+  floor_ -= 1e-5;  // the FP32 products' rounding
+  int count = 0;
+  for (int s = 0; s < ncell; ++s) {
+    bounds(gen[s], lo, hi);
+    if (!(hi >= floor_)) continue;
+    if (count >= kBinMax) {
+      count = -1;
+      break;
+    }
+    bins[b].cell[count++] = s;
+  }
+  bins[b].count = count;
+}
+
+__global__ __launch_bounds__(256) void ff_locate(int n, int ncell, int g, const lpm::Vec4<float>* __restrict__ gen,
+                                                 const LocBin* __restrict__ bins, const double* __restrict__ x,
+                                                 const double* __restrict__ y, const double* __restrict__ z,
+                                                 const int* __restrict__ active, int* __restrict__ cellof,
+                                                 lpm::CellSort sort) {
+  const int i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i >= n) return;
+  const float px = (float)x[i], py = (float)y[i], pz = (float)z[i];
+  float best = -3.f;
+  int bs = 0;
+  auto visit = [&](const lpm::Vec4<float>& q, int s) {
+    const float d = fmaf(q.a, px, fmaf(q.b, py, q.c * pz));
+    if (d > best) {  // strict: the lowest index wins a tie
+      best = d;
+      bs = s;
     }
   };
-  int s = 0;
-  for (; s + 8 <= ncell; s += 8) {
-    lpm::Vec4<float> g[8];
-#pragma unroll
-    for (int e = 0; e < 8; ++e) g[e] = gen[s + e];
-#pragma unroll
-    for (int e = 0; e < 8; ++e) visit(g[e], s + e);
+  const float size = fabsf(px) + fabsf(py) + fabsf(pz);
+  const LocBin* bin = nullptr;
+  if (size > 1e-15f && size < 1e15f) {  // false for NaN
+    bin = bins + loc_bin(px, py, pz, g);
+    if (bin->count < 0) bin = nullptr;
   }
-  for (; s < ncell; ++s) visit(gen[s], s);
-#pragma unroll
-  for (int r = 0; r < kLocR; ++r) {
-    const int i = i0 + r * (int)blockDim.x;
-    if (i < n) {
-      cellof[i] = bs[r];
-      key_t[i] = bs[r];
-      key_s[i] = active[i] ? bs[r] : ncell;
-      iota[i] = i;
+  if (bin) {
+    const int count = bin->count;
+    for (int k = 0; k < count; ++k) {
+      const int s = bin->cell[k];
+      visit(gen[s], s);
     }
+  } else {
+    for (int s = 0; s < ncell; ++s) visit(gen[s], s);
   }
+  cellof[i] = bs;
+  sort.tgt_key[i] = bs;
+  sort.src_key[i] = active[i] ? bs : ncell;
+  sort.tgt_val[i] = i;
+  sort.src_val[i] = i;
 }
 
-__device__ __forceinline__ int lower_bound_dev(const int* __restrict__ a, int n, int key) {
-  int lo = 0, hi = n;
-  while (lo < hi) {
-    const int mid = (lo + hi) >> 1;
-    if (a[mid] < key) lo = mid + 1;
-    else hi = mid;
-  }
-  return lo;
-}
-
-// Start of every cell (and the end, index ncell) in the sorted key arrays.
-__global__ __launch_bounds__(256) void ff_bounds(int n, int ncell, const int* __restrict__ tkey,
-                                                 const int* __restrict__ skey, int* __restrict__ tgt_start,
+// Start of every cell (and the end, index ncell) in the sorted key arrays: item i
+// starts the cells after its predecessor's, up to its own.
+__global__ __launch_bounds__(256) void ff_bounds(int n, int ncell, const unsigned* __restrict__ tkey,
+                                                 const unsigned* __restrict__ skey, int* __restrict__ tgt_start,
                                                  int* __restrict__ src_start) {
-  const int c = blockIdx.x * blockDim.x + threadIdx.x;
-  if (c > ncell) return;
-  tgt_start[c] = lower_bound_dev(tkey, n, c);
-  src_start[c] = lower_bound_dev(skey, n, c);
+  const int i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i > n) return;
+  auto mark = [&](const unsigned* key, int* start) {
+    const int prev = i > 0 ? (int)key[i - 1] : -1, cur = i < n ? (int)key[i] : ncell;
+    for (int c = prev + 1; c <= cur; ++c) start[c] = i;
+  };
+  mark(tkey, tgt_start);
+  mark(skey, src_start);
 }
 
 // Work items (cell, tile) for tiles of tileA and of tileB targets, in cell
@@ -396,28 +464,41 @@ struct GeomArgs {
   double* geo;         // [ncell][8]: src dir (3), src rho, tgt dir (3), tgt rho
   double* cen64;       // [ncell][3] FP64 source centroids
   double* mom64;       // [ncell][kNMom]
+  double* pgeo;        // [npar][4]: the parents' source dir (3), rho
 };
 
-__device__ double block_sum(double v, double* sh) {
-  sh[threadIdx.x] = v;
-  __syncthreads();
-  for (int k = blockDim.x / 2; k > 0; k >>= 1) {
-    if ((int)threadIdx.x < k) sh[threadIdx.x] += sh[threadIdx.x + k];
+// Sums of K values over the block, in a fixed order, to every thread: eight values
+// at a time through LDS, 32 lanes to a value.  `sh` holds kRedWords doubles.
+constexpr int kRedWords = 8 * 256 + 48;
+template <int K>
+__device__ __forceinline__ void block_sums(double (&v)[K], double* sh) {
+  double* res = sh + 8 * 256;
+#pragma unroll
+  for (int k0 = 0; k0 < K; k0 += 8) {
+#pragma unroll
+    for (int e = 0; e < 8; ++e)
+      if (k0 + e < K) sh[e * 256 + threadIdx.x] = v[k0 + e];
+    __syncthreads();
+    const int e = threadIdx.x >> 5, l = threadIdx.x & 31;
+    if (k0 + e < K) {
+      double s = 0.0;
+#pragma unroll
+      for (int j = 0; j < 8; ++j) s += sh[e * 256 + l + 32 * j];
+      for (int m = 16; m > 0; m >>= 1) s += __shfl_xor(s, m);
+      if (l == 0) res[k0 + e] = s;
+    }
     __syncthreads();
   }
-  double r = sh[0];
-  __syncthreads();
-  return r;
+#pragma unroll
+  for (int k = 0; k < K; ++k) v[k] = res[k];
 }
 
-__device__ double block_max(double v, double* sh) {
-  sh[threadIdx.x] = v;
+// Smallest of a value over the block (NaN ignored), to every thread.
+__device__ __forceinline__ double block_min(double v, double* sh) {
+  for (int m = 32; m > 0; m >>= 1) v = fmin(v, __shfl_xor(v, m));
+  if ((threadIdx.x & 63) == 0) sh[threadIdx.x >> 6] = v;
   __syncthreads();
-  for (int k = blockDim.x / 2; k > 0; k >>= 1) {
-    if ((int)threadIdx.x < k) sh[threadIdx.x] = fmax(sh[threadIdx.x], sh[threadIdx.x + k]);
-    __syncthreads();
-  }
-  double r = sh[0];
+  const double r = fmin(fmin(sh[0], sh[1]), fmin(sh[2], sh[3]));
   __syncthreads();
   return r;
 }
@@ -430,58 +511,47 @@ struct SourceMoments {
   double m[kNMom];
 };
 
-__device__ void source_moments(const int* __restrict__ src_perm, const double* __restrict__ x,
-                               const double* __restrict__ y, const double* __restrict__ z,
-                               const double* __restrict__ q, const double* __restrict__ area, int s0, int s1,
-                               double* sh, SourceMoments& r) {
-  double ax = 0, ay = 0, az = 0, aa = 0;
+// The centroid alone (v: area-weighted x, y, z and the area).
+__device__ __forceinline__ void set_centroid(const double v[4], SourceMoments& r) {
+  r.cx = v[3] > 0 ? v[0] / v[3] : 0.0;
+  r.cy = v[3] > 0 ? v[1] / v[3] : 0.0;
+  r.cz = v[3] > 0 ? v[2] / v[3] : 1.0;
+  const double cn = sqrt(r.cx * r.cx + r.cy * r.cy + r.cz * r.cz);
+  r.ux = r.cx / cn;
+  r.uy = r.cy / cn;
+  r.uz = r.cz / cn;
+}
+
+// Moments, sum |w| and angular radius about the centroid in r.  The radius is the
+// arc cosine of the smallest cosine: one arc cosine a block, not one a source.
+__device__ void source_moments(const GeomArgs& a, int s0, int s1, double* sh, SourceMoments& r) {
+  double v[kNMom + 1];
+#pragma unroll
+  for (int k = 0; k <= kNMom; ++k) v[k] = 0.0;
+  double cosmin = 1.0;
   for (int j = s0 + threadIdx.x; j < s1; j += 256) {
-    const int p = src_perm[j];
-    const double w = area[p];
-    ax += w * x[p];
-    ay += w * y[p];
-    az += w * z[p];
-    aa += w;
-  }
-  ax = block_sum(ax, sh);
-  ay = block_sum(ay, sh);
-  az = block_sum(az, sh);
-  aa = block_sum(aa, sh);
-  const double cx = aa > 0 ? ax / aa : 0.0, cy = aa > 0 ? ay / aa : 0.0, cz = aa > 0 ? az / aa : 1.0;
-  const double cn = sqrt(cx * cx + cy * cy + cz * cz);
-  const double ux = cx / cn, uy = cy / cn, uz = cz / cn;
-  double* m = r.m;
-  for (int k = 0; k < kNMom; ++k) m[k] = 0.0;
-  double wabs = 0.0, rho = 0.0;
-  for (int j = s0 + threadIdx.x; j < s1; j += 256) {
-    const int p = src_perm[j];
-    const double w = q[p] * area[p];
-    const double d[3] = {x[p] - cx, y[p] - cy, z[p] - cz};
-    m[0] += w;
+    const int p = a.src_perm[j];
+    const double x = a.x[p], y = a.y[p], z = a.z[p];
+    const double w = a.q[p] * a.area[p];
+    const double d[3] = {x - r.cx, y - r.cy, z - r.cz};
+    v[0] += w;
 #pragma unroll
-    for (int i = 0; i < 3; ++i) m[1 + i] += w * d[i];
+    for (int i = 0; i < 3; ++i) v[1 + i] += w * d[i];
 #pragma unroll
-    for (int i = 0; i < 6; ++i) m[kMomOff[2] + i] += w * d[kPair[i][0]] * d[kPair[i][1]];
+    for (int i = 0; i < 6; ++i) v[kMomOff[2] + i] += w * d[kPair[i][0]] * d[kPair[i][1]];
 #pragma unroll
-    for (int i = 0; i < 10; ++i) m[kMomOff[3] + i] += w * d[kTri[i][0]] * d[kTri[i][1]] * d[kTri[i][2]];
+    for (int i = 0; i < 10; ++i) v[kMomOff[3] + i] += w * d[kTri[i][0]] * d[kTri[i][1]] * d[kTri[i][2]];
 #pragma unroll
     for (int i = 0; i < 15; ++i)
-      m[kMomOff[4] + i] += w * d[kQuad[i][0]] * d[kQuad[i][1]] * d[kQuad[i][2]] * d[kQuad[i][3]];
-    wabs += fabs(w);
-    const double rr = sqrt(x[p] * x[p] + y[p] * y[p] + z[p] * z[p]);
-    const double cosang = (x[p] * ux + y[p] * uy + z[p] * uz) / rr;
-    rho = fmax(rho, acos(fmin(1.0, fmax(-1.0, cosang))));
+      v[kMomOff[4] + i] += w * d[kQuad[i][0]] * d[kQuad[i][1]] * d[kQuad[i][2]] * d[kQuad[i][3]];
+    v[kNMom] += fabs(w);
+    cosmin = fmin(cosmin, (x * r.ux + y * r.uy + z * r.uz) / sqrt(x * x + y * y + z * z));
   }
+  block_sums(v, sh);
 #pragma unroll
-  for (int k = 0; k < kNMom; ++k) m[k] = block_sum(m[k], sh);
-  r.wabs = block_sum(wabs, sh);
-  r.rho = block_max(rho, sh);
-  r.cx = cx;
-  r.cy = cy;
-  r.cz = cz;
-  r.ux = ux;
-  r.uy = uy;
-  r.uz = uz;
+  for (int k = 0; k < kNMom; ++k) r.m[k] = v[k];
+  r.wabs = v[kNMom];
+  r.rho = acos(fmax(-1.0, block_min(cosmin, sh)));
 }
 
 // The FP32 far record of far_expansion_acc: c, e_c = R^2 - |c|^2, the moments
@@ -497,27 +567,52 @@ __device__ void write_far_record(float* fr, const SourceMoments& sm, double R) {
   fr[4 + kNMom] = (float)sm.rho;
 }
 
+// One block per cell, then one per parent.  Parent p is the four cells 4p .. 4p+3,
+// whose sources are contiguous in cell order; it has a far record (after the
+// cells' records) and its geometry only.  Both kinds wait on gathers and on the
+// block's sums; at 491,522 particles and 1,280 + 320 blocks 36 us, against 88 + 42 with
+// a sum of its own, nine barriers long, for each of the 45 values.
 __global__ __launch_bounds__(256) void ff_cell_geometry(GeomArgs a) {
-  __shared__ double sh[256];
-  const int c = blockIdx.x;
-  const int s0 = a.src_start[c], s1 = a.src_start[c + 1];
-  const int t0 = a.tgt_start[c], t1 = a.tgt_start[c + 1];
+  __shared__ double sh[kRedWords];
+  const bool cell = (int)blockIdx.x < a.ncell;
+  const int c = cell ? blockIdx.x : blockIdx.x - a.ncell;
+  const int s0 = a.src_start[cell ? c : 4 * c], s1 = a.src_start[cell ? c + 1 : 4 * c + 4];
+  const int t0 = cell ? a.tgt_start[c] : 0, t1 = cell ? a.tgt_start[c + 1] : 0;
+  double v[7] = {};
+  for (int j = s0 + threadIdx.x; j < s1; j += 256) {
+    const int p = a.src_perm[j];
+    const double w = a.area[p];
+    v[0] += w * a.x[p];
+    v[1] += w * a.y[p];
+    v[2] += w * a.z[p];
+    v[3] += w;
+  }
+  for (int k = t0 + threadIdx.x; k < t1; k += 256) {
+    const int p = a.tgt_perm[k];
+    v[4] += a.x[p];
+    v[5] += a.y[p];
+    v[6] += a.z[p];
+  }
+  block_sums(v, sh);
   SourceMoments sm;
-  source_moments(a.src_perm, a.x, a.y, a.z, a.q, a.area, s0, s1, sh, sm);
+  set_centroid(v, sm);
+  source_moments(a, s0, s1, sh, sm);
+  if (!cell) {
+    if (threadIdx.x == 0) {
+      write_far_record(a.far_rec + (size_t)(a.ncell + c) * kCellRec, sm, a.radius);
+      double* g = a.pgeo + (size_t)c * 4;
+      g[0] = sm.ux;
+      g[1] = sm.uy;
+      g[2] = sm.uz;
+      g[3] = sm.rho;
+    }
+    return;
+  }
   const double cx = sm.cx, cy = sm.cy, cz = sm.cz, ux = sm.ux, uy = sm.uy, uz = sm.uz;
   const double* m = sm.m;
   const double wabs = sm.wabs, rho = sm.rho;
   // target cell direction and radius
-  double tx = 0, ty = 0, tz = 0;
-  for (int k = t0 + threadIdx.x; k < t1; k += 256) {
-    const int p = a.tgt_perm[k];
-    tx += a.x[p];
-    ty += a.y[p];
-    tz += a.z[p];
-  }
-  tx = block_sum(tx, sh);
-  ty = block_sum(ty, sh);
-  tz = block_sum(tz, sh);
+  double tx = v[4], ty = v[5], tz = v[6];
   double tn = sqrt(tx * tx + ty * ty + tz * tz);
   if (!(tn > 0)) {
     tx = ux;
@@ -526,14 +621,13 @@ __global__ __launch_bounds__(256) void ff_cell_geometry(GeomArgs a) {
     tn = 1.0;
   }
   const double vx = tx / tn, vy = ty / tn, vz = tz / tn;
-  double trho = 0.0;
+  double cosmin = 1.0;
   for (int k = t0 + threadIdx.x; k < t1; k += 256) {
     const int p = a.tgt_perm[k];
-    const double r = sqrt(a.x[p] * a.x[p] + a.y[p] * a.y[p] + a.z[p] * a.z[p]);
-    const double cosang = (a.x[p] * vx + a.y[p] * vy + a.z[p] * vz) / r;
-    trho = fmax(trho, acos(fmin(1.0, fmax(-1.0, cosang))));
+    const double x = a.x[p], y = a.y[p], z = a.z[p];
+    cosmin = fmin(cosmin, (x * vx + y * vy + z * vz) / sqrt(x * x + y * y + z * z));
   }
-  trho = block_max(trho, sh);
+  const double trho = acos(fmax(-1.0, block_min(cosmin, sh)));
   if (threadIdx.x == 0) {
     const double R = a.radius;
     const double inv = 1.0 / (4.0 * kPi * R);
@@ -601,32 +695,6 @@ __global__ __launch_bounds__(256) void ff_cell_geometry(GeomArgs a) {
     a.cen64[(size_t)c * 3 + 1] = cy;
     a.cen64[(size_t)c * 3 + 2] = cz;
     for (int k = 0; k < kNMom; ++k) a.mom64[(size_t)c * kNMom + k] = m[k];
-  }
-}
-
-// Coarse level: parent p is the four cells 4p .. 4p+3, whose sources are
-// contiguous in cell order.  Its far record (after the cells' records) and its
-// geometry {direction of c (3), rho}.
-struct ParentArgs {
-  const int *src_perm, *src_start;
-  const double *x, *y, *z, *q, *area;
-  double radius;
-  float* far_rec;  // [npar][kCellRec]
-  double* pgeo;    // [npar][4]
-};
-
-__global__ __launch_bounds__(256) void ff_parent_geometry(ParentArgs a) {
-  __shared__ double sh[256];
-  const int p = blockIdx.x;
-  SourceMoments sm;
-  source_moments(a.src_perm, a.x, a.y, a.z, a.q, a.area, a.src_start[4 * p], a.src_start[4 * p + 4], sh, sm);
-  if (threadIdx.x == 0) {
-    write_far_record(a.far_rec + (size_t)p * kCellRec, sm, a.radius);
-    double* g = a.pgeo + (size_t)p * 4;
-    g[0] = sm.ux;
-    g[1] = sm.uy;
-    g[2] = sm.uz;
-    g[3] = sm.rho;
   }
 }
 
@@ -947,16 +1015,6 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(7))) void f
   }
 }
 
-// V = the near partials, then the far partials, summed in this fixed order.
-__global__ __launch_bounds__(256) void ff_sum_parts(int nt, int nparts, const double* __restrict__ part,
-                                                    double* __restrict__ V) {
-  const int k = blockIdx.x * blockDim.x + threadIdx.x;
-  if (k >= 3 * nt) return;
-  double v = part[k];
-  for (int sp = 1; sp < nparts; ++sp) v += part[(size_t)sp * 3 * nt + k];
-  V[k] = v;
-}
-
 // --------------------------------------------------- MLP correction (MFMA)
 // Target position in the cell frame, Q (x - c) / l.
 __device__ __forceinline__ void mlp_local(const float* mr, float x, float y, float z, float loc[3]) {
@@ -995,7 +1053,7 @@ struct MlpCorrArgs {
   int ncell, nt, order;
   const lpm::mlp_t* frag;
   const float* bias;
-  double* out;        // [3][nt] accumulated into
+  double* part;       // [3][nt] this launch's partial
 };
 
 // 512 threads: 8 waves (2 per SIMD) share one LDS copy of the weights, which
@@ -1068,21 +1126,30 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
         const int k = k0 + 16 * ct + lane;
         if (k < k_end)
 #pragma unroll
-          for (int c = 0; c < 3; ++c) a.out[(size_t)c * a.nt + k] += (double)acc[ct][c];
+          for (int c = 0; c < 3; ++c) a.part[(size_t)c * a.nt + k] = (double)acc[ct][c];
       }
     }
   }
 }
 
 // ---------------------------------------------------------------- epilogue
-__global__ __launch_bounds__(256) void ff_epilogue(int nt, const int* __restrict__ perm, const double* __restrict__ V,
-                                                   const double* __restrict__ x, const double* __restrict__ y,
-                                                   const double* __restrict__ z, double* __restrict__ u,
-                                                   double* __restrict__ v, double* __restrict__ w) {
+// V = the near partials, the far partials, then the network's, summed in this
+// fixed order; u = V x x, in the particles' own order.
+__global__ __launch_bounds__(256) void ff_epilogue(int nt, int nparts, const int* __restrict__ perm,
+                                                   const double* __restrict__ part, const double* __restrict__ x,
+                                                   const double* __restrict__ y, const double* __restrict__ z,
+                                                   double* __restrict__ u, double* __restrict__ v,
+                                                   double* __restrict__ w) {
   int k = blockIdx.x * blockDim.x + threadIdx.x;
   if (k >= nt) return;
   const int p = perm[k];
-  const double A0 = V[k], A1 = V[(size_t)nt + k], A2 = V[(size_t)2 * nt + k];
+  double V[3];
+#pragma unroll
+  for (int c = 0; c < 3; ++c) V[c] = part[(size_t)c * nt + k];
+  for (int sp = 1; sp < nparts; ++sp)
+#pragma unroll
+    for (int c = 0; c < 3; ++c) V[c] += part[(size_t)(3 * sp + c) * nt + k];
+  const double A0 = V[0], A1 = V[1], A2 = V[2];
   const double px = x[p], py = y[p], pz = z[p];
   u[p] = A1 * pz - A2 * py;
   v[p] = A2 * px - A0 * pz;
@@ -1098,7 +1165,9 @@ struct SampleArgs {
   int n_samples;
   unsigned long long seed;
   int nt, ncell, order;
-  const int *tgt_perm, *tgt_cell, *src_perm, *src_start, *band_list, *band_count;
+  const int* tgt_perm;
+  const unsigned* tgt_cell;
+  const int *src_perm, *src_start, *band_list, *band_count;
   const double *x, *y, *z, *q, *area;
   const double *cen64, *mom64;
   const float* mlp_rec;
@@ -1134,7 +1203,7 @@ __global__ __launch_bounds__(256) void ff_make_samples(SampleArgs a) {
   for (int attempt = 0; attempt < 8 && !ok; ++attempt) {
     const int k = (int)(h % (unsigned long long)a.nt);
     h = mix64(h);
-    const int t = a.tgt_cell[k];
+    const int t = (int)a.tgt_cell[k];
     const int nb = a.band_count[t];
     if (nb == 0) continue;
     const int p = a.tgt_perm[k];
@@ -1287,11 +1356,11 @@ struct lpm_bve_ff {
   DevBuf xi, yi, zi, qi;
   DevBuf pu, pv, pw;  // plain-sum velocity (judge)
   // binning: cell-ordered particle lists rebuilt at every evaluation
-  DevBuf src_perm, src_key, src_start, tgt_perm, tgt_cell, tgt_start;
-  DevBuf key_t, key_s, iota, cellof, active, sort_tmp, item_count;
+  DevBuf src_perm, src_start, tgt_perm, tgt_start;
+  DevBuf cellof, active, sort_tmp, item_count;
+  const unsigned* tgt_cell = nullptr;  // cell of each ordered target, in sort_tmp
   DevBuf gen, adir;  // cell generator directions (float4), frame anchor directions (FP64)
-  int end_bit = 0;
-  size_t sort_bytes = 0;
+  DevBuf bins;       // LocBin per direction bin: the generators' search, laid out once
   DevBuf trec, srec, far_rec, mlp_rec, geo, cen64, mom64;
   DevBuf near_list, near_count, band_list, band_count;
   DevBuf far_list, far_count;  // expansion records per target cell (cells or parents)
@@ -1299,8 +1368,7 @@ struct lpm_bve_ff {
   int npar = 0;                // parents in use (0: no coarse level)
   double r_par = 0.0;          // a parent replaces its 4 cells beyond this radius
   DevBuf items, mlp_items;
-  DevBuf V;
-  DevBuf Vpart;        // FP64 partials [near_split + far_split][3][n]: near, then far
+  DevBuf Vpart;        // FP64 partials [near_split + far_split + 1][3][n]: near, far, network
   int near_split = 1;  // near lists split in this many parts (fills the chip)
   int far_split = 1;   // far cells split in this many ranges
   DevBuf list_plain;  // ascending active list for the plain path
@@ -1331,19 +1399,15 @@ int ff_upload(lpm_ctx* ctx, DevBuf& b, const void* host, size_t bytes) {
 int ff_bin(lpm_bve_ff* f, const double* x, const double* y, const double* z) {
   lpm_ctx* ctx = f->ctx;
   const int n = f->n, nc = f->ncell;
-  hipLaunchKernelGGL(ff_locate, dim3((n + 256 * kLocR - 1) / (256 * kLocR)), dim3(256), 0, ctx->stream, n, nc,
-                     f->gen.as<lpm::Vec4<float>>(), x, y, z, f->active.as<int>(), f->cellof.as<int>(),
-                     f->key_t.as<int>(), f->key_s.as<int>(), f->iota.as<int>());
-  size_t bytes = f->sort_bytes;
-  LPM_HIP(ctx, hipcub::DeviceRadixSort::SortPairs(f->sort_tmp.p, bytes, f->key_t.as<int>(), f->tgt_cell.as<int>(),
-                                                  f->iota.as<int>(), f->tgt_perm.as<int>(), n, 0, f->end_bit,
-                                                  ctx->stream));
-  bytes = f->sort_bytes;
-  LPM_HIP(ctx, hipcub::DeviceRadixSort::SortPairs(f->sort_tmp.p, bytes, f->key_s.as<int>(), f->src_key.as<int>(),
-                                                  f->iota.as<int>(), f->src_perm.as<int>(), n, 0, f->end_bit,
-                                                  ctx->stream));
-  hipLaunchKernelGGL(ff_bounds, dim3((nc + 1 + 255) / 256), dim3(256), 0, ctx->stream, n, nc, f->tgt_cell.as<int>(),
-                     f->src_key.as<int>(), f->tgt_start.as<int>(), f->src_start.as<int>());
+  const lpm::CellSort sort = lpm::cell_sort_input(f->sort_tmp, n);
+  hipLaunchKernelGGL(ff_locate, dim3((n + 255) / 256), dim3(256), 0, ctx->stream, n, nc, loc_grid(nc),
+                     f->gen.as<lpm::Vec4<float>>(), f->bins.as<LocBin>(), x, y, z, f->active.as<int>(),
+                     f->cellof.as<int>(), sort);
+  const unsigned* src_key = nullptr;
+  lpm::cell_sort(ctx->stream, f->sort_tmp, n, 32 - __builtin_clz((unsigned)nc), f->tgt_perm.as<int>(),
+                 f->src_perm.as<int>(), &f->tgt_cell, &src_key);  // keys 0..ncell
+  hipLaunchKernelGGL(ff_bounds, dim3((n + 1 + 255) / 256), dim3(256), 0, ctx->stream, n, nc, f->tgt_cell, src_key,
+                     f->tgt_start.as<int>(), f->src_start.as<int>());
   hipLaunchKernelGGL(ff_make_items, dim3(1), dim3(1024), 0, ctx->stream, nc, f->tgt_start.as<int>(), 64 * kR, kMlpTile,
                      f->items.as<int2>(), f->mlp_items.as<int2>(), f->item_count.as<int>());
   LPM_HIP(ctx, hipGetLastError());
@@ -1387,13 +1451,9 @@ int ff_eval(lpm_bve_ff* f, int mode, const double* x, const double* y, const dou
   lpm::launch_pack(LPM_K_SPHERE_BS, LPM_PREC_FP32_KAHAN, pa, f->srec.p, nullptr, f->ns, 0, ctx->stream);
   GeomArgs ga{nc, f->src_perm.as<int>(), f->src_start.as<int>(), f->tgt_perm.as<int>(), f->tgt_start.as<int>(),
               x, y, z, q, f->area.as<double>(), f->radius, f->far_rec.as<float>(), f->mlp_rec.as<float>(),
-              f->adir.as<double>(), f->geo.as<double>(), f->cen64.as<double>(), f->mom64.as<double>()};
-  hipLaunchKernelGGL(ff_cell_geometry, dim3(nc), b256, 0, ctx->stream, ga);
-  if (f->npar) {
-    ParentArgs pa2{f->src_perm.as<int>(), f->src_start.as<int>(), x, y, z, q, f->area.as<double>(), f->radius,
-                   f->far_rec.as<float>() + (size_t)nc * kCellRec, f->pgeo.as<double>()};
-    hipLaunchKernelGGL(ff_parent_geometry, dim3(f->npar), b256, 0, ctx->stream, pa2);
-  }
+              f->adir.as<double>(), f->geo.as<double>(), f->cen64.as<double>(), f->mom64.as<double>(),
+              f->pgeo.as<double>()};
+  hipLaunchKernelGGL(ff_cell_geometry, dim3(nc + f->npar), b256, 0, ctx->stream, ga);
   ClassArgs ca{nc, f->geo.as<double>(), f->r_near, f->r_band, f->near_list.as<int>(),
                f->near_count.as<int>(), f->band_list.as<int>(), f->band_count.as<int>()};
   hipLaunchKernelGGL(ff_classify, dim3(nc), b256, 0, ctx->stream, ca);
@@ -1417,21 +1477,21 @@ int ff_eval(lpm_bve_ff* f, int mode, const double* x, const double* y, const dou
   if (f->order == 2) hipLaunchKernelGGL(ff_far_kernel<2>, gfar, b256, 0, ctx->stream, fa);
   else if (f->order == 3) hipLaunchKernelGGL(ff_far_kernel<3>, gfar, b256, 0, ctx->stream, fa);
   else hipLaunchKernelGGL(ff_far_kernel<4>, gfar, b256, 0, ctx->stream, fa);
-  hipLaunchKernelGGL(ff_sum_parts, dim3((3 * f->n + 255) / 256), b256, 0, ctx->stream, f->n,
-                     f->near_split + f->far_split, f->Vpart.as<double>(), f->V.as<double>());
+  int nparts = f->near_split + f->far_split;
   if (mode == 2 && f->trained) {
     MlpCorrArgs ma{f->trec.as<lpm::Vec4<float>>(), f->tgt_start.as<int>(), f->mlp_rec.as<float>(),
                    f->band_list.as<int>(), f->band_count.as<int>(), f->mlp_items.as<int2>(), f->item_count.as<int>() + 1, nc, f->n,
                    f->order,
-                   f->net.frag.as<lpm::mlp_t>(), f->net.bias.as<float>(), f->V.as<double>()};
+                   f->net.frag.as<lpm::mlp_t>(), f->net.bias.as<float>(), f->Vpart.as<double>() + (size_t)3 * nparts * f->n};
+    ++nparts;
     hipLaunchKernelGGL(ff_mlp_kernel, dim3(ctx->num_cus), dim3(512), 0, ctx->stream, ma);
   }
   if (ctx->timing && e0 && e1) {
     LPM_HIP(ctx, hipEventRecord(e1, ctx->stream));
     ctx->pending.push_back({e0, e1, LPM_K_FAR_FIELD});
   }
-  hipLaunchKernelGGL(ff_epilogue, dim3((f->n + 255) / 256), b256, 0, ctx->stream, f->n, f->tgt_perm.as<int>(),
-                     f->V.as<double>(), x, y, z, u, v, w);
+  hipLaunchKernelGGL(ff_epilogue, dim3((f->n + 255) / 256), b256, 0, ctx->stream, f->n, nparts, f->tgt_perm.as<int>(),
+                     f->Vpart.as<double>(), x, y, z, u, v, w);
   LPM_HIP(ctx, hipGetLastError());
   return LPM_OK;
 }
@@ -1516,17 +1576,9 @@ int ff_load(lpm_bve_ff* f, int n, const double* x, const double* y, const double
                              : f->order == 3 ? reinterpret_cast<const void*>(ff_far_kernel<3>)
                                              : reinterpret_cast<const void*>(ff_far_kernel<4>));
   }
-  const int end_bit = 32 - __builtin_clz((unsigned)ncell);  // keys 0..ncell
-  size_t sort_bytes = 0;
-  const hipError_t sort_query =
-      hipcub::DeviceRadixSort::SortPairs(nullptr, sort_bytes, (const int*)nullptr, (int*)nullptr, (const int*)nullptr,
-                                         (int*)nullptr, n, 0, end_bit, ctx->stream);
-  f->end_bit = end_bit;
-  f->sort_bytes = sort_bytes;
   const size_t nb = (size_t)n * sizeof(double);
   const size_t ni = (size_t)n * sizeof(int);
-  int rc = sort_query == hipSuccess ? LPM_OK
-                                    : fail(ctx, LPM_ERR_HIP, "lpm_bve_ff_new: radix-sort workspace query failed");
+  int rc = LPM_OK;
   auto chk = [&](int r) {
     if (r && !rc) rc = r;
     return rc == LPM_OK;
@@ -1538,14 +1590,13 @@ int ff_load(lpm_bve_ff* f, int n, const double* x, const double* y, const double
       chk(ff_upload(ctx, f->pv, nullptr, nb)) && chk(ff_upload(ctx, f->pw, nullptr, nb)) &&
       chk(ff_upload(ctx, f->xi, nullptr, nb)) && chk(ff_upload(ctx, f->yi, nullptr, nb)) &&
       chk(ff_upload(ctx, f->zi, nullptr, nb)) && chk(ff_upload(ctx, f->qi, nullptr, nb)) &&
-      chk(ff_upload(ctx, f->src_perm, nullptr, ni)) && chk(ff_upload(ctx, f->src_key, nullptr, ni)) &&
+      chk(ff_upload(ctx, f->src_perm, nullptr, ni)) &&
       chk(ff_upload(ctx, f->src_start, nullptr, ((size_t)ncell + 1) * 4)) &&
-      chk(ff_upload(ctx, f->tgt_perm, nullptr, ni)) && chk(ff_upload(ctx, f->tgt_cell, nullptr, ni)) &&
+      chk(ff_upload(ctx, f->tgt_perm, nullptr, ni)) &&
       chk(ff_upload(ctx, f->tgt_start, nullptr, ((size_t)ncell + 1) * 4)) &&
-      chk(ff_upload(ctx, f->key_t, nullptr, ni)) && chk(ff_upload(ctx, f->key_s, nullptr, ni)) &&
-      chk(ff_upload(ctx, f->iota, nullptr, ni)) && chk(ff_upload(ctx, f->cellof, nullptr, ni)) &&
+      chk(ff_upload(ctx, f->cellof, nullptr, ni)) &&
       chk(ff_upload(ctx, f->active, act.data(), ni)) &&
-      chk(ff_upload(ctx, f->sort_tmp, nullptr, std::max<size_t>(sort_bytes, 16))) &&
+      chk(ff_upload(ctx, f->sort_tmp, nullptr, lpm::cell_sort_bytes(n))) &&
       chk(ff_upload(ctx, f->item_count, nullptr, 2 * 4)) &&
       chk(ff_upload(ctx, f->list_plain, plain.data(), std::max<size_t>(plain.size(), 1) * 4)) &&
       chk(ff_upload(ctx, f->items, nullptr, (size_t)f->n_items * sizeof(int2))) &&
@@ -1562,8 +1613,8 @@ int ff_load(lpm_bve_ff* f, int n, const double* x, const double* y, const double
       chk(ff_upload(ctx, f->near_list, nullptr, (size_t)ncell * ncell * 4)) &&
       chk(ff_upload(ctx, f->near_count, nullptr, (size_t)ncell * 4)) &&
       chk(ff_upload(ctx, f->band_list, nullptr, (size_t)ncell * ncell * 4)) &&
-      chk(ff_upload(ctx, f->band_count, nullptr, (size_t)ncell * 4)) && chk(ff_upload(ctx, f->V, nullptr, 3 * nb)) &&
-      chk(ff_upload(ctx, f->Vpart, nullptr, (size_t)(f->near_split + f->far_split) * 3 * nb));
+      chk(ff_upload(ctx, f->band_count, nullptr, (size_t)ncell * 4)) &&
+      chk(ff_upload(ctx, f->Vpart, nullptr, (size_t)(f->near_split + f->far_split + 1) * 3 * nb));
   for (int s = 0; s < 4 && rc == LPM_OK; ++s)
     for (int c = 0; c < 4 && rc == LPM_OK; ++c) chk(ff_upload(ctx, f->k[s][c], nullptr, nb));
   if (rc == LPM_OK) {
@@ -1679,8 +1730,15 @@ int lpm_bve_ff_new(lpm_ctx* ctx, lpm_bve_ff** out, int n, const double* x, const
     if (r && !rc) rc = r;
     return rc == LPM_OK;
   };
-  chk(ff_upload(ctx, f->gen, gen.data(), (size_t)ncell * sizeof(lpm::Vec4<float>))) &&
-      chk(ff_upload(ctx, f->adir, adir.data(), adir.size() * 8)) && chk(f->net.init(ctx, 13, 128, 3, 3, LPM_ACT_ISRU, 12345)) &&
+  const int g = loc_grid(ncell), nbins = 6 * g * g;
+  if (chk(ff_upload(ctx, f->gen, gen.data(), (size_t)ncell * sizeof(lpm::Vec4<float>))) &&
+      chk(ff_upload(ctx, f->bins, nullptr, (size_t)nbins * sizeof(LocBin)))) {
+    hipLaunchKernelGGL(ff_locate_bins, dim3((nbins + 255) / 256), dim3(256), 0, ctx->stream, ncell, g,
+                       f->gen.as<lpm::Vec4<float>>(), f->bins.as<LocBin>());
+    const hipError_t e = hipGetLastError();
+    if (e != hipSuccess) rc = lpm::hip_fail(ctx, e, "ff_locate_bins");
+  }
+  chk(rc) && chk(ff_upload(ctx, f->adir, adir.data(), adir.size() * 8)) && chk(f->net.init(ctx, 13, 128, 3, 3, LPM_ACT_ISRU, 12345)) &&
       chk(ff_load(f, n, x, y, z, relvort, area, active));
   if (rc != LPM_OK) {
     lpm_bve_ff_delete(f);
@@ -1741,7 +1799,7 @@ int lpm_bve_ff_collect(lpm_bve_ff* f, int n_samples, uint64_t seed, int64_t* tot
     nx.p = ny.p = ni.p = nullptr;
     f->cap_collected = cap;
   }
-  SampleArgs sa{n_samples, (unsigned long long)seed, f->n, f->ncell, f->order, f->tgt_perm.as<int>(), f->tgt_cell.as<int>(),
+  SampleArgs sa{n_samples, (unsigned long long)seed, f->n, f->ncell, f->order, f->tgt_perm.as<int>(), f->tgt_cell,
                 f->src_perm.as<int>(), f->src_start.as<int>(), f->band_list.as<int>(), f->band_count.as<int>(),
                 f->x.as<double>(), f->y.as<double>(), f->z.as<double>(), f->q.as<double>(), f->area.as<double>(),
                 f->cen64.as<double>(), f->mom64.as<double>(), f->mlp_rec.as<float>(), f->radius,
@@ -1976,12 +2034,12 @@ int lpm_bve_ff_delete(lpm_bve_ff* f) {
   if (!f) return LPM_ERR_ARG;
   (void)hipStreamSynchronize(f->ctx->stream);
   DevBuf* all[] = {&f->x, &f->y, &f->z, &f->q, &f->u, &f->v, &f->w, &f->area, &f->xi, &f->yi, &f->zi, &f->qi,
-                   &f->pu, &f->pv, &f->pw, &f->src_perm, &f->src_start, &f->tgt_perm, &f->tgt_start, &f->tgt_cell,
+                   &f->pu, &f->pv, &f->pw, &f->src_perm, &f->src_start, &f->tgt_perm, &f->tgt_start,
                    &f->trec, &f->srec, &f->far_rec, &f->mlp_rec, &f->geo, &f->cen64, &f->mom64, &f->far_list, &f->far_count, &f->pgeo,
-                   &f->near_list, &f->near_count, &f->band_list, &f->band_count, &f->items, &f->mlp_items, &f->V,
+                   &f->near_list, &f->near_count, &f->band_list, &f->band_count, &f->items, &f->mlp_items,
                    &f->list_plain, &f->tgt_plain, &f->src_plain, &f->partial_plain, &f->ptrs, &f->err_part, &f->sx,
-                   &f->sy, &f->sid, &f->src_key, &f->key_t, &f->key_s, &f->iota, &f->cellof, &f->active,
-                   &f->sort_tmp, &f->item_count, &f->gen, &f->adir, &f->Vpart};
+                   &f->sy, &f->sid, &f->cellof, &f->active,
+                   &f->sort_tmp, &f->item_count, &f->gen, &f->bins, &f->adir, &f->Vpart};
   for (DevBuf* b : all) b->release();
   for (auto& row : f->k)
     for (auto& b : row) b.release();

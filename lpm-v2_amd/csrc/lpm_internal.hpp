@@ -236,6 +236,17 @@ struct OrderInput {
 size_t order_bytes(int nt, int ns);  // spatial_order allocates nothing in a buffer of this size
 int spatial_order(lpm_ctx* ctx, const OrderInput& in, DevBuf& buf, int** tgt_order, int** src_order);
 
+// The same stable sort on n targets and n sources with keys of the caller's:
+// `buf` holds cell_sort_bytes(n); fill the input, then sort by `bits` bits.
+struct CellSort {
+  unsigned *tgt_key, *src_key;
+  int *tgt_val, *src_val;
+};
+size_t cell_sort_bytes(int n);
+CellSort cell_sort_input(DevBuf& buf, int n);
+void cell_sort(hipStream_t st, DevBuf& buf, int n, int bits, int* tgt_perm, int* src_perm, const unsigned** tgt_key,
+               const unsigned** src_key);
+
 int blocks_per_cu(const void* kernel);
 hipEvent_t take_event(lpm_ctx* ctx);
 

@@ -11,7 +11,7 @@
 // digit counts, a scan per digit, stable scatter.  Targets and sources go through the same
 // launches (two segments), keys have 16-24 bits, so ordering both takes 7-11 short
 // launches.  It is deterministic, allocates nothing and holds no memset, so it may
-// be captured.  The library sort that it stands beside takes a merge-sort path of
+// be captured.  rocPRIM's sort takes a merge-sort path of
 // about 24 launches (130 us) at these sizes.
 #include "lpm_internal.hpp"
 
@@ -57,7 +57,6 @@ struct Segment {
 
 struct OrderDev {
   Segment seg[2];
-  int blocks0;  // sort blocks of segment 0
   int k;        // bits per coordinate
   int sphere;
   const double* box;  // plane: kBoxBlocks x {xmin, ymin, xmax, ymax}
@@ -308,7 +307,61 @@ __global__ __launch_bounds__(kSortThreads) void sort_scatter(SortDev a) {
 int sort_blocks(int n) { return (n + kSortItems - 1) / kSortItems; }
 size_t up256(size_t b) { return (b + 255) / 256 * 256; }
 
+// Buffers of a sort of n0 + n1 items, laid out from p.
+struct SortSpace {
+  unsigned* key[2];
+  int* val[2];
+  int *hist, *total;
+};
+
+SortSpace sort_space(char* p, int n0, int n1) {
+  auto take = [&](size_t b) {
+    char* r = p;
+    p += up256(b);
+    return r;
+  };
+  const size_t items = (size_t)n0 + n1;
+  SortSpace w;
+  for (int q = 0; q < 2; ++q) w.key[q] = reinterpret_cast<unsigned*>(take(items * 4));
+  for (int q = 0; q < 2; ++q) w.val[q] = reinterpret_cast<int*>(take(items * 4));
+  w.hist = reinterpret_cast<int*>(take(((size_t)sort_blocks(n0) + sort_blocks(n1)) * kBins * 4));
+  w.total = reinterpret_cast<int*>(take(2 * kBins * 4));
+  return w;
+}
+
+// Sort key[0], val[0] (segment 0, then segment 1) by `bits` bits; the values go to
+// out0 and out1, the sorted keys to key[passes & 1].
+const unsigned* sort_pairs(hipStream_t st, const SortSpace& w, int n0, int n1, int bits, int* out0, int* out1) {
+  const int b0 = sort_blocks(n0), b1 = sort_blocks(n1);
+  const int passes = (bits + 7) / 8;
+  for (int q = 0; q < passes; ++q) {
+    const bool last = q == passes - 1;
+    SortDev s{n0, n1, b0, b1, 8 * q, w.key[q & 1], w.val[q & 1], w.key[(q + 1) & 1],
+              last ? out0 : w.val[(q + 1) & 1], last ? out1 : w.val[(q + 1) & 1] + n0, w.hist, w.total};
+    hipLaunchKernelGGL(sort_count, dim3(b0 + b1), dim3(kSortThreads), 0, st, s);
+    hipLaunchKernelGGL(sort_scan, dim3(2 * kBins), dim3(256), 0, st, s);
+    hipLaunchKernelGGL(sort_scatter, dim3(b0 + b1), dim3(kSortThreads), 0, st, s);
+  }
+  return w.key[passes & 1];
+}
+
 }  // namespace
+
+size_t cell_sort_bytes(int n) {
+  return 4 * up256(2 * (size_t)n * 4) + up256(2 * (size_t)sort_blocks(n) * kBins * 4) + up256(2 * kBins * 4);
+}
+
+CellSort cell_sort_input(DevBuf& buf, int n) {
+  const SortSpace w = sort_space(buf.as<char>(), n, n);
+  return CellSort{w.key[0], w.key[0] + n, w.val[0], w.val[0] + n};
+}
+
+void cell_sort(hipStream_t st, DevBuf& buf, int n, int bits, int* tgt_perm, int* src_perm, const unsigned** tgt_key,
+               const unsigned** src_key) {
+  const unsigned* k = sort_pairs(st, sort_space(buf.as<char>(), n, n), n, n, bits, tgt_perm, src_perm);
+  *tgt_key = k;
+  *src_key = k + n;
+}
 
 size_t order_bytes(int nt, int ns) {
   const size_t items = (size_t)nt + ns;
@@ -329,14 +382,8 @@ int spatial_order(lpm_ctx* ctx, const OrderInput& in, DevBuf& buf, int** tgt_ord
   // the results first: their place depends on nt and ns alone
   int* tout = reinterpret_cast<int*>(take((size_t)in.nt * 4));
   int* sout = reinterpret_cast<int*>(take((size_t)in.ns * 4));
-  unsigned* key[2];
-  int* val[2];
-  for (int q = 0; q < 2; ++q) key[q] = reinterpret_cast<unsigned*>(take((size_t)items * 4));
-  for (int q = 0; q < 2; ++q) val[q] = reinterpret_cast<int*>(take((size_t)items * 4));
-  const int b0 = sort_blocks(in.nt), b1 = sort_blocks(in.ns);
-  int* hist = reinterpret_cast<int*>(take((size_t)(b0 + b1) * kBins * 4));
-  int* total = reinterpret_cast<int*>(take(2 * kBins * 4));
   double* box = reinterpret_cast<double*>(take(kBoxBlocks * 4 * sizeof(double)));
+  const SortSpace w = sort_space(p, in.nt, in.ns);
   *tgt_order = tout;
   *src_order = sout;
   if (items == 0) return LPM_OK;
@@ -354,23 +401,14 @@ int spatial_order(lpm_ctx* ctx, const OrderInput& in, DevBuf& buf, int** tgt_ord
   OrderDev a;
   a.seg[0] = Segment{in.tx, in.ty, in.tz, nullptr, in.i0, in.nt};
   a.seg[1] = Segment{in.x, in.y, in.z, in.list, 0, in.ns};
-  a.blocks0 = b0;
   a.k = k;
   a.sphere = in.sphere ? 1 : 0;
   a.box = box;
   a.prob = in.prob;
   a.sorted = in.sorted;
   if (!in.sphere) hipLaunchKernelGGL(box_partial, dim3(kBoxBlocks), dim3(256), 0, ctx->stream, a, box);
-  hipLaunchKernelGGL(make_keys, dim3((items + 255) / 256), dim3(256), 0, ctx->stream, a, key[0], val[0]);
-  const int passes = (bits + 7) / 8;
-  for (int q = 0; q < passes; ++q) {
-    const bool last = q == passes - 1;
-    SortDev s{in.nt, in.ns, b0, b1, 8 * q, key[q & 1], val[q & 1], key[(q + 1) & 1],
-              last ? tout : val[(q + 1) & 1], last ? sout : val[(q + 1) & 1] + in.nt, hist, total};
-    hipLaunchKernelGGL(sort_count, dim3(b0 + b1), dim3(kSortThreads), 0, ctx->stream, s);
-    hipLaunchKernelGGL(sort_scan, dim3(2 * kBins), dim3(256), 0, ctx->stream, s);
-    hipLaunchKernelGGL(sort_scatter, dim3(b0 + b1), dim3(kSortThreads), 0, ctx->stream, s);
-  }
+  hipLaunchKernelGGL(make_keys, dim3((items + 255) / 256), dim3(256), 0, ctx->stream, a, w.key[0], w.val[0]);
+  sort_pairs(ctx->stream, w, in.nt, in.ns, bits, tout, sout);
   LPM_HIP(ctx, hipGetLastError());
   return LPM_OK;
 }

@@ -51,6 +51,37 @@ def test_binning_is_nearest_generator(ctx):
     f.delete()
 
 
+@pytest.mark.parametrize("cells,radius", [("level 0", 1.0), ("level 4", 1.0), ("level 2", 4.0), ("cap", 1.0)])
+def test_binning_by_direction_bins(ctx, cells, radius):
+    """The search among a direction bin's generators finds the nearest of all: few
+    and many cells, radii where the products pass 3, and single-face cells in a
+    cap, whose bins list too many and fall back to all generators.  The FP32
+    products are within 4 roundings of |g| |p| of these."""
+    m, zeta = _case(5, int(cells[-1]) if cells != "cap" else 0)
+    P = m.xyz()
+    if cells == "cap":
+        leaf = P[m.face_centre]
+        own = np.flatnonzero(leaf[:, 2] > np.cos(0.1))
+        m.face_cell = np.zeros(len(leaf), np.int64)
+        m.face_cell[own] = 1 + np.arange(len(own))
+    m.x, m.y, m.z, m.area = m.x * radius, m.y * radius, m.z * radius, m.area * radius**2
+    f = FarFieldBVE(ctx, m, zeta, near_radius=0.1, band_radius=0.45, radius=radius)
+    got = f.binning()
+    act = m.active == 1
+    gen = np.zeros((f.ncell, 3))
+    np.add.at(gen, f.cell[act], P[act] * m.area[act, None])
+    gen /= np.linalg.norm(gen, axis=1)[:, None]
+    dots = P @ gen.T
+    best = dots.max(axis=1)
+    assert (best - dots[np.arange(m.n), got]).max() < 4 * 2.0**-24 * 3
+    again = FarFieldBVE(ctx, m, zeta, near_radius=0.1, band_radius=0.45, radius=radius)
+    assert np.array_equal(again.binning(), got)
+    counts = np.bincount(got, minlength=f.ncell)
+    assert counts.sum() == m.n
+    again.delete()
+    f.delete()
+
+
 def test_expansion_error_bounded_over_time(ctx):
     """Cells are re-binned at every evaluation, so the flow cannot stretch them:
     the expansion error after 30 steps stays near its initial value."""
