@@ -1,7 +1,7 @@
 // lpm_pair.hip -- pack, pair-sum and finalize kernels; the pair-sum driver.
 //
 // Data flow of one sum (all on the context stream, inputs already in HBM):
-//   pack_targets / pack_sources : FP64 SoA particles -> FP32 (or FP64) records
+//   pack_records : FP64 SoA particles -> FP32 (or FP64) records
 //   pair_sum_kernel             : all pairs, per-split FP64 partials
 //   source_totals (green only)  : FP64 sums of the source weights
 //   finalize                    : ordered sum over splits + FP64 epilogue
@@ -16,6 +16,7 @@
 #include "cull_kernels.hpp"
 #include "far_kernels.hpp"
 #include "lpm_internal.hpp"
+#include "finalize.hpp"
 #include "pair_kernels.hpp"
 
 namespace lpm {
@@ -46,8 +47,7 @@ __device__ __forceinline__ T idx_word(int p) {
 }
 
 template <typename T, int KIND>
-__global__ __launch_bounds__(256) void pack_sources(PackArgs a, T* __restrict__ rec) {
-  int j = blockIdx.x * blockDim.x + threadIdx.x;
+__device__ __forceinline__ void pack_source(const PackArgs& a, int j, T* __restrict__ rec) {
   const int count = a.count_dev ? *a.count_dev : a.count;
   if (j >= count) return;
   const int p = a.list[j];
@@ -106,8 +106,7 @@ __global__ __launch_bounds__(256) void pack_sources(PackArgs a, T* __restrict__ 
 }
 
 template <typename T, int KIND>
-__global__ __launch_bounds__(256) void pack_targets(PackArgs a, Vec4<T>* __restrict__ rec) {
-  int i = blockIdx.x * blockDim.x + threadIdx.x;
+__device__ __forceinline__ void pack_target(const PackArgs& a, int i, Vec4<T>* __restrict__ rec) {
   if (i >= a.count) return;
   const int p = a.tgt_order ? a.tgt_order[i] : a.i0 + i;
   const double x = a.x[p], y = a.y[p];
@@ -135,6 +134,18 @@ __global__ __launch_bounds__(256) void pack_targets(PackArgs a, Vec4<T>* __restr
     t.c = (T)a.q0[p];
   }
   rec[i] = t;
+}
+
+// Source records by the first `src_blocks` blocks, target records by the others:
+// one launch instead of two, about 4 us of a small sum's 60.
+template <typename T, int KIND>
+__global__ __launch_bounds__(256) void pack_records(int src_blocks, PackArgs as, T* __restrict__ srec, PackArgs at,
+                                                    Vec4<T>* __restrict__ trec) {
+  const int b = blockIdx.x;
+  if (b < src_blocks)
+    pack_source<T, KIND>(as, b * 256 + threadIdx.x, srec);
+  else
+    pack_target<T, KIND>(at, (b - src_blocks) * 256 + threadIdx.x, trec);
 }
 
 __global__ __launch_bounds__(256) void zero_fill(size_t n, double* __restrict__ p) {
@@ -174,18 +185,11 @@ __global__ __launch_bounds__(256) void source_totals(int ns, const int* __restri
 }
 
 // ---------------------------------------------------------------- finalize
-template <int KIND, int NO>
-__global__ __launch_bounds__(256) void finalize_kernel(FinArgs f) {
-  int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= f.nt) return;
+template <int KIND, int NO, int W>
+__global__ __launch_bounds__(fin_threads(W)) void finalize_kernel(FinArgs f) {
+  int i;
   double A[NO];
-#pragma unroll
-  for (int k = 0; k < NO; ++k) A[k] = 0.0;
-  for (int s = 0; s < f.nsplit; ++s) {
-    const double* ps = f.partial + (size_t)s * NO * f.nt;
-#pragma unroll
-    for (int k = 0; k < NO; ++k) A[k] += ps[(size_t)k * f.nt + i];
-  }
+  if (!sum_partials<NO, W>(f, i, A)) return;
   const int p = f.tgt_order ? f.tgt_order[i] : f.i0 + i;
   if constexpr (KIND == LPM_K_SPHERE_BS) {
     const double x = f.x[p], y = f.y[p], z = f.z[p];
@@ -318,15 +322,14 @@ static KernelFn pick_kernel(int kind, int prec, int r, int variant) {
 template <typename T>
 static void launch_pack_t(int kind, const PackArgs& a_src, const PackArgs& a_tgt, void* srec, void* trec,
                           int ns, int nt, hipStream_t st) {
-  dim3 b(256);
-  dim3 gs((ns + 255) / 256), gt((nt + 255) / 256);
+  const int gs = (ns + 255) / 256, gt = (nt + 255) / 256;
+  if (gs + gt == 0) return;
   PackArgs as = a_src, at = a_tgt;
   as.count = ns;
   at.count = nt;
-#define LPM_PACK_CASE(K)                                                                    \
-  case K:                                                                                   \
-    if (ns > 0) hipLaunchKernelGGL((pack_sources<T, K>), gs, b, 0, st, as, (T*)srec);      \
-    if (nt > 0) hipLaunchKernelGGL((pack_targets<T, K>), gt, b, 0, st, at, (Vec4<T>*)trec); \
+#define LPM_PACK_CASE(K)                                                                                           \
+  case K:                                                                                                          \
+    hipLaunchKernelGGL((pack_records<T, K>), dim3(gs + gt), dim3(256), 0, st, gs, as, (T*)srec, at, (Vec4<T>*)trec); \
     break;
   switch (kind) {
     LPM_PACK_CASE(LPM_K_SPHERE_BS)
@@ -354,15 +357,14 @@ void launch_pack(int kind, int precision, const PackArgs& a, void* srec, void* t
 }
 
 static void launch_finalize(int kind, const FinArgs& f, hipStream_t st) {
-  dim3 b(256), g((f.nt + 255) / 256);
   switch (kind) {
-    case LPM_K_SPHERE_BS: hipLaunchKernelGGL((finalize_kernel<LPM_K_SPHERE_BS, 3>), g, b, 0, st, f); break;
-    case LPM_K_PLANE_BS: hipLaunchKernelGGL((finalize_kernel<LPM_K_PLANE_BS, 2>), g, b, 0, st, f); break;
-    case LPM_K_PSE8: hipLaunchKernelGGL((finalize_kernel<LPM_K_PSE8, 1>), g, b, 0, st, f); break;
-    case LPM_K_PSE2: hipLaunchKernelGGL((finalize_kernel<LPM_K_PSE2, 1>), g, b, 0, st, f); break;
-    case LPM_K_PSE_SPHERE8: hipLaunchKernelGGL((finalize_kernel<LPM_K_PSE_SPHERE8, 1>), g, b, 0, st, f); break;
-    case LPM_K_SPHERE_GREEN: hipLaunchKernelGGL((finalize_kernel<LPM_K_SPHERE_GREEN, 2>), g, b, 0, st, f); break;
-    default: hipLaunchKernelGGL((finalize_kernel<LPM_K_PLANE_GREEN, 1>), g, b, 0, st, f); break;
+    case LPM_K_SPHERE_BS: LPM_LAUNCH_FIN(f, st, finalize_kernel, LPM_K_SPHERE_BS, 3); break;
+    case LPM_K_PLANE_BS: LPM_LAUNCH_FIN(f, st, finalize_kernel, LPM_K_PLANE_BS, 2); break;
+    case LPM_K_PSE8: LPM_LAUNCH_FIN(f, st, finalize_kernel, LPM_K_PSE8, 1); break;
+    case LPM_K_PSE2: LPM_LAUNCH_FIN(f, st, finalize_kernel, LPM_K_PSE2, 1); break;
+    case LPM_K_PSE_SPHERE8: LPM_LAUNCH_FIN(f, st, finalize_kernel, LPM_K_PSE_SPHERE8, 1); break;
+    case LPM_K_SPHERE_GREEN: LPM_LAUNCH_FIN(f, st, finalize_kernel, LPM_K_SPHERE_GREEN, 2); break;
+    default: LPM_LAUNCH_FIN(f, st, finalize_kernel, LPM_K_PLANE_GREEN, 1); break;
   }
 }
 

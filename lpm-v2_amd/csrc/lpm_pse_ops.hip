@@ -12,6 +12,7 @@
 
 #include "cull_kernels.hpp"
 #include "lpm_internal.hpp"
+#include "finalize.hpp"
 #include "pair_kernels.hpp"
 
 namespace lpm {
@@ -34,8 +35,7 @@ __host__ __device__ constexpr bool sphere_kind(int kind) {
 
 // Source records (see PseDeriv, PseInterp, SwePlane for the layouts).
 template <typename T, int KIND>
-__global__ __launch_bounds__(256) void ops_pack_sources(PackArgs a, int nw, T* __restrict__ rec) {
-  const int j = blockIdx.x * blockDim.x + threadIdx.x;
+__device__ __forceinline__ void ops_pack_source(const PackArgs& a, int j, int nw, T* __restrict__ rec) {
   if (j >= a.count) return;
   const int p = a.list[j];
   T* r = rec + (size_t)j * nw;  // written in place: the field count is a runtime value
@@ -85,8 +85,7 @@ __global__ __launch_bounds__(256) void ops_pack_sources(PackArgs a, int nw, T* _
 }
 
 template <typename T, int KIND>
-__global__ __launch_bounds__(256) void ops_pack_targets(PackArgs a, Vec4<T>* __restrict__ rec) {
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
+__device__ __forceinline__ void ops_pack_target(const PackArgs& a, int i, Vec4<T>* __restrict__ rec) {
   if (i >= a.count) return;
   const int p = a.tgt_order ? a.tgt_order[i] : a.i0 + i;
   const double x = a.x[p], y = a.y[p];
@@ -108,23 +107,27 @@ __global__ __launch_bounds__(256) void ops_pack_targets(PackArgs a, Vec4<T>* __r
   rec[i] = t;
 }
 
+// Source records by the first `src_blocks` blocks, target records by the others.
+template <typename T, int KIND>
+__global__ __launch_bounds__(256) void ops_pack_records(int src_blocks, PackArgs as, int nw, T* __restrict__ srec,
+                                                        PackArgs at, Vec4<T>* __restrict__ trec) {
+  const int b = blockIdx.x;
+  if (b < src_blocks)
+    ops_pack_source<T, KIND>(as, b * 256 + threadIdx.x, nw, srec);
+  else
+    ops_pack_target<T, KIND>(at, (b - src_blocks) * 256 + threadIdx.x, trec);
+}
+
 // Epilogues.  NO = number of sums per target, OP the derivative operator.
 // OP is a template parameter rather than a runtime switch: with the output
 // pointer chosen by a runtime switch (a pointer phi), the gfx950 back end of
 // the ROCm 7.2 compiler stored the double dot through the pointer of another
 // case (the LLVM IR was correct).
-template <int KIND, int NO, int OP>
-__global__ __launch_bounds__(256) void ops_finalize(FinArgs f) {
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= f.nt) return;
+template <int KIND, int NO, int OP, int W>
+__global__ __launch_bounds__(fin_threads(W)) void ops_finalize(FinArgs f) {
+  int i;
   double A[NO];
-#pragma unroll
-  for (int k = 0; k < NO; ++k) A[k] = 0.0;
-  for (int s = 0; s < f.nsplit; ++s) {
-    const double* ps = f.partial + (size_t)s * NO * f.nt;
-#pragma unroll
-    for (int k = 0; k < NO; ++k) A[k] += ps[(size_t)k * f.nt + i];
-  }
+  if (!sum_partials<NO, W>(f, i, A)) return;
   const int p = f.tgt_order ? f.tgt_order[i] : f.i0 + i;
   if constexpr (KIND == LPM_K_PSE_INTERP_PLANE || KIND == LPM_K_PSE_INTERP_SPHERE) {
     f.out0[p] = A[0] * f.scale;
@@ -264,14 +267,15 @@ CullFn pick_cull(int kind, int m, int series) {
 template <typename T>
 void pack_t(int kind, int nw, const PackArgs& as, const PackArgs& at, void* srec, void* trec, int ns, int nt,
             hipStream_t st) {
-  dim3 b(256), gs((ns + 255) / 256), gt((nt + 255) / 256);
+  const int gs = (ns + 255) / 256, gt = (nt + 255) / 256;
+  if (gs + gt == 0) return;
   PackArgs s = as, t = at;
   s.count = ns;
   t.count = nt;
-#define LPM_OPS_PACK(K)                                                                             \
-  case K:                                                                                           \
-    if (ns > 0) hipLaunchKernelGGL((ops_pack_sources<T, K>), gs, b, 0, st, s, nw, (T*)srec);       \
-    if (nt > 0) hipLaunchKernelGGL((ops_pack_targets<T, K>), gt, b, 0, st, t, (Vec4<T>*)trec);     \
+#define LPM_OPS_PACK(K)                                                                                         \
+  case K:                                                                                                       \
+    hipLaunchKernelGGL((ops_pack_records<T, K>), dim3(gs + gt), dim3(256), 0, st, gs, s, nw, (T*)srec, t,        \
+                       (Vec4<T>*)trec);                                                                         \
     break;
   switch (kind) {
     LPM_OPS_PACK(LPM_K_PSE_DERIV_PLANE)
@@ -321,26 +325,25 @@ void ops_launch_pack(int kind, int prec, const PackArgs& s, const PackArgs& t, v
 }
 
 int ops_launch_finalize(int kind, int m, const FinArgs& f, hipStream_t st) {
-  dim3 b(256), g((f.nt + 255) / 256);
   constexpr int kPlane = LPM_K_PSE_DERIV_PLANE, kSphere = LPM_K_PSE_DERIV_SPHERE;
   if (kind == kPlane && m == 1 && f.op == kOpGradient)
-    hipLaunchKernelGGL((ops_finalize<kPlane, 4, kOpGradient>), g, b, 0, st, f);
+    LPM_LAUNCH_FIN(f, st, ops_finalize, kPlane, 4, kOpGradient);
   else if (kind == kPlane && m == 2 && f.op == kOpSecondPartials)
-    hipLaunchKernelGGL((ops_finalize<kPlane, 6, kOpSecondPartials>), g, b, 0, st, f);
+    LPM_LAUNCH_FIN(f, st, ops_finalize, kPlane, 6, kOpSecondPartials);
   else if (kind == kPlane && m == 2 && f.op == kOpDoubleDot)
-    hipLaunchKernelGGL((ops_finalize<kPlane, 6, kOpDoubleDot>), g, b, 0, st, f);
+    LPM_LAUNCH_FIN(f, st, ops_finalize, kPlane, 6, kOpDoubleDot);
   else if (kind == kSphere && m == 1 && f.op == kOpGradient)
-    hipLaunchKernelGGL((ops_finalize<kSphere, 6, kOpGradient>), g, b, 0, st, f);
+    LPM_LAUNCH_FIN(f, st, ops_finalize, kSphere, 6, kOpGradient);
   else if (kind == kSphere && m == 3 && f.op == kOpDoubleDot)
-    hipLaunchKernelGGL((ops_finalize<kSphere, 12, kOpDoubleDot>), g, b, 0, st, f);
+    LPM_LAUNCH_FIN(f, st, ops_finalize, kSphere, 12, kOpDoubleDot);
   else if (kind == kSphere && m == 3 && f.op == kOpDivergence)
-    hipLaunchKernelGGL((ops_finalize<kSphere, 12, kOpDivergence>), g, b, 0, st, f);
+    LPM_LAUNCH_FIN(f, st, ops_finalize, kSphere, 12, kOpDivergence);
   else if (kind == LPM_K_PSE_INTERP_PLANE)
-    hipLaunchKernelGGL((ops_finalize<LPM_K_PSE_INTERP_PLANE, 1, 0>), g, b, 0, st, f);
+    LPM_LAUNCH_FIN(f, st, ops_finalize, LPM_K_PSE_INTERP_PLANE, 1, 0);
   else if (kind == LPM_K_PSE_INTERP_SPHERE)
-    hipLaunchKernelGGL((ops_finalize<LPM_K_PSE_INTERP_SPHERE, 1, 0>), g, b, 0, st, f);
+    LPM_LAUNCH_FIN(f, st, ops_finalize, LPM_K_PSE_INTERP_SPHERE, 1, 0);
   else if (kind == LPM_K_SWE_PLANE)
-    hipLaunchKernelGGL((ops_finalize<LPM_K_SWE_PLANE, 5, 0>), g, b, 0, st, f);
+    LPM_LAUNCH_FIN(f, st, ops_finalize, LPM_K_SWE_PLANE, 5, 0);
   else
     return LPM_ERR_ARG;  // no epilogue for this kind / field count / operator
   return LPM_OK;

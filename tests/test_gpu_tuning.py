@@ -121,3 +121,26 @@ def test_small_sums_match_forced_shapes(ctx, prec, n):
             ctx.set_tuning(kind, prec, 0, 0, 0)
         for g, r in zip(got, ref):
             assert np.abs(g - r).max() <= tol * max(np.abs(r).max(), 1e-300)
+
+
+@pytest.mark.parametrize("splits", [2, 15, 16, 17, 40, 64])
+@pytest.mark.parametrize("nt", [1, 63, 65, 300])
+def test_partials_add_up_whatever_their_number(ctx, splits, nt):
+    """One thread a target below 16 splits, eight waves to 64 targets from there on
+    (remainders of 8 and of 4 x 8), against a sum that is not split.  The FP64 sums
+    differ by their order only: 5,120 terms, 5,120 * 2^-53 = 6e-13 at most."""
+    m = mesh.icosahedral_mesh(4)
+    f = m.z + 0.3 * m.x
+
+    def run(s):
+        for kind in (L.K_SPHERE_BS, L.K_PSE_DERIV_SPHERE):
+            ctx.set_tuning(kind, "fp64", 1, 32, s)
+        return (np.stack(ctx.bve_sphere_velocity(m.x, m.y, m.z, f, m.area, m.active, i1=nt)),
+                np.stack(ctx.pse_sphere_gradient(m.x, m.y, m.z, f, m.area, m.active, 0.2, i1=nt)))
+
+    try:
+        for got, ref in zip(run(splits), run(1)):
+            assert np.abs(got - ref).max() < 6e-13 * np.abs(ref).max()
+    finally:
+        for kind in (L.K_SPHERE_BS, L.K_PSE_DERIV_SPHERE):
+            ctx.set_tuning(kind, "fp64", 0, 0, 0)
