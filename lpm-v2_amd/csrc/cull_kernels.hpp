@@ -32,6 +32,10 @@ struct CullArgs {
   const int* tgt_order;   // particle of every target record, null where no pair is a self pair
   int nt, ns, nsplit, n_wtiles, n_stiles;
   float reach;            // separation in record units beyond which terms are zero
+  // shallow water: balls per FAR_TILE; the tiles that are far of each other are not
+  // this kernel's (null: all are)
+  const float4* far_tballs = nullptr;
+  const float4* far_sballs = nullptr;
 };
 
 // The sums of one source tile, records [j0, j1), for the wave's targets.
@@ -125,6 +129,10 @@ static __global__ __launch_bounds__(256) void cull_sum_kernel(const void* __rest
       near = !(d2 > th * th);
       touch = a.tgt_order && balls_touch(d2, tb, sb);
       own = (mine & (a.nsplit - 1)) == split;
+      if constexpr (!__is_same(FAR, void)) {
+        constexpr int W = FAR_TILE / (64 * R), B = FAR_TILE / CULL_TILE;
+        if (a.far_tballs) own = own && !tiles_far_swe(a.far_tballs[wtile / W], a.far_sballs[mine / B], a.reach);
+      }
     }
     const unsigned long long m_near = __ballot(near), m_touch = __ballot(touch);
     unsigned long long todo = __ballot(own);

@@ -1,5 +1,5 @@
-// far_kernels.hpp -- the FP32 Biot-Savart and Green sums with the well-separated
-// source tiles on the matrix units.
+// far_kernels.hpp -- the FP32 Biot-Savart, Green and shallow-water sums with the
+// well-separated source tiles on the matrix units.
 //
 // The all-VALU pair (pair_kernels.hpp) is bound by VALU issue: 11-12 instructions,
 // 31-36 cycles per 64 pairs and SIMD on MI355X.  Only the reciprocal (or log) has
@@ -32,22 +32,9 @@ typedef float f32x4 __attribute__((ext_vector_type(4)));
 typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 
-constexpr int FAR_TILE = 256;     // sources per tile, targets per block
 constexpr int FAR_COLS = 4;       // 16-target column tiles per wave
 constexpr int FAR_FOLD = 1024;    // sources per group, the unit of the source splits
 constexpr int FAR_PART = 512;     // sources per FP32 partial sum (128 terms a lane)
-
-// Well separated: every target-source distance is at least the radius of the target
-// block (|Y| >= 2 rho_t).  The norms and products above are then at most 9 times the
-// denominator for the closest pairs and about equal to it for nearly all; errors
-// against FP64 are the same with 3 rho_t, and fewer tiles go the VALU way.  The
-// margins keep a pair of equal points (a self pair) out for any rounding of centres
-// and radii; the lower bound keeps the split's low parts normal.
-__device__ __forceinline__ bool tiles_far(const float4& t, const float4& s) {
-  const float d2 = ball_d2(t, s);
-  const float th = 1.001f * s.w + 2.002f * t.w;
-  return d2 > th * th && d2 > 1e-28f;
-}
 
 // Exact split v = h + m + l into bf16 values, each in the high half of its word.
 __device__ __forceinline__ void split3(float v, unsigned& h, unsigned& m, unsigned& l) {
@@ -87,39 +74,69 @@ __device__ __forceinline__ u32x4 frag_tgt(float v, bool norm) {
 
 // ----------------------------------------------------------- far policies
 // DIMS coordinates; E: record word 3 holds e; W0 (and W1): weight words; NW weight
-// sums accumulated by FMAs (0: Biot-Savart, by MFMA); trans: the VALU function.
+// sums accumulated by FMAs (0: by MFMA); trans: the VALU function; BLOCKS per CU.
 template <bool USE_E>
 struct FarSphereBS {
   using Near = SphereBS<float, USE_E>;
-  static constexpr int DIMS = 3, W0 = 4, W1 = 4, NW = 0;
+  static constexpr int DIMS = 3, W0 = 4, W1 = 4, NW = 0, BLOCKS = 4;
   static constexpr bool E = USE_E;
   __device__ __forceinline__ static float trans(float r2) { return fast_rcp(r2); }
 };
 struct FarPlaneBS {
   using Near = PlaneBS<float>;
-  static constexpr int DIMS = 2, W0 = 2, W1 = 2, NW = 0;
+  static constexpr int DIMS = 2, W0 = 2, W1 = 2, NW = 0, BLOCKS = 4;
   static constexpr bool E = false;
   __device__ __forceinline__ static float trans(float r2) { return fast_rcp(r2); }
 };
 template <bool USE_E>
 struct FarSphereGreen {
   using Near = SphereGreen<float, USE_E>;
-  static constexpr int DIMS = 3, W0 = 4, W1 = 5, NW = 2;
+  static constexpr int DIMS = 3, W0 = 4, W1 = 5, NW = 2, BLOCKS = 4;
   static constexpr bool E = USE_E;
   __device__ __forceinline__ static float trans(float r2) { return fast_log2(r2); }
 };
 struct FarPlaneGreen {
   using Near = PlaneGreen<float>;
-  static constexpr int DIMS = 2, W0 = 2, W1 = 2, NW = 1;
+  static constexpr int DIMS = 2, W0 = 2, W1 = 2, NW = 1, BLOCKS = 4;
   static constexpr bool E = false;
   __device__ __forceinline__ static float trans(float r2) { return fast_log2(r2); }
 };
+
+// The shallow-water sums beyond the reach of the Laplacian's exponential, where only
+// the vortex and divergence terms are left.  With z = X + i Y (target minus source),
+// f = 1 / |z|^2 and c = vorticity + i divergence weight, the two velocity sums are
+// those of c conj(z) f and the two gradient sums those of -c conj(z)^2 f^2; conj(z)
+// is the difference of target and source, so both are matrix products of f and f^2
+// with the source weights c, c conj(Z), c conj(Z)^2: three 4-row products, 42 cycles
+// per 64 pairs against 66 on the VALU.  The other tiles are left to cull_sum_kernel,
+// whose smaller tiles know the exponential's reach and which keeps more waves (sums
+// of both: 301^2 3,480 -> 2,780 us, 512^2 26.1 -> 20.3 ms; with the near tiles in this
+// kernel a reach over the whole domain cost 25 %).
+struct FarSwePlane {
+  using Near = SwePlane<float, true>;
+  static constexpr int DIMS = 2, W0 = 2, W1 = 3, NW = 0, BLOCKS = 3;
+  static constexpr bool E = false;
+  __device__ __forceinline__ static float trans(float r2) { return fast_rcp(r2); }
+};
+template <class P>
+inline constexpr bool kSwe = __is_same(P, FarSwePlane);
 
 // LDS of one staged source tile: 16 steps of 16 sources, the MFMA A fragments
 // (64 x 16 bytes a step) and the weights (16 x 16 bytes a step).
 struct FarStage {
   u32x4 frag[16 * 64];
   f32x4 wgt[16 * 16];
+};
+struct FarStageSwe : FarStage {
+  f32x4 wgt2[16 * 16];
+};
+template <class P>
+struct FarStageOf {
+  using T = FarStage;
+};
+template <>
+struct FarStageOf<FarSwePlane> {
+  using T = FarStageSwe;
 };
 
 // The direct VALU sum of one near tile for the wave's 64 targets (lane = target);
@@ -201,12 +218,15 @@ template <class P>
 struct FarStep {
   u32x4 a;
   f32x4 w, w2;
-  __device__ __forceinline__ void read(const FarStage& st, int s, int lane, int wl, int grp) {
+  __device__ __forceinline__ void read(const typename FarStageOf<P>::T& st, int s, int lane, int wl, int grp) {
     a = st.frag[s * 64 + lane];
     w = st.wgt[s * 16 + wl];
+    if constexpr (kSwe<P>) w2 = st.wgt2[s * 16 + wl];
     if constexpr (P::NW == 2) w2 = st.wgt[s * 16 + grp * 4 + 1];
   }
-  __device__ __forceinline__ void add(const u32x4 B[FAR_COLS], f32x4 D[FAR_COLS]) const {
+  // D: FAR_COLS accumulators; the shallow-water sums have 3 FAR_COLS (f with the
+  // first weights, f^2 with both)
+  __device__ __forceinline__ void add(const u32x4 B[FAR_COLS], f32x4* D) const {
     f32x4 r[FAR_COLS];
     __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
@@ -223,6 +243,20 @@ struct FarStep {
       for (int v = 0; v < 4; ++v)
 #pragma unroll
         for (int c = 0; c < FAR_COLS; ++c) D[c] = __builtin_amdgcn_mfma_f32_4x4x1f32(w[v], r[c][v], D[c], 0, 0, 0);
+      if constexpr (kSwe<P>) {
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int c = 0; c < FAR_COLS; ++c) r[c] *= r[c];
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int v = 0; v < 4; ++v)
+#pragma unroll
+          for (int c = 0; c < FAR_COLS; ++c) {
+            f32x4 &D1 = D[FAR_COLS + c], &D2 = D[2 * FAR_COLS + c];
+            D1 = __builtin_amdgcn_mfma_f32_4x4x1f32(w[v], r[c][v], D1, 0, 0, 0);
+            D2 = __builtin_amdgcn_mfma_f32_4x4x1f32(w2[v], r[c][v], D2, 0, 0, 0);
+          }
+      }
     } else {
 #pragma unroll
       for (int c = 0; c < FAR_COLS; ++c)
@@ -245,10 +279,19 @@ template <class P>
 __device__ __forceinline__ void far_block(const Vec4<float>* __restrict__ tg, int nt, int t_block,
                                           const int* __restrict__ order, const float4 tm, const float* __restrict__ src,
                                           const float4* __restrict__ smeta, int ns, int first_group,
-                                          int group_step, double* __restrict__ out, int out_stride, FarStage* stage) {
+                                          int group_step, double* __restrict__ out, int out_stride,
+                                          typename FarStageOf<P>::T* stage, float reach = 0.f) {
   using N = typename P::Near;
   constexpr int NO = N::NOUT;
   constexpr int NACC = P::NW == 0 ? 4 : P::NW;
+  constexpr int ND = kSwe<P> ? 3 * FAR_COLS : FAR_COLS;  // accumulators
+  constexpr int NFAR = kSwe<P> ? 12 : NACC;              // far sums of a target
+  auto is_far = [&](const float4& sm) {
+    if constexpr (kSwe<P>)
+      return tiles_far_swe(tm, sm, reach);
+    else
+      return tiles_far(tm, sm);
+  };
   const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
   const int grp = lane >> 4;
   const int t_begin = t_block + wid * 64;
@@ -270,18 +313,23 @@ __device__ __forceinline__ void far_block(const Vec4<float>* __restrict__ tg, in
   int n_far = 0;
   for (int jt = j_begin; jt < ns; jt = next_tile(jt)) {
     const float4 sm = smeta[jt / FAR_TILE];
-    if (tiles_far(tm, sm)) {
+    if (is_far(sm)) {
       ++n_far;
       continue;
     }
-    if (t_begin >= nt) continue;
+    if (kSwe<P> || t_begin >= nt) continue;
     const int jt_end = min(ns, jt + FAR_TILE);
-    if (balls_touch(ball_d2(tm, sm), tm, sm))
-      near_tile<N, true>(t, tid, src, jt, jt_end, near_sum);
-    else
-      near_tile<N, false>(t, tid, src, jt, jt_end, near_sum);
+    if constexpr (!kSwe<P>) {
+      if (balls_touch(ball_d2(tm, sm), tm, sm))
+        near_tile<N, true>(t, tid, src, jt, jt_end, near_sum);
+      else
+        near_tile<N, false>(t, tid, src, jt, jt_end, near_sum);
+    }
   }
 
+  double far_sum[NFAR];
+#pragma unroll
+  for (int k = 0; k < NFAR; ++k) far_sum[k] = 0.0;
   double sum[FAR_COLS][NACC];
 #pragma unroll
   for (int c = 0; c < FAR_COLS; ++c)
@@ -300,12 +348,12 @@ __device__ __forceinline__ void far_block(const Vec4<float>* __restrict__ tg, in
       const float v = grp == 0 ? a0 : grp == 1 ? a1 : grp == 2 ? a2 : a3;
       B[c] = frag_tgt(v, grp == 3);
     }
-    f32x4 D[FAR_COLS];
+    f32x4 D[ND];
 #pragma unroll
-    for (int c = 0; c < FAR_COLS; ++c) D[c] = f32x4{0.f, 0.f, 0.f, 0.f};
+    for (int c = 0; c < ND; ++c) D[c] = f32x4{0.f, 0.f, 0.f, 0.f};
 
     auto next_far = [&](int jt) {
-      while (jt < ns && !tiles_far(tm, smeta[jt / FAR_TILE])) jt = next_tile(jt);
+      while (jt < ns && !is_far(smeta[jt / FAR_TILE])) jt = next_tile(jt);
       return jt;
     };
     float rec[SREC];
@@ -322,7 +370,7 @@ __device__ __forceinline__ void far_block(const Vec4<float>* __restrict__ tg, in
     load(jt);
     int buf = 0;
     while (jt < ns) {
-      FarStage& st = stage[buf];
+      typename FarStageOf<P>::T& st = stage[buf];
       {
         // this thread's source: row threadIdx % 16 of step threadIdx / 16; past the
         // end a source of weight 0 at distance 1
@@ -336,7 +384,18 @@ __device__ __forceinline__ void far_block(const Vec4<float>* __restrict__ tg, in
         st.frag[s * 64 + 32 + r] = frag_src(-2.f * d[2]);
         st.frag[s * 64 + 48 + r] = frag_src_norm(n2);
         float* w = reinterpret_cast<float*>(st.wgt + s * 16 + (r >> 2) * 4) + (r & 3);
-        if constexpr (P::NW == 0) {
+        if constexpr (kSwe<P>) {
+          // c, c conj(Z); c conj(Z)^2
+          float* wb = reinterpret_cast<float*>(st.wgt2 + s * 16 + (r >> 2) * 4) + (r & 3);
+          const float vr = fmaf(w0, d[0], w1 * d[1]), vi = fmaf(w1, d[0], -w0 * d[1]);
+          w[0] = w0;
+          w[4] = w1;
+          w[8] = vr;
+          w[12] = vi;
+          wb[0] = fmaf(vr, d[0], vi * d[1]);
+          wb[4] = fmaf(vi, d[0], -vr * d[1]);
+          wb[8] = wb[12] = 0.f;
+        } else if constexpr (P::NW == 0) {
           w[0] = w0 * d[0];
           w[4] = w0 * d[1];
           w[8] = w0 * d[2];
@@ -365,13 +424,30 @@ __device__ __forceinline__ void far_block(const Vec4<float>* __restrict__ tg, in
       // fold at fixed places of the source array, so that the split leaves no trace
       // beyond FP64 rounding
       if (jn >= ns || jn / FAR_PART != jt / FAR_PART) {
+        if constexpr (kSwe<P>) {
+          // FP64 sums of all four columns would take 96 registers: add the four row
+          // groups here, each group keeping one column tile
+          const bool hi = grp & 2, odd = grp & 1;
 #pragma unroll
-        for (int c = 0; c < FAR_COLS; ++c)
+          for (int k = 0; k < NFAR; ++k) {
+            f32x4* d = D + (k >> 2) * FAR_COLS;
+            const int e = k & 3;
+            const float k0 = hi ? d[2][e] : d[0][e], k1 = hi ? d[3][e] : d[1][e];
+            const float s0 = hi ? d[0][e] : d[2][e], s1 = hi ? d[1][e] : d[3][e];
+            const double a = (double)k0 + (double)__shfl_xor(s0, 32), b = (double)k1 + (double)__shfl_xor(s1, 32);
+            far_sum[k] += (odd ? b : a) + __shfl_xor(odd ? a : b, 16);
 #pragma unroll
-          for (int k = 0; k < NACC; ++k) {
-            sum[c][k] += (double)D[c][k];
-            D[c][k] = 0.f;
+            for (int c = 0; c < FAR_COLS; ++c) d[c][e] = 0.f;
           }
+        } else {
+#pragma unroll
+          for (int c = 0; c < FAR_COLS; ++c)
+#pragma unroll
+            for (int k = 0; k < NACC; ++k) {
+              sum[c][k] += (double)D[c][k];
+              D[c][k] = 0.f;
+            }
+        }
       }
       buf ^= 1;
       jt = jn;
@@ -379,10 +455,7 @@ __device__ __forceinline__ void far_block(const Vec4<float>* __restrict__ tg, in
   }
 
   // add the four row groups, then give lane l target t_begin + l its column tile
-  double far_sum[NACC];
-#pragma unroll
-  for (int k = 0; k < NACC; ++k) far_sum[k] = 0.0;
-  if (n_far > 0) {
+  if (!kSwe<P> && n_far > 0) {
 #pragma unroll
     for (int c = 0; c < FAR_COLS; ++c)
 #pragma unroll
@@ -395,7 +468,16 @@ __device__ __forceinline__ void far_block(const Vec4<float>* __restrict__ tg, in
   }
   if (i < nt) {
     double o[NO];
-    if constexpr (P::NW == 0) {
+    if constexpr (kSwe<P>) {
+      const double x = X[0], y = X[1], xx = x * x - y * y, xy = 2.0 * x * y;
+      const double* u1 = far_sum;     // f c, f c conj(Z)
+      const double* u2 = far_sum + 4;  // f^2 c, f^2 c conj(Z), f^2 c conj(Z)^2
+      o[0] = x * u1[1] - y * u1[0] - u1[3];
+      o[1] = x * u1[0] + y * u1[1] - u1[2];
+      o[2] = -(xx * u2[1] - xy * u2[0] - 2.0 * (x * u2[3] - y * u2[2]) + u2[5]);
+      o[3] = -(xx * u2[0] + xy * u2[1] - 2.0 * (x * u2[2] + y * u2[3]) + u2[4]);
+      o[4] = 0.0;
+    } else if constexpr (P::NW == 0) {
       double v[3];
 #pragma unroll
       for (int k = 0; k < 3; ++k) v[k] = (double)X[k] * far_sum[3] - far_sum[k];
@@ -416,18 +498,18 @@ __device__ __forceinline__ void far_block(const Vec4<float>* __restrict__ tg, in
 }
 
 template <class P>
-static __global__ __launch_bounds__(256, 4) void far_sum_kernel(const void* __restrict__ tgt, const void* __restrict__ srcv,
+static __global__ __launch_bounds__(256, P::BLOCKS) void far_sum_kernel(const void* __restrict__ tgt, const void* __restrict__ srcv,
                                                          double* __restrict__ partial,
                                                          const float4* __restrict__ tmeta,
                                                          const float4* __restrict__ smeta,
                                                          const int* __restrict__ order, PairArgs a) {
-  __shared__ FarStage stage[2];
+  __shared__ typename FarStageOf<P>::T stage[2];
   const int nblk_t = (a.nt + FAR_TILE - 1) / FAR_TILE;
   const int split = blockIdx.x / nblk_t;
   const int tb = blockIdx.x - split * nblk_t;
   far_block<P>(reinterpret_cast<const Vec4<float>*>(tgt), a.nt, tb * FAR_TILE, order, tmeta[tb],
                reinterpret_cast<const float*>(srcv), smeta, a.ns, split, a.nsplit,
-               partial + (size_t)split * P::Near::NOUT * a.nt, a.nt, stage);
+               partial + (size_t)split * P::Near::NOUT * a.nt, a.nt, stage, a.reach);
 }
 
 // Batched problems: a persistent launch whose blocks take (problem, target block,

@@ -209,7 +209,7 @@ void launch_pack(int kind, int precision, const PackArgs& a, void* srec, void* t
                  hipStream_t st);
 Tuning default_tuning(int kind, int prec);
 // Where the far path starts, in pairs (see sum_path).
-constexpr double kFarMinPairsSphere = 2e9, kFarMinPairsPlane = 4e9;
+constexpr double kFarMinPairsSphere = 2e9, kFarMinPairsPlane = 4e9, kFarMinPairsSwe = 4e9;
 
 // How a sum is scheduled: over all pairs (pair_kernels.hpp), with the
 // well-separated tiles on the MFMA (far_kernels.hpp), or without the tiles whose

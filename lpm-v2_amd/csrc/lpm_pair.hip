@@ -465,6 +465,7 @@ static FarFn pick_far(int kind, bool on_sphere) {
     case LPM_K_SPHERE_GREEN:
       return on_sphere ? far_sum_kernel<FarSphereGreen<false>> : far_sum_kernel<FarSphereGreen<true>>;
     case LPM_K_PLANE_GREEN: return far_sum_kernel<FarPlaneGreen>;
+    case LPM_K_SWE_PLANE: return far_sum_kernel<FarSwePlane>;
     default: return nullptr;
   }
 }
@@ -501,7 +502,9 @@ static CullFn pick_cull(int kind, int prec, int m, int series) {
 // far tiles, sphere velocity 0.95 of the all-pairs rate at 1.2e9 pairs, 1.01 at 2.5e9,
 // 1.23 at 1e10; plane velocity 0.92 at 1.6e9, 1.07 at 4.3e9.  Culled PSE sums: plane
 // 80^2 (4e7 pairs) 0.88, 110^2 (1.5e8) 1.0, 150^2 (5e8) 1.3; sphere FP32 1.0 at 7.5e7
-// and 1.6 at 6e8.  On the sphere the sum must also reach less than kCullMaxReach radii
+// and 1.6 at 6e8.  Shallow water, far tiles against culled ones: 200^2 (1.6e9) 1.05 at
+// eps = 2 h and 0.91 at 20 h, 301^2 (8e9) 1.27 and 1.0, and 0.99 where nothing is
+// beyond reach.  On the sphere the sum must also reach less than kCullMaxReach radii
 // (chord): in FP64 at level 5 it reaches every particle.
 SumPath sum_path(const lpm_ctx* ctx, int kind, int prec, int nt, int ns, double reach) {
   const Tuning& ov = ctx->tune[kind][prec == LPM_PREC_FP32_KAHAN ? 1 : 0];
@@ -512,6 +515,8 @@ SumPath sum_path(const lpm_ctx* ctx, int kind, int prec, int nt, int ns, double 
     const double least = plane ? kFarMinPairsPlane : kFarMinPairsSphere;
     return prec == LPM_PREC_FP32_KAHAN && (double)nt * ns >= least ? kFarTiles : kAllPairs;
   }
+  if (kind == LPM_K_SWE_PLANE && prec == LPM_PREC_FP32_KAHAN && !ov.splits && (double)nt * ns >= kFarMinPairsSwe)
+    return kFarTiles;
   return !ov.splits && (double)nt * ns >= kCullMinPairs && reach < kCullMaxReach ? kCullTiles : kAllPairs;
 }
 
@@ -651,7 +656,9 @@ int run_pair_sum(lpm_ctx* ctx, const PairProblem& pp) {
                           kind == LPM_K_PSE_INTERP_SPHERE;
   const int variant = sphere_pse ? series_terms(fp32, 7.0 * pp.eps / pp.radius) : pp.on_sphere ? 1 : 0;
   FarFn far_fn = far ? pick_far(kind, pp.on_sphere) : nullptr;
-  CullFn cull_fn = cull ? pick_cull(kind, prec, pp.m, variant) : nullptr;
+  // the shallow-water far path shares the pairs with the cull kernel
+  const bool both = far && kind == LPM_K_SWE_PLANE;
+  CullFn cull_fn = cull || both ? pick_cull(kind, prec, pp.m, variant) : nullptr;
   KernelFn fn = far ? reinterpret_cast<KernelFn>(far_fn) : ops ? reinterpret_cast<KernelFn>(const_cast<void*>(ops_pick_kernel(kind, prec, tu.r, pp.m, variant)))
                     : pick_kernel(kind, prec, tu.r, variant);
   if (!fn) return fail(ctx, LPM_ERR_ARG, "no pair kernel for this kind, precision and field count");
@@ -668,12 +675,18 @@ int run_pair_sum(lpm_ctx* ctx, const PairProblem& pp) {
     want = std::min<long long>(want, groups);
     const int per = std::min<int>(kFarGroups, std::max<int>(1, (int)(groups / want)));
     nsplit = ov.splits > 0 ? (int)want : (int)std::min<long long>((groups + per - 1) / per, cap);
-  } else if (cull) {
-    // enough waves for kCullWaves a SIMD; a split takes every nsplit-th tile
+  }
+  int cull_split = 1;
+  if (cull || both) {
+    // enough waves for kCullWaves a SIMD; a split takes every cull_split-th tile
     const size_t split_bytes = (size_t)no * nt * sizeof(double);
-    while (nsplit < 64 && (long long)n_wtiles * nsplit < (long long)kCullWaves * 4 * ctx->num_cus &&
-           (size_t)(2 * nsplit) * split_bytes <= kPartialCap && ns >= 2 * nsplit * CULL_TILE)
-      nsplit *= 2;
+    while (cull_split < 64 && (long long)n_wtiles * cull_split < (long long)kCullWaves * 4 * ctx->num_cus &&
+           (size_t)(2 * cull_split) * split_bytes <= kPartialCap && ns >= 2 * cull_split * CULL_TILE)
+      cull_split *= 2;
+    if (cull) nsplit = cull_split;
+  }
+  if (path != kAllPairs) {
+    // splits are set
   } else if (ns > 0) {
     const size_t split_bytes = (size_t)no * nt * sizeof(double);
     size_t cap = std::min<size_t>(4096, kPartialCap / split_bytes);
@@ -694,9 +707,12 @@ int run_pair_sum(lpm_ctx* ctx, const PairProblem& pp) {
   const size_t tgt_bytes = (size_t)nt * TREC * wsz, src_bytes = (size_t)std::max(ns, 1) * nw * wsz;
   const size_t tball_bytes = path == kAllPairs ? 0 : (size_t)((nt + t_tile - 1) / t_tile) * sizeof(float4);
   const size_t sball_bytes = path == kAllPairs ? 0 : (size_t)((ns + s_tile - 1) / s_tile) * sizeof(float4);
-  LPM_HIP(ctx, tb.ensure(tgt_bytes + tball_bytes));
-  LPM_HIP(ctx, sb.ensure(src_bytes + sball_bytes));
-  LPM_HIP(ctx, pb.ensure((size_t)nsplit * no * nt * sizeof(double)));
+  const size_t tball2_bytes = both ? (size_t)n_wtiles * sizeof(float4) : 0;
+  const size_t sball2_bytes = both ? (size_t)((ns + CULL_TILE - 1) / CULL_TILE) * sizeof(float4) : 0;
+  const int parts = nsplit + (both ? cull_split : 0);
+  LPM_HIP(ctx, tb.ensure(tgt_bytes + tball_bytes + tball2_bytes));
+  LPM_HIP(ctx, sb.ensure(src_bytes + sball_bytes + sball2_bytes));
+  LPM_HIP(ctx, pb.ensure((size_t)parts * no * nt * sizeof(double)));
 
   const int *tgt_order = nullptr, *src_list = pp.src_list;
   if (path != kAllPairs) {
@@ -739,8 +755,13 @@ int run_pair_sum(lpm_ctx* ctx, const PairProblem& pp) {
     launch_pack2(kind, prec, pa, pt, sb.p, tb.p, ns, nt, ctx->stream);
   LPM_HIP(ctx, hipGetLastError());
 
+  // records of the scaled kinds hold separations in units of eps / sqrt(log2 e)
+  // (FP32) or eps (FP64); SWE records are unscaled
+  const double unit = kind == LPM_K_SWE_PLANE ? 1.0 / std::sqrt(pa.aux) : 1.0;
+  const float reach = (float)(std::sqrt(fp32 ? (double)CULL_Q32 : CULL_Q64) * unit);
   if (ns > 0) {
     PairArgs a;
+    a.reach = reach;
     a.tgt = tb.p;
     a.src = sb.p;
     a.partial = pb.as<double>();
@@ -757,31 +778,33 @@ int run_pair_sum(lpm_ctx* ctx, const PairProblem& pp) {
     dim3 grid((unsigned)(nblk_t * nsplit)), block(256);
     float4* tballs = reinterpret_cast<float4*>(static_cast<char*>(tb.p) + tgt_bytes);
     float4* sballs = reinterpret_cast<float4*>(static_cast<char*>(sb.p) + src_bytes);
+    float4* tballs2 = reinterpret_cast<float4*>(static_cast<char*>(tb.p) + tgt_bytes + tball_bytes);
+    float4* sballs2 = reinterpret_cast<float4*>(static_cast<char*>(sb.p) + src_bytes + sball_bytes);
     if (path != kAllPairs) {
       if (fp32)
         launch_balls<float>(kind, pp.m, nw, tb.p, sb.p, tballs, sballs, nt, ns, t_tile, s_tile, ctx->stream);
       else
         launch_balls<double>(kind, pp.m, nw, tb.p, sb.p, tballs, sballs, nt, ns, t_tile, s_tile, ctx->stream);
     }
+    if (both)
+      launch_balls<float>(kind, pp.m, nw, tb.p, sb.p, tballs2, sballs2, nt, ns, 64, CULL_TILE, ctx->stream);
     hipEvent_t e0 = nullptr, e1 = nullptr;
     if (ctx->timing && !pp.ns_dev) {
       e0 = take_event(ctx);
       e1 = take_event(ctx);
       if (e0 && e1) LPM_HIP(ctx, hipEventRecord(e0, ctx->stream));
     }
-    if (far) {
+    if (far)
       hipLaunchKernelGGL(far_fn, grid, block, 0, ctx->stream, tb.p, sb.p, pb.as<double>(), tballs, sballs, tgt_order,
                          a);
-    } else if (cull) {
-      // records of the scaled kinds hold separations in units of eps / sqrt(log2 e)
-      // (FP32) or eps (FP64); SWE records are unscaled
-      const double unit = kind == LPM_K_SWE_PLANE ? 1.0 / std::sqrt(pa.aux) : 1.0;
-      CullArgs ca{tb.p, sb.p, pb.as<double>(), tballs, sballs, pp.tx ? nullptr : tgt_order, nt, ns, nsplit,
-                  n_wtiles, (ns + CULL_TILE - 1) / CULL_TILE,
-                  (float)(std::sqrt(fp32 ? (double)CULL_Q32 : CULL_Q64) * unit)};
-      hipLaunchKernelGGL(cull_fn, grid, block, 0, ctx->stream, tb.p, sb.p, pb.as<double>(), ca);
-    } else
-      hipLaunchKernelGGL(fn, grid, block, 0, ctx->stream, a);
+    if (cull || both) {
+      double* out = pb.as<double>() + (both ? (size_t)nsplit * no * nt : 0);
+      CullArgs ca{tb.p, sb.p, out, both ? tballs2 : tballs, both ? sballs2 : sballs, pp.tx ? nullptr : tgt_order, nt, ns,
+                  cull_split, n_wtiles, (ns + CULL_TILE - 1) / CULL_TILE, reach};
+      if (both) ca.far_tballs = tballs, ca.far_sballs = sballs;
+      hipLaunchKernelGGL(cull_fn, dim3((unsigned)(nblk_t * cull_split)), block, 0, ctx->stream, tb.p, sb.p, out, ca);
+    }
+    if (path == kAllPairs) hipLaunchKernelGGL(fn, grid, block, 0, ctx->stream, a);
     LPM_HIP(ctx, hipGetLastError());
     if (ctx->timing && e0 && e1) {
       LPM_HIP(ctx, hipEventRecord(e1, ctx->stream));
@@ -799,7 +822,7 @@ int run_pair_sum(lpm_ctx* ctx, const PairProblem& pp) {
   f.partial = pb.as<double>();
   f.nt = nt;
   f.i0 = pp.i0;
-  f.nsplit = nsplit;
+  f.nsplit = ns > 0 ? parts : 1;
   f.x = pp.x;
   f.y = pp.y;
   f.z = pp.z;

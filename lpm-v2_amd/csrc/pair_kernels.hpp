@@ -525,6 +525,7 @@ struct PairArgs {
   // when set, the number of sources is read here and ns is only the bound
   // that sized chunk * nsplit (splits past the count sum nothing)
   const int* ns_dev = nullptr;
+  float reach = 0.f;  // far path, shallow water: separation beyond which the exponential is zero
 };
 
 template <typename T>

@@ -96,4 +96,25 @@ __device__ __forceinline__ bool balls_touch(float d2, const float4& a, const flo
   return !(d2 > th * th);
 }
 
+constexpr int FAR_TILE = 256;     // sources per tile, targets per block of the far path
+
+// Well separated: every target-source distance is at least the radius of the target
+// block (|Y| >= 2 rho_t).  The norms and products above are then at most 9 times the
+// denominator for the closest pairs and about equal to it for nearly all; errors
+// against FP64 are the same with 3 rho_t, and fewer tiles go the VALU way.  The
+// margins keep a pair of equal points (a self pair) out for any rounding of centres
+// and radii; the lower bound keeps the split's low parts normal.
+__device__ __forceinline__ bool tiles_far(const float4& t, const float4& s) {
+  const float d2 = ball_d2(t, s);
+  const float th = 1.001f * s.w + 2.002f * t.w;
+  return d2 > th * th && d2 > 1e-28f;
+}
+
+// f^2 stays a normal number: pair distances are at least 1e-3 of the centres'
+__device__ __forceinline__ bool tiles_far_swe(const float4& t, const float4& s, float reach) {
+  const float d2 = ball_d2(t, s);
+  const float th = 1.0001f * (reach + t.w + s.w);
+  return tiles_far(t, s) && d2 > th * th && d2 > 1e-12f && d2 < 1e16f;
+}
+
 }  // namespace lpm

@@ -249,3 +249,68 @@ def test_culled_sums_spread_non_finite_values_like_all_pairs(ctx, prec, bad, whe
             continue  # does not read f
         for g, r in zip(_rows(call()), _all_pairs(ctx, kind, prec, call)):
             assert np.array_equal(np.isfinite(g), np.isfinite(r)), name
+
+
+# ------------------------------------------------------- shallow water on far tiles
+def _swe(ctx, x, y, area, act, eps, **kw):
+    vort, div = np.sin(3 * x) + y, np.cos(2 * y) * x
+
+    def call(prec="fp32"):
+        return ctx.swe_plane_rhs(x, y, vort, div, 1.0 + 0.1 * x, 0.05 * y, area, act, eps, precision=prec, **kw)
+
+    return call
+
+
+@pytest.mark.parametrize("shape", ["grid", "strip", "duplicates", "units"])
+@pytest.mark.parametrize("eps_h", [2.0, 40.0])
+def test_far_tiles_shallow_water(ctx, shape, eps_h):
+    """Far tiles by the matrix products of f and f^2, the others by the culled sum
+    (4e9 pairs on): shuffled, passive particles, a block of targets that starts inside
+    a tile, and lengths at which f^2 would leave the normal numbers.  As far off the
+    FP64 sums as the all-pairs kernel is, or within the FP32 bar."""
+    rng = np.random.default_rng(11)
+    x, y, area, h = mesh.grid_centres(270, 1.0, jitter=1e-3, seed=3)
+    n = x.size
+    if shape == "strip":
+        x, y = rng.uniform(-50, 50, n), rng.uniform(-0.01, 0.01, n)
+    elif shape == "duplicates":
+        x, y = np.repeat(x[::300], 300), np.repeat(y[::300], 300)
+        n = x.size
+        area = area[:n]
+    elif shape == "units":
+        x, y, area, h = x * 1e-9, y * 1e-9, area * 1e-18, h * 1e-9
+    idx = rng.permutation(n)
+    x, y, area = x[idx], y[idx], area[idx]
+    act = (rng.uniform(size=n) < 0.93).astype(np.int32)
+    tgt = np.ones(n, bool)
+    if shape == "duplicates":  # one active particle a point, compared on itself
+        order = np.lexsort((y, x))
+        act = np.zeros(n, np.int32)
+        act[order[::300]] = 1
+        tgt = act == 1
+    kw = {"i0": 333, "i1": n - 70} if shape == "grid" else {}
+    call = _swe(ctx, x, y, area, act, eps_h * h, **kw)
+    got, again = _rows(call()), _rows(call())
+    pairs = _all_pairs(ctx, L.K_SWE_PLANE, "fp32", call)
+    for k, (g, e, r, a) in enumerate(zip(got, pairs, _rows(call("fp64")), again)):
+        own = rel_err_max(e[tgt], r[tgt])
+        assert rel_err_max(g[tgt], r[tgt]) < max(TOL32, 1.5 * own), (shape, k, own)
+        assert np.array_equal(g, a, equal_nan=True)  # the passive copies sit on a source
+
+
+@pytest.mark.parametrize("bad", [np.inf, np.nan])
+@pytest.mark.parametrize("what", ["vort", "depth", "target"])
+def test_far_shallow_water_spreads_non_finite_values_like_all_pairs(ctx, bad, what):
+    x, y, area, h = mesh.grid_centres(256, 1.0, jitter=1e-3, seed=3)
+    vort, depth = np.sin(3 * x) + y, 1.0 + 0.1 * x
+    act = np.ones(x.size, np.int32)
+    j = 7000
+    if what == "target":
+        act[j] = 0
+    (vort if what == "vort" else depth)[j] = bad
+
+    def call():
+        return ctx.swe_plane_rhs(x, y, vort, 0.2 * vort, depth, 0.05 * y, area, act, 2 * h, precision="fp32")
+
+    for g, r in zip(_rows(call()), _all_pairs(ctx, L.K_SWE_PLANE, "fp32", call)):
+        assert np.array_equal(np.isfinite(g), np.isfinite(r))
