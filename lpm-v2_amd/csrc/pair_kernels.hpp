@@ -58,6 +58,21 @@ __device__ __forceinline__ double rcp_refined(double x) {
   const double e = fma(-x, r, 1.0);
   return fma(r, fma(e, e, e), r);
 }
+// Four reciprocals for the price of one: r = 1 / (z0 z1 z2 z3) and nine products, 72
+// cycles against 120 for four refined ones.  The products' roundings stay far below
+// the sums' (icosahedral L4, 600 targets in extended precision: rms 1.95e-15 either
+// way).  Where the product leaves the range of FP64 (coincident points, separations
+// beyond 1e38 or below 1e-38) all four are NaN, and pair_tile takes the wave's sums
+// again one by one.
+__device__ __forceinline__ void rcp_four(const double z[4], double f[4]) {
+  const double a = z[0] * z[1], b = z[2] * z[3], p = a * b;
+  const double r = rcp_refined(p);
+  const double ra = r * b, rb = r * a;
+  f[0] = ra * z[1];
+  f[1] = ra * z[0];
+  f[2] = rb * z[3];
+  f[3] = rb * z[2];
+}
 // FP64 exponential and logarithm by table.  The FP64 vector rate is 4.6 cycles per
 // instruction and SIMD, so the sums below are bound by the length of these: a table
 // entry from LDS (512 or 2,048 bytes, filled once per block) takes the place of half
@@ -559,11 +574,23 @@ template <>
 inline constexpr int LOAD_GROUP<PlaneBS<double>, double> = 4;
 template <>
 inline constexpr int LOAD_GROUP<PlaneGreen<double>, double> = 4;
+// FP64 Biot-Savart sums take the reciprocals of a load group together (never of two
+// targets: a value that is not finite stays with its target).  Kernels at icosahedral
+// L4 / L5 / L6: 39.5 / 410 / 5,100 us one by one, 37 / 355 / 4,500 in fours; plane 300^2
+// 3,280 / 2,720.  With R targets a lane the groups are kept apart by a scheduling
+// barrier: interleaved they took 120 registers at R = 2, 86 apart, and 3 % longer.
+template <class P, typename T>
+inline constexpr bool RCP_FOUR = false;
+template <bool E>
+inline constexpr bool RCP_FOUR<SphereBS<double, E>, double> = true;
+template <>
+inline constexpr bool RCP_FOUR<PlaneBS<double>, double> = true;
 
 // One wavefront's work: targets [t_begin, t_begin + 64 R) of the record array
 // tg[0, nt) (particle index tgt_idx0 + local) against sources [j_begin, j_end)
 // of src; FP64 results go to out[k * out_stride + i] for valid targets i.
-template <class P, typename T, int R, bool COMPENSATED>
+// FOUR: reciprocals in fours; sums that are not finite are taken again without.
+template <class P, typename T, int R, bool COMPENSATED, bool FOUR = RCP_FOUR<P, T>>
 __device__ __forceinline__ void pair_tile(const Vec4<T>* __restrict__ tg, int nt, int t_begin,
                                           int tgt_idx0, const T* __restrict__ src, int j_begin,
                                           int j_end, int kt, double* __restrict__ out,
@@ -622,16 +649,34 @@ __device__ __forceinline__ void pair_tile(const Vec4<T>* __restrict__ tg, int nt
           for (int g = 0; g < G; ++g)
 #pragma unroll
             for (int q = 0; q < P::NW; ++q) sn[g][q] = src[(size_t)(jn + g) * P::NW + q];
+          if constexpr (FOUR) {
+            static_assert(G == 4);
 #pragma unroll
-          for (int g = 0; g < G; ++g) {
-            W4<T> w[R];
-            T f[R];
+            for (int r = 0; r < R; ++r) {
+              W4<T> w[G];
+              T z[G], f[G];
 #pragma unroll
-            for (int r = 0; r < R; ++r) P::arg(t[r], sv[g], w[r]);
+              for (int g = 0; g < G; ++g) {
+                P::arg(t[r], sv[g], w[g]);
+                z[g] = w[g].z;
+              }
+              rcp_four(z, f);
 #pragma unroll
-            for (int r = 0; r < R; ++r) f[r] = P::trans(w[r]);
+              for (int g = 0; g < G; ++g) P::acc(sv[g], w[g], f[g], p[r]);
+              if (r + 1 < R) __builtin_amdgcn_sched_barrier(0);
+            }
+          } else {
 #pragma unroll
-            for (int r = 0; r < R; ++r) P::acc(sv[g], w[r], f[r], p[r]);
+            for (int g = 0; g < G; ++g) {
+              W4<T> w[R];
+              T f[R];
+#pragma unroll
+              for (int r = 0; r < R; ++r) P::arg(t[r], sv[g], w[r]);
+#pragma unroll
+              for (int r = 0; r < R; ++r) f[r] = P::trans(w[r]);
+#pragma unroll
+              for (int r = 0; r < R; ++r) P::acc(sv[g], w[r], f[r], p[r]);
+            }
           }
 #pragma unroll
           for (int g = 0; g < G; ++g)
@@ -683,6 +728,17 @@ __device__ __forceinline__ void pair_tile(const Vec4<T>* __restrict__ tg, int nt
       }
   }
 
+  if constexpr (FOUR) {
+    bool bad = false;
+#pragma unroll
+    for (int r = 0; r < R; ++r)
+#pragma unroll
+      for (int k = 0; k < NO; ++k) bad = bad || !__builtin_isfinite(S[r][k]);
+    if (__any(bad)) {
+      pair_tile<P, T, R, COMPENSATED, false>(tg, nt, t_begin, tgt_idx0, src, j_begin, j_end, kt, out, out_stride);
+      return;
+    }
+  }
 #pragma unroll
   for (int r = 0; r < R; ++r) {
     int i = t_begin + r * 64 + lane;
@@ -744,8 +800,12 @@ struct BatchArgs {
 // item, and only kernel-level noalias lets the compiler keep the source reads
 // on the scalar unit (wave-uniform s_load, SGPR operands) across those stores.
 // Through a struct, it issued per-lane vector loads of the same addresses.
+// Waves a SIMD must hold: 6 in FP32; FP64 at the registers its reciprocals in fours
+// take without spills (86, 166 and 256 at R = 2, 4 and 8).
+template <typename T, int R>
+inline constexpr int batch_waves = sizeof(T) == 4 || R == 1 ? 6 : R == 2 ? 5 : R == 4 ? 3 : 1;
 template <class P, typename T, int R, bool COMPENSATED>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(6))) void pair_batch_kernel(
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(batch_waves<T, R>))) void pair_batch_kernel(
     const void* __restrict__ tgt, const void* __restrict__ srcv, double* __restrict__ partial,
     const BatchProblem* __restrict__ probs, const BatchItem* __restrict__ items, int n_items, int kt,
     unsigned int* __restrict__ counter) {

@@ -128,3 +128,42 @@ def test_fp64_exponential_in_pse_sums(ctx):
     assert (rel < 2.3e-16 * (8 + 6 * q[ok])).all()
     far = q > 760
     assert far.any() and not lap[far].any()
+
+
+@pytest.mark.parametrize("scale", [1e-100, 1e-60, 1e-30, 1.0, 1e30, 1e60, 1e70])
+@pytest.mark.parametrize("n", [3, 64, 5000, 30011])
+def test_fp64_reciprocals_in_fours(ctx, n, scale):
+    """Four reciprocals from one of their product, taken one by one where the product
+    leaves the range (separations from 1e38 on or below 1e-38).  Against numpy for 40
+    targets: n terms of a few roundings each, 8 + sqrt(n) of 2^-53 of the terms' sum."""
+    rng = np.random.default_rng(n)
+    x, y = rng.uniform(-1, 1, n) * scale, rng.uniform(-1, 1, n) * scale
+    w, area = rng.normal(size=n), np.full(n, scale / n)
+    act = (rng.uniform(size=n) < 0.9).astype(np.int32)
+    u, v = ctx.plane_velocity(x, y, w, area, act, precision="fp64")
+    src = np.flatnonzero(act)
+    for i in rng.integers(0, n, 40):
+        j = src[src != i]
+        dx, dy = (x[i] - x[j]) / scale, (y[i] - y[j]) / scale
+        k = w[j] / n / (2 * np.pi * (dx * dx + dy * dy))
+        tol = (8 + np.sqrt(n)) * 2.0**-53
+        assert abs(u[i] + (k * dy).sum()) <= tol * np.abs(k * dy).sum()
+        assert abs(v[i] - (k * dx).sum()) <= tol * np.abs(k * dx).sum()
+
+
+def test_fp64_reciprocals_in_fours_keep_a_bad_value_to_its_target(ctx):
+    """A passive particle on top of a source, and one that is not a number: NaN there,
+    and every other target as without them."""
+    n = 5000
+    rng = np.random.default_rng(5)
+    p = _sphere_points(rng, n)
+    act = np.ones(n, np.int32)
+    act[[70, 71]] = 0
+    q, area = rng.normal(size=n), np.full(n, 4 * np.pi / n)
+    ref = np.stack(ctx.bve_sphere_velocity(*p, q, area, act, precision="fp64"))
+    p[:, 70] = p[:, 4000]
+    p[0, 71] = np.nan
+    got = np.stack(ctx.bve_sphere_velocity(*p, q, area, act, precision="fp64"))
+    assert np.isnan(got[:, 71]).all() and not np.isfinite(got[:, 70]).any()
+    rest = np.delete(np.arange(n), [70, 71])
+    assert np.abs(got - ref)[:, rest].max() <= 1e-13 * np.abs(ref[:, rest]).max()
