@@ -190,59 +190,44 @@ __device__ __forceinline__ void expansion(const T c[3], T e_c, const T* m, const
 //   a_k = x . b_k (k >= 1), so alpha = phi (M_0 + x . beta) needs no a_k, and
 //   phi = 2 psi with psi = 1 / (|x-c|^2 + e_c),
 // so with the record's moments scaled by 2^k (M'_k = 2^k M_k / (4 pi R)) and
-// B_k = M'_k[., x^(k-1)]:
-//   beta = psi h,  h = B_1 + psi (B_2 + ... + psi B_P)
-//   alpha = psi (M'_0 + psi (2x) . h)
+// X = psi x the contractions nest:
+//   h = M'_1 + X . (M'_2 + X . (M'_3 + X . M'_4)),  beta = psi h
+//   alpha = psi (M'_0 + 2 X . h)
 //   p += c alpha + psi h.
-// cv = {c (3), e_c, M'_0..M'_P}; x2 = 2x.  84 vector instructions per target
-// and cell at P = 4 against 102 for expansion<4, float> and the sum into p.
+// cv = {c (3), e_c, M'_0..M'_P}.  78 vector instructions per target and cell at
+// P = 4, none of which needs a product of coordinates kept in registers.
 template <int P>
-__device__ __forceinline__ void far_expansion_acc(const float* cv, const float x[3], const float x2[3], float p[3]) {
+__device__ __forceinline__ void far_expansion_acc(const float* cv, const float x[3], float p[3]) {
   const float dx = x[0] - cv[0], dy = x[1] - cv[1], dz = x[2] - cv[2];
   const float psi = recip(fmaf(dx, dx, fmaf(dy, dy, fmaf(dz, dz, cv[3]))));
   const float* m = cv + 4;
-  float B[5][3] = {};
+  const float X[3] = {psi * x[0], psi * x[1], psi * x[2]};
+  float t3[10], t2[6], h[3];
+  if constexpr (P >= 3) {
 #pragma unroll
-  for (int k = 0; k < 3; ++k) B[1][k] = m[1 + k];
-  if (P >= 2) {
+    for (int i = 0; i < 10; ++i) {
+      t3[i] = m[kMomOff[3] + i];
+      if constexpr (P >= 4)
 #pragma unroll
-    for (int k = 0; k < 3; ++k)
-      B[2][k] = fmaf(m[kMomIdx.b2[k][2]], x[2], fmaf(m[kMomIdx.b2[k][1]], x[1], m[kMomIdx.b2[k][0]] * x[0]));
-  }
-  if (P >= 3) {
-    float q[6];
-#pragma unroll
-    for (int i = 0; i < 6; ++i) q[i] = kPairMul[i] * x[kPair[i][0]] * x[kPair[i][1]];
-#pragma unroll
-    for (int k = 0; k < 3; ++k) {
-      float s = m[kMomIdx.b3[k][0]] * q[0];
-#pragma unroll
-      for (int i = 1; i < 6; ++i) s = fmaf(m[kMomIdx.b3[k][i]], q[i], s);
-      B[3][k] = s;
+        for (int l = 0; l < 3; ++l)
+          t3[i] = fmaf(X[l], m[kMomIdx.b4[l][i]], t3[i]);
     }
   }
-  if (P >= 4) {
-    float q[10];
 #pragma unroll
-    for (int i = 0; i < 10; ++i) q[i] = kTriMul[i] * x[kTri[i][0]] * x[kTri[i][1]] * x[kTri[i][2]];
+  for (int i = 0; i < 6; ++i) {
+    t2[i] = m[kMomOff[2] + i];
+    if constexpr (P >= 3)
 #pragma unroll
-    for (int k = 0; k < 3; ++k) {
-      float s = m[kMomIdx.b4[k][0]] * q[0];
-#pragma unroll
-      for (int i = 1; i < 10; ++i) s = fmaf(m[kMomIdx.b4[k][i]], q[i], s);
-      B[4][k] = s;
-    }
+      for (int l = 0; l < 3; ++l) t2[i] = fmaf(X[l], t3[kMomIdx.b3[l][i] - kMomOff[3]], t2[i]);
   }
-  float h[3];
 #pragma unroll
   for (int i = 0; i < 3; ++i) {
-    float s = B[P][i];
+    h[i] = m[1 + i];
 #pragma unroll
-    for (int k = P - 1; k >= 1; --k) s = fmaf(psi, s, B[k][i]);
-    h[i] = s;
+    for (int l = 0; l < 3; ++l) h[i] = fmaf(X[l], t2[kMomIdx.b2[l][i] - kMomOff[2]], h[i]);
   }
-  const float xh = fmaf(x2[0], h[0], fmaf(x2[1], h[1], x2[2] * h[2]));
-  const float alpha = psi * fmaf(psi, xh, m[0]);
+  const float xh = fmaf(X[0], h[0], fmaf(X[1], h[1], X[2] * h[2]));
+  const float alpha = psi * fmaf(2.f, xh, m[0]);
 #pragma unroll
   for (int i = 0; i < 3; ++i) p[i] = fmaf(cv[i], alpha, fmaf(psi, h[i], p[i]));
 }
@@ -953,18 +938,31 @@ struct FarArgs {
   double* part;               // [gridDim.y][3][nt] this launch's partials
 };
 
+// Records pass through LDS, kFarBatch at a time and per wave, to vector registers: a
+// vector instruction with a scalar operand takes 4.2 cycles, one without 2.9, and
+// each of a record's words is an operand of kR targets.  At 491,522 targets and some
+// 460 records each (P = 4): 411 us, against 532 with scalar records and the
+// products of coordinates in registers; 467 at 3 and 4 targets a lane, whose tiles
+// leave more of a cell's last one empty, 443 at 4 waves a SIMD.  (The near sums take
+// 8 words a source for 11 instructions: there the LDS reads cost what they save,
+// 863 against 815 us.)
+constexpr int kRec4 = kCellRec / 4;
+constexpr int kFarBatch = 64 / kRec4;  // a 16-byte word a lane
+
 template <int P>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(7))) void ff_far_kernel(FarArgs a) {
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(5))) void ff_far_kernel(FarArgs a) {
+  __shared__ float4 stage[4][2][kFarBatch * kRec4];
   // the wave's item index is wave-uniform: readfirstlane puts it (and every
-  // index and record address derived from it) in scalar registers
-  const int item = __builtin_amdgcn_readfirstlane(blockIdx.x * 4 + (threadIdx.x >> 6));
+  // index derived from it) in scalar registers
+  const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int item = blockIdx.x * 4 + wid;
   if (item >= *a.n_items) return;
   const int lane = threadIdx.x & 63;
   const int2 it = a.items[item];
   const int t = it.x;
   const int k0 = a.tgt_start[t] + it.y * 64 * kR;
   const int k_end = a.tgt_start[t + 1];
-  float X[kR][3], X2[kR][3];
+  float X[kR][3];
 #pragma unroll
   for (int r = 0; r < kR; ++r) {
     const int k = k0 + 64 * r + lane;
@@ -972,8 +970,6 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(7))) void f
     X[r][0] = v.a;
     X[r][1] = v.b;
     X[r][2] = v.c;
-#pragma unroll
-    for (int c = 0; c < 3; ++c) X2[r][c] = 2.f * X[r][c];
   }
   float S[kR][3], C[kR][3];
 #pragma unroll
@@ -984,26 +980,46 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(7))) void f
   const int cnt = a.far_count[t];
   const int q_lo = (int)((long long)cnt * blockIdx.y / gridDim.y);
   const int q_hi = (int)((long long)cnt * (blockIdx.y + 1) / gridDim.y);
-  // one compensated block per 64 records of this part of the list
-  for (int b0 = q_lo; b0 < q_hi; b0 += 64) {
-    const int b1 = min(q_hi, b0 + 64);
-    float p[kR][3];
+  // a lane fetches one 16-byte word of the batch; past the end of the list the last
+  // record's again
+  const float4* cell4 = reinterpret_cast<const float4*>(a.cell);
+  float4 next;
+  auto fetch = [&](int q) {
+    next = cell4[(size_t)list[min(q + lane / kRec4, q_hi - 1)] * kRec4 + lane % kRec4];
+  };
+  float p[kR][3];
 #pragma unroll
-    for (int r = 0; r < kR; ++r) p[r][0] = p[r][1] = p[r][2] = 0.f;
-    for (int qi = b0; qi < b1; ++qi) {
-      const int s = list[qi];
-      const float* cr = a.cell + (size_t)s * kCellRec;
+  for (int r = 0; r < kR; ++r) p[r][0] = p[r][1] = p[r][2] = 0.f;
+  if (q_lo < q_hi) fetch(q_lo);
+  int buf = 0, done = 0;
+  for (int q = q_lo; q < q_hi; q += kFarBatch, buf ^= 1) {
+    float4* st = stage[wid][buf];
+    if (lane < kFarBatch * kRec4) st[lane] = next;
+    __builtin_amdgcn_wave_barrier();  // LDS serves a wave's accesses in order
+    if (q + kFarBatch < q_hi) fetch(q + kFarBatch);
+    const int n = min(kFarBatch, q_hi - q);
+    for (int e = 0; e < n; ++e) {
       constexpr int NV = 4 + kMomOff[P] + (P + 1) * (P + 2) / 2;  // c, e_c, M'0..M'P
-      float cv[NV];
+      float cv[(NV + 3) / 4 * 4];
 #pragma unroll
-      for (int e = 0; e < NV; ++e) cv[e] = cr[e];
+      for (int w = 0; w < (NV + 3) / 4; ++w) {
+        const float4 v = st[e * kRec4 + w];
+        cv[4 * w] = v.x, cv[4 * w + 1] = v.y, cv[4 * w + 2] = v.z, cv[4 * w + 3] = v.w;
+      }
 #pragma unroll
-      for (int r = 0; r < kR; ++r) far_expansion_acc<P>(cv, X[r], X2[r], p[r]);
+      for (int r = 0; r < kR; ++r) far_expansion_acc<P>(cv, X[r], p[r]);
     }
+    // one compensated block per 10 batches of this part of the list
+    if (++done == 10 || q + kFarBatch >= q_hi) {
+      done = 0;
 #pragma unroll
-    for (int r = 0; r < kR; ++r)
+      for (int r = 0; r < kR; ++r)
 #pragma unroll
-      for (int c = 0; c < 3; ++c) lpm::two_sum_acc(S[r][c], C[r][c], p[r][c]);
+        for (int c = 0; c < 3; ++c) {
+          lpm::two_sum_acc(S[r][c], C[r][c], p[r][c]);
+          p[r][c] = 0.f;
+        }
+    }
   }
   double* out = a.part + (size_t)blockIdx.y * 3 * a.nt;
 #pragma unroll
