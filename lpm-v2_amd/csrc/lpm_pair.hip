@@ -261,6 +261,9 @@ Tuning default_tuning(int kind, int prec) {
 
 constexpr double kCullMinPairs = 1.5e8;
 constexpr double kCullMaxReach = 1.6;
+// The tested tiles leave about this reach, in eps, of the 10.2 (FP32) and 27.3 (FP64)
+// at which terms are zero.
+constexpr double kTestedReach = 8.5;
 constexpr int kFarRounds = 8;   // rounds of resident blocks wanted of a far-tile sum
 constexpr int kFarGroups = 8;   // at most so many groups of FAR_FOLD sources per split
 constexpr int kCullWaves = 12;  // waves per SIMD wanted of a culled sum
@@ -420,6 +423,13 @@ constexpr size_t kPartialCap = size_t(2) << 30;  // bytes of FP64 split partials
 // cubed level 5 FP64 92 -> 65 us, level 5 FP64 (6e8 pairs) 420 -> 360 us.  In FP32, and
 // for the longer PSE pairs, 2 targets per lane are as fast at 7.5e7 pairs and 3-6 %
 // faster at 3e8.
+// Source tiles from which a PSE sum looks at groups of 64 first (512^2 PSE-8 in FP32:
+// 350 us over all tiles, 321 over groups; a launch of 4 us).
+constexpr int kGroupTiles = 512;
+// PSE sums: tiles within sqrt(kNearQ) eps are added without a test (the bound needs at
+// least 16; 20 to 60 are within 3 %).
+constexpr double kNearQ = 36.0;
+
 constexpr double kSmallPairs = 1.2e8, kSmallPairsVortex64 = 1e9;
 constexpr int kSmallChunk = 64;
 constexpr int kSmallWaves = 24576;
@@ -500,12 +510,12 @@ static CullFn pick_cull(int kind, int prec, int m, int series) {
 
 // Where the tile paths start, by whole calls (ordering and balls cost 45 us there):
 // far tiles, sphere velocity 0.95 of the all-pairs rate at 1.2e9 pairs, 1.01 at 2.5e9,
-// 1.23 at 1e10; plane velocity 0.92 at 1.6e9, 1.07 at 4.3e9.  Culled PSE sums: plane
-// 80^2 (4e7 pairs) 0.88, 110^2 (1.5e8) 1.0, 150^2 (5e8) 1.3; sphere FP32 1.0 at 7.5e7
-// and 1.6 at 6e8.  Shallow water, far tiles against culled ones: 200^2 (1.6e9) 1.05 at
+// 1.23 at 1e10; plane velocity 0.92 at 1.6e9, 1.07 at 4.3e9.  Culled PSE sums at
+// eps = 2 h: plane 80^2 (4e7 pairs) 0.56-0.68, 110^2 (1.5e8) 1.0, 150^2 (5e8) 1.3 in FP32
+// and 1.6 in FP64, 200^2 2.0-2.4 and 3.2-3.4; sphere level 5 (6e8) 1.5 and 1.85.  Shallow water, far tiles against culled ones: 200^2 (1.6e9) 1.05 at
 // eps = 2 h and 0.91 at 20 h, 301^2 (8e9) 1.27 and 1.0, and 0.99 where nothing is
 // beyond reach.  On the sphere the sum must also reach less than kCullMaxReach radii
-// (chord): in FP64 at level 5 it reaches every particle.
+// (chord): 1.0-1.1 at eps = 0.18 and 0.22 (reach 1.6 and 1.85), 0.86-0.97 at 0.37.
 SumPath sum_path(const lpm_ctx* ctx, int kind, int prec, int nt, int ns, double reach) {
   const Tuning& ov = ctx->tune[kind][prec == LPM_PREC_FP32_KAHAN ? 1 : 0];
   if (ov.r || ov.kt) return kAllPairs;  // a forced tile shape is one of the all-pairs kernel
@@ -546,10 +556,25 @@ static bool sphere_kind(int kind) {
          kind == LPM_K_PSE_DERIV_SPHERE || kind == LPM_K_PSE_INTERP_SPHERE;
 }
 
+// Words that bound a term: the target's value, the source's two weights.
+static void weight_words(int kind, int m, unsigned tgt[2], unsigned src[2]) {
+  const int d = sphere_kind(kind) ? 3 : 2;
+  if (kind == LPM_K_PSE8 || kind == LPM_K_PSE2 || kind == LPM_K_PSE_SPHERE8) {
+    tgt[0] = 1u << d;
+    src[1] = 2u << d;
+  } else if (kind == LPM_K_PSE_DERIV_PLANE || kind == LPM_K_PSE_DERIV_SPHERE) {
+    src[1] = ((1u << m) - 1u) << (d + 1);
+  }
+  src[0] = 1u << d;
+}
+
 template <typename T>
 static void launch_balls(int kind, int m, int nw, const void* trec, const void* srec, float4* tballs, float4* sballs,
-                         int nt, int ns, int t_tile, int s_tile, hipStream_t st) {
+                         int nt, int ns, int t_tile, int s_tile, float2* tmag, float2* smag, hipStream_t st) {
   BallSet<T> t, s;
+  t.mag = tmag;
+  s.mag = smag;
+  if (smag) weight_words(kind, m, t.mag_mask, s.mag_mask);
   t.rec = static_cast<const T*>(trec);
   t.out = tballs;
   t.words = TREC;
@@ -644,10 +669,9 @@ int run_pair_sum(lpm_ctx* ctx, const PairProblem& pp) {
     tu.kt = fp32 ? 64 : 32;
   }
   // a device-side source count cannot be ordered
-  const double reach_eps = fp32 ? std::sqrt(CULL_Q32 / kLog2e) : std::sqrt(CULL_Q64);  // in eps
   const SumPath path = pp.ns_dev ? kAllPairs
                                  : sum_path(ctx, kind, prec, nt, ns,
-                                            sphere_kind(kind) ? reach_eps * pp.eps / pp.radius : 0.0);
+                                            sphere_kind(kind) ? kTestedReach * pp.eps / pp.radius : 0.0);
   const bool far = path == kFarTiles, cull = path == kCullTiles;
   const int t_tile = far ? FAR_TILE : 64, s_tile = far ? FAR_TILE : CULL_TILE;
   const int per_wave = path != kAllPairs ? 64 : 64 * tu.r;
@@ -709,9 +733,15 @@ int run_pair_sum(lpm_ctx* ctx, const PairProblem& pp) {
   const size_t sball_bytes = path == kAllPairs ? 0 : (size_t)((ns + s_tile - 1) / s_tile) * sizeof(float4);
   const size_t tball2_bytes = both ? (size_t)n_wtiles * sizeof(float4) : 0;
   const size_t sball2_bytes = both ? (size_t)((ns + CULL_TILE - 1) / CULL_TILE) * sizeof(float4) : 0;
+  const bool mags = cull && kind != LPM_K_SWE_PLANE;
+  const size_t tmag_bytes = mags ? (size_t)n_wtiles * sizeof(float2) : 0;
+  const int n_stiles = (ns + CULL_TILE - 1) / CULL_TILE;
+  const size_t smag_bytes = mags ? (size_t)(n_stiles + (n_stiles & 1)) * sizeof(float2) : 0;
+  const int n_groups = mags && n_stiles >= kGroupTiles ? (n_stiles + 63) / 64 : 0;
   const int parts = nsplit + (both ? cull_split : 0);
-  LPM_HIP(ctx, tb.ensure(tgt_bytes + tball_bytes + tball2_bytes));
-  LPM_HIP(ctx, sb.ensure(src_bytes + sball_bytes + sball2_bytes));
+  LPM_HIP(ctx, tb.ensure(tgt_bytes + tball_bytes + tball2_bytes + tmag_bytes));
+  LPM_HIP(ctx, sb.ensure(src_bytes + sball_bytes + sball2_bytes + smag_bytes +
+                         n_groups * sizeof(float4)));
   LPM_HIP(ctx, pb.ensure((size_t)parts * no * nt * sizeof(double)));
 
   const int *tgt_order = nullptr, *src_list = pp.src_list;
@@ -780,14 +810,22 @@ int run_pair_sum(lpm_ctx* ctx, const PairProblem& pp) {
     float4* sballs = reinterpret_cast<float4*>(static_cast<char*>(sb.p) + src_bytes);
     float4* tballs2 = reinterpret_cast<float4*>(static_cast<char*>(tb.p) + tgt_bytes + tball_bytes);
     float4* sballs2 = reinterpret_cast<float4*>(static_cast<char*>(sb.p) + src_bytes + sball_bytes);
+    float2* tmag = mags ? reinterpret_cast<float2*>(tballs2) : nullptr;  // one or the other
+    float2* smag = mags ? reinterpret_cast<float2*>(sballs2) : nullptr;
     if (path != kAllPairs) {
       if (fp32)
-        launch_balls<float>(kind, pp.m, nw, tb.p, sb.p, tballs, sballs, nt, ns, t_tile, s_tile, ctx->stream);
+        launch_balls<float>(kind, pp.m, nw, tb.p, sb.p, tballs, sballs, nt, ns, t_tile, s_tile, tmag, smag,
+                            ctx->stream);
       else
-        launch_balls<double>(kind, pp.m, nw, tb.p, sb.p, tballs, sballs, nt, ns, t_tile, s_tile, ctx->stream);
+        launch_balls<double>(kind, pp.m, nw, tb.p, sb.p, tballs, sballs, nt, ns, t_tile, s_tile, tmag, smag,
+                             ctx->stream);
     }
+    float4* gballs = n_groups ? reinterpret_cast<float4*>(smag + n_stiles + (n_stiles & 1)) : nullptr;
+    if (gballs)
+      hipLaunchKernelGGL(group_balls, dim3((n_groups + 3) / 4), block, 0, ctx->stream, n_stiles, sballs, gballs);
     if (both)
-      launch_balls<float>(kind, pp.m, nw, tb.p, sb.p, tballs2, sballs2, nt, ns, 64, CULL_TILE, ctx->stream);
+      launch_balls<float>(kind, pp.m, nw, tb.p, sb.p, tballs2, sballs2, nt, ns, 64, CULL_TILE, nullptr, nullptr,
+                          ctx->stream);
     hipEvent_t e0 = nullptr, e1 = nullptr;
     if (ctx->timing && !pp.ns_dev) {
       e0 = take_event(ctx);
@@ -802,6 +840,11 @@ int run_pair_sum(lpm_ctx* ctx, const PairProblem& pp) {
       CullArgs ca{tb.p, sb.p, out, both ? tballs2 : tballs, both ? sballs2 : sballs, pp.tx ? nullptr : tgt_order, nt, ns,
                   cull_split, n_wtiles, (ns + CULL_TILE - 1) / CULL_TILE, reach};
       if (both) ca.far_tballs = tballs, ca.far_sballs = sballs;
+      ca.gballs = gballs;
+      ca.tmag = tmag;
+      ca.smag = smag;
+      ca.product = kind == LPM_K_PSE_DERIV_PLANE || kind == LPM_K_PSE_DERIV_SPHERE;
+      ca.near_reach = (float)std::sqrt(kNearQ * (fp32 ? kLog2e : 1.0));
       hipLaunchKernelGGL(cull_fn, dim3((unsigned)(nblk_t * cull_split)), block, 0, ctx->stream, tb.p, sb.p, out, ca);
     }
     if (path == kAllPairs) hipLaunchKernelGGL(fn, grid, block, 0, ctx->stream, a);

@@ -21,7 +21,18 @@ struct BallSet {
   unsigned finite_mask = 0;
   const int2* desc = nullptr;  // when set: (first record, count) of every ball
   int balls = 0;
+  // when set: binary exponents e of the largest magnitudes among the words of each
+  // mask, |word| < 2^e in the tile (-inf where all are zero)
+  float2* mag = nullptr;
+  unsigned mag_mask[2] = {0, 0};
 };
+
+// e with |v| < 2^e, -inf for 0 and +inf where v is not finite.
+template <typename T>
+__device__ __forceinline__ float exponent_above(T v) {
+  if (v == (T)0) return -__builtin_huge_valf();
+  return isfinite(v) ? (float)(ilogb(v) + 1) : __builtin_huge_valf();
+}
 
 template <typename T>
 __device__ __forceinline__ void ball_of(const BallSet<T>& a, int b) {
@@ -30,6 +41,7 @@ __device__ __forceinline__ void ball_of(const BallSet<T>& a, int b) {
   const int count = a.desc ? a.desc[b].y : min(a.tile, a.n - first);
   T c[4][3];
   bool bad = false;
+  T big[2] = {(T)0, (T)0};
   T lo[3] = {(T)3e38, (T)3e38, (T)3e38}, hi[3] = {(T)-3e38, (T)-3e38, (T)-3e38};
 #pragma unroll
   for (int q = 0; q < 4; ++q) {
@@ -39,7 +51,11 @@ __device__ __forceinline__ void ball_of(const BallSet<T>& a, int b) {
     if (i < count) {
       const T* r = a.rec + (size_t)(first + i) * a.words;
       for (int k = 0; k < a.words; ++k)
+      {
         if ((a.finite_mask >> k) & 1u) bad = bad || !isfinite(r[k]);
+        if ((a.mag_mask[0] >> k) & 1u) big[0] = fmax(big[0], fabs(r[k]));
+        if ((a.mag_mask[1] >> k) & 1u) big[1] = fmax(big[1], fabs(r[k]));
+      }
       for (int k = 0; k < a.dims; ++k) c[q][k] = r[k];
 #pragma unroll
       for (int k = 0; k < 3; ++k) {
@@ -67,6 +83,13 @@ __device__ __forceinline__ void ball_of(const BallSet<T>& a, int b) {
     }
 #pragma unroll
   for (int m = 32; m > 0; m >>= 1) d2 = fmax(d2, __shfl_xor(d2, m));
+  if (a.mag) {
+#pragma unroll
+    for (int m = 32; m > 0; m >>= 1)
+#pragma unroll
+      for (int q = 0; q < 2; ++q) big[q] = fmax(big[q], __shfl_xor(big[q], m));
+    if (lane == 0) a.mag[b] = make_float2(exponent_above(big[0]), exponent_above(big[1]));
+  }
   bad = __any(bad) || count <= 0;
   if (lane == 0) {
     const float rad = bad ? __builtin_huge_valf() : (float)sqrt(d2) * 1.000001f;
@@ -82,6 +105,27 @@ static __global__ __launch_bounds__(256) void tile_balls(BallSet<T> tgt, BallSet
     ball_of(tgt, b);
   else if (b - tgt.balls < src.balls)
     ball_of(src, b - tgt.balls);
+}
+
+// Balls around 64 balls each, one wave per group.
+static __global__ __launch_bounds__(256) void group_balls(int n, const float4* __restrict__ balls,
+                                                          float4* __restrict__ out) {
+  const int g = blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
+  if (g * 64 >= n) return;
+  const float4 b = balls[min(g * 64 + lane, n - 1)];
+  float lo[3] = {b.x, b.y, b.z}, hi[3] = {b.x, b.y, b.z};
+  for (int m = 32; m > 0; m >>= 1)
+#pragma unroll
+    for (int k = 0; k < 3; ++k) {
+      lo[k] = fminf(lo[k], __shfl_xor(lo[k], m));
+      hi[k] = fmaxf(hi[k], __shfl_xor(hi[k], m));
+    }
+  const float x = 0.5f * (lo[0] + hi[0]), y = 0.5f * (lo[1] + hi[1]), z = 0.5f * (lo[2] + hi[2]);
+  const float dx = b.x - x, dy = b.y - y, dz = b.z - z;
+  float rad = 1.000001f * (sqrtf(dx * dx + dy * dy + dz * dz) + b.w);
+  if (!(rad < __builtin_huge_valf())) rad = __builtin_huge_valf();  // also where a centre is not a number
+  for (int m = 32; m > 0; m >>= 1) rad = fmaxf(rad, __shfl_xor(rad, m));
+  if (lane == 0) out[g] = make_float4(x, y, z, rad);
 }
 
 // Separation of two balls: squared centre distance.

@@ -314,3 +314,54 @@ def test_far_shallow_water_spreads_non_finite_values_like_all_pairs(ctx, bad, wh
 
     for g, r in zip(_rows(call()), _all_pairs(ctx, L.K_SWE_PLANE, "fp32", call)):
         assert np.array_equal(np.isfinite(g), np.isfinite(r))
+
+
+# ------------------------------------------- tiles too small to change a sum
+@pytest.mark.parametrize("field", ["patch", "jump", "lattice"])
+@pytest.mark.parametrize("space", ["plane", "sphere"])
+def test_tiles_passed_over_never_matter(ctx, field, space):
+    """A tile is passed over only where adding it would round away, so every target keeps
+    its own accuracy, however small its sum: a field that is zero but for a patch (sums
+    down to 1e-290 around it), one that jumps by 1e200, and a regular lattice whose
+    sums cancel.  FP64 against all pairs, each target by itself: 2^-53 of the sum of
+    its terms' magnitudes times their number, for terms of one sign 1e-11 of the sum."""
+    rng = np.random.default_rng(4)
+    if space == "plane":
+        x, y, area, h = mesh.grid_centres(128, 1.0, jitter=0.0 if field == "lattice" else 1e-3, seed=3)
+        z, eps, r = None, 2 * h, np.hypot(x, y)
+    else:
+        m = mesh.icosahedral_mesh(5)
+        x, y, z, area, eps, r = m.x, m.y, m.z, m.area, 0.03, np.arccos(np.clip(m.z, -1, 1))
+    if field == "patch":
+        f = np.where(r < 0.2, 1.0 + 0.1 * x, 0.0)
+    elif field == "jump":
+        f = np.where(x > 0.05, 1e100, 1e-100)
+    else:
+        f = np.ones(x.size)
+    act = np.ones(x.size, np.int32) if z is None else m.active
+    idx = rng.permutation(x.size)
+    pts = (0.97 * x[idx], 0.97 * y[idx]) if z is None else (y[::3], z[::3], x[::3])
+    if z is None:
+        def interpolate():
+            return ctx.pse_plane_interpolate(x, y, f, area, act, eps, *pts, precision="fp64")
+
+        def lap():
+            return ctx.pse_plane_laplacian(x, y, f, area, act, eps, order=2, precision="fp64")
+        kinds = ((L.K_PSE_INTERP_PLANE, interpolate), (L.K_PSE2, lap))
+    else:
+        def interpolate():
+            return ctx.pse_sphere_interpolate(x, y, z, f, area, act, eps, *pts, precision="fp64")
+        kinds = ((L.K_PSE_INTERP_SPHERE, interpolate),)
+    for kind, call in kinds:
+        got, ref = np.asarray(call()), _all_pairs(ctx, kind, "fp64", call)[0]
+        if field == "lattice" and kind == L.K_PSE2:  # zero terms: f_j - f_i
+            assert not got.any() and not ref.any()
+            continue
+        seen = np.abs(ref) > 1e-290
+        print(space, field, kind, "smallest", np.abs(ref[seen]).min(), "zeros", (~seen).sum())
+        if kind == L.K_PSE2 and field == "jump":
+            assert rel_err_max(got, ref) < 1e-11  # both signs within a target
+        # the delta kernel changes sign where its cubic does, far inside the near tiles
+        err = np.abs(got - ref)[seen] / np.abs(ref[seen])
+        assert np.quantile(err, 0.99) < 1e-11 and err.max() < 1e-7
+        assert np.abs(got[~seen]).max(initial=0.0) < 1e-289
