@@ -26,10 +26,9 @@ int64_t mlp_param_count(int nin, int width, int nhidden, int nout) {
 
 namespace {
 
-// Blocks a split product aims at, one per CU: 128 x 128 over 32,768 samples takes
-// 19.4 us at 256 blocks, 18.2 at 512 and 17.2 at 1024, whose partials cost twice
-// and four times the memory.
-constexpr int kGemmBlocks = 256;
+// Blocks the weight gradients aim at: three per CU, as many as their LDS lets run
+// together.
+constexpr int kDwBlocks = 768;
 
 // dY = 2 (Y - T) / (B nout); per-block partial loss (fixed order -> deterministic)
 __global__ __launch_bounds__(256) void mse_grad(int n, float scale, const float* __restrict__ Y,
@@ -132,32 +131,19 @@ __global__ __launch_bounds__(256) void mlp_mfma_forward_kernel(int n, int nin, i
   }
 }
 
-// Products with a long K and few output tiles (the weight gradients dZ^T H over
-// a minibatch) are split along K when `part` has room (`part_elems` floats) and
-// the results (C, then sums) are one contiguous run.
-void gemm(hipStream_t st, bool ta, bool tb, const GemmArgs& g0, float* part = nullptr, size_t part_elems = 0) {
-  GemmArgs g = g0;
-  g.part = nullptr;
-  g.kchunk = 0;
-  const int mt = (g.M + kGemmTile - 1) / kGemmTile, nt = (g.N + kGemmTile - 1) / kGemmTile;
-  const int tiles = mt * nt;
-  const size_t outs = (size_t)g.M * g.N + (g.sums ? g.M : 0);
-  int splits = 1;
-  if (part && tiles < 128 && g.K >= 512) {
-    splits = std::min((kGemmBlocks + tiles - 1) / tiles, g.K / 256);
-    while (splits > 1 && (size_t)splits * outs > part_elems) --splits;
-  }
-  if (splits > 1) {
-    g.kchunk = ((g.K + splits - 1) / splits + kGemmK - 1) / kGemmK * kGemmK;
-    splits = (g.K + g.kchunk - 1) / g.kchunk;
-    g.part = part;
-  }
-  dim3 grid(mt, nt, splits), blk(256);
-  if (ta) hipLaunchKernelGGL((gemm_f32<true, false>), grid, blk, 0, st, g);
-  else if (tb) hipLaunchKernelGGL((gemm_f32<false, true>), grid, blk, 0, st, g);
+void gemm(hipStream_t st, bool tb, const GemmArgs& g) {
+  dim3 grid((g.M + kGemmTile - 1) / kGemmTile, (g.N + kGemmTile - 1) / kGemmTile), blk(256);
+  if (tb) hipLaunchKernelGGL((gemm_f32<false, true>), grid, blk, 0, st, g);
   else hipLaunchKernelGGL((gemm_f32<false, false>), grid, blk, 0, st, g);
-  if (g.part)
-    hipLaunchKernelGGL(gemm_splitk_reduce, dim3((unsigned)((outs + 63) / 64)), blk, 0, st, splits, (int)outs, g.part, g.C);
+}
+
+// 64 samples a block where that gives every CU two, else 32.
+template <bool FORWARD>
+void chain(lpm_ctx* ctx, const ChainArgs& a) {
+  if (a.n >= 64 * 2 * ctx->num_cus)
+    hipLaunchKernelGGL((mlp_chain<4, FORWARD>), dim3((a.n + 63) / 64), dim3(256), 0, ctx->stream, a);
+  else
+    hipLaunchKernelGGL((mlp_chain<2, FORWARD>), dim3((a.n + 31) / 32), dim3(256), 0, ctx->stream, a);
 }
 
 }  // namespace
@@ -206,6 +192,8 @@ int Mlp::init(lpm_ctx* c, int nin_, int width_, int nhidden_, int nout_, int act
 
 bool Mlp::mfma_ok() const { return nin <= 32 && width == 128 && nhidden == 3 && nout <= 4; }
 
+bool Mlp::chained() const { return std::max(nin, std::max(width, nout)) <= kChainWidth; }
+
 int Mlp::pack() {
   if (!mfma_ok()) return LPM_OK;
   hipLaunchKernelGGL(mlp_pack_fragments, dim3(64), dim3(256), 0, ctx->stream, p.as<float>(), nin, nout,
@@ -217,10 +205,6 @@ int Mlp::pack() {
 int Mlp::ensure_batch(int n) {
   const size_t per = (size_t)(nhidden + 1) * (size_t)std::max(width, nout);
   LPM_HIP(ctx, act.ensure((size_t)n * per * 4));
-  LPM_HIP(ctx, scratch.ensure((size_t)n * std::max(width, nout) * 2 * 4));
-  LPM_HIP(ctx, loss_part.ensure(1024 * 8));
-  // split-K partials of the weight and bias gradients: up to 64 splits of the largest layer
-  LPM_HIP(ctx, splitk.ensure((size_t)64 * (std::max(width, nin) + 1) * std::max(width, nout) * 4));
   return LPM_OK;
 }
 
@@ -232,6 +216,12 @@ int Mlp::forward_f32(int n, const float* X) {
   int din = nin;
   int64_t off = 0;
   const size_t slot = (size_t)n * std::max(width, nout);
+  if (chained()) {
+    ChainArgs a{n, nin, width, nout, nhidden + 1, act_kind, p.as<float>(), X, nullptr, act.as<float>(), nullptr, slot};
+    chain<true>(ctx, a);
+    LPM_HIP(ctx, hipGetLastError());
+    return LPM_OK;
+  }
   for (int l = 0; l <= nhidden; ++l) {
     const int dout = l == nhidden ? nout : width;
     GemmArgs g{};
@@ -246,7 +236,7 @@ int Mlp::forward_f32(int n, const float* X) {
     g.ldb = din;
     g.ldc = dout;
     g.act = l == nhidden ? 0 : act_kind;
-    gemm(ctx->stream, false, true, g);
+    gemm(ctx->stream, true, g);
     in = g.C;
     din = dout;
     off += (int64_t)(l == 0 ? nin : width) * dout + dout;
@@ -260,52 +250,74 @@ int Mlp::loss_grad(int n, const float* X, const float* T, double* loss) {
   cur_n = n;
   const size_t slot = (size_t)n * std::max(width, nout);
   float* Y = act.as<float>() + (size_t)nhidden * slot;
-  float* dcur = scratch.as<float>();
-  float* dnext = scratch.as<float>() + slot;
+  LPM_HIP(ctx, scratch.ensure((size_t)(nhidden + 1) * slot * 4));
+  LPM_HIP(ctx, loss_part.ensure(1024 * 8));
+  float* dZ = scratch.as<float>();  // layer l's dZ at dZ + l slot
+  float* dY = dZ + (size_t)nhidden * slot;
   const int nb = std::min(1024, (n * nout + 255) / 256);
   hipLaunchKernelGGL(mse_grad, dim3(nb), dim3(256), 0, ctx->stream, n * nout, 1.0f / (float)(n * nout), Y, T,
-                     dcur, loss_part.as<double>());
+                     dY, loss_part.as<double>());
   // layer offsets
   std::vector<int64_t> offs((size_t)nhidden + 2, 0);
   for (int l = 0; l <= nhidden; ++l) {
     const int di = l == 0 ? nin : width, dout = l == nhidden ? nout : width;
     offs[(size_t)l + 1] = offs[(size_t)l] + (int64_t)di * dout + dout;
   }
-  for (int l = nhidden; l >= 0; --l) {
-    const int di = l == 0 ? nin : width, dout = l == nhidden ? nout : width;
-    const float* Hin = l == 0 ? X : act.as<float>() + (size_t)(l - 1) * slot;
-    float* gW = grad.as<float>() + offs[(size_t)l];
-    // dW = dZ^T H  ([dout][n] x [n][di]) and, after it in grad, db = column sums of dZ
-    GemmArgs g{};
-    g.A = dcur;
-    g.B = Hin;
-    g.C = gW;
-    g.sums = gW + (int64_t)di * dout;
-    g.M = dout;
-    g.N = di;
-    g.K = n;
-    g.lda = dout;
-    g.ldb = di;
-    g.ldc = di;
-    gemm(ctx->stream, true, false, g, splitk.as<float>(), splitk.bytes / sizeof(float));
-    if (l > 0) {
-      // dH = dZ W  ([n][dout] x [dout][di]), then times act'(H)
+  // dZ_(l-1) = (dZ_l W_l) act'(H_(l-1))
+  if (chained()) {
+    ChainArgs a{n, nin, width, nout, nhidden + 1, act_kind, p.as<float>(), nullptr, dY, act.as<float>(), dZ, slot};
+    chain<false>(ctx, a);
+  } else {
+    for (int l = nhidden; l > 0; --l) {
       GemmArgs h{};
-      h.A = dcur;
+      h.A = dZ + (size_t)l * slot;
       h.B = p.as<float>() + offs[(size_t)l];
-      h.C = dnext;
-      h.H = Hin;
+      h.C = dZ + (size_t)(l - 1) * slot;
+      h.H = act.as<float>() + (size_t)(l - 1) * slot;
       h.act = act_kind;
       h.M = n;
-      h.N = di;
-      h.K = dout;
-      h.lda = dout;
-      h.ldb = di;
-      h.ldc = di;
-      gemm(ctx->stream, false, false, h);
-      std::swap(dcur, dnext);
+      h.N = width;
+      h.K = l == nhidden ? nout : width;
+      h.lda = h.K;
+      h.ldb = width;
+      h.ldc = width;
+      gemm(ctx->stream, false, h);
     }
   }
+  // dW_l = dZ_l^T H_(l-1)  ([dout][n] x [n][di]) and, after it in grad, db_l
+  DwArgs d{};
+  int tiles = 0;
+  for (int l = 0; l <= nhidden; ++l) {
+    GemmArgs& g = d.layer[l];
+    g.A = dZ + (size_t)l * slot;
+    g.B = l == 0 ? X : act.as<float>() + (size_t)(l - 1) * slot;
+    g.C = grad.as<float>() + offs[(size_t)l];
+    g.M = l == nhidden ? nout : width;
+    g.N = l == 0 ? nin : width;
+    g.K = n;
+    g.lda = g.M;
+    g.ldb = g.N;
+    g.ldc = g.N;
+    g.sums = g.C + (int64_t)g.M * g.N;
+    d.first[l] = tiles;
+    tiles += ((g.M + kGemmTile - 1) / kGemmTile) * ((g.N + kGemmTile - 1) / kGemmTile);
+  }
+  for (int l = nhidden + 1; l <= kMaxLayers; ++l) d.first[l] = tiles;
+  int splits = std::max(1, std::min((kDwBlocks + tiles - 1) / tiles, n / 256));
+  const int kchunk = ((n + splits - 1) / splits + kGemmK - 1) / kGemmK * kGemmK;
+  splits = (n + kchunk - 1) / kchunk;
+  if (splits > 1) {
+    LPM_HIP(ctx, splitk.ensure((size_t)splits * np * 4));
+    for (int l = 0; l <= nhidden; ++l) {
+      d.layer[l].part = splitk.as<float>() + offs[(size_t)l];
+      d.layer[l].part_stride = (size_t)np;
+      d.layer[l].kchunk = kchunk;
+    }
+  }
+  hipLaunchKernelGGL(gemm_dw, dim3(tiles, splits), dim3(256), 0, ctx->stream, d);
+  if (splits > 1)
+    hipLaunchKernelGGL(gemm_splitk_reduce, dim3((unsigned)((np + 63) / 64)), dim3(256), 0, ctx->stream, splits, (int)np,
+                       splitk.as<float>(), grad.as<float>());
   LPM_HIP(ctx, hipGetLastError());
   if (loss) {
     std::vector<double> part((size_t)nb);

@@ -26,6 +26,7 @@ struct Mlp {
   void release();
   int init(lpm_ctx* c, int nin, int width, int nhidden, int nout, int act, uint64_t seed);
   bool mfma_ok() const;
+  bool chained() const;  // every layer fits the chain kernels
   int pack();  // FP32 params -> FP16 fragments
   int ensure_batch(int n);
   int forward_f32(int n, const float* X);  // device X [n][nin]; output in act slot nhidden

@@ -4,8 +4,9 @@
 // ISRU x / sqrt(1 + x^2), parameters per layer W[out][in] (row-major) then
 // b[out], FP32 master copy.
 //
-// Training path (FP32 matrix instructions): tiled GEMMs C = A op(B) with the
-// bias + activation, the activation's derivative or the bias gradient fused in, and Adam.
+// Training path (FP32 matrix instructions): all layers forward and all back in one
+// launch each, or a tiled GEMM C = A op(B) a layer where they are too wide, the weight
+// and bias gradients in one launch, and Adam.
 // Inference path (FP16 MFMA, FP32 accumulate), specialised for the
 // 13 -> 128 -> 128 -> 128 -> 3 surrogate: activations are kept transposed
 // (features = MFMA rows, samples = MFMA columns), so the D registers of one
@@ -104,15 +105,14 @@ __host__ __device__ inline float mlp_hidden_scale(int act) {
 // block needs 4 LDS reads per 16 matrix instructions; a row pitch of 36
 // floats spreads the reads over the banks.  B's rows are the instruction's
 // rows: a lane's four results are four consecutive n, one 16-byte store.
-// Split K: with part != nullptr, block z covers k in [z kchunk, (z+1) kchunk)
+// Split K: with part != nullptr, split z covers k in [z kchunk, (z+1) kchunk)
 // and writes its partial product (and, after it, its partial sums) to
-// part[z][M N (+ M)]; gemm_splitk_reduce adds them in a fixed order.
-// At 32,768 samples and width 128 (1.07 GFLOP, 6.8 us of matrix time; the
-// operands' 34 MB take 7 us) a layer's forward takes 22 us, its input gradient
-// 19.5 and its weight and bias gradient 24 with the reduction; the same on the
-// vector units, with the derivative and the sums in kernels of their own, took
-// 51, 52 and 188.  What is left is the serial load, product, store of a block
-// with 4 K tiles.
+// part + z part_stride; gemm_splitk_reduce adds them in a fixed order.
+// The weight and bias gradients of all layers are one launch (gemm_dw): at 32,768
+// samples, 13 -> 128 x 3 -> 3, 768 blocks and 49 us with the reduction (20 us of matrix
+// time), against 24 us a layer in launches of their own and 188 on the vector units
+// with the sums in a kernel of its own.  Layers up to 128 wide go through mlp_chain
+// instead of one product each.
 constexpr int kGemmTile = 64;
 constexpr int kGemmK = 32;
 constexpr int kGemmPitch = kGemmK + 4;
@@ -128,6 +128,7 @@ struct GemmArgs {
   int lda, ldb, ldc;
   int act;  // 0 none, kActTanh, kActIsru
   float* part;
+  size_t part_stride;
   int kchunk;
 };
 
@@ -136,6 +137,15 @@ struct GemmArgs {
 __device__ __forceinline__ float act_slope(int act, float h) {
   const float t = 1.0f - h * h;
   return act == kActIsru ? t * sqrtf(fmaxf(t, 0.0f)) : t;
+}
+
+// x / sqrt(1 + x^2): the hardware's reciprocal square root with one Newton step, a
+// fifth of the 38 instructions of the library's square root and division and as close
+// to the exact value.
+__device__ __forceinline__ float isru(float x) {
+  const float t = fmaf(x, x, 1.0f), r = __builtin_amdgcn_rsqf(t), h = 0.5f * r;
+  const float n = fmaf(h, fmaf(-t * r, r, 1.0f), r);
+  return x * (t < 1e38f ? n : r);  // t may overflow
 }
 
 // Eight floats of one operand's 64 x 32 tile (rows r0 .., k0 ..) for this thread.
@@ -183,19 +193,25 @@ __device__ __forceinline__ void gemm_stage(float* __restrict__ S, const floatx4_
   }
 }
 
+// One block's 64 x 64 outputs: tile (mb, nb), split z.
+struct GemmStage {
+  float A[2][kGemmTile * kGemmPitch], B[2][kGemmTile * kGemmPitch];
+};
+
 template <bool TA, bool TB>
-__global__ __launch_bounds__(256) void gemm_f32(GemmArgs g) {
-  __shared__ __attribute__((aligned(16))) float As[2][kGemmTile * kGemmPitch];
-  __shared__ __attribute__((aligned(16))) float Bs[2][kGemmTile * kGemmPitch];
+__device__ __forceinline__ void gemm_block(const GemmArgs& g, int mb, int nb, int z, GemmStage& st) {
+  auto& As = st.A;
+  auto& Bs = st.B;
   const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
   const int i16 = lane & 15, g4 = lane >> 4;
-  const int m0 = blockIdx.x * kGemmTile, n0 = blockIdx.y * kGemmTile;
+  const int m0 = mb * kGemmTile, n0 = nb * kGemmTile;
   const int wm = 32 * (w & 1), wn = 32 * (w >> 1);
-  const int kb = g.part ? (int)blockIdx.z * g.kchunk : 0;
+  const int kb = g.part ? z * g.kchunk : 0;
   const int ke = g.part ? min(g.K, kb + g.kchunk) : g.K;
   const bool va = !TA && (g.lda & 3) == 0 && (reinterpret_cast<uintptr_t>(g.A) & 15) == 0;
   const bool vb = TB && (g.ldb & 3) == 0 && (reinterpret_cast<uintptr_t>(g.B) & 15) == 0;
   const bool sums = TA && g.sums && n0 == 0;
+  const bool idle = m0 + wm >= g.M || n0 + wn >= g.N;  // a wave of nothing but padding
   floatx4_t acc[2][2] = {};  // [n tile][m tile]
   floatx4_t fa[2], fb[2];
   float sum = 0.f;
@@ -214,6 +230,7 @@ __global__ __launch_bounds__(256) void gemm_f32(GemmArgs g) {
       gemm_fetch<!TA>(g.A, g.lda, g.M, ke, m0, k0 + kGemmK, va, fa);
       gemm_fetch<TB>(g.B, g.ldb, g.N, ke, n0, k0 + kGemmK, vb, fb);
     }
+    if (idle) continue;
     const float* a = As[cur] + (wm + i16) * kGemmPitch + 4 * g4;
     const float* b = Bs[cur] + (wn + i16) * kGemmPitch + 4 * g4;
 #pragma unroll
@@ -234,7 +251,7 @@ __global__ __launch_bounds__(256) void gemm_f32(GemmArgs g) {
     }
   }
   const size_t mn = (size_t)g.M * g.N;
-  float* P = g.part ? g.part + (size_t)blockIdx.z * (mn + (g.sums ? g.M : 0)) : nullptr;
+  float* P = g.part ? g.part + z * g.part_stride : nullptr;
   if (sums) {  // 4 waves' sums of each row, in order; the staging buffers are free after the barrier
     __syncthreads();
     As[0][threadIdx.x] = sum;
@@ -273,13 +290,240 @@ __global__ __launch_bounds__(256) void gemm_f32(GemmArgs g) {
           for (int e = 0; e < 4; ++e) v[e] = tanhf(v[e]);
         } else if (g.act == kActIsru) {
 #pragma unroll
-          for (int e = 0; e < 4; ++e) v[e] = v[e] / sqrtf(fmaf(v[e], v[e], 1.0f));
+          for (int e = 0; e < 4; ++e) v[e] = isru(v[e]);
         }
       }
       if (vc && cols == 4) *reinterpret_cast<floatx4_t*>(C + at) = v;
       else
         for (int e = 0; e < cols; ++e) C[at + e] = v[e];
     }
+  }
+}
+
+template <bool TA, bool TB>
+__global__ __launch_bounds__(256) void gemm_f32(GemmArgs g) {
+  __shared__ __attribute__((aligned(16))) GemmStage st;
+  gemm_block<TA, TB>(g, blockIdx.x, blockIdx.y, blockIdx.z, st);
+}
+
+// Weight and bias gradients of all layers, dW_l = dZ_l^T H_(l-1) and db_l = column sums
+// of dZ_l: block x is a tile of some layer, block y a split.
+constexpr int kMaxLayers = 17;  // 16 hidden layers and the output
+struct DwArgs {
+  GemmArgs layer[kMaxLayers];
+  int first[kMaxLayers + 1];  // first tile of each layer
+};
+
+static __global__ __launch_bounds__(256) void gemm_dw(DwArgs a) {
+  __shared__ __attribute__((aligned(16))) GemmStage st;
+  int l = 0;
+  while ((int)blockIdx.x >= a.first[l + 1]) ++l;
+  const GemmArgs& g = a.layer[l];
+  const int tile = blockIdx.x - a.first[l], mt = (g.M + kGemmTile - 1) / kGemmTile;
+  gemm_block<true, false>(g, tile % mt, tile / mt, blockIdx.y, st);
+}
+
+// ------------------------------------------------- chains of layers up to 128 wide
+// A block takes 16 MT samples through all layers, forward (from the inputs) or
+// backward (from the output's gradient to every layer's dZ), its activations in LDS
+// between layers and stored once for the products that need them later.  Wave w
+// computes columns 32 w .. + 31 with the layer's weights in registers, in the matrix
+// instruction's operand order.  As one product a layer, each launch wrote 17 MB that
+// the next one read back behind a launch of 4 us: 70 us forward and 56 backward at
+// 32,768 samples (16 us of matrix time each), against 47 and 48 here, where a layer's
+// loads and stores still alternate with its products (32 samples a block: 58 and 49).
+// A training step on 4,096 samples took 133 us and takes 80.
+constexpr int kChainWidth = 128;
+constexpr int kChainPitch = kChainWidth + 4;
+
+struct ChainArgs {
+  int n, nin, width, nout, layers, act;
+  const float* P;     // parameters
+  const float* X;     // forward: inputs [n][nin]
+  const float* dY;    // backward: output gradient [n][nout]
+  float* H;           // layer l's output at H + l slot
+  float* dZ;          // backward: layer l's dZ at dZ + l slot
+  size_t slot;
+};
+
+__device__ __forceinline__ int64_t chain_offset(const ChainArgs& a, int l) {
+  return l == 0 ? 0 : (int64_t)a.width * a.nin + a.width + (int64_t)(l - 1) * (a.width * (a.width + 1));
+}
+
+// 16-k blocks a product of length k is unrolled for.
+__host__ __device__ constexpr int chain_blocks(int k) { return k <= 16 ? 1 : k <= 32 ? 2 : k <= 64 ? 4 : 8; }
+
+// LDS rows m0 .. of X [n][k], zero past the end and up to the product's length.
+template <int MT>
+__device__ __forceinline__ void chain_load(float (*Hs)[kChainPitch], const float* __restrict__ X, int n, int m0, int k) {
+  const int blocks = chain_blocks(k), shift = 4 + (blocks > 1) + (blocks > 2) + (blocks > 4);
+  for (int t = threadIdx.x; t < (16 * MT) << shift; t += 256) {
+    const int r = t >> shift, c = t & ((1 << shift) - 1);
+    Hs[r][c] = m0 + r < n && c < k ? X[(size_t)(m0 + r) * k + c] : 0.f;
+  }
+}
+
+// acc = LDS rows times the wave's 32 columns of B(k, n) = TB ? W[n][k] : W[k][n], for
+// K <= 16 KK.  Row r of product p is column n0 + 2 r + p, so that a lane reads W[k][n]
+// two columns at a time and its results are eight consecutive columns.  Columns past
+// the end repeat the last (they are not kept), k past the end is zero; without a
+// branch among them all loads are in flight together.
+template <int MT, bool TB, int KK>
+__device__ __forceinline__ void chain_product_k(const float (*Hs)[kChainPitch], const float* __restrict__ W, int K,
+                                                int N, int n0, floatx4_t acc[MT][2]) {
+  const int lane = threadIdx.x & 63, i16 = lane & 15, g4 = lane >> 4;
+  typedef float floatx2_t __attribute__((ext_vector_type(2)));
+  floatx4_t bv[2][KK];
+  const int n = n0 + 2 * i16;
+  if (TB && K == 16 * KK && (reinterpret_cast<uintptr_t>(W) & 15) == 0) {
+#pragma unroll
+    for (int kk = 0; kk < KK; ++kk)
+#pragma unroll
+      for (int p = 0; p < 2; ++p)
+        bv[p][kk] = *reinterpret_cast<const floatx4_t*>(W + (size_t)min(n + p, N - 1) * K + 16 * kk + 4 * g4);
+  } else if (!TB && (N & 1) == 0 && (reinterpret_cast<uintptr_t>(W) & 7) == 0) {
+#pragma unroll
+    for (int kk = 0; kk < KK; ++kk)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const int k = 16 * kk + 4 * g4 + e;
+        const floatx2_t y = *reinterpret_cast<const floatx2_t*>(W + (size_t)min(k, K - 1) * N + min(n, N - 2));
+        bv[0][kk][e] = k < K ? y[0] : 0.f;
+        bv[1][kk][e] = k < K ? y[1] : 0.f;
+      }
+  } else {
+#pragma unroll
+    for (int kk = 0; kk < KK; ++kk)
+#pragma unroll
+      for (int p = 0; p < 2; ++p)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          const int k = 16 * kk + 4 * g4 + e, kc = min(k, K - 1), nc = min(n + p, N - 1);
+          const float y = TB ? W[(size_t)nc * K + kc] : W[(size_t)kc * N + nc];
+          bv[p][kk][e] = k < K ? y : 0.f;
+        }
+  }
+#pragma unroll
+  for (int kk = 0; kk < KK; ++kk) {
+    floatx4_t av[MT];
+#pragma unroll
+    for (int q = 0; q < MT; ++q)
+      av[q] = *reinterpret_cast<const floatx4_t*>(&Hs[16 * q + i16][16 * kk + 4 * g4]);
+#pragma unroll
+    for (int s = 0; s < 4; ++s)
+#pragma unroll
+      for (int q = 0; q < MT; ++q)
+#pragma unroll
+        for (int p = 0; p < 2; ++p)
+          acc[q][p] = __builtin_amdgcn_mfma_f32_16x16x4f32(bv[p][kk][s], av[q][s], acc[q][p], 0, 0, 0);
+  }
+}
+
+template <int MT, bool TB>
+__device__ __forceinline__ void chain_product(const float (*Hs)[kChainPitch], const float* __restrict__ W, int K, int N,
+                                              int n0, floatx4_t acc[MT][2]) {
+  if (chain_blocks(K) == 1) chain_product_k<MT, TB, 1>(Hs, W, K, N, n0, acc);
+  else if (chain_blocks(K) == 2) chain_product_k<MT, TB, 2>(Hs, W, K, N, n0, acc);
+  else if (chain_blocks(K) == 4) chain_product_k<MT, TB, 4>(Hs, W, K, N, n0, acc);
+  else chain_product_k<MT, TB, 8>(Hs, W, K, N, n0, acc);
+}
+
+__device__ __forceinline__ floatx4_t chain_read(const float* __restrict__ row, int n, int N, bool vec) {
+  floatx4_t v = {0.f, 0.f, 0.f, 0.f};
+  if (vec && n + 4 <= N) v = *reinterpret_cast<const floatx4_t*>(row + n);
+  else
+    for (int e = 0; e < 4; ++e)
+      if (n + e < N) v[e] = row[n + e];
+  return v;
+}
+// The block's rows of a layer's result from LDS to X [n][k].
+template <int MT>
+__device__ __forceinline__ void chain_store(const float (*Hs)[kChainPitch], float* __restrict__ X, int n, int m0, int k) {
+  const int rows = min(16 * MT, n - m0);
+  if ((k & 3) == 0 && (reinterpret_cast<uintptr_t>(X) & 15) == 0) {
+    const int c = 4 * (threadIdx.x & 31);
+    if (c < k)
+      for (int r = threadIdx.x >> 5; r < rows; r += 8)
+        *reinterpret_cast<floatx4_t*>(X + (size_t)(m0 + r) * k + c) = *reinterpret_cast<const floatx4_t*>(&Hs[r][c]);
+  } else {
+    for (int r = threadIdx.x >> 5; r < rows; r += 8)
+      for (int c = threadIdx.x & 31; c < k; c += 32) X[(size_t)(m0 + r) * k + c] = Hs[r][c];
+  }
+}
+
+// One layer of mlp_chain: samples m0 .. m0 + 16 MT - 1 (LDS rows Hs), columns n0 ..
+// n0 + 31.  idle: the wave has no part in it; zero: but its columns are set to zero.
+template <int MT, bool FORWARD>
+__device__ __forceinline__ void chain_layer(const ChainArgs& a, float (*Hs)[kChainPitch], int l, int m0, int n0,
+                                            bool idle, bool zero) {
+  const int lane = threadIdx.x & 63, i16 = lane & 15, g4 = lane >> 4;
+  const int last = a.layers - 1;
+  const int din = l == 0 ? a.nin : a.width, dout = l == last ? a.nout : a.width;
+  const float* W = a.P + chain_offset(a, l);
+  const int N = FORWARD ? dout : din;
+  const bool vec = (N & 3) == 0 && ((reinterpret_cast<uintptr_t>(a.H) | reinterpret_cast<uintptr_t>(a.dZ)) & 15) == 0 &&
+                   (a.slot & 3) == 0;
+  floatx4_t acc[MT][2] = {}, h[MT][2], bias[2] = {};
+  const int n8 = n0 + 8 * g4;  // the lane's columns n8 .. n8 + 7 of rows 16 q + i16
+  if (!idle) {
+    if constexpr (FORWARD) {
+#pragma unroll
+      for (int e = 0; e < 8; ++e) bias[e >> 2][e & 3] = W[(size_t)din * dout + min(n8 + e, N - 1)];
+      chain_product<MT, true>(Hs, W, din, N, n0, acc);
+    } else {
+      // the outputs that the slope needs, under the products
+#pragma unroll
+      for (int q = 0; q < MT; ++q)
+#pragma unroll
+        for (int c = 0; c < 2; ++c)
+          h[q][c] = chain_read(a.H + (l - 1) * a.slot + (size_t)min(m0 + 16 * q + i16, a.n - 1) * N, n8 + 4 * c, N, vec);
+      chain_product<MT, false>(Hs, W, dout, N, n0, acc);
+    }
+  }
+  __syncthreads();  // every wave has read this layer's rows
+  if (!idle || zero) {
+#pragma unroll
+    for (int q = 0; q < MT; ++q)
+#pragma unroll
+      for (int c = 0; c < 2; ++c) {
+        floatx4_t v = {acc[q][0][2 * c], acc[q][1][2 * c], acc[q][0][2 * c + 1], acc[q][1][2 * c + 1]};
+        if (!idle) {
+#pragma unroll
+          for (int e = 0; e < 4; ++e) {
+            if constexpr (FORWARD) {
+              v[e] += bias[c][e];
+              if (l != last) {
+                if (a.act == kActTanh) v[e] = tanhf(v[e]);
+                else if (a.act == kActIsru) v[e] = isru(v[e]);
+              }
+            } else {
+              v[e] *= act_slope(a.act, h[q][c][e]);
+            }
+            if (n8 + 4 * c + e >= N) v[e] = 0.f;
+          }
+        }
+        *reinterpret_cast<floatx4_t*>(&Hs[16 * q + i16][n8 + 4 * c]) = v;
+      }
+  }
+  __syncthreads();
+}
+
+template <int MT, bool FORWARD>
+__global__ __launch_bounds__(256, 2) void mlp_chain(ChainArgs a) {
+  __shared__ __attribute__((aligned(16))) float Hs[16 * MT][kChainPitch];
+  const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int m0 = blockIdx.x * 16 * MT;
+  const int last = a.layers - 1;
+  chain_load<MT>(Hs, FORWARD ? a.X : a.dY, a.n, m0, FORWARD ? a.nin : a.nout);
+  __syncthreads();
+  for (int i = 0; i < (FORWARD ? a.layers : last); ++i) {
+    const int l = FORWARD ? i : last - i;
+    const int N = FORWARD ? (l == last ? a.nout : a.width) : (l == 0 ? a.nin : a.width);
+    if (N <= 32)  // a 16-row tile to each wave instead of 32 columns
+      chain_layer<1, FORWARD>(a, Hs + 16 * (w % MT), l, m0 + 16 * (w % MT), 0, w >= MT, false);
+    else
+      chain_layer<MT, FORWARD>(a, Hs, l, m0, 32 * w, 32 * w >= N, true);
+    chain_store<MT>(Hs, FORWARD ? a.H + l * a.slot : a.dZ + (l - 1) * a.slot, a.n, m0, N);
   }
 }
 
