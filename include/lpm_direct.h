@@ -347,13 +347,16 @@ int lpm_bve_batch_steps(lpm_bve_batch *batch, double dt, int nsteps);
 int lpm_bve_batch_get_state(lpm_bve_batch *batch, double *x, double *y, double *z,
                             double *relvort, double *u, double *v, double *w);
 /* Tile shape: targets per lane (2, 4, 8), sources per compensated tile and
- * sources per work item. */
+ * sources per work item.  A shape set here is used for all problems; otherwise
+ * FP32 problems of 2e9 pairs or more take their well-separated tiles on the
+ * matrix units and the shape is that of the smaller ones. */
 int lpm_bve_batch_set_tuning(lpm_bve_batch *batch, int targets_per_lane, int tile_sources,
                              int chunk_sources);
 int lpm_bve_batch_get_tuning(lpm_bve_batch *batch, int *targets_per_lane, int *tile_sources,
                              int *chunk_sources, int *n_items);
-/* Autotuner: times one velocity evaluation for each candidate tile shape and
- * keeps the fastest (any output pointer may be NULL). */
+/* Autotuner: times one velocity evaluation for each candidate tile shape, with
+ * and without the matrix-unit path, and keeps the fastest (any output pointer
+ * may be NULL). */
 int lpm_bve_batch_autotune(lpm_bve_batch *batch, int *targets_per_lane, int *tile_sources,
                            int *chunk_sources, double *best_ms);
 /* Pair interactions of one velocity evaluation (sum over problems of T*S - S). */
@@ -508,8 +511,9 @@ int lpm_reset_kernel_stats(lpm_ctx *ctx);
  * chunks of about 2,048 sources, at least enough splits to fill the GPU,
  * at most 2 GiB of FP64 split partials; a forced count is not capped, and
  * its partials take splits x outputs x targets x 8 bytes of device memory).
- * Values 0 restore the per-kind
- * defaults.  The FP64 PSE derivative, interpolation and SWE kinds have no
+ * Values 0 restore the per-kind defaults.  A forced targets_per_lane or
+ * tile_sources also keeps a large sum on the all-pairs kernel; a forced split
+ * count keeps a PSE or shallow-water sum there.  The FP64 PSE derivative, interpolation and SWE kinds have no
  * 8-targets-per-lane kernel: their calls then fail with LPM_ERR_ARG.  The
  * shape changes the schedule, not the result beyond FP32 (FP64) rounding. */
 int lpm_set_tuning(lpm_ctx *ctx, int kind, int precision, int targets_per_lane,

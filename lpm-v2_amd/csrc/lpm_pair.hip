@@ -267,6 +267,12 @@ constexpr double kTestedReach = 8.5;
 constexpr int kFarRounds = 8;   // rounds of resident blocks wanted of a far-tile sum
 constexpr int kFarGroups = 8;   // at most so many groups of FAR_FOLD sources per split
 constexpr int kCullWaves = 12;  // waves per SIMD wanted of a culled sum
+// Source tiles from which a PSE sum looks at groups of 64 first (512^2 PSE-8 in FP32:
+// 350 us over all tiles, 321 over groups; a launch of 4 us).
+constexpr int kGroupTiles = 512;
+// PSE sums: tiles within sqrt(kNearQ) eps are added without a test (the bound needs at
+// least 16; 20 to 60 are within 3 %).
+constexpr double kNearQ = 36.0;
 
 using KernelFn = void (*)(PairArgs);
 
@@ -420,16 +426,10 @@ constexpr size_t kPartialCap = size_t(2) << 30;  // bytes of FP64 split partials
 // and short chunks over more waves win: one target per lane, at least kSmallChunk
 // sources and about kSmallWaves waves.  Kernel times against 2 targets per lane and
 // 256 sources: level 3 FP64 82 -> 16 us, level 4 FP64 82 -> 42 us and FP32 57 -> 30 us,
-// cubed level 5 FP64 92 -> 65 us, level 5 FP64 (6e8 pairs) 420 -> 360 us.  In FP32, and
+// cubed level 5 FP64 92 -> 65 us, level 5 FP64 (6e8 pairs) 420 -> 360 us (13, 36, 57 and
+// 350 with the reciprocals in fours).  In FP32, and
 // for the longer PSE pairs, 2 targets per lane are as fast at 7.5e7 pairs and 3-6 %
 // faster at 3e8.
-// Source tiles from which a PSE sum looks at groups of 64 first (512^2 PSE-8 in FP32:
-// 350 us over all tiles, 321 over groups; a launch of 4 us).
-constexpr int kGroupTiles = 512;
-// PSE sums: tiles within sqrt(kNearQ) eps are added without a test (the bound needs at
-// least 16; 20 to 60 are within 3 %).
-constexpr double kNearQ = 36.0;
-
 constexpr double kSmallPairs = 1.2e8, kSmallPairsVortex64 = 1e9;
 constexpr int kSmallChunk = 64;
 constexpr int kSmallWaves = 24576;
@@ -650,7 +650,7 @@ int run_pair_sum(lpm_ctx* ctx, const PairProblem& pp) {
     // targets per lane from a sweep of R in {1, 2, 4, 8} on MI355X (512^2
     // plane, icosahedral L7): in FP32 the sphere operators (series distance)
     // at R = 1, the plane derivative sums and interpolation at R = 2, the
-    // 7-sum SWE kernel at R = 1; in FP64 every operator at R = 2 (R = 1 was
+    // SWE kernel at R = 1; in FP64 every operator at R = 2 (R = 1 was
     // 3-7 % slower for the sphere gradient and divergence, R = 4 up to 25 %)
     if (prec == LPM_PREC_FP32_KAHAN)
       tu.r = kind == LPM_K_PSE_DERIV_SPHERE || kind == LPM_K_PSE_INTERP_SPHERE || kind == LPM_K_SWE_PLANE ? 1 : 2;
