@@ -144,7 +144,7 @@ struct PairProblem {
   DevBuf* tgt_buf = nullptr;
   DevBuf* src_buf = nullptr;
   DevBuf* partial_buf = nullptr;
-  DevBuf* red_buf = nullptr;  // FP32 sphere Green: the two FP64 source totals
+  DevBuf* red_buf = nullptr;  // FP32 sphere Green: the two FP64 source totals and their partials
   DevBuf* order_buf = nullptr;
   // Spatial order of targets and sources when the caller has it (a solver keeps
   // one for the four sums of a step); else run_pair_sum makes one where it is used.

@@ -365,3 +365,17 @@ def test_tiles_passed_over_never_matter(ctx, field, space):
         err = np.abs(got - ref)[seen] / np.abs(ref[seen])
         assert np.quantile(err, 0.99) < 1e-11 and err.max() < 1e-7
         assert np.abs(got[~seen]).max(initial=0.0) < 1e-289
+
+
+@pytest.mark.parametrize("active", [0, 1, 1023, 1024, 1025, 2049, 20480])
+def test_stream_source_totals(ctx, active):
+    """The FP32 stream function adds the sources' total in FP64: none, one block of
+    1,024 sources, a remainder, many.  FP64 sums of the same sources, the FP32 bar."""
+    m = mesh.icosahedral_mesh(5)
+    act = np.zeros(m.n, np.int32)
+    act[np.flatnonzero(m.active)[:active]] = 1
+    q = 1.0 + 0.5 * m.z  # one sign: the total is as large as it can be
+    got = ctx.bve_sphere_stream(m.x, m.y, m.z, q, q + m.x, m.area, act, precision="fp32")
+    ref = ctx.bve_sphere_stream(m.x, m.y, m.z, q, q + m.x, m.area, act, precision="fp64")
+    for g, r in zip(got, ref):
+        assert np.abs(g - r).max() <= 2e-6 * np.abs(r).max()
