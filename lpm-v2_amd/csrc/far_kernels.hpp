@@ -140,10 +140,11 @@ struct FarStageOf<FarSwePlane> {
 };
 
 // The direct VALU sum of one near tile for the wave's 64 targets (lane = target);
-// SELF: the tile may hold the targets' own particles.  The records of the next
-// NEAR_AHEAD sources load (scalar) under the arithmetic of these: with 64 targets
-// per source, one record ahead does not cover the latency of the load.
-constexpr int NEAR_AHEAD = 4;
+// SELF: the tile may hold the targets' own particles.  The near tiles are a tenth of
+// the pairs at 1e10 and wait for their records more than for their arithmetic: with
+// scalar loads 2, 4 and 6 sources ahead the velocity at level 6 took 1,791, 1,714 and
+// 1,676 us, with the tile in LDS, loaded one tile ahead, 1,684, and the same at 61,441
+// targets 964 (4 ahead) and 937.  Without near tiles it would take 1,404.
 // Sources per FP32 partial sum.  Sources in spatial order push a partial sum in one
 // direction, so it rounds more than one over scattered sources: with 256 per partial
 // the 100^2 plane velocity was off by 1.05e-7 against 6.1e-8 in the caller's order.
@@ -167,50 +168,25 @@ __device__ __forceinline__ void near_source(const Vec4<float>& t, int tid, const
   }
 }
 
+// `rec`: the tile's records in LDS, two 16-byte words each.
 template <class N, bool SELF>
-__device__ __forceinline__ void near_tile(const Vec4<float>& t, int tid, const float* __restrict__ src, int jt,
-                                          int jt_end, double S[N::NOUT]) {
-  constexpr int NO = N::NOUT, G = NEAR_AHEAD;
-  float p[NO];
+__device__ __forceinline__ void near_tile(const Vec4<float>& t, int tid, const float4* rec, int count,
+                                          double S[N::NOUT]) {
+  constexpr int NO = N::NOUT;
+  for (int j0 = 0; j0 < count; j0 += NEAR_FOLD) {
+    const int j1 = min(count, j0 + NEAR_FOLD);
+    float p[NO];
 #pragma unroll
-  for (int k = 0; k < NO; ++k) p[k] = 0.f;
-  int j = jt;
-  if (jt + G <= jt_end) {
-    float sv[G][SREC];
-#pragma unroll
-    for (int g = 0; g < G; ++g)
-#pragma unroll
-      for (int q = 0; q < SREC; ++q) sv[g][q] = src[(size_t)(jt + g) * SREC + q];
-    for (; j + G <= jt_end; j += G) {
-      const int jn = j + 2 * G <= jt_end ? j + G : j;
-      float sn[G][SREC];
-#pragma unroll
-      for (int g = 0; g < G; ++g)
-#pragma unroll
-        for (int q = 0; q < SREC; ++q) sn[g][q] = src[(size_t)(jn + g) * SREC + q];
-#pragma unroll
-      for (int g = 0; g < G; ++g) near_source<N, SELF>(t, tid, sv[g], p);
-#pragma unroll
-      for (int g = 0; g < G; ++g)
-#pragma unroll
-        for (int q = 0; q < SREC; ++q) sv[g][q] = sn[g][q];
-      if (((j - jt) & (NEAR_FOLD - 1)) == NEAR_FOLD - G) {
-#pragma unroll
-        for (int k = 0; k < NO; ++k) {
-          S[k] += (double)p[k];
-          p[k] = 0.f;
-        }
-      }
+    for (int k = 0; k < NO; ++k) p[k] = 0.f;
+#pragma unroll 4
+    for (int j = j0; j < j1; ++j) {
+      const float4 lo = rec[2 * j], hi = rec[2 * j + 1];
+      const float sv[SREC] = {lo.x, lo.y, lo.z, lo.w, hi.x, hi.y, hi.z, hi.w};
+      near_source<N, SELF>(t, tid, sv, p);
     }
-  }
-  for (; j < jt_end; ++j) {
-    float sv[SREC];
 #pragma unroll
-    for (int q = 0; q < SREC; ++q) sv[q] = src[(size_t)j * SREC + q];
-    near_source<N, SELF>(t, tid, sv, p);
+    for (int k = 0; k < NO; ++k) S[k] += (double)p[k];
   }
-#pragma unroll
-  for (int k = 0; k < NO; ++k) S[k] += (double)p[k];
 }
 
 // One step: 16 staged sources against the wave's column tiles.
@@ -309,21 +285,50 @@ __device__ __forceinline__ void far_block(const Vec4<float>* __restrict__ tg, in
   };
   const int j_begin = first_group * FAR_FOLD;
 
-  // near tiles first: no staging, no barriers
+  float rec[SREC];
+  bool have;
+  auto load = [&](int jt) {  // this thread's source of the tile at jt
+    const int j = jt + (int)threadIdx.x;
+    have = j < ns;
+    const float4* r = reinterpret_cast<const float4*>(src + (size_t)(have ? j : ns - 1) * SREC);
+    const float4 lo = r[0], hi = r[1];
+    rec[0] = lo.x, rec[1] = lo.y, rec[2] = lo.z, rec[3] = lo.w;
+    rec[4] = hi.x, rec[5] = hi.y, rec[6] = hi.z, rec[7] = hi.w;
+  };
+  int buf = 0;
   int n_far = 0;
-  for (int jt = j_begin; jt < ns; jt = next_tile(jt)) {
-    const float4 sm = smeta[jt / FAR_TILE];
-    if (is_far(sm)) {
-      ++n_far;
-      continue;
-    }
-    if (kSwe<P> || t_begin >= nt) continue;
-    const int jt_end = min(ns, jt + FAR_TILE);
-    if constexpr (!kSwe<P>) {
-      if (balls_touch(ball_d2(tm, sm), tm, sm))
-        near_tile<N, true>(t, tid, src, jt, jt_end, near_sum);
-      else
-        near_tile<N, false>(t, tid, src, jt, jt_end, near_sum);
+  // near tiles first, through the stages' memory.  Here and below one barrier a tile: a
+  // wave writes a buffer again only after the barrier of the tile between, which every
+  // wave reaches after its reads of this one.
+  if constexpr (kSwe<P>) {
+    for (int jt = j_begin; jt < ns; jt = next_tile(jt)) n_far += is_far(smeta[jt / FAR_TILE]) ? 1 : 0;
+  } else {
+    auto next_near = [&](int jt) {
+      while (jt < ns && is_far(smeta[jt / FAR_TILE])) {
+        jt = next_tile(jt);
+        ++n_far;
+      }
+      return jt;
+    };
+    int jt = next_near(j_begin);
+    if (jt < ns) load(jt);
+    while (jt < ns) {  // block-uniform
+      float4* st = reinterpret_cast<float4*>(&stage[buf]);
+      st[2 * threadIdx.x] = make_float4(rec[0], rec[1], rec[2], rec[3]);
+      st[2 * threadIdx.x + 1] = make_float4(rec[4], rec[5], rec[6], rec[7]);
+      const int jn = next_near(next_tile(jt));
+      if (jn < ns) load(jn);
+      __syncthreads();
+      if (t_begin < nt) {
+        const float4 sm = smeta[jt / FAR_TILE];
+        const int count = min(FAR_TILE, ns - jt);
+        if (balls_touch(ball_d2(tm, sm), tm, sm))
+          near_tile<N, true>(t, tid, st, count, near_sum);
+        else
+          near_tile<N, false>(t, tid, st, count, near_sum);
+      }
+      buf ^= 1;
+      jt = jn;
     }
   }
 
@@ -356,19 +361,8 @@ __device__ __forceinline__ void far_block(const Vec4<float>* __restrict__ tg, in
       while (jt < ns && !is_far(smeta[jt / FAR_TILE])) jt = next_tile(jt);
       return jt;
     };
-    float rec[SREC];
-    bool have;
-    auto load = [&](int jt) {
-      const int j = jt + (int)threadIdx.x;
-      have = j < ns;
-      const float4* r = reinterpret_cast<const float4*>(src + (size_t)(have ? j : ns - 1) * SREC);
-      const float4 lo = r[0], hi = r[1];
-      rec[0] = lo.x, rec[1] = lo.y, rec[2] = lo.z, rec[3] = lo.w;
-      rec[4] = hi.x, rec[5] = hi.y, rec[6] = hi.z, rec[7] = hi.w;
-    };
     int jt = next_far(j_begin);
     load(jt);
-    int buf = 0;
     while (jt < ns) {
       typename FarStageOf<P>::T& st = stage[buf];
       {
@@ -407,8 +401,6 @@ __device__ __forceinline__ void far_block(const Vec4<float>* __restrict__ tg, in
       }
       const int jn = next_far(next_tile(jt));
       if (jn < ns) load(jn);
-      // one barrier a tile: a wave writes a buffer again only after the barrier of
-      // the tile between, which every wave reaches after its reads of this one
       __syncthreads();
       // two register sets in turn: the next step's LDS reads run under this step
       const int wl = grp * 4 + (P::NW == 0 ? lane & 3 : 0);
