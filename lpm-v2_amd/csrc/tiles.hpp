@@ -128,10 +128,14 @@ static __global__ __launch_bounds__(256) void group_balls(int n, const float4* _
   if (lane == 0) out[g] = make_float4(x, y, z, rad);
 }
 
-// Separation of two balls: squared centre distance.
+// Separation of two balls: squared centre distance.  Here and in the rules below no
+// product is left for the compiler to fuse with a sum or not: the far and the cull
+// kernel share out the tiles of a shallow-water sum by the same rule, each for itself,
+// and with 1.001 s + 2.002 t fused one way in one and the other way in the other a tile
+// pair on the line was summed twice or not at all.
 __device__ __forceinline__ float ball_d2(const float4& a, const float4& b) {
   const float dx = a.x - b.x, dy = a.y - b.y, dz = a.z - b.z;
-  return dx * dx + dy * dy + dz * dz;
+  return fmaf(dz, dz, fmaf(dy, dy, dx * dx));
 }
 // Whether a point may lie in both balls (for any rounding; true for infinite radii):
 // only then can the tile hold a target's own particle.
@@ -150,7 +154,7 @@ constexpr int FAR_TILE = 256;     // sources per tile, targets per block of the 
 // and radii; the lower bound keeps the split's low parts normal.
 __device__ __forceinline__ bool tiles_far(const float4& t, const float4& s) {
   const float d2 = ball_d2(t, s);
-  const float th = 1.001f * s.w + 2.002f * t.w;
+  const float th = fmaf(1.001f, s.w, 2.002f * t.w);
   return d2 > th * th && d2 > 1e-28f;
 }
 

@@ -379,3 +379,60 @@ def test_stream_source_totals(ctx, active):
     ref = ctx.bve_sphere_stream(m.x, m.y, m.z, q, q + m.x, m.area, act, precision="fp64")
     for g, r in zip(got, ref):
         assert np.abs(g - r).max() <= 2e-6 * np.abs(r).max()
+
+
+# ---------------------------------------- tiles on the line between near and far
+def _clusters_on_the_far_line():
+    """16 x 16 clusters of 256 points, each on a line along x inside its own cell of the
+    order's curve, so that each is one tile: radius a (1 + 1e-6) about c, both multiples
+    of 2^-24.  Half-widths and distances of every second pair of neighbours in a row,
+    about 1/8 apart, are chosen so that the far rule, distance > 1.001 a_s + 2.002 a_t,
+    holds by one way of rounding it with one fused multiply-add and not by the other."""
+    f32 = np.float32
+    rng = np.random.default_rng(8)
+
+    def fma(a, b, c):
+        return f32(float(a) * float(b) + float(c))  # the product is exact in 64 bits
+
+    def radius(k):
+        a = f32(k * 2.0**-24)
+        return f32(np.sqrt(f32(a * a)) * f32(1.000001))
+
+    def pair():
+        while True:
+            kt, d = int(rng.integers(690000, 710000)), 2**21 + int(rng.integers(-2000, 2000))
+            ks = int(round(d / 1.001001)) - 2 * kt
+            t, s, dist = radius(kt), radius(ks), f32(d * 2.0**-24)
+            one = fma(s, f32(1.001), f32(f32(2.002) * t))
+            two = fma(t, f32(2.002), f32(f32(1.001) * s))
+            if (dist * dist > one * one) != (dist * dist > two * two):
+                return kt, ks, d
+
+    x, y = [], []
+    for row in range(16):
+        for col in range(0, 16, 2):
+            kt, ks, d = pair()
+            for side, k in enumerate((kt, ks)):
+                u = np.rint(np.linspace(-1.0, 1.0, 256) * k) + side * d
+                x.append(-1.0 + (col + 0.5) / 8 + u * 2.0**-24)
+                y.append(np.full(256, -1.0 + row / 8))
+    return np.concatenate(x), np.concatenate(y)
+
+
+def test_tiles_on_the_far_line_belong_to_one_kernel(ctx):
+    """Far and near tiles of the shallow-water sums are two kernels' work: every tile
+    pair is summed once, also where its distance is the far rule's threshold to the last
+    bit.  A cluster summed twice or not at all is off by 1e-3 and more."""
+    x, y = _clusters_on_the_far_line()
+    n = x.size
+    idx = np.random.default_rng(1).permutation(n)
+    x, y = x[idx], y[idx]
+    area = np.full(n, 4.0 / n)
+    call = _swe(ctx, x, y, area, np.ones(n, np.int32), 1e-3)
+    for g, e, r in zip(_rows(call()), _all_pairs(ctx, L.K_SWE_PLANE, "fp32", call), _rows(call("fp64"))):
+        own = rel_err_max(e, r)
+        assert rel_err_max(g, r) < max(TOL32, 1.5 * own), own
+    for kind, call in ((L.K_PLANE_BS, lambda p: ctx.plane_velocity(x, y, 1.0 + x, area, np.ones(n, np.int32),
+                                                                   precision=p)),):
+        for g, r in zip(_rows(call("fp32")), _rows(call("fp64"))):
+            assert rel_err_max(g, r) < 4 * TOL32
