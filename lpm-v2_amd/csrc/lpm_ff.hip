@@ -478,7 +478,13 @@ __device__ __forceinline__ void block_sums(double (&v)[K], double* sh) {
   for (int k = 0; k < K; ++k) v[k] = res[k];
 }
 
-// Smallest of a value over the block (NaN ignored), to every thread.
+// Cosine of the angle between (x, y, z) and a unit vector d for an angular radius; -1
+// where either is not a number, so that the radius is pi and every pair near.
+__device__ __forceinline__ double radius_cos(double x, double y, double z, double dx, double dy, double dz) {
+  return fmax(-1.0, (x * dx + y * dy + z * dz) / sqrt(x * x + y * y + z * z));
+}
+
+// Smallest of a value over the block (no NaN), to every thread.
 __device__ __forceinline__ double block_min(double v, double* sh) {
   for (int m = 32; m > 0; m >>= 1) v = fmin(v, __shfl_xor(v, m));
   if ((threadIdx.x & 63) == 0) sh[threadIdx.x >> 6] = v;
@@ -530,13 +536,13 @@ __device__ void source_moments(const GeomArgs& a, int s0, int s1, double* sh, So
     for (int i = 0; i < 15; ++i)
       v[kMomOff[4] + i] += w * d[kQuad[i][0]] * d[kQuad[i][1]] * d[kQuad[i][2]] * d[kQuad[i][3]];
     v[kNMom] += fabs(w);
-    cosmin = fmin(cosmin, (x * r.ux + y * r.uy + z * r.uz) / sqrt(x * x + y * y + z * z));
+    cosmin = fmin(cosmin, radius_cos(x, y, z, r.ux, r.uy, r.uz));
   }
   block_sums(v, sh);
 #pragma unroll
   for (int k = 0; k < kNMom; ++k) r.m[k] = v[k];
   r.wabs = v[kNMom];
-  r.rho = acos(fmax(-1.0, block_min(cosmin, sh)));
+  r.rho = acos(block_min(cosmin, sh));
 }
 
 // The FP32 far record of far_expansion_acc: c, e_c = R^2 - |c|^2, the moments
@@ -610,9 +616,9 @@ __global__ __launch_bounds__(256) void ff_cell_geometry(GeomArgs a) {
   for (int k = t0 + threadIdx.x; k < t1; k += 256) {
     const int p = a.tgt_perm[k];
     const double x = a.x[p], y = a.y[p], z = a.z[p];
-    cosmin = fmin(cosmin, (x * vx + y * vy + z * vz) / sqrt(x * x + y * y + z * z));
+    cosmin = fmin(cosmin, radius_cos(x, y, z, vx, vy, vz));
   }
-  const double trho = acos(fmax(-1.0, block_min(cosmin, sh)));
+  const double trho = acos(block_min(cosmin, sh));
   if (threadIdx.x == 0) {
     const double R = a.radius;
     const double inv = 1.0 / (4.0 * kPi * R);

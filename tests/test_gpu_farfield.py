@@ -340,3 +340,31 @@ def test_online_fine_tuning_threshold(ctx):
     with pytest.raises(Exception):
         f.set_online(2000, above=1.5)
     f.delete()
+
+
+def test_particle_that_is_not_a_number_spoils_no_other(ctx):
+    """A passive particle whose coordinates are not numbers falls in cell 0, whose extent
+    is then unknown: the cell's other targets take every cell directly, not by
+    expansions of their own neighbourhood."""
+    m, zeta = _case(5, 2)
+    # a position of its own: the far field's other targets keep theirs
+    j = int(np.flatnonzero(m.active == 0)[100])
+    x, y, z = m.x.copy(), m.y.copy(), m.z.copy()
+    f = FarFieldBVE(ctx, m, zeta, near_radius=0.1, band_radius=0.45)
+    want = np.array(f.velocity(EXPANSION))
+    exact = np.array(ctx.bve_sphere_velocity(m.x, m.y, m.z, zeta, m.area, m.active, precision="fp64"))
+    for bad in (np.nan, np.inf):
+        x[j] = y[j] = z[j] = bad
+        f.set_particles(x, y, z, zeta, m.area, m.active)
+        got = np.array(f.velocity(EXPANSION))
+        cell = f.binning()
+        assert cell[j] == 0 and np.isnan(got[:, j]).all()
+        other = np.arange(m.n) != j
+        assert np.isfinite(got[:, other]).all()
+        near = other & (cell == 0)
+        assert near.sum() > 10
+        # cell 0 is all direct sums (the FP32 bar), the other targets stay as far off as they were
+        err = np.linalg.norm(got - exact, axis=0) / np.linalg.norm(exact, axis=0).max()
+        assert err[near].max() < 1e-6
+        assert err[other].max() <= 1.5 * rel_err_max(want, exact)
+    f.delete()
