@@ -341,6 +341,11 @@ __device__ __forceinline__ void far_block(const Vec4<float>* __restrict__ tg, in
 #pragma unroll
     for (int k = 0; k < NACC; ++k) sum[c][k] = 0.0;
   const float X[3] = {t.a - tm.x, t.b - tm.y, P::DIMS == 3 ? t.c - tm.z : 0.f};
+  // A weight w times a position, or its square, leaves the normal numbers long before
+  // the all-pairs kernel's w / d^2 does (at lengths of 1e-13, of 1e18, or of 1e-6 with weak
+  // fields).  In units of the first far tile's distance, a power of two, w / d comes
+  // before the product, which lies between w and w / d^2; results keep their bits.
+  float unit = 1.f;
 
   if (n_far > 0) {  // block-uniform
     const float n2t = fmaf(X[0], X[0], fmaf(X[1], X[1], fmaf(X[2], X[2], P::E ? t.d : 0.f)));
@@ -363,6 +368,7 @@ __device__ __forceinline__ void far_block(const Vec4<float>* __restrict__ tg, in
     };
     int jt = next_far(j_begin);
     load(jt);
+    unit = inverse_length(ball_d2(tm, smeta[jt / FAR_TILE]));
     while (jt < ns) {
       typename FarStageOf<P>::T& st = stage[buf];
       {
@@ -381,18 +387,21 @@ __device__ __forceinline__ void far_block(const Vec4<float>* __restrict__ tg, in
         if constexpr (kSwe<P>) {
           // c, c conj(Z); c conj(Z)^2
           float* wb = reinterpret_cast<float*>(st.wgt2 + s * 16 + (r >> 2) * 4) + (r & 3);
-          const float vr = fmaf(w0, d[0], w1 * d[1]), vi = fmaf(w1, d[0], -w0 * d[1]);
+          const float a0 = w0 * unit, a1 = w1 * unit;
+          const float vr = fmaf(a0, d[0], a1 * d[1]), vi = fmaf(a1, d[0], -a0 * d[1]);
+          const float br = vr * unit, bi = vi * unit;
           w[0] = w0;
           w[4] = w1;
           w[8] = vr;
           w[12] = vi;
-          wb[0] = fmaf(vr, d[0], vi * d[1]);
-          wb[4] = fmaf(vi, d[0], -vr * d[1]);
+          wb[0] = fmaf(br, d[0], bi * d[1]);
+          wb[4] = fmaf(bi, d[0], -br * d[1]);
           wb[8] = wb[12] = 0.f;
         } else if constexpr (P::NW == 0) {
-          w[0] = w0 * d[0];
-          w[4] = w0 * d[1];
-          w[8] = w0 * d[2];
+          const float a0 = w0 * unit;
+          w[0] = a0 * d[0];
+          w[4] = a0 * d[1];
+          w[8] = a0 * d[2];
           w[12] = w0;
         } else {
           w[0] = w0;
@@ -460,19 +469,20 @@ __device__ __forceinline__ void far_block(const Vec4<float>* __restrict__ tg, in
   }
   if (i < nt) {
     double o[NO];
+    const double length = 1.0 / unit;
     if constexpr (kSwe<P>) {
-      const double x = X[0], y = X[1], xx = x * x - y * y, xy = 2.0 * x * y;
       const double* u1 = far_sum;     // f c, f c conj(Z)
       const double* u2 = far_sum + 4;  // f^2 c, f^2 c conj(Z), f^2 c conj(Z)^2
-      o[0] = x * u1[1] - y * u1[0] - u1[3];
-      o[1] = x * u1[0] + y * u1[1] - u1[2];
-      o[2] = -(xx * u2[1] - xy * u2[0] - 2.0 * (x * u2[3] - y * u2[2]) + u2[5]);
-      o[3] = -(xx * u2[0] + xy * u2[1] - 2.0 * (x * u2[2] + y * u2[3]) + u2[4]);
+      const double x = (double)X[0] * unit, y = (double)X[1] * unit, xx = x * x - y * y, xy = 2.0 * x * y;
+      o[0] = (x * u1[1] - y * u1[0] - u1[3]) * length;
+      o[1] = (x * u1[0] + y * u1[1] - u1[2]) * length;
+      o[2] = -(xx * u2[1] - xy * u2[0] - 2.0 * (x * u2[3] - y * u2[2]) + u2[5]) * (length * length);
+      o[3] = -(xx * u2[0] + xy * u2[1] - 2.0 * (x * u2[2] + y * u2[3]) + u2[4]) * (length * length);
       o[4] = 0.0;
     } else if constexpr (P::NW == 0) {
       double v[3];
 #pragma unroll
-      for (int k = 0; k < 3; ++k) v[k] = (double)X[k] * far_sum[3] - far_sum[k];
+      for (int k = 0; k < 3; ++k) v[k] = (double)X[k] * far_sum[3] - far_sum[k] * length;
       if constexpr (P::DIMS == 3) {
 #pragma unroll
         for (int k = 0; k < 3; ++k) o[k] = v[k];

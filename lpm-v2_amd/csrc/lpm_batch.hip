@@ -386,6 +386,7 @@ int eval_velocity(lpm_bve_batch* b, const double* x, const double* y, const doub
     sr.desc = t.desc + b->n_tballs;
     sr.balls = b->n_sballs;
     t.dims = sr.dims = 3;
+    t.limit = sr.limit = lpm::kFarLimit;
     hipLaunchKernelGGL(lpm::tile_balls<float>, dim3((b->n_tballs + b->n_sballs + 3) / 4), dim3(256), 0, ctx->stream,
                        t, sr);
     hipLaunchKernelGGL(pick_far(on_sphere), dim3((unsigned)std::min(b->far_grid, b->n_far_items)), dim3(256), 0,

@@ -597,6 +597,7 @@ static void launch_balls(int kind, int m, int nw, const void* trec, const void* 
   t.dims = s.dims = sphere_kind(kind) ? 3 : 2;
   t.finite_mask = finite_words(kind, m, true);
   t.balls = (nt + t_tile - 1) / t_tile;
+  if (is_vortex_kind(kind)) t.limit = s.limit = kFarLimit;
   s.rec = static_cast<const T*>(srec);
   s.out = sballs;
   s.words = nw;

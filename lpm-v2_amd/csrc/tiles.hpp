@@ -11,14 +11,16 @@ namespace lpm {
 
 // One set of records: n records of `words` values, `tile` records to a ball (at most
 // 256), coordinates in the first `dims` words.  A ball is {centre, radius}; its radius
-// is infinite when any word of `finite_mask` is not finite, so that the tile gets no
-// shortcut and its infinities and NaN spread as in the sum over all pairs.
+// is infinite when any word of `finite_mask` is not finite, or a coordinate beyond
+// `limit`, so that the tile gets no shortcut and its infinities and NaN spread as in the
+// sum over all pairs.
 template <typename T>
 struct BallSet {
   const T* rec = nullptr;
   float4* out = nullptr;
   int words = 0, n = 0, tile = 64, dims = 2;
   unsigned finite_mask = 0;
+  float limit = __builtin_huge_valf();
   const int2* desc = nullptr;  // when set: (first record, count) of every ball
   int balls = 0;
   // when set: binary exponents e of the largest magnitudes among the words of each
@@ -56,7 +58,10 @@ __device__ __forceinline__ void ball_of(const BallSet<T>& a, int b) {
         if ((a.mag_mask[0] >> k) & 1u) big[0] = fmax(big[0], fabs(r[k]));
         if ((a.mag_mask[1] >> k) & 1u) big[1] = fmax(big[1], fabs(r[k]));
       }
-      for (int k = 0; k < a.dims; ++k) c[q][k] = r[k];
+      for (int k = 0; k < a.dims; ++k) {
+        c[q][k] = r[k];
+        bad = bad || fabs(r[k]) > (T)a.limit;
+      }
 #pragma unroll
       for (int k = 0; k < 3; ++k) {
         lo[k] = fmin(lo[k], c[q][k]);
@@ -145,17 +150,25 @@ __device__ __forceinline__ bool balls_touch(float d2, const float4& a, const flo
 }
 
 constexpr int FAR_TILE = 256;     // sources per tile, targets per block of the far path
+// Coordinates of far tiles: squared distances stay below 1.2e37, norms below 5e37.
+constexpr float kFarLimit = 1e18f;
 
 // Well separated: every target-source distance is at least the radius of the target
 // block (|Y| >= 2 rho_t).  The norms and products above are then at most 9 times the
 // denominator for the closest pairs and about equal to it for nearly all; errors
 // against FP64 are the same with 3 rho_t, and fewer tiles go the VALU way.  The
 // margins keep a pair of equal points (a self pair) out for any rounding of centres
-// and radii; the lower bound keeps the split's low parts normal.
+// and radii; the lower bound keeps the split's low parts normal (kFarLimit: the norms finite).
 __device__ __forceinline__ bool tiles_far(const float4& t, const float4& s) {
   const float d2 = ball_d2(t, s);
   const float th = fmaf(1.001f, s.w, 2.002f * t.w);
   return d2 > th * th && d2 > 1e-28f;
+}
+
+// Power of two about 1 / d, for the d2 of a far tile.
+__device__ __forceinline__ float inverse_length(float d2) {
+  const int e = ((int)(__float_as_uint(d2) >> 23) - 127) >> 1;
+  return __uint_as_float((unsigned)(127 - e) << 23);
 }
 
 // f^2 stays a normal number: pair distances are at least 1e-3 of the centres'

@@ -436,3 +436,49 @@ def test_tiles_on_the_far_line_belong_to_one_kernel(ctx):
                                                                    precision=p)),):
         for g, r in zip(_rows(call("fp32")), _rows(call("fp64"))):
             assert rel_err_max(g, r) < 4 * TOL32
+
+
+# ------------------------------------------------------- lengths and weights of any unit
+@pytest.mark.parametrize("length,weight", [(1e-13, 1.0), (1e-11, 1.0), (1e-6, 1e-15), (1e6, 1e-5), (1e18, 1.0),
+                                           (3e19, 1.0)])
+@pytest.mark.parametrize("space", ["plane", "sphere"])
+def test_far_tiles_in_any_unit(ctx, space, length, weight):
+    """Far tiles multiply weights by positions and squares by each other: lengths at which
+    those products leave the normal numbers, where a pair of the all-pairs kernel does
+    not.  As far off the FP64 sums as that kernel is, or within the FP32 bar."""
+    if space == "plane":
+        x, y, area, _ = mesh.grid_centres(270, 1.0, jitter=5e-4, seed=2)
+        x, y, area, q, act = x * length, y * length, area * length**2, weight * (1 + 0.5 * np.sin(5 * x)), np.ones(
+            x.size, np.int32)
+        calls = ((L.K_PLANE_BS, lambda p: ctx.plane_velocity(x, y, q, area, act, precision=p)),
+                 (L.K_PLANE_GREEN, lambda p: ctx.plane_stream(x, y, q, area, act, precision=p)))
+    else:
+        x, y, z, q, area, act = _sphere("mesh")
+        x, y, z, q, area = x * length, y * length, z * length, q * weight, area * length**2
+        i1 = 50000
+        calls = ((L.K_SPHERE_BS, lambda p: ctx.bve_sphere_velocity(x, y, z, q, area, act, i1=i1, radius=length,
+                                                                   precision=p)),
+                 (L.K_SPHERE_GREEN, lambda p: ctx.bve_sphere_stream(x, y, z, q, q, area, act, i1=i1, radius=length,
+                                                                    precision=p)))
+    for kind, call in calls:
+        got, pairs, exact = _rows(call("fp32")), _all_pairs(ctx, kind, "fp32", lambda: call("fp32")), _rows(call("fp64"))
+        for g, e, r in zip(got, pairs, exact):
+            assert np.array_equal(np.isfinite(g), np.isfinite(e))
+            if np.isfinite(e).all():  # (logarithms of squares beyond the FP32 range are not)
+                own = rel_err_max(e, r)
+                assert rel_err_max(g, r) < max(TOL32, 1.5 * own), own
+
+
+def test_far_shallow_water_with_weak_fields(ctx):
+    """As above for the products c conj(Z)^2: lengths of 1e-5 and fields of 1e-14."""
+    x, y, area, h = mesh.grid_centres(270, 1.0, jitter=1e-3, seed=3)
+    s, act = 1e-5, np.ones(x.size, np.int32)
+    vort, div = 1e-14 * (np.sin(3 * x) + y), 1e-14 * np.cos(2 * y) * x
+
+    def call(prec="fp32"):
+        return ctx.swe_plane_rhs(s * x, s * y, vort, div, 1.0 + 0.1 * x, 0.05 * y, s * s * area, act, 2 * s * h,
+                                 precision=prec)
+
+    for g, e, r in zip(_rows(call()), _all_pairs(ctx, L.K_SWE_PLANE, "fp32", call), _rows(call("fp64"))):
+        own = rel_err_max(e, r)
+        assert rel_err_max(g, r) < max(TOL32, 1.5 * own), own
