@@ -482,3 +482,84 @@ def test_far_shallow_water_with_weak_fields(ctx):
     for g, e, r in zip(_rows(call()), _all_pairs(ctx, L.K_SWE_PLANE, "fp32", call), _rows(call("fp64"))):
         own = rel_err_max(e, r)
         assert rel_err_max(g, r) < max(TOL32, 1.5 * own), own
+
+
+# ------------------------------------------------------- groups of 64 source tiles
+def _assert_culled(pairs):
+    """Calls of fewer pairs take the all-pairs kernel (kCullMinPairs of lpm_pair.hip)."""
+    assert pairs >= 1.5e8
+
+
+@pytest.mark.parametrize("prec", ["fp64", "fp32"])
+@pytest.mark.parametrize("eps_h", [2.0, 9.0])
+@pytest.mark.parametrize("side,block", [(182, 5000), (520, 1000)])
+def test_culled_plane_sums_over_groups(ctx, prec, eps_h, side, block):
+    """From 512 source tiles on, groups of 64 are tested first: 518 tiles, the last group
+    of 6, and 4,225, more than the 64 groups that one mask holds.  Shuffled, a block of
+    targets, then one source that is not finite."""
+    x, y, area, h = mesh.grid_centres(side, 1.0, jitter=0.2 / side, seed=3)
+    n = x.size
+    rng = np.random.default_rng(5)
+    idx = rng.permutation(n)
+    x, y, area = x[idx], y[idx], area[idx]
+    f = np.exp(-4.0 * (x * x + y * y)) + 0.3 * x
+    act = np.ones(n, np.int32)
+    act[rng.permutation(n)[:50]] = 0
+    _assert_culled((n - 50) * block)
+    i0, eps = n // 3, eps_h * h
+    px, py = rng.uniform(-1, 1, block), rng.uniform(-1, 1, block)
+    calls = ((L.K_PSE8, lambda: ctx.pse_plane_laplacian(x, y, f, area, act, eps, order=8, i0=i0, i1=i0 + block,
+                                                        precision=prec)),
+             (L.K_PSE_DERIV_PLANE, lambda: ctx.pse_plane_gradient(x, y, f, area, act, eps, i0=i0, i1=i0 + block,
+                                                                  precision=prec)),
+             (L.K_PSE_INTERP_PLANE, lambda: ctx.pse_plane_interpolate(x, y, f, area, act, eps, px, py,
+                                                                      precision=prec)))
+    for kind, call in calls:
+        for g, r in zip(_rows(call()), _all_pairs(ctx, kind, prec, call)):
+            assert rel_err_max(g, r) <= CULL_TOL[prec], kind
+    j = int(np.flatnonzero(act)[77])
+    f[j] = np.inf
+    for kind, call in calls:
+        for g, r in zip(_rows(call()), _all_pairs(ctx, kind, prec, call)):
+            assert np.array_equal(np.isfinite(g), np.isfinite(r)), kind
+
+
+@pytest.mark.parametrize("prec", ["fp64", "fp32"])
+@pytest.mark.parametrize("eps", [0.01, 0.04])
+def test_culled_sphere_sums_over_groups(ctx, prec, eps):
+    """5,120 source tiles (icosahedral level 7), a block of targets or points."""
+    m = mesh.icosahedral_mesh(7)
+    f = np.sin(3 * m.x) * m.y + m.z
+    i0, i1 = 200001, 201000
+    _assert_culled(int(m.active.sum()) * (i1 - i0))
+    p = [np.ascontiguousarray(c[i0:i1]) for c in (m.y, m.z, m.x)]
+    a = (m.area, m.active, eps)
+    for kind, call in (
+            (L.K_PSE_SPHERE8, lambda: ctx.pse_sphere_laplacian(m.x, m.y, m.z, f, *a, i0=i0, i1=i1, precision=prec)),
+            (L.K_PSE_DERIV_SPHERE, lambda: ctx.pse_sphere_gradient(m.x, m.y, m.z, f, *a, i0=i0, i1=i1, precision=prec)),
+            (L.K_PSE_INTERP_SPHERE, lambda: ctx.pse_sphere_interpolate(m.x, m.y, m.z, f, *a, *p, precision=prec))):
+        for g, r in zip(_rows(call()), _all_pairs(ctx, kind, prec, call)):
+            assert rel_err_max(g, r) <= 4 * CULL_TOL[prec], kind
+
+
+@pytest.mark.parametrize("prec", ["fp64", "fp32"])
+@pytest.mark.parametrize("eps_h", [0.7, 2.0, 4.0])
+def test_culled_plane_interpolation(ctx, prec, eps_h):
+    """Interpolation at as many points as there are sources, shuffled, with passive
+    particles; then sources that are not finite."""
+    x, y, area, h = mesh.grid_centres(131, 1.0, jitter=1e-3, seed=3)
+    rng = np.random.default_rng(9)
+    f = np.exp(-4.0 * (x * x + y * y)) + 0.3 * x
+    act = (rng.uniform(size=x.size) < 0.93).astype(np.int32)
+    idx = rng.permutation(x.size)
+    px, py = 0.9 * x[idx] + 1e-3, 0.9 * y[idx]
+    _assert_culled(int(act.sum()) * px.size)
+
+    def call():
+        return ctx.pse_plane_interpolate(x, y, f, area, act, eps_h * h, px, py, precision=prec)
+
+    assert rel_err_max(call(), _all_pairs(ctx, L.K_PSE_INTERP_PLANE, prec, call)[0]) <= CULL_TOL[prec]
+    act[7000] = 1
+    for bad in (np.inf, np.nan):
+        f[7000] = bad
+        assert np.array_equal(np.isfinite(call()), np.isfinite(_all_pairs(ctx, L.K_PSE_INTERP_PLANE, prec, call)[0]))
