@@ -150,6 +150,7 @@ class CallIO {
       for (const double* a : arrays) gather(a, n, nb);
       for (const double* a : points) gather(a, npts, pb);
       list_ = reinterpret_cast<int*>(d + at);
+      sources_ = reinterpret_cast<int*>(h + at);
       ns_ = compact(active, n, reinterpret_cast<int*>(h + at));
       at += lb;
       if (flags) {
@@ -180,6 +181,7 @@ class CallIO {
     host_list_.reset(new (std::nothrow) int[(size_t)std::max(n, 1)]);
     if (!host_list_) return fail(ctx_, LPM_ERR_NOMEM, "no host memory for the active list");
     ns_ = compact(active, n, host_list_.get());
+    sources_ = host_list_.get();
     LPM_HIP(ctx_, ctx_->list.ensure((size_t)std::max(ns_, 1) * 4));
     list_ = ctx_->list.as<int>();
     if (ns_ > 0)
@@ -221,6 +223,33 @@ class CallIO {
   CallIO(const CallIO&) = delete;
   CallIO& operator=(const CallIO&) = delete;
 
+  // Share of the pairs of targets t [t0, t1) and active sources at x, y that lie within
+  // `reach`, as a plane PSE sum wants it (sum_path): from 32 x 64 pairs picked by two
+  // sequences that spread evenly over any order of the particles, under the copies.
+  // 0 where the sum has too few pairs for it to matter.
+  double share_within(double reach, const double* tx, const double* ty, int t0, int t1, const double* x,
+                      const double* y) const {
+    if ((double)(t1 - t0) * ns_ < lpm::kCullMinPairs) return 0.0;
+    auto pick = [](unsigned k, unsigned step, int count) { return (int)(((uint64_t)(k * step) * (unsigned)count) >> 32); };
+    constexpr int T = 32, S = 64;
+    double sx[S], sy[S];
+    for (int k = 0; k < S; ++k) {
+      const int p = sources_[pick(k + 1, 0x6a09e667u, ns_)];
+      sx[k] = x[p];
+      sy[k] = y[p];
+    }
+    int in = 0;
+    for (int k = 0; k < T; ++k) {
+      const int p = t0 + pick(k + 1, 0x9e3779b9u, t1 - t0);
+      const double px = tx[p], py = ty[p];
+      for (int j = 0; j < S; ++j) {
+        const double dx = px - sx[j], dy = py - sy[j];
+        in += dx * dx + dy * dy < reach * reach;
+      }
+    }
+    return (double)in / (T * S);
+  }
+
   const double* arg(int k) const { return arg_[k]; }
   double* res(int k) const { return k < nout_ ? res_[k] : nullptr; }
   const int* list() const { return list_; }
@@ -252,6 +281,7 @@ class CallIO {
   double* res_[4] = {};
   int *list_ = nullptr, *flags_ = nullptr;
   size_t out_at_ = 0;
+  const int* sources_ = nullptr;  // the active list on the host
   std::unique_ptr<int[]> host_list_;
 };
 
@@ -317,6 +347,10 @@ int run_ops_call(lpm_ctx* ctx, const OpsCall& c, Bind bind) {
     pp.tq = c.points.size() > 3 ? in(k_pts + 3) : nullptr;
   }
   bind(pp, in);
+  if (pp.kind == LPM_K_PSE_DERIV_PLANE || pp.kind == LPM_K_PSE_INTERP_PLANE) {
+    const double *const *src = c.inputs.begin(), *const *tgt = at_points ? c.points.begin() : src;
+    pp.reach_share = io.share_within(lpm::kTestedReach * c.eps, tgt[0], tgt[1], t0, t1, src[0], src[1]);
+  }
   if (int rc = lpm::run_pair_sum(ctx, pp)) return rc;
   return io.close(t0, t1, c.outputs);
 }
@@ -585,6 +619,7 @@ int lpm_pse_plane_laplacian(lpm_ctx* ctx, double* lap, const double* x, const do
   pp.src_list = io.list();
   pp.ns = io.ns();
   pp.eps = eps;
+  pp.reach_share = io.share_within(lpm::kTestedReach * eps, x, y, i0, i1, x, y);
   pp.out0 = io.res(0);
   if (int rc = lpm::run_pair_sum(ctx, pp)) return rc;
   return io.close(i0, i1, {lap});

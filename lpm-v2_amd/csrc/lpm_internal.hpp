@@ -150,6 +150,9 @@ struct PairProblem {
   // one for the four sums of a step); else run_pair_sum makes one where it is used.
   const int* tgt_order = nullptr;
   const int* src_order = nullptr;
+  // Plane PSE kinds: share of the pairs within kTestedReach eps, as far as the caller
+  // knows it (see sum_path)
+  double reach_share = 0.0;
   // Source count on the device (set by a device-side compaction): ns is then
   // an upper bound that sizes the launches, and the kernels read the count.
   // Such a sum also records no timing events.
@@ -215,8 +218,12 @@ constexpr double kFarMinPairsSphere = 2e9, kFarMinPairsPlane = 4e9, kFarMinPairs
 // well-separated tiles on the MFMA (far_kernels.hpp), or without the tiles whose
 // terms are zero (cull_kernels.hpp).  The last two want the records in spatial order.
 enum SumPath { kAllPairs = 0, kFarTiles = 1, kCullTiles = 2 };
-// reach: of a PSE kernel on the sphere, in radii
-SumPath sum_path(const lpm_ctx* ctx, int kind, int prec, int nt, int ns, double reach = 0.0);
+// reach_share: of a PSE sum, the share of the pairs within kTestedReach eps
+SumPath sum_path(const lpm_ctx* ctx, int kind, int prec, int nt, int ns, double reach_share = 0.0);
+constexpr double kCullMinPairs = 1.5e8;
+// The tested tiles leave about this reach, in eps, of the 10.2 (FP32) and 27.3 (FP64)
+// at which terms are zero.
+constexpr double kTestedReach = 8.5;
 
 // Spatial order (lpm_order.hip) of targets tx.. [i0, i0 + nt) and of the sources
 // x..[list[0, ns)]: device arrays of particle indices inside `buf`.

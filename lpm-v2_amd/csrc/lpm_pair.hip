@@ -273,11 +273,6 @@ Tuning default_tuning(int kind, int prec) {
   return t;
 }
 
-constexpr double kCullMinPairs = 1.5e8;
-constexpr double kCullMaxReach = 1.6;
-// The tested tiles leave about this reach, in eps, of the 10.2 (FP32) and 27.3 (FP64)
-// at which terms are zero.
-constexpr double kTestedReach = 8.5;
 constexpr int kFarRounds = 8;   // rounds of resident blocks wanted of a far-tile sum
 constexpr int kFarGroups = 8;   // at most so many groups of FAR_FOLD sources per split
 constexpr int kCullWaves = 12;  // waves per SIMD wanted of a culled sum
@@ -528,9 +523,24 @@ static CullFn pick_cull(int kind, int prec, int m, int series) {
 // eps = 2 h: plane 80^2 (4e7 pairs) 0.56-0.68, 110^2 (1.5e8) 1.0, 150^2 (5e8) 1.3 in FP32
 // and 1.6 in FP64, 200^2 2.0-2.4 and 3.2-3.4; sphere level 5 (6e8) 1.5 and 1.85.  Shallow water, far tiles against culled ones: 200^2 (1.6e9) 1.05 at
 // eps = 2 h and 0.91 at 20 h, 301^2 (8e9) 1.27 and 1.0, and 0.99 where nothing is
-// beyond reach.  On the sphere the sum must also reach less than kCullMaxReach radii
-// (chord): 1.0-1.1 at eps = 0.18 and 0.22 (reach 1.6 and 1.85), 0.86-0.97 at 0.37.
-SumPath sum_path(const lpm_ctx* ctx, int kind, int prec, int nt, int ns, double reach) {
+// beyond reach.  A PSE sum must also leave enough pairs out of reach.  Time over all
+// pairs by time culled, at shares in reach of 0.44 / 0.56 / 0.67 / 0.77 / 0.89 on the plane:
+// Laplacian 300^2 1.4 / 1.15 / 1.0 / 0.94 / 0.86 in FP32, 1.7 / 1.4 / 1.25 / 1.06 / 0.94 in
+// FP64, 170^2 1.0 / 0.94 / 0.88 / 0.83 / 0.80 and 1.35 / 1.2 / 1.1 / 1.05 / 0.95, gradient
+// 300^2 in FP32 1.5 / 1.3 / 1.15 / 1.06 / 0.98, and 0.66-0.92 where all pairs are in reach; on
+// the sphere 1.0-1.1 at 0.64 and 0.85, 0.86-0.97 at 1.
+static double cull_max_share(int kind, int prec) {
+  switch (kind) {
+    case LPM_K_SWE_PLANE: return 2.0;  // the velocity takes all pairs either way
+    case LPM_K_PSE_SPHERE8:
+    case LPM_K_PSE_DERIV_SPHERE:
+    case LPM_K_PSE_INTERP_SPHERE: return 0.64;
+    case LPM_K_PSE_DERIV_PLANE: return prec == LPM_PREC_FP32_KAHAN ? 0.75 : 0.8;
+    default: return prec == LPM_PREC_FP32_KAHAN ? 0.6 : 0.8;
+  }
+}
+
+SumPath sum_path(const lpm_ctx* ctx, int kind, int prec, int nt, int ns, double reach_share) {
   const Tuning& ov = ctx->tune[kind][prec == LPM_PREC_FP32_KAHAN ? 1 : 0];
   if (ov.r || ov.kt) return kAllPairs;  // a forced tile shape is one of the all-pairs kernel
   if ((long long)nt + ns > (1 << 30)) return kAllPairs;  // item counts of the sort are ints
@@ -541,7 +551,8 @@ SumPath sum_path(const lpm_ctx* ctx, int kind, int prec, int nt, int ns, double 
   }
   if (kind == LPM_K_SWE_PLANE && prec == LPM_PREC_FP32_KAHAN && !ov.splits && (double)nt * ns >= kFarMinPairsSwe)
     return kFarTiles;
-  return !ov.splits && (double)nt * ns >= kCullMinPairs && reach < kCullMaxReach ? kCullTiles : kAllPairs;
+  return !ov.splits && (double)nt * ns >= kCullMinPairs && reach_share < cull_max_share(kind, prec) ? kCullTiles
+                                                                                                    : kAllPairs;
 }
 
 // Words of a source / target record that must be finite for a tile to be treated
@@ -684,9 +695,9 @@ int run_pair_sum(lpm_ctx* ctx, const PairProblem& pp) {
     tu.kt = fp32 ? 64 : 32;
   }
   // a device-side source count cannot be ordered
-  const SumPath path = pp.ns_dev ? kAllPairs
-                                 : sum_path(ctx, kind, prec, nt, ns,
-                                            sphere_kind(kind) ? kTestedReach * pp.eps / pp.radius : 0.0);
+  const double cap = 0.5 * kTestedReach * pp.eps / pp.radius;  // a cap's share of the sphere: (chord / 2)^2
+  const SumPath path =
+      pp.ns_dev ? kAllPairs : sum_path(ctx, kind, prec, nt, ns, sphere_kind(kind) ? cap * cap : pp.reach_share);
   const bool far = path == kFarTiles, cull = path == kCullTiles;
   const int t_tile = far ? FAR_TILE : 64, s_tile = far ? FAR_TILE : CULL_TILE;
   const int per_wave = path != kAllPairs ? 64 : 64 * tu.r;

@@ -563,3 +563,41 @@ def test_culled_plane_interpolation(ctx, prec, eps_h):
     for bad in (np.inf, np.nan):
         f[7000] = bad
         assert np.array_equal(np.isfinite(call()), np.isfinite(_all_pairs(ctx, L.K_PSE_INTERP_PLANE, prec, call)[0]))
+
+
+# ------------------------------------------------------- wide kernels
+@pytest.mark.parametrize("prec", ["fp64", "fp32"])
+@pytest.mark.parametrize("order", ["grid", "shuffled", "two_far_clusters"])
+def test_wide_plane_kernels_take_all_pairs(ctx, prec, order):
+    """A kernel that reaches nearly all pairs has no tile to pass over: the sum is the
+    all-pairs kernel's, bit for bit.  A narrow one is not."""
+    x, y, area, h = mesh.grid_centres(140, 1.0, jitter=1e-3, seed=3)
+    if order == "shuffled":
+        idx = np.random.default_rng(1).permutation(x.size)
+        x, y, area = x[idx], y[idx], area[idx]
+    elif order == "two_far_clusters":
+        x = np.where(x > 0, x + 1e5, x)
+    f = np.exp(-4.0 * (x * x + y * y)) + y
+    act = np.ones(x.size, np.int32)
+    _assert_culled(x.size**2)
+    r = {L.K_PSE8: 4, L.K_PSE_DERIV_PLANE: 2, L.K_PSE_INTERP_PLANE: 2} if prec == "fp64" else {
+        L.K_PSE8: 2, L.K_PSE_DERIV_PLANE: 2, L.K_PSE_INTERP_PLANE: 2}
+
+    def calls(eps):
+        return ((L.K_PSE8, lambda: ctx.pse_plane_laplacian(x, y, f, area, act, eps, order=8, precision=prec)),
+                (L.K_PSE_DERIV_PLANE, lambda: ctx.pse_plane_gradient(x, y, f, area, act, eps, precision=prec)),
+                (L.K_PSE_INTERP_PLANE, lambda: ctx.pse_plane_interpolate(x, y, f, area, act, eps, 0.97 * x, 0.97 * y,
+                                                                         precision=prec)))
+
+    def forced(kind, call):
+        ctx.set_tuning(kind, prec, r[kind], 256 if prec == "fp32" else 64, 0)
+        try:
+            return _rows(call())
+        finally:
+            ctx.set_tuning(kind, prec, 0, 0, 0)
+
+    for kind, call in calls(0.8):
+        same = all(np.array_equal(g, e) for g, e in zip(_rows(call()), forced(kind, call)))
+        assert same == (order != "two_far_clusters"), kind  # half of the pairs are out of reach there
+    for kind, call in calls(2 * h):
+        assert not all(np.array_equal(g, e) for g, e in zip(_rows(call()), forced(kind, call))), kind
