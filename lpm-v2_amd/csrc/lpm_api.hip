@@ -126,15 +126,20 @@ class CallIO {
  public:
   explicit CallIO(lpm_ctx* ctx) : ctx_(ctx) {}
 
+  // What a call reads of the active mask: the list of active particles, the flags
+  // themselves, or both.
+  enum Mask { kList = 1, kFlags = 2 };
+
   // Inputs: the active mask and `arrays` of n values, then `points` of npts values;
   // room for nout outputs of `rows` values.
-  int open(int n, const int32_t* active, bool flags, std::initializer_list<const double*> arrays, int rows, int nout,
+  int open(int n, const int32_t* active, int mask, std::initializer_list<const double*> arrays, int rows, int nout,
            int npts = 0, std::initializer_list<const double*> points = {}) {
+    const bool list = mask & kList, flags = mask & kFlags;
     rows_ = rows;
     nout_ = nout;
     const size_t nb = up((size_t)std::max(n, 1) * 8), pb = up((size_t)std::max(npts, 1) * 8);
     const size_t lb = up((size_t)std::max(n, 1) * 4);
-    const size_t in_bytes = arrays.size() * nb + points.size() * pb + lb + (flags ? lb : 0);
+    const size_t in_bytes = arrays.size() * nb + points.size() * pb + (list ? lb : 0) + (flags ? lb : 0);
     const size_t out_bytes = nout * up((size_t)std::max(rows, 1) * 8);
     staged_ = in_bytes + out_bytes <= kStageBytes;
     if (staged_) {
@@ -149,10 +154,12 @@ class CallIO {
       };
       for (const double* a : arrays) gather(a, n, nb);
       for (const double* a : points) gather(a, npts, pb);
-      list_ = reinterpret_cast<int*>(d + at);
-      sources_ = reinterpret_cast<int*>(h + at);
-      ns_ = compact(active, n, reinterpret_cast<int*>(h + at));
-      at += lb;
+      if (list) {
+        list_ = reinterpret_cast<int*>(d + at);
+        sources_ = reinterpret_cast<int*>(h + at);
+        ns_ = compact(active, n, reinterpret_cast<int*>(h + at));
+        at += lb;
+      }
       if (flags) {
         flags_ = reinterpret_cast<int*>(d + at);
         if (n > 0) memcpy(h + at, active, (size_t)n * 4);
@@ -177,15 +184,17 @@ class CallIO {
       if (int rc = copy(a, n)) return rc;
     for (const double* a : points)
       if (int rc = copy(a, npts)) return rc;
-    // built under the copies above, in memory that lasts until the call ends
-    host_list_.reset(new (std::nothrow) int[(size_t)std::max(n, 1)]);
-    if (!host_list_) return fail(ctx_, LPM_ERR_NOMEM, "no host memory for the active list");
-    ns_ = compact(active, n, host_list_.get());
-    sources_ = host_list_.get();
-    LPM_HIP(ctx_, ctx_->list.ensure((size_t)std::max(ns_, 1) * 4));
-    list_ = ctx_->list.as<int>();
-    if (ns_ > 0)
-      LPM_HIP(ctx_, hipMemcpyAsync(list_, host_list_.get(), (size_t)ns_ * 4, hipMemcpyHostToDevice, ctx_->stream));
+    if (list) {
+      // built under the copies above, in memory that lasts until the call ends
+      host_list_.reset(new (std::nothrow) int[(size_t)std::max(n, 1)]);
+      if (!host_list_) return fail(ctx_, LPM_ERR_NOMEM, "no host memory for the active list");
+      ns_ = compact(active, n, host_list_.get());
+      sources_ = host_list_.get();
+      LPM_HIP(ctx_, ctx_->list.ensure((size_t)std::max(ns_, 1) * 4));
+      list_ = ctx_->list.as<int>();
+      if (ns_ > 0)
+        LPM_HIP(ctx_, hipMemcpyAsync(list_, host_list_.get(), (size_t)ns_ * 4, hipMemcpyHostToDevice, ctx_->stream));
+    }
     if (flags) {
       LPM_HIP(ctx_, ctx_->flags.ensure((size_t)std::max(n, 1) * 4));
       flags_ = ctx_->flags.as<int>();
@@ -322,7 +331,7 @@ int run_ops_call(lpm_ctx* ctx, const OpsCall& c, Bind bind) {
   const int t0 = at_points ? 0 : c.i0, t1 = at_points ? c.npts : c.i1;
   if (t1 == t0) return LPM_OK;
   CallIO io(ctx);
-  if (int rc = io.open(c.n, c.active, false, c.inputs, at_points ? c.npts : c.n, (int)c.outputs.size(),
+  if (int rc = io.open(c.n, c.active, CallIO::kList, c.inputs, at_points ? c.npts : c.n, (int)c.outputs.size(),
                        at_points ? c.npts : 0, c.points))
     return rc;
   const int k_pts = (int)c.inputs.size();
@@ -459,7 +468,7 @@ int lpm_bve_sphere_velocity(lpm_ctx* ctx, double* u, double* v, double* w, const
   LPM_HIP(ctx, hipSetDevice(ctx->device));
   if (i1 == i0) return LPM_OK;
   CallIO io(ctx);
-  if (int rc = io.open(n, active, false, {x, y, z, relvort, area}, n, 3)) return rc;
+  if (int rc = io.open(n, active, CallIO::kList, {x, y, z, relvort, area}, n, 3)) return rc;
   lpm::PairProblem pp;
   pp.kind = LPM_K_SPHERE_BS;
   pp.precision = precision;
@@ -571,7 +580,7 @@ int lpm_plane_velocity(lpm_ctx* ctx, double* u, double* v, const double* x, cons
   LPM_HIP(ctx, hipSetDevice(ctx->device));
   if (i1 == i0) return LPM_OK;
   CallIO io(ctx);
-  if (int rc = io.open(n, active, false, {x, y, vort, area}, n, 2)) return rc;
+  if (int rc = io.open(n, active, CallIO::kList, {x, y, vort, area}, n, 2)) return rc;
   lpm::PairProblem pp;
   pp.kind = LPM_K_PLANE_BS;
   pp.precision = precision;
@@ -605,7 +614,7 @@ int lpm_pse_plane_laplacian(lpm_ctx* ctx, double* lap, const double* x, const do
   LPM_HIP(ctx, hipSetDevice(ctx->device));
   if (i1 == i0) return LPM_OK;
   CallIO io(ctx);
-  if (int rc = io.open(n, active, false, {x, y, f, area}, n, 1)) return rc;
+  if (int rc = io.open(n, active, CallIO::kList, {x, y, f, area}, n, 1)) return rc;
   lpm::PairProblem pp;
   pp.kind = order == 8 ? LPM_K_PSE8 : LPM_K_PSE2;
   pp.precision = precision;
@@ -639,7 +648,7 @@ int lpm_pse_sphere_laplacian(lpm_ctx* ctx, double* lap, const double* x, const d
   LPM_HIP(ctx, hipSetDevice(ctx->device));
   if (i1 == i0) return LPM_OK;
   CallIO io(ctx);
-  if (int rc = io.open(n, active, false, {x, y, z, f, area}, n, 1)) return rc;
+  if (int rc = io.open(n, active, CallIO::kList, {x, y, z, f, area}, n, 1)) return rc;
   lpm::PairProblem pp;
   pp.kind = LPM_K_PSE_SPHERE8;
   pp.precision = precision;
@@ -817,7 +826,7 @@ int lpm_bve_sphere_stream(lpm_ctx* ctx, double* psi_rel, double* psi_abs, const 
   LPM_HIP(ctx, hipSetDevice(ctx->device));
   if (i1 == i0) return LPM_OK;
   CallIO io(ctx);
-  if (int rc = io.open(n, active, true, {x, y, z, relvort, absvort, area}, n, 2)) return rc;
+  if (int rc = io.open(n, active, CallIO::kList | CallIO::kFlags, {x, y, z, relvort, absvort, area}, n, 2)) return rc;
   lpm::PairProblem pp;
   pp.kind = LPM_K_SPHERE_GREEN;
   pp.precision = precision;
@@ -852,7 +861,7 @@ int lpm_plane_stream(lpm_ctx* ctx, double* psi, const double* x, const double* y
   LPM_HIP(ctx, hipSetDevice(ctx->device));
   if (i1 == i0) return LPM_OK;
   CallIO io(ctx);
-  if (int rc = io.open(n, active, false, {x, y, vort, area}, n, 1)) return rc;
+  if (int rc = io.open(n, active, CallIO::kList, {x, y, vort, area}, n, 1)) return rc;
   lpm::PairProblem pp;
   pp.kind = LPM_K_PLANE_GREEN;
   pp.precision = precision;
@@ -900,7 +909,7 @@ int lpm_diagnostics(lpm_ctx* ctx, const double* u, const double* v, const double
     return fail(ctx, LPM_ERR_ARG, "lpm_diagnostics: null argument");
   LPM_HIP(ctx, hipSetDevice(ctx->device));
   CallIO io(ctx);
-  if (int rc = io.open(n, active, true, {u, v, w, vort, area}, 0, 0)) return rc;
+  if (int rc = io.open(n, active, CallIO::kFlags, {u, v, w, vort, area}, 0, 0)) return rc;
   double out[3];
   if (int rc = lpm::run_diagnostics(ctx, n, io.arg(0), io.arg(1), io.arg(2), io.arg(3), io.arg(4), io.flags(), out))
     return rc;
