@@ -9,9 +9,10 @@
 //
 // The sort is a stable least-significant-digit radix sort, 8 bits a pass: per-block
 // digit counts, a scan per digit, stable scatter.  Targets and sources go through the same
-// launches (two segments), keys have 16-24 bits, so ordering both takes 7-11 short
-// launches.  It is deterministic, allocates nothing and holds no memset, so it may
-// be captured.  rocPRIM's sort takes a merge-sort path of
+// launches (two segments), three a pass beside the keys' one and, on the plane, the
+// bounding box's: keys have 8-24 bits on the plane, 11-27 on the sphere and up to 32 in
+// batches, 5-11 and 7-13 short launches for both.  It is deterministic, allocates nothing
+// and holds no memset, so it may be captured.  rocPRIM's sort takes a merge-sort path of
 // about 24 launches (130 us) at these sizes.
 #include "lpm_internal.hpp"
 

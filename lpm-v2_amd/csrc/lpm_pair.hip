@@ -521,9 +521,9 @@ static CullFn pick_cull(int kind, int prec, int m, int series) {
 // far tiles, sphere velocity 0.95 of the all-pairs rate at 1.2e9 pairs, 1.01 at 2.5e9,
 // 1.23 at 1e10; plane velocity 0.92 at 1.6e9, 1.07 at 4.3e9.  Culled PSE sums at
 // eps = 2 h: plane 80^2 (4e7 pairs) 0.56-0.68, 110^2 (1.5e8) 1.0, 150^2 (5e8) 1.3 in FP32
-// and 1.6 in FP64, 200^2 2.0-2.4 and 3.2-3.4; sphere level 5 (6e8) 1.5 and 1.85.  Shallow water, far tiles against culled ones: 200^2 (1.6e9) 1.05 at
-// eps = 2 h and 0.91 at 20 h, 301^2 (8e9) 1.27 and 1.0, and 0.99 where nothing is
-// beyond reach.  A PSE sum must also leave enough pairs out of reach.  Time over all
+// and 1.6 in FP64, 200^2 2.0-2.4 and 3.2-3.4; sphere level 5 (6e8) 1.5 and 1.85.  Shallow
+// water, far tiles against culled ones: 200^2 (1.6e9) 1.05 at eps = 2 h and 0.91 at 20 h,
+// 301^2 (8e9) 1.27 and 1.0, and 0.99 where nothing is beyond reach.  A PSE sum must also leave enough pairs out of reach.  Time over all
 // pairs by time culled, at shares in reach of 0.44 / 0.56 / 0.67 / 0.77 / 0.89 on the plane:
 // Laplacian 300^2 1.4 / 1.15 / 1.0 / 0.94 / 0.86 in FP32, 1.7 / 1.4 / 1.25 / 1.06 / 0.94 in
 // FP64, 170^2 1.0 / 0.94 / 0.88 / 0.83 / 0.80 and 1.35 / 1.2 / 1.1 / 1.05 / 0.95, gradient
